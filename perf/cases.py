@@ -1,0 +1,469 @@
+"""Timed cases: the multiwavelet Green's-function work an SCF program asks of this package.
+
+Every case goes through the package's public calls (apply, apply_batch,
+build_operators, multiply, add, ApplyPlan) on Gaussian-sum functions in the
+[-20, 20]^3 world of the benchmark configurations, with the orders,
+precisions and exponents of those configurations and of the tests.
+
+    apply          one Coulomb (Poisson, relative precision) or Helmholtz
+                   (absolute precision) apply, in the context's FP64, mixed or
+                   split16 arithmetic; on device-resident trees (the SCF loop
+                   keeps its functions there) or on host trees (the default)
+    helmholtz_scf  one HelmholtzVector step: operators for the iteration's
+                   orbital energies, then all orbitals in one batch
+    exchange       the Poisson applies of all orbital pairs in one batch, each
+                   with the orbitals as precision trees
+    exchange_kij   calcExchange_kij and its sum: multiply, apply, two
+                   multiplies, linear combination, in-place add, crop
+    product        one tree product (a pair density)
+    sum            a linear combination on the union grid
+    frozen         one execution of a plan on a kept grid, raw blocks read back
+
+Results are read whole: of a resident tree through its device pack, into a
+torch buffer on the GPU, of a host tree through nodes().
+"""
+import math
+
+import numpy as np
+import torch
+
+import mrchem_amd as mw
+from mrchem_amd import workloads
+
+_WORLD = workloads.WORLD
+_MAX_DEPTH = 14
+_contexts = {}
+
+
+def _context(mode):
+    """The program's context for one arithmetic, made once (one stream and its tables)."""
+    if mode not in _contexts:
+        _contexts[mode] = mw.Context(0)
+        _contexts[mode].set_precision(mode)
+    return _contexts[mode]
+
+
+def _case(name, kind, order, prec, n_gauss, exp_lo, exp_hi, box, **more):
+    c = dict(name=name, kind=kind, order=order, prec=prec, n_gauss=n_gauss, exp_lo=exp_lo, exp_hi=exp_hi, box=box,
+             mode="fp64", molecule=1000 + order)
+    c.update(more)
+    return c
+
+
+def listed():
+    return [
+        # the smallest call: a loose-precision potential of one compact
+        # charge, a few refinement levels of a few hundred nodes
+        _case("coulomb_k4_small", "apply", 4, 1e-3, 1, 2.0, 10.0, 1.0, kernel="poisson", resident=True),
+        # the single-Gaussian Coulomb potential at order 7
+        _case("coulomb_k7", "apply", 7, 1e-5, 1, 10.0, 10.0, 1.0, kernel="poisson", resident=True),
+        # the default call: host trees in and out, and the potential at points
+        _case("coulomb_k8_host", "apply", 8, 1e-5, 4, 1.0, 50.0, 3.0, kernel="poisson", resident=False),
+        # one orbital's Helmholtz apply at order 9 (the benchmark's workload),
+        # in FP64 and in the low-precision mode
+        _case("helmholtz_k9", "apply", 9, 1e-6, 10, 0.5, 50.0, 3.0, kernel="helmholtz", mu=1.2, resident=True),
+        _case("helmholtz_k9_split16", "apply", 9, 1e-6, 10, 0.5, 50.0, 3.0, kernel="helmholtz", mu=1.2,
+              resident=True, mode="split16"),
+        # a molecule's Coulomb potential at an even order, mixed arithmetic
+        _case("coulomb_k10_mixed", "apply", 10, 1e-6, 6, 1.0, 50.0, 3.0, kernel="poisson", resident=True,
+              mode="mixed"),
+        # the largest: one SCF iteration's Helmholtz step at order 11
+        _case("helmholtz_scf_k11", "helmholtz_scf", 11, 1e-7, 8, 0.3, 30.0, 6.0, n=6),
+        # the pair potentials of four orbitals (10 pairs)
+        _case("exchange_k7", "exchange", 7, 1e-5, 6, 0.3, 30.0, 4.0, n=4),
+        # one exchange contribution, from orbitals to the cropped sum
+        _case("exchange_kij_k7", "exchange_kij", 7, 1e-4, 4, 0.5, 20.0, 2.0),
+        # one pair density
+        _case("product_k7", "product", 7, 1e-5, 6, 0.3, 30.0, 4.0),
+        # a sum of eight functions
+        _case("sum_k7", "sum", 7, 1e-5, 6, 0.3, 30.0, 4.0, n=8),
+        # a kept grid: the calculator alone, and its raw blocks
+        _case("frozen_k9", "frozen", 9, 1e-6, 8, 1.0, 100.0, 3.0, kernel="poisson"),
+    ]
+
+
+def draw(rng):
+    kind = rng.choice(["apply", "apply", "apply", "helmholtz_scf", "exchange", "exchange_kij", "product", "sum",
+                       "frozen"])
+    # precision, and the order that goes with it (about 1.5 digits an order)
+    digits = rng.uniform(3.0, 5.5 if kind in ("exchange", "exchange_kij") else 6.8)
+    order = min(11, max(3, int(round(1.6 * digits)) - 1 + rng.choice([-1, 0, 0, 1])))
+    lo = math.exp(rng.uniform(math.log(0.3), math.log(3.0)))
+    c = dict(kind=kind, order=order, prec=10.0 ** -digits, n_gauss=rng.randint(1, 8), exp_lo=lo,
+             exp_hi=lo * math.exp(rng.uniform(math.log(2.0), math.log(30.0))), box=rng.uniform(1.0, 4.0), mode="fp64",
+             molecule=rng.randrange(1 << 20))
+    if kind in ("apply", "frozen"):
+        c["kernel"] = rng.choice(["poisson", "helmholtz"])
+        if c["kernel"] == "helmholtz":
+            c["mu"] = rng.uniform(0.5, 2.5)
+    if kind == "apply":
+        c["resident"] = rng.random() < 0.75
+        c["mode"] = rng.choice(["fp64", "fp64", "mixed", "split16"])
+    if kind == "helmholtz_scf":
+        c["n"] = rng.randint(1, 4)
+    if kind == "exchange":
+        c["n"] = rng.randint(2, 3)
+    if kind == "sum":
+        c["n"] = rng.randint(2, 8)
+    return c
+
+
+def _turn(seed):
+    """One of the cube's 48 symmetries (a permutation of the axes and their signs)."""
+    perm = [(0, 1, 2), (1, 2, 0), (2, 0, 1), (0, 2, 1), (2, 1, 0), (1, 0, 2)][seed // 8 % 6]
+    return list(perm), np.array([1.0 - 2.0 * ((seed >> d) & 1) for d in range(3)])
+
+
+def _functions(case, seed, count):
+    """count Gaussian sums (coefficients, exponents, centres): normal coefficients
+    (a density: positive ones), exponents uniform in their logarithm.  The
+    case fixes the molecule and so the sizes of its grids; the seed its
+    orientation in the world and the functions' signs."""
+    rng = np.random.default_rng(case["molecule"])
+    perm, sign = _turn(seed)
+    signs = np.random.default_rng(seed).choice([-1.0, 1.0], count)
+    n = case["n_gauss"]
+    out = []
+    for i in range(count):
+        c = rng.standard_normal(n)
+        if case.get("kernel") == "poisson":
+            c = np.abs(c) + 0.1
+        a = np.exp(rng.uniform(math.log(case["exp_lo"]), math.log(case["exp_hi"]), n))
+        out.append((c * signs[i], a, rng.uniform(-case["box"], case["box"], (n, 3))[:, perm] * sign))
+    return out
+
+
+def _points(case, seed):
+    return np.random.default_rng(seed + 7919).uniform(-8.0, 8.0, (64, 3))
+
+
+def _mu(case):
+    return np.random.default_rng(case["molecule"] + 1).uniform(0.5, 2.5, case["n"])
+
+
+def prepare(case, seed):
+    kind, prec = case["kind"], case["prec"]
+    ctx = _context(case["mode"])
+    mra = mw.MultiResolutionAnalysis(order=case["order"], max_depth=_MAX_DEPTH, **_WORLD)
+    s = dict(case=case, ctx=ctx, mra=mra)
+
+    def project(f, p, resident=True):
+        t = mw.FunctionTree(mra).project_gaussians(p, *f)
+        return t.set_resident(ctx) if resident else t
+
+    def out(resident=True):
+        t = mw.FunctionTree(mra)
+        return t.set_resident(ctx) if resident else t
+
+    if kind in ("apply", "frozen"):
+        f = _functions(case, seed, 1)[0]
+        s["resident"] = kind == "frozen" or case["resident"]
+        s["inp"] = project(f, prec, s["resident"])
+        mu = case.get("mu", 0.0)
+        if s["resident"]:
+            s["op"] = mw.build_operators(mra, [mu], prec, ctx=ctx)[0]
+        else:
+            s["op"] = mw.HelmholtzOperator(mra, mu, prec) if mu else mw.PoissonOperator(mra, prec)
+        # MRChem: the Coulomb potential to relative, the Helmholtz apply to absolute precision
+        s["abs"] = case["kernel"] == "helmholtz"
+        s["prec"] = prec if s["abs"] else prec / s["inp"].norm()
+        if kind == "apply":
+            s["out"] = out(s["resident"])
+            s["points"] = _points(case, seed)
+        else:
+            s["grid"] = out(False)
+            mw.apply(s["prec"], s["grid"], s["op"], s["inp"], abs_prec=s["abs"], ctx=ctx)
+            s["plan"] = mw.ApplyPlan(s["grid"], s["op"], s["inp"], s["grid"].thresholds(), mode=case["mode"], ctx=ctx)
+    elif kind == "helmholtz_scf":
+        s["inps"] = [project(f, prec) for f in _functions(case, seed, case["n"])]
+        s["outs"] = [out() for _ in s["inps"]]
+        s["mus"] = _mu(case)
+    elif kind == "exchange":
+        orbs = _functions(case, seed, case["n"])
+        pairs = [(i, j) for i in range(case["n"]) for j in range(i, case["n"])]
+        s["phi"] = [project(f, prec) for f in orbs]
+        s["rho"] = [project(workloads.pair_density(orbs[i], orbs[j]), prec) for i, j in pairs]
+        s["pairs"] = pairs
+        s["outs"] = [out() for _ in pairs]
+        s["op"] = mw.build_operators(mra, [0.0], prec, ctx=ctx)[0]
+    elif kind == "exchange_kij":
+        s["phi"] = [project(f, prec / 10) for f in _functions(case, seed, 3)]
+        s["op"] = mw.build_operators(mra, [0.0], prec / 10, ctx=ctx)[0]
+        s["trees"] = [out() for _ in range(5)]
+    elif kind == "product":
+        s["a"], s["b"] = [project(f, prec) for f in _functions(case, seed, 2)]
+        s["out"] = out()
+    else:
+        fs = _functions(case, seed, case["n"])
+        s["inps"] = [project(f, prec) for f in fs]
+        s["coefs"] = [(-1.0) ** i / (1.0 + i) for i in range(len(fs))]
+        s["out"] = out()
+    return s
+
+
+def _whole(tree, ctx):
+    """A resident tree's grid and blocks, packed on the device into a torch buffer."""
+    n = tree.size()
+    size = tree.pack_size()
+    buf = torch.empty(size // 8, dtype=torch.float64, device="cuda")
+    tree.pack_device(buf.data_ptr(), size, ctx=ctx)
+    at = 9 + (n + 1) // 2  # 72-byte header, int32 depths padded to 8 bytes, int64 translations, blocks
+    return {"depth": buf[9:at].view(torch.int32)[:n], "l": buf[at:at + 3 * n].view(torch.int64).view(n, 3),
+            "blocks": buf[at + 3 * n:].view(n, tree.mra.block)}
+
+
+def run(s):
+    case, ctx = s["case"], s["ctx"]
+    kind, prec = case["kind"], case["prec"]
+    if kind == "apply":
+        mw.apply(s["prec"], s["out"], s["op"], s["inp"], abs_prec=s["abs"], ctx=ctx)
+        if s["resident"]:
+            return _whole(s["out"], ctx)
+        depth, l, blocks = s["out"].nodes()
+        return {"depth": depth, "l": l, "blocks": blocks, "values": s["out"].evaluate(s["points"])}
+    if kind == "helmholtz_scf":
+        ops = mw.build_operators(s["mra"], s["mus"], prec, ctx=ctx)
+        mw.apply_batch([dict(prec=prec, out=o, oper=h, inp=f, abs_prec=True)
+                        for o, h, f in zip(s["outs"], ops, s["inps"])], ctx=ctx)
+        return [_whole(o, ctx) for o in s["outs"]]
+    if kind == "exchange":
+        mw.apply_batch([dict(prec=prec, out=o, oper=s["op"], inp=r, abs_prec=True,
+                             prec_trees=[s["phi"][i], s["phi"][j]])
+                        for o, r, (i, j) in zip(s["outs"], s["rho"], s["pairs"])], ctx=ctx)
+        return [_whole(o, ctx) for o in s["outs"]]
+    if kind == "exchange_kij":
+        pk, pi, pj = s["phi"]
+        rho, V, xk, xj, ex = s["trees"]
+        mw.multiply(prec / 10, rho, pi, pj, abs_prec=True, ctx=ctx)
+        mw.apply(prec * 10, V, s["op"], rho, abs_prec=True, prec_trees=[pk, pj, pi], ctx=ctx)
+        mw.multiply(prec / 100, xk, pk, V, abs_prec=True, ctx=ctx)
+        mw.multiply(prec / 100, xj, pj, V, abs_prec=True, ctx=ctx)
+        mw.add(prec, ex, [1.0, 0.5], [xk, xj], abs_prec=True, ctx=ctx)
+        ex.add(1.0, xk, ctx=ctx)
+        ex.crop(prec, 1.0, True)
+        return [_whole(t, ctx) for t in s["trees"]]
+    if kind == "product":
+        mw.multiply(prec, s["out"], s["a"], s["b"], abs_prec=True, ctx=ctx)
+        return _whole(s["out"], ctx)
+    if kind == "sum":
+        mw.add(-1.0, s["out"], s["coefs"], s["inps"], ctx=ctx)
+        return _whole(s["out"], ctx)
+    stats = s["plan"].execute()
+    return {"blocks": s["plan"].download_ns(), "term_apps": stats["term_apps"]}
+
+
+def work(case):
+    """Input and output blocks once each; 6 N^4 operations for each term-application
+    that passes the screening rule, 4 N multiply-adds a value and direction for the
+    transforms of products and sums (counted on one pass)."""
+    s = prepare(case, 1)
+    n, n3 = case["order"] + 1, (case["order"] + 1) ** 3
+    blk = 8 * n3
+    size = lambda trees: sum(t.size() for t in trees)
+    r = run(s)
+    kind = case["kind"]
+    if kind == "frozen":
+        return {"bytes": 8.0 * blk * (s["inp"].size() + len(r["blocks"])), "flops": 6.0 * n ** 4 * r["term_apps"]}
+    step = 3 * 2.0 * 2 * n * blk  # one two-scale transform of a node's block, three directions
+    if kind == "apply":
+        trees, branch = [s["inp"], s["out"]], size([s["out"]]) / 8
+    elif kind == "helmholtz_scf":
+        trees, branch = s["inps"] + s["outs"], size(s["outs"]) / 8
+    elif kind == "exchange":
+        trees, branch = s["phi"] + s["rho"] + s["outs"], size(s["outs"]) / 8
+    elif kind == "exchange_kij":
+        trees, branch = s["phi"] + s["trees"], size([s["trees"][1]]) / 8 + 3 * size(s["trees"][::2]) * 7 / 8
+    elif kind == "product":
+        trees, branch = [s["a"], s["b"], s["out"]], 3 * size([s["out"]]) * 7 / 8
+        return {"bytes": 8.0 * blk * size(trees), "flops": step * branch}
+    else:
+        trees = s["inps"] + [s["out"]]
+        return {"bytes": 8.0 * blk * size(trees), "flops": 2.0 * blk * case["n"] * s["out"].size()}
+    apps = s["ctx"].last_stats()["term_apps"]
+    return {"bytes": 8.0 * blk * size(trees), "flops": 6.0 * n ** 4 * apps + step * branch}
+
+
+# ---- values in 64 bits, numpy alone ----
+#
+# The adaptive applies have none: their blocks are defined by the screening of
+# a fitted kernel, and differ from the continuous convolution by the requested
+# precision.  Where a program evaluates the potential at points, the closed
+# form of the Gaussians' potential is given for those.
+
+
+def _erf(x):
+    return np.vectorize(math.erf)(x)
+
+
+def _filter(n):
+    """Two-scale filter [H0 H1; G0 G1] of the interpolating basis of n points: the
+    scaling part by Gauss-Legendre quadrature, the wavelets the orthonormal
+    complement built from the left half's functions in turn."""
+    x, w = np.polynomial.legendre.leggauss(n)
+    x, w = (x + 1) / 2, w / 2
+
+    def phi(t):  # [i][q]
+        leg = lambda u: np.array([math.sqrt(2 * p + 1) * np.polynomial.legendre.Legendre.basis(p)(2 * u - 1)
+                                  for p in range(n)])
+        return (np.sqrt(w)[:, None] * leg(x).T) @ leg(t)
+
+    q, v = np.polynomial.legendre.leggauss(2 * n)
+    q, v = (q + 1) / 2, v / 2
+    F = np.zeros((2 * n, 2 * n))
+    F[:n, :n] = (phi(q / 2) * v) @ phi(q).T / math.sqrt(2)
+    F[:n, n:] = (phi((q + 1) / 2) * v) @ phi(q).T / math.sqrt(2)
+    for g in range(n):
+        u = np.zeros(2 * n)
+        u[g] = 1.0
+        for _ in range(3):
+            u -= F[:n + g].T @ (F[:n + g] @ u)
+        F[n + g] = u / np.linalg.norm(u)
+    return F
+
+
+def _transform(blocks, M, n):
+    """[nodes][8][z][y][x] -> the three directions of M on (t, t | bit) pairs."""
+    b = blocks.reshape(-1, 2, 2, 2, n, n, n)  # [node][tz][ty][tx][z][y][x]
+    Mr = M.reshape(2, n, 2, n)
+    b = np.einsum("aibj,Nzybqrj->Nzyaqri", Mr, b, optimize=True)
+    b = np.einsum("aibj,Nzbxqjs->Nzaxqis", Mr, b, optimize=True)
+    b = np.einsum("aibj,Nbyxjrs->Nayxirs", Mr, b, optimize=True)
+    return b.reshape(-1, 8, n, n, n)
+
+
+class _Ref:
+    """Trees in numpy: keys in the order in which the package's trees grow (level
+    by level from the roots, 8 children at a time), one block per key."""
+
+    def __init__(self, case):
+        self.n = case["order"] + 1
+        self.F = _filter(self.n)
+        x, w = np.polynomial.legendre.leggauss(self.n)
+        self.x, self.w = (x + 1) / 2, w / 2
+        W = _WORLD
+        c, b = W["corner"], W["boxes"]
+        self.roots = [(0, c[0] + i, c[1] + j, c[2] + k) for k in range(b[2]) for j in range(b[1]) for i in range(b[0])]
+
+    def side(self, depth):
+        return _WORLD["scaling_factor"] * 2.0 ** -(_WORLD["min_scale"] + depth)
+
+    def kids(self, k):
+        return [(k[0] + 1, 2 * k[1] + (t & 1), 2 * k[2] + ((t >> 1) & 1), 2 * k[3] + (t >> 2)) for t in range(8)]
+
+    def _integrals(self, a, r, depth, ls):
+        """int phi_i(x) g(x) dx over the boxes ls of the depth, g the normalised 1D Gaussian."""
+        h, n = self.side(depth), self.n
+        pieces = max(1, int(math.ceil(h * math.sqrt(a))))
+        q, v = np.polynomial.legendre.leggauss(n + 16)
+        t = ((np.arange(pieces)[:, None] + (q + 1) / 2) / pieces).ravel()
+        g = np.sqrt(a / math.pi) * np.exp(-a * ((ls[:, None] + t) * h - r) ** 2) * np.tile(v / 2 / pieces, pieces)
+        norm = np.sqrt(2 * np.arange(n) + 1)
+        P = np.polynomial.legendre.legvander(2 * t - 1, n - 1) * norm
+        PX = np.polynomial.legendre.legvander(2 * self.x - 1, n - 1) * norm
+        return math.sqrt(h) * np.sqrt(self.w) * ((g @ P) @ PX.T)
+
+    def project(self, f, prec, max_depth=_MAX_DEPTH):
+        c, a, R = f
+        n = self.n
+        p = a[:, None] + a[None]
+        d2 = np.sum((R[:, None] - R[None]) ** 2, axis=2)
+        q = a[:, None] * a[None] / p
+        tnorm = math.sqrt(max(0.0, float(np.sum(c[:, None] * c[None] * (q / math.pi) ** 1.5 * np.exp(-q * d2)))))
+        keys, blocks, work = [], [], list(self.roots)
+        while work:
+            depth = work[0][0] + 1
+            kids = np.array([self.kids(k) for k in work])[:, :, 1:].reshape(-1, 3)
+            s = np.zeros((len(kids), n, n, n))
+            for g in range(len(c)):
+                I = []
+                for d in range(3):
+                    ls, at = np.unique(kids[:, d], return_inverse=True)
+                    I.append(self._integrals(a[g], R[g, d], depth, ls)[at])
+                s += c[g] * I[2][:, :, None, None] * I[1][:, None, :, None] * I[0][:, None, None, :]
+            b = _transform(s.reshape(-1, 8, n, n, n), self.F, n)
+            keys += work
+            blocks.append(b)
+            wn = np.sqrt(np.sum(b[:, 1:] ** 2, axis=(1, 2, 3, 4)))
+            work = [kid for k, x in zip(work, wn) if depth - 1 < max_depth and x > self.cut(k[0], prec, tnorm)
+                    for kid in self.kids(k)]
+        return {k: b for k, b in zip(keys, np.concatenate(blocks))}
+
+    def cut(self, depth, prec, tnorm):
+        return max(2 * 2.220446049250313e-16, prec * tnorm * 2.0 ** (-0.5 * (_WORLD["min_scale"] + depth + 1)))
+
+    def union(self, trees):
+        have = dict.fromkeys(self.roots)
+        for t in trees:
+            for k in t:
+                if k not in have:
+                    for kid in self.kids((k[0] - 1, k[1] >> 1, k[2] >> 1, k[3] >> 1)):
+                        have.setdefault(kid)
+        return list(have)
+
+    def block_at(self, t, k, made):
+        """t's block at k; below its finest node the scaling part alone."""
+        if k in t:
+            return t[k]
+        if k not in made:
+            up = (k[0] - 1, k[1] >> 1, k[2] >> 1, k[3] >> 1)
+            b = np.zeros((8,) + (self.n,) * 3)
+            child = (k[1] & 1) | ((k[2] & 1) << 1) | ((k[3] & 1) << 2)
+            b[0] = _transform(self.block_at(t, up, made)[None], self.F.T, self.n)[0, child]
+            made[k] = b
+        return made[k]
+
+    def product(self, ta, tb, prec):
+        n = self.n
+        pw = 1.0 / np.sqrt(np.einsum("k,j,i->kji", self.w, self.w, self.w))
+        keys = self.union([ta, tb])
+        kids_of = lambda k: self.kids(k)[0]
+        have = set(keys)
+        work = [k for k in keys if kids_of(k) not in have]
+        blocks, ma, mb = {}, {}, {}
+        while work:
+            A = _transform(np.stack([self.block_at(ta, k, ma) for k in work]), self.F.T, n)
+            B = _transform(np.stack([self.block_at(tb, k, mb) for k in work]), self.F.T, n)
+            h = np.array([self.side(k[0] + 1) ** -1.5 for k in work])
+            P = _transform(A * B * h[:, None, None, None, None] * pw, self.F, n)
+            blocks.update(zip(work, P))
+            wn = np.sqrt(np.sum(P[:, 1:] ** 2, axis=(1, 2, 3, 4)))
+            work = [kid for k, x in zip(work, wn) if k[0] < _MAX_DEPTH and x > self.cut(k[0], prec, 1.0)
+                    for kid in self.kids(k)]
+            keys += work
+        for k in sorted((k for k in keys if k not in blocks or kids_of(k) in blocks), key=lambda k: -k[0]):
+            if kids_of(k) in blocks:
+                blocks[k] = _transform(np.stack([blocks[x][0] for x in self.kids(k)])[None], self.F, n)[0]
+        return keys, np.stack([blocks[k].ravel() for k in keys])
+
+    def sum(self, coefs, trees):
+        keys = self.union(trees)
+        made = [{} for _ in trees]
+        return keys, np.stack([sum(c * self.block_at(t, k, m) for c, t, m in zip(coefs, trees, made)).ravel()
+                               for k in keys])
+
+
+def _potential(case, f, points):
+    """sum_i c_i of the normalised Gaussians' Coulomb potentials erf(sqrt(a) r) / r."""
+    c, a, R = f
+    r = np.sqrt(np.sum((points[:, None] - R[None]) ** 2, axis=2))
+    return np.sum(c * _erf(np.sqrt(a) * r) / r, axis=1)
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "apply" and not case["resident"] and case["kernel"] == "poisson":
+        return {"depth": None, "l": None, "blocks": None,
+                "values": _potential(case, _functions(case, seed, 1)[0], _points(case, seed))}
+    if kind not in ("product", "sum"):
+        return None
+    fs = _functions(case, seed, 2 if kind == "product" else case["n"])
+    ref = _Ref(case)
+    trees = [ref.project(f, case["prec"]) for f in fs]
+    if sum(len(t) for t in trees) * (case["order"] + 1) ** 3 > 6e6:
+        return None  # over the time a check may take
+    if kind == "product":
+        keys, blocks = ref.product(trees[0], trees[1], case["prec"])
+    else:
+        keys, blocks = ref.sum([(-1.0) ** i / (1.0 + i) for i in range(len(fs))], trees)
+    k = np.array(keys)
+    return {"depth": k[:, 0].astype(np.int32), "l": k[:, 1:].astype(np.int64), "blocks": blocks}
