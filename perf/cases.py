@@ -53,8 +53,8 @@ def _case(name, kind, order, prec, n_gauss, exp_lo, exp_hi, box, **more):
 def listed():
     return [
         # the smallest call: a loose-precision potential of one compact
-        # charge, a few refinement levels of a few hundred nodes
-        _case("coulomb_k4_small", "apply", 4, 1e-3, 1, 2.0, 10.0, 1.0, kernel="poisson", resident=True),
+        # charge, a few refinement levels of few nodes
+        _case("coulomb_k4_small", "apply", 4, 1e-3, 1, 30.0, 30.0, 1.0, kernel="poisson", resident=True),
         # the single-Gaussian Coulomb potential at order 7
         _case("coulomb_k7", "apply", 7, 1e-5, 1, 10.0, 10.0, 1.0, kernel="poisson", resident=True),
         # the default call: host trees in and out, and the potential at points
