@@ -1353,6 +1353,8 @@ struct DevicePlan {
     PostPair *post_pairs = nullptr;
     std::vector<long long> post_off;
     double *post_F = nullptr, *post_norms = nullptr;
+    // the root level's dense products (n_items 0: none)
+    RootLaunch root;
     // the captured step (step_graph) and what it was captured for
     hipGraphExec_t graph = nullptr;
     int graph_mode = -1;
@@ -1776,6 +1778,34 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
     const size_t f_sj = place(sizeof(int) * n_all), f_s0 = place(sizeof(int) * n_all), f_s1 = place(sizeof(int) * n_all);
     const size_t f_apps = place(sizeof(AppDesc) * parts.size());
     const size_t f_cnt = place(sizeof(unsigned long long) * 8);
+    // root boxes and (apply, term) items of the dense root kernels
+    std::vector<RootApp> root_apps;
+    std::vector<RootItem> root_items;
+    std::vector<long long> root_slot_off;
+    std::vector<int> root_out;
+    {
+        long long o_out = 0, o_pool = 0;
+        for (size_t ai = 0; ai < parts.size(); ai++) {
+            const ApplyPlan &pl = *parts[ai].plan;
+            if (pl.root_dense) {
+                const OperFlat &f = *parts[ai].flat;
+                for (int m = 0; m < f.M; m++)
+                    if (f.L[(size_t)m * f.ndepth] >= 0) root_items.push_back(RootItem{(int)root_apps.size(), m});
+                root_apps.push_back(RootApp{opers[ai]->L, opers[ai]->boff, opers[ai]->blocks, f.ndepth,
+                                            (int)root_out.size()});
+                for (size_t r = 0; r < pl.root_q.size(); r++) {
+                    root_out.push_back((int)o_out + pl.root_q[r]);
+                    root_slot_off.push_back(o_pool + pl.slot_off[pl.root_slot[r]]);
+                }
+                p->root.geo = RootGeo{N, {pl.boxes[0], pl.boxes[1], pl.boxes[2]}};
+                p->root.apps_count += (unsigned long long)pl.root_apps;
+            }
+            o_out += (long long)pl.out_node.size();
+            o_pool += pl.device_pool ? pl.pool_values : (long long)pl.in_coefs.size();
+        }
+    }
+    const size_t f_ra = place(sizeof(RootApp) * root_apps.size()), f_ri = place(sizeof(RootItem) * root_items.size());
+    const size_t f_rs = place(sizeof(long long) * root_slot_off.size()), f_ro = place(sizeof(int) * root_out.size());
     std::vector<size_t> f_mt(parts.size());
     for (size_t ai = 0; ai < parts.size(); ai++) f_mt[ai] = place(sizeof(double) * mtabs[ai].size());
     if (adopt_pool) {
@@ -1799,6 +1829,12 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
     }
     p->out_bytes = sizeof(double) * (size_t)std::max<long long>(n_out, 1) * 8 * N * N * N;
     if (!rc) rc = plan_alloc(p, p->out_bytes / sizeof(double), &a.out_ns, err);
+    if (!rc && !root_items.empty()) {
+        size_t na = 0, ny = 0;
+        root_work_values(N, p->root.geo.boxes, (long long)root_items.size(), &na, &ny);
+        rc = plan_alloc(p, na, &p->root.A, err);
+        if (!rc) rc = plan_alloc(p, ny, &p->root.Y, err);
+    }
     if (rc) {
         delete p;
         return rc;
@@ -1913,6 +1949,10 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
     if (!rc) {
         std::memcpy(at(f_apps), p->apps.data(), sizeof(AppDesc) * p->apps.size());
         std::memset(at(f_cnt), 0, sizeof(unsigned long long) * 8);
+        put(f_ra, 0, root_apps);
+        put(f_ri, 0, root_items);
+        put(f_rs, 0, root_slot_off);
+        put(f_ro, 0, root_out);
         hipError_t e = hipMemcpyAsync(dev, stage.data(), arena, hipMemcpyHostToDevice, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) {
@@ -1942,6 +1982,16 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
     a.seg_job = reinterpret_cast<const int *>(dev + f_sj);
     a.seg_p0 = reinterpret_cast<const int *>(dev + f_s0);
     a.seg_p1 = reinterpret_cast<const int *>(dev + f_s1);
+    if (!root_items.empty()) {
+        RootLaunch &r = p->root;
+        r.apps = reinterpret_cast<const RootApp *>(dev + f_ra);
+        r.items = reinterpret_cast<const RootItem *>(dev + f_ri);
+        r.n_items = (int)root_items.size();
+        r.slot_off = reinterpret_cast<const long long *>(dev + f_rs);
+        r.root_out = reinterpret_cast<const int *>(dev + f_ro);
+        r.pool = p->pool;
+        r.counter = a.counters;
+    }
     if (adopt_pool) p->bufs.push_back(adopt_pool);
     *out = p;
     return 0;
@@ -2277,6 +2327,11 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         HIP_TRY(hipGetLastError());
     }
     int rc = 0;
+    if (p->root.n_items > 0) {
+        p->root.out_ns = p->args.out_ns;
+        rc = dev_root_launch(c->stream, p->root, err);
+        if (rc) return rc;
+    }
     const double inf = HUGE_VAL;
     // queue heads of the persistent launches: counters[2] (first stream),
     // counters[3] (second stream)

@@ -225,6 +225,40 @@ void dev_set_noalloc(DeviceCtx *c, void *base, size_t bytes);
 void *dev_noalloc_base(DeviceCtx *c);
 size_t dev_noalloc_bytes(DeviceCtx *c);
 
+// The root level as dense products (mw_root.hip): output blocks of every root
+// box of `apps` from all their terms, added into out_ns.
+struct RootGeo {
+    int n, boxes[3];  // k + 1, root boxes per direction
+};
+// One apply: its operator's tables and the start of its boxes (x fastest) in
+// the launch's slot_off (pool offsets of their blocks) and root_out (output
+// nodes).
+struct RootApp {
+    const int *L;
+    const long long *boff;
+    const double *blocks;
+    int ndepth, root0;
+};
+struct RootItem {
+    int app, m;  // root apply, term
+};
+struct RootLaunch {
+    RootGeo geo{};
+    const RootApp *apps = nullptr;
+    const RootItem *items = nullptr;  // of one apply after another
+    int n_items = 0;
+    const long long *slot_off = nullptr;
+    const int *root_out = nullptr;
+    const double *pool = nullptr;
+    double *A = nullptr, *Y = nullptr;  // work areas (root_work_values)
+    double *out_ns = nullptr;
+    unsigned long long *counter = nullptr;  // += apps_count
+    unsigned long long apps_count = 0;
+};
+void root_work_values(int n, const int *boxes, long long n_items, size_t *a_values, size_t *y_values);
+// Launches only, on `stream`.
+int dev_root_launch(void *stream, const RootLaunch &r, std::string &err);
+
 // Helpers shared by the HIP sources.
 struct DevOperTables {
     int *L = nullptr;

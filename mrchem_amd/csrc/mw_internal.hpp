@@ -287,6 +287,16 @@ struct ApplyPlan {
     bool device_pool = false;
     std::vector<int> slot_src, gen_parent, gen_child, gen_level_off;
     long long pool_values = 0;  // doubles of the pool
+    // The root boxes when all of them are output nodes with threshold zero
+    // (an apply's first level) and their tensor fits the dense root kernels
+    // (2 (k+1) boxes <= 48 per direction): output position and input slot of
+    // each box, x fastest; else empty.  root_dense (finish_plan_counts): the
+    // roots are computed by those kernels and hold no segments, root_apps
+    // their passing term-applications.
+    int boxes[3] = {0, 0, 0};
+    std::vector<int> root_q, root_slot;
+    bool root_dense = false;
+    long long root_apps = 0;
 };
 
 struct ApplyStats {

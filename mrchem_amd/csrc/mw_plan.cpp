@@ -174,6 +174,32 @@ void build_plan(ApplyPlan &plan, const Operator &op, const Tree &inp, const Tree
                 }
     }
 
+    // Root boxes for the dense root kernels (48: three 16-wide tiles a
+    // direction, the widest they hold in registers).
+    for (int d = 0; d < 3; d++) plan.boxes[d] = mra.boxes[d];
+    const int n_roots = mra.boxes[0] * mra.boxes[1] * mra.boxes[2];
+    if (2 * mra.kp1() * std::max(mra.boxes[0], std::max(mra.boxes[1], mra.boxes[2])) <= 48) {
+        plan.root_q.assign(n_roots, -1);
+        plan.root_slot.assign(n_roots, -1);
+        int found = 0;
+        for (size_t q = 0; q < nodes.size(); q++) {
+            const NodeKey &k = out.keys[nodes[q]];
+            if (k.depth != 0 || thr[q] != 0.0) continue;
+            long long b[3];
+            for (int d = 0; d < 3; d++) b[d] = k.l[d] - mra.corner[d];
+            const int r = (int)((b[2] * mra.boxes[1] + b[1]) * mra.boxes[0] + b[0]);
+            const int side = 2 * plan.band_w[q] + 1, s = plan.band[plan.band_off[q] + (side * side * side - 1) / 2];
+            if (plan.root_q[r] >= 0 || s < 0 || slot_real[s] < 0) continue;
+            plan.root_q[r] = (int)q;
+            plan.root_slot[r] = s;
+            found++;
+        }
+        if (found < n_roots) {
+            plan.root_q.clear();
+            plan.root_slot.clear();
+        }
+    }
+
     // Coefficient pool: real slots keep the full block, generated slots the
     // scaling part only.
     const int ns = (int)slot_keys.size();
@@ -462,12 +488,24 @@ void finish_plan_counts(ApplyPlan &plan, const Operator &op, int seg_target, boo
         }
     }
     plan.term_apps = napps;
+    // The roots go to the dense root kernels in plain FP64, and in the mixed
+    // and split modes where no threshold is positive (then every term is of
+    // the FP64 class); with positive thresholds those modes class the roots'
+    // terms by bound, and the roots keep their segments.
+    plan.root_dense = !plan.root_q.empty() && (!fine_segments || plan.thr_floor == 0.0);
+    std::vector<char> dense(nq, 0);
+    plan.root_apps = 0;
+    if (plan.root_dense)
+        for (int q : plan.root_q) {
+            dense[q] = 1;
+            for (long long e = cof[q]; e < cof[q + 1]; e++) plan.root_apps += counts[e];
+        }
     // A small launch (an adaptive apply's level) is cut finer, into about
     // 2048 segments of at least 32 terms, so that it still has work for every
     // compute unit's workgroups; launches with 2048 x seg_target passing terms
     // or more (this plan's count times n_share) keep seg_target.
     const int target_in = seg_target;
-    const long long launch_apps = napps * std::max(1, n_share);
+    const long long launch_apps = (napps - plan.root_apps) * std::max(1, n_share);
     seg_target = (int)std::min<long long>(seg_target, std::max<long long>(32, launch_apps / 2048));
     // In such a small plan a band position holding more passing terms than a
     // segment is cut inside, at input-component boundaries (an adaptive
@@ -554,7 +592,7 @@ void finish_plan_counts(ApplyPlan &plan, const Operator &op, int seg_target, boo
             mine.clear();
             const int q0 = (int)((long long)nq * t / T), q1 = (int)((long long)nq * (t + 1) / T);
             for (int q = q0; q < q1; q++)
-                for (int gt = 0; gt < (kind == 1 ? 4 : 8); gt++) {
+                for (int gt = 0; gt < (kind == 1 ? 4 : 8) && !dense[q]; gt++) {
                     const int comps[2] = {gt, gt | 4};
                     cut(q, comps, kind == 1 ? 2 : 1, kind == 0 ? fine_target : seg_target, mine);
                 }
