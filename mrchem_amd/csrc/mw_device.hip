@@ -12,6 +12,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
 #include <thread>
 #include <type_traits>
@@ -1290,7 +1291,32 @@ struct DevOper {
     int M = 0, ndepth = 0;
 };
 
+// Device memory of one context.  hipMalloc and hipFree cost 0.1-1 ms each
+// for the tens to hundreds of MB of an apply's pools and levels (hipFree also
+// waits for the device), a dozen pairs a refinement level (without -> with the
+// pool: one k = 9 apply on resident trees 34.7 -> 25.1 ms, ten exchange
+// densities at k = 7 43.9 -> 31.3 ms, one k = 7 product 2.24 -> 1.39 ms).
+// Blocks are kept by
+// size class (an eighth of a power of two, so at most 12.5 % is unused) and
+// given back to the driver when more than kIdleMax bytes are idle, when an
+// allocation fails on any context of the device, and with the context.
+struct MemPool {
+    static constexpr size_t kIdleMax = (size_t)8 << 30;
+    std::mutex mtx;
+    std::map<void *, size_t> live;         // handed out: class size
+    std::multimap<size_t, void *> idle;
+    size_t idle_bytes = 0;
+    static size_t size_class(size_t b) {
+        b = std::max<size_t>(b, 512);
+        int e = 0;
+        while ((b >> e) > 8) e++;  // b in (8, 16] x 2^(e - 1) and more
+        const size_t q = (size_t)1 << (e > 0 ? e - 1 : 0);
+        return (b + q - 1) / q * q;
+    }
+};
+
 struct DeviceCtx {
+    MemPool mem;
     int device = 0;
     int n_cu = 0;       // compute units
     int lds_max = 0;    // LDS bytes a workgroup may use
@@ -1315,6 +1341,90 @@ struct DeviceCtx {
     void *stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
+
+namespace {
+// contexts of the process, for dev_mem_get's second try
+std::mutex g_ctx_mtx;
+std::set<DeviceCtx *> g_ctxs;
+
+void mem_trim(MemPool &m) {
+    std::lock_guard<std::mutex> g(m.mtx);
+    for (auto &kv : m.idle) (void)hipFree(kv.second);
+    m.idle.clear();
+    m.idle_bytes = 0;
+}
+}  // namespace
+
+int dev_mem_get(DeviceCtx *c, size_t bytes, void **p, std::string &err) {
+    *p = nullptr;
+    HIP_TRY(hipSetDevice(c->device));
+    MemPool &m = c->mem;
+    const size_t cls = MemPool::size_class(bytes);
+    {
+        std::lock_guard<std::mutex> g(m.mtx);
+        auto it = m.idle.lower_bound(cls);
+        // the class itself or the next one up
+        if (it != m.idle.end() && it->first <= cls + cls / 7) {
+            *p = it->second;
+            m.idle_bytes -= it->first;
+            m.live[*p] = it->first;
+            m.idle.erase(it);
+            return 0;
+        }
+    }
+    hipError_t e = hipMalloc(p, cls);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        {
+            std::lock_guard<std::mutex> g(g_ctx_mtx);
+            for (DeviceCtx *o : g_ctxs)
+                if (o->device == c->device) mem_trim(o->mem);
+        }
+        e = hipMalloc(p, cls);
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        err = "hipMalloc(" + std::to_string(cls) + " bytes): " + hipGetErrorString(e);
+        return -2;
+    }
+    std::lock_guard<std::mutex> g(m.mtx);
+    m.live[*p] = cls;
+    return 0;
+}
+
+void dev_mem_put(DeviceCtx *c, void *p) {
+    if (!p) return;
+    MemPool &m = c->mem;
+    {
+        std::lock_guard<std::mutex> g(m.mtx);
+        auto it = m.live.find(p);
+        if (it == m.live.end()) return;
+        const size_t cls = it->second;
+        m.live.erase(it);
+        if (m.idle_bytes + cls <= MemPool::kIdleMax) {
+            m.idle.emplace(cls, p);
+            m.idle_bytes += cls;
+            return;
+        }
+    }
+    (void)hipSetDevice(c->device);
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(p);
+}
+
+int dev_raw_alloc(DeviceCtx *c, size_t bytes, void **p, std::string &err) {
+    *p = nullptr;
+    HIP_TRY(hipSetDevice(c->device));
+    HIP_TRY(hipMalloc(p, std::max<size_t>(bytes, 8)));
+    return 0;
+}
+
+void dev_raw_free(DeviceCtx *c, void *p) {
+    if (!p) return;
+    (void)hipSetDevice(c->device);
+    (void)hipStreamSynchronize(c->stream);
+    (void)hipFree(p);
+}
 
 struct DevicePlan {
     DeviceCtx *ctx = nullptr;
@@ -1363,13 +1473,9 @@ struct DevicePlan {
     unsigned ran_eager = 0;  // bit 2 mode + post: an eager run of that step happened
     ~DevicePlan() {
         if (graph) (void)hipGraphExecDestroy(graph);
-        for (void *p : bufs)
-            if (p) (void)hipFree(p);
-        if (pool32) (void)hipFree(pool32);
-        if (pool_h) (void)hipFree(pool_h);
-        if (pool_hsc) (void)hipFree(pool_hsc);
-        if (list_hi) (void)hipFree(list_hi);
-        if (list_lo) (void)hipFree(list_lo);
+        for (void *p : bufs) dev_mem_put(ctx, p);
+        for (void *p : {(void *)pool32, (void *)pool_h, (void *)pool_hsc, (void *)list_hi, (void *)list_lo})
+            dev_mem_put(ctx, p);
     }
 };
 
@@ -1408,19 +1514,18 @@ int dev_create(int device, DeviceCtx **out, std::string &err) {
         dev_destroy(c);
         return -2;
     }
+    {
+        std::lock_guard<std::mutex> g(g_ctx_mtx);
+        g_ctxs.insert(c);
+    }
     *out = c;
     return 0;
 }
 
-static void free_oper(DevOper &o) {
-    if (o.L) (void)hipFree(o.L);
-    if (o.boff) (void)hipFree(o.boff);
-    if (o.noff) (void)hipFree(o.noff);
-    if (o.blocks) (void)hipFree(o.blocks);
-    if (o.norms) (void)hipFree(o.norms);
-    if (o.blocks32) (void)hipFree(o.blocks32);
-    if (o.blocks_h) (void)hipFree(o.blocks_h);
-    if (o.blocks_hsc) (void)hipFree(o.blocks_hsc);
+static void free_oper(DeviceCtx *c, DevOper &o) {
+    for (void *p : {(void *)o.L, (void *)o.boff, (void *)o.noff, (void *)o.blocks, (void *)o.norms,
+                    (void *)o.blocks32, (void *)o.blocks_h, (void *)o.blocks_hsc})
+        dev_mem_put(c, p);
     o = DevOper();
 }
 
@@ -1428,7 +1533,7 @@ void dev_destroy(DeviceCtx *c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (auto &kv : c->opers) free_oper(kv.second);
+    for (auto &kv : c->opers) free_oper(c, kv.second);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->evm) (void)hipEventDestroy(c->evm);
@@ -1445,6 +1550,12 @@ void dev_destroy(DeviceCtx *c) {
         (void)hipStreamSynchronize(c->stream2);
         (void)hipStreamDestroy(c->stream2);
     }
+    {
+        std::lock_guard<std::mutex> g(g_ctx_mtx);
+        g_ctxs.erase(c);
+    }
+    mem_trim(c->mem);
+    for (auto &kv : c->mem.live) (void)hipFree(kv.first);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -1550,19 +1661,22 @@ void dev_forget_operator(DeviceCtx *c, const void *key) {
     if (it == c->opers.end()) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
-    free_oper(it->second);
+    free_oper(c, it->second);
     c->opers.erase(it);
 }
 
 template <typename T>
-static int alloc_copy(const std::vector<T> &v, T **out, hipStream_t s, std::string &err) {
-    HIP_TRY(hipMalloc((void **)out, sizeof(T) * std::max<size_t>(v.size(), 1)));
-    if (!v.empty()) HIP_TRY(hipMemcpyAsync(*out, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, s));
+static int alloc_copy(DeviceCtx *c, const std::vector<T> &v, T **out, std::string &err) {
+    int rc = dev_mem(c, v.size(), out, err);
+    if (rc) return rc;
+    if (!v.empty()) HIP_TRY(hipMemcpyAsync(*out, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, c->stream));
     return 0;
 }
 
-static int to_f32(const double *src, float **dst, long long n, hipStream_t s, std::string &err) {
-    HIP_TRY(hipMalloc((void **)dst, sizeof(float) * std::max<long long>(n, 1)));
+static int to_f32(DeviceCtx *c, const double *src, float **dst, long long n, std::string &err) {
+    hipStream_t s = c->stream;
+    int rc = dev_mem(c, (size_t)n, dst, err);
+    if (rc) return rc;
     if (n > 0) {
         const int bs = 256;
         hipLaunchKernelGGL(k_to_f32, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, s, src, *dst, n);
@@ -1583,16 +1697,16 @@ static int get_oper(DeviceCtx *c, const void *key, const OperFlat &f, DevOper **
         return -1;
     }
     DevOper o;
-    int rc = alloc_copy(f.L, &o.L, c->stream, err);
-    if (!rc) rc = alloc_copy(f.boff, &o.boff, c->stream, err);
-    if (!rc) rc = alloc_copy(f.noff, &o.noff, c->stream, err);
-    if (!rc) rc = alloc_copy(f.blocks, &o.blocks, c->stream, err);
-    if (!rc) rc = alloc_copy(f.norms, &o.norms, c->stream, err);
+    int rc = alloc_copy(c, f.L, &o.L, err);
+    if (!rc) rc = alloc_copy(c, f.boff, &o.boff, err);
+    if (!rc) rc = alloc_copy(c, f.noff, &o.noff, err);
+    if (!rc) rc = alloc_copy(c, f.blocks, &o.blocks, err);
+    if (!rc) rc = alloc_copy(c, f.norms, &o.norms, err);
     o.nblk = (long long)f.blocks.size();
     o.M = f.M;
     o.ndepth = f.ndepth;
     if (rc) {
-        free_oper(o);
+        free_oper(c, o);
         return rc;
     }
     c->opers[key] = o;
@@ -1611,13 +1725,14 @@ void *dev_stream(DeviceCtx *c) { return c->stream; }
 
 int dev_alloc_oper_tables(DeviceCtx *c, const OperFlat &f, DevOperTables &t, std::string &err) {
     t = DevOperTables();
-    HIP_TRY(hipMalloc((void **)&t.blocks, sizeof(double) * std::max<long long>(f.device_blocks, 1)));
-    HIP_TRY(hipMalloc((void **)&t.norms, sizeof(double) * std::max<size_t>(f.norms.size(), 1)));
+    int rc = dev_mem(c, (size_t)f.device_blocks, &t.blocks, err);
+    if (!rc) rc = dev_mem(c, f.norms.size(), &t.norms, err);
+    if (rc) return rc;
     HIP_TRY(hipMemsetAsync(t.blocks, 0, sizeof(double) * std::max<long long>(f.device_blocks, 1), c->stream));
     HIP_TRY(hipMemsetAsync(t.norms, 0, sizeof(double) * std::max<size_t>(f.norms.size(), 1), c->stream));
-    int rc = alloc_copy(f.L, &t.L, c->stream, err);
-    if (!rc) rc = alloc_copy(f.boff, &t.boff, c->stream, err);
-    if (!rc) rc = alloc_copy(f.noff, &t.noff, c->stream, err);
+    rc = alloc_copy(c, f.L, &t.L, err);
+    if (!rc) rc = alloc_copy(c, f.boff, &t.boff, err);
+    if (!rc) rc = alloc_copy(c, f.noff, &t.noff, err);
     return rc;
 }
 
@@ -1627,7 +1742,7 @@ int dev_register_operator(DeviceCtx *c, const void *key, const OperFlat &f, cons
     auto it = c->opers.find(key);
     if (it != c->opers.end()) {
         (void)hipStreamSynchronize(c->stream);
-        free_oper(it->second);
+        free_oper(c, it->second);
         c->opers.erase(it);
     }
     DevOper o;
@@ -1665,11 +1780,9 @@ int dev_download_operator_blocks(DeviceCtx *c, const void *key, double *out, lon
 // Device buffer of n elements owned by the plan.
 template <typename T>
 static int plan_alloc(DevicePlan *p, size_t n, T **out, std::string &err) {
-    void *d = nullptr;
-    HIP_TRY(hipMalloc(&d, sizeof(T) * std::max<size_t>(n, 1)));
-    p->bufs.push_back(d);
-    *out = static_cast<T *>(d);
-    return 0;
+    int rc = dev_mem(p->ctx, n, out, err);
+    if (!rc) p->bufs.push_back(*out);
+    return rc;
 }
 
 template <typename T, typename A>
@@ -2150,12 +2263,12 @@ static int make_lists(DevicePlan *p, int mode, double tau, std::string &err) {
     int rc0 = drop_graph(p, err);
     if (rc0) return rc0;
     HIP_TRY(hipStreamSynchronize(p->ctx->stream));
-    if (p->list_hi) HIP_TRY(hipFree(p->list_hi));
-    if (p->list_lo) HIP_TRY(hipFree(p->list_lo));
+    dev_mem_put(p->ctx, p->list_hi);
+    dev_mem_put(p->ctx, p->list_lo);
     p->list_hi = p->list_lo = nullptr;
     p->list_tau = -1.0;
-    int rc = alloc_copy(hi, &p->list_hi, p->ctx->stream, err);
-    if (!rc) rc = alloc_copy(lo, &p->list_lo, p->ctx->stream, err);
+    int rc = alloc_copy(p->ctx, hi, &p->list_hi, err);
+    if (!rc) rc = alloc_copy(p->ctx, lo, &p->list_lo, err);
     if (rc) return rc;
     p->n_hi = (int)hi.size();
     p->n_lo = (int)lo.size();
@@ -2178,7 +2291,7 @@ static int ensure_f32(DevicePlan *p, std::string &err) {
         }
         DevOper &o = it->second;
         if (!o.blocks32) {
-            int rc = to_f32(o.blocks, &o.blocks32, o.nblk, c->stream, err);
+            int rc = to_f32(c, o.blocks, &o.blocks32, o.nblk, err);
             if (rc) return rc;
         }
         if (p->apps[i].blk32 != o.blocks32) {
@@ -2190,7 +2303,7 @@ static int ensure_f32(DevicePlan *p, std::string &err) {
         int rc = upload_at(p->d_apps, p->apps, c->stream, err);
         if (rc) return rc;
     }
-    if (!p->pool32) return to_f32(p->pool, &p->pool32, p->npool, c->stream, err);
+    if (!p->pool32) return to_f32(c, p->pool, &p->pool32, p->npool, err);
     return 0;
 }
 
@@ -2198,10 +2311,12 @@ static int ensure_f32(DevicePlan *p, std::string &err) {
 static int split_rh(int N) { return N > 10 ? 32 : 24; }
 
 template <int N>
-static int split_rows_n(const double *src, long long nblocks, int rows, bool data, _Float16 **dst, double **scale,
-                        hipStream_t s, std::string &err) {
-    HIP_TRY(hipMalloc((void **)dst, sizeof(_Float16) * (size_t)std::max<long long>(nblocks, 1) * rows * SplitShape<N>::RH));
-    HIP_TRY(hipMalloc((void **)scale, sizeof(double) * (size_t)std::max<long long>(nblocks, 1)));
+static int split_rows_n(DeviceCtx *c, const double *src, long long nblocks, int rows, bool data, _Float16 **dst,
+                        double **scale, std::string &err) {
+    hipStream_t s = c->stream;
+    int rc = dev_mem(c, (size_t)nblocks * rows * SplitShape<N>::RH, dst, err);
+    if (!rc) rc = dev_mem(c, (size_t)nblocks, scale, err);
+    if (rc) return rc;
     if (nblocks == 0) return 0;
     if (data)
         hipLaunchKernelGGL((k_split_rows<N, true>), dim3((unsigned)nblocks), dim3(64), 0, s, src, nblocks, rows, *dst,
@@ -2214,24 +2329,24 @@ static int split_rows_n(const double *src, long long nblocks, int rows, bool dat
 }
 
 // FP16 split rows of FP64 blocks of `rows` x N values (data or operator side).
-static int split_rows(int N, const double *src, long long nblocks, int rows, bool data, _Float16 **dst,
-                      double **scale, hipStream_t s, std::string &err) {
+static int split_rows(DeviceCtx *c, int N, const double *src, long long nblocks, int rows, bool data, _Float16 **dst,
+                      double **scale, std::string &err) {
     if (nblocks + 1 >= (1LL << 31)) {
         err = "too many blocks for the FP16 split conversion";
         return -1;
     }
     switch (N) {
-        case 2: return split_rows_n<2>(src, nblocks, rows, data, dst, scale, s, err);
-        case 3: return split_rows_n<3>(src, nblocks, rows, data, dst, scale, s, err);
-        case 4: return split_rows_n<4>(src, nblocks, rows, data, dst, scale, s, err);
-        case 5: return split_rows_n<5>(src, nblocks, rows, data, dst, scale, s, err);
-        case 6: return split_rows_n<6>(src, nblocks, rows, data, dst, scale, s, err);
-        case 7: return split_rows_n<7>(src, nblocks, rows, data, dst, scale, s, err);
-        case 8: return split_rows_n<8>(src, nblocks, rows, data, dst, scale, s, err);
-        case 9: return split_rows_n<9>(src, nblocks, rows, data, dst, scale, s, err);
-        case 10: return split_rows_n<10>(src, nblocks, rows, data, dst, scale, s, err);
-        case 11: return split_rows_n<11>(src, nblocks, rows, data, dst, scale, s, err);
-        case 12: return split_rows_n<12>(src, nblocks, rows, data, dst, scale, s, err);
+        case 2: return split_rows_n<2>(c, src, nblocks, rows, data, dst, scale, err);
+        case 3: return split_rows_n<3>(c, src, nblocks, rows, data, dst, scale, err);
+        case 4: return split_rows_n<4>(c, src, nblocks, rows, data, dst, scale, err);
+        case 5: return split_rows_n<5>(c, src, nblocks, rows, data, dst, scale, err);
+        case 6: return split_rows_n<6>(c, src, nblocks, rows, data, dst, scale, err);
+        case 7: return split_rows_n<7>(c, src, nblocks, rows, data, dst, scale, err);
+        case 8: return split_rows_n<8>(c, src, nblocks, rows, data, dst, scale, err);
+        case 9: return split_rows_n<9>(c, src, nblocks, rows, data, dst, scale, err);
+        case 10: return split_rows_n<10>(c, src, nblocks, rows, data, dst, scale, err);
+        case 11: return split_rows_n<11>(c, src, nblocks, rows, data, dst, scale, err);
+        case 12: return split_rows_n<12>(c, src, nblocks, rows, data, dst, scale, err);
         default: err = "unsupported basis size"; return -1;
     }
 }
@@ -2257,7 +2372,7 @@ static int ensure_h16(DevicePlan *p, std::string &err) {
         DevOper &o = it->second;
         if (!o.blocks_h) {
             const long long nb = o.nblk / ((long long)N * N);
-            int rc = split_rows(N, o.blocks, nb, N, false, &o.blocks_h, &o.blocks_hsc, c->stream, err);
+            int rc = split_rows(c, N, o.blocks, nb, N, false, &o.blocks_h, &o.blocks_hsc, err);
             if (rc) return rc;
         }
         if (p->apps[i].blk_h != o.blocks_h) {
@@ -2272,7 +2387,7 @@ static int ensure_h16(DevicePlan *p, std::string &err) {
     }
     if (!p->pool_h) {
         const long long nb = p->npool / ((long long)N * N * N);
-        return split_rows(N, p->pool, nb, N * N, true, &p->pool_h, &p->pool_hsc, c->stream, err);
+        return split_rows(c, N, p->pool, nb, N * N, true, &p->pool_h, &p->pool_hsc, err);
     }
     return 0;
 }
@@ -2446,13 +2561,13 @@ int dev_plan_max_diff(DevicePlan *p, const double *ref, double *max_diff, double
     const long long n = (long long)p->n_out * 8 * p->kp1 * p->kp1 * p->kp1;
     constexpr int nb = 1024;
     double *part = nullptr;
-    HIP_TRY(hipMalloc((void **)&part, sizeof(double) * 2 * nb));
+    if (int rc = dev_mem(c, 2 * (size_t)nb, &part, err)) return rc;
     hipLaunchKernelGGL(k_max_diff, dim3(nb), dim3(256), 0, c->stream, p->args.out_ns, ref, n, part);
     std::vector<double> h(2 * nb);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(h.data(), part, sizeof(double) * 2 * nb, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(part);
+    dev_mem_put(c, part);
     if (e != hipSuccess) {
         err = std::string("max difference: ") + hipGetErrorString(e);
         return -2;
@@ -2585,11 +2700,11 @@ int dev_plan_clone_output(DevicePlan *p, double **out, std::string &err) {
     HIP_TRY(hipSetDevice(c->device));
     const size_t n = (size_t)std::max(p->n_out, 1) * 8 * p->kp1 * p->kp1 * p->kp1;
     double *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, sizeof(double) * n));
+    if (int rc = dev_mem(c, n, &d, err)) return rc;
     hipError_t e = hipMemcpyAsync(d, p->args.out_ns, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
-        (void)hipFree(d);
+        dev_mem_put(c, d);
         err = std::string("output copy: ") + hipGetErrorString(e);
         return -2;
     }

@@ -189,6 +189,23 @@ int dev_copy_d2h(DeviceCtx *c, void *dst, const void *src, size_t bytes, std::st
 // copies go through the same pinned staging buffers.
 int dev_copy_h2d(DeviceCtx *c, void *dst, const void *src, size_t bytes, std::string &err);
 void dev_free(DeviceCtx *c, void *p);
+// Device memory from the context's pool (mw_device.hip): a block put back is
+// handed out again without a call to the driver.  Blocks are used by work on
+// the context's stream (or joined to it), so a block may be put back while
+// such work still runs: what its next holder enqueues comes after.
+int dev_mem_get(DeviceCtx *c, size_t bytes, void **p, std::string &err);
+void dev_mem_put(DeviceCtx *c, void *p);
+template <typename T>
+int dev_mem(DeviceCtx *c, size_t n, T **p, std::string &err) {
+    void *v = nullptr;
+    const int rc = dev_mem_get(c, sizeof(T) * (n ? n : 1), &v, err);
+    *p = static_cast<T *>(v);
+    return rc;
+}
+// Memory that callers outside the library hold (and may use on streams of
+// their own): straight from and back to the driver.
+int dev_raw_alloc(DeviceCtx *c, size_t bytes, void **p, std::string &err);
+void dev_raw_free(DeviceCtx *c, void *p);
 
 // Node-wise sums (mw_multiply.hip): for one output node and one input, the
 // input's source node (its deepest node on the path: block offset in the

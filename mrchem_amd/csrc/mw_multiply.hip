@@ -860,7 +860,7 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
     const size_t up_bytes = bytes;
     const size_t f_gen = place(sizeof(double) * n_gen * (size_t)n3), f_nrm = place(sizeof(double) * 8 * n_slot);
     unsigned char *dev = nullptr;
-    HIP_TRY(hipMalloc((void **)&dev, bytes));
+    if (int rc = dev_mem(c, bytes, &dev, err)) return rc;
     double *gen_s = reinterpret_cast<double *>(dev + f_gen), *norms = reinterpret_cast<double *>(dev + f_nrm);
     std::vector<unsigned char, UninitAlloc<unsigned char>> stage(up_bytes);
     std::memcpy(stage.data() + f_F, mra.basis.F.data(), sizeof(double) * mra.basis.F.size());
@@ -885,7 +885,7 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
                 }
                 const int t = pl.gen_child[g];
                 if ((cur->mask >> t) & 1) {
-                    (void)hipFree(dev);
+                    dev_mem_put(c, dev);
                     err = "pool fill: a generated node twice";
                     return -1;
                 }
@@ -932,7 +932,7 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
     if (e == hipSuccess && n_slot > 0)
         e = hipMemcpyAsync(norms_h.data(), norms, sizeof(double) * 8 * n_slot, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(dev);
+    dev_mem_put(c, dev);
     if (e != hipSuccess) {
         err = std::string("pool fill: ") + hipGetErrorString(e);
         return -2;
@@ -972,10 +972,7 @@ int dev_scale(DeviceCtx *c, double *p, size_t n, double f, std::string &err) {
 }
 
 int dev_alloc(DeviceCtx *c, size_t n, double **dst, std::string &err) {
-    HIP_TRY(hipSetDevice(dev_device(c)));
-    *dst = nullptr;
-    HIP_TRY(hipMalloc((void **)dst, sizeof(double) * std::max<size_t>(n, 1)));
-    return 0;
+    return dev_mem(c, n, dst, err);
 }
 
 static int move_blocks(DeviceCtx *c, const double *src, const std::vector<int> *src_idx,
@@ -984,7 +981,7 @@ static int move_blocks(DeviceCtx *c, const double *src, const std::vector<int> *
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
     int *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, sizeof(int) * n));
+    if (int rc = dev_mem(c, n, &d, err)) return rc;
     const std::vector<int> &idx = src_idx ? *src_idx : *dst_idx;
     hipError_t e = hipMemcpyAsync(d, idx.data(), sizeof(int) * n, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
@@ -993,7 +990,7 @@ static int move_blocks(DeviceCtx *c, const double *src, const std::vector<int> *
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(d);
+    dev_mem_put(c, d);
     if (e != hipSuccess) {
         err = std::string("block move: ") + hipGetErrorString(e);
         return -2;
@@ -1025,12 +1022,11 @@ int dev_d2d(DeviceCtx *c, double *dst, const double *src, size_t n, std::string 
 }
 
 int dev_upload(DeviceCtx *c, const double *src, size_t n, double **dst, std::string &err) {
-    HIP_TRY(hipSetDevice(dev_device(c)));
-    *dst = nullptr;
-    HIP_TRY(hipMalloc((void **)dst, sizeof(double) * std::max<size_t>(n, 1)));
-    const int rc = dev_copy_h2d(c, *dst, src, sizeof(double) * n, err);
+    int rc = dev_mem(c, n, dst, err);
+    if (rc) return rc;
+    rc = dev_copy_h2d(c, *dst, src, sizeof(double) * n, err);
     if (rc) {
-        (void)hipFree(*dst);
+        dev_mem_put(c, *dst);
         *dst = nullptr;
         err = "upload: " + err;
     }
@@ -1043,13 +1039,13 @@ int dev_node_norms(DeviceCtx *c, int kp1, const double *blocks, long long n, dou
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
     double *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, sizeof(double) * 2 * (size_t)n));
+    if (int rc = dev_mem(c, 2 * (size_t)n, &d, err)) return rc;
     hipLaunchKernelGGL(k_node_norms, dim3((unsigned)n), dim3(256), 0, s, blocks, n, kp1 * kp1 * kp1, d, d + n);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(host_s2, d, sizeof(double) * n, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipMemcpyAsync(host_w2, d + n, sizeof(double) * n, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(d);
+    dev_mem_put(c, d);
     if (e != hipSuccess) {
         err = std::string("node norms: ") + hipGetErrorString(e);
         return -2;
@@ -1062,12 +1058,12 @@ int dev_component_norms(DeviceCtx *c, int kp1, const double *blocks, long long n
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
     double *d = nullptr;
-    HIP_TRY(hipMalloc((void **)&d, sizeof(double) * 8 * (size_t)n));
+    if (int rc = dev_mem(c, 8 * (size_t)n, &d, err)) return rc;
     hipLaunchKernelGGL(k_component_norms, dim3((unsigned)n), dim3(64), 0, s, blocks, n, kp1 * kp1 * kp1, d);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(host8, d, sizeof(double) * 8 * (size_t)n, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(d);
+    dev_mem_put(c, d);
     if (e != hipSuccess) {
         err = std::string("component norms: ") + hipGetErrorString(e);
         return -2;
@@ -1098,17 +1094,17 @@ int dev_post_transform(DeviceCtx *c, const MRA &mra, const std::vector<std::vect
         all.insert(all.end(), l.begin(), l.end());
         off.push_back((long long)all.size());
     }
-    hipError_t e = hipMalloc((void **)&F, sizeof(double) * mra.basis.F.size());
-    if (e == hipSuccess) e = hipMalloc((void **)&pairs, sizeof(PostPair) * all.size());
-    if (e == hipSuccess)
+    int rc = dev_mem(c, mra.basis.F.size(), &F, err);
+    if (!rc) rc = dev_mem(c, all.size(), &pairs, err);
+    hipError_t e = hipSuccess;
+    if (!rc)
         e = hipMemcpyAsync(F, mra.basis.F.data(), sizeof(double) * mra.basis.F.size(), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess)
+    if (!rc && e == hipSuccess)
         e = hipMemcpyAsync(pairs, all.data(), sizeof(PostPair) * all.size(), hipMemcpyHostToDevice, s);
-    int rc = 0;
-    if (e == hipSuccess) rc = dev_post_launch(s, mra.kp1(), pairs, off, F, err, topdown);
-    if (e == hipSuccess && rc == 0) e = hipStreamSynchronize(s);
-    for (void *p : {(void *)F, (void *)pairs})
-        if (p) (void)hipFree(p);
+    if (!rc && e == hipSuccess) rc = dev_post_launch(s, mra.kp1(), pairs, off, F, err, topdown);
+    if (!rc && e == hipSuccess) e = hipStreamSynchronize(s);
+    dev_mem_put(c, F);
+    dev_mem_put(c, pairs);
     if (rc) return rc;
     if (e != hipSuccess) {
         err = std::string("post transforms: ") + hipGetErrorString(e);
@@ -1146,10 +1142,7 @@ int dev_download(DeviceCtx *c, const double *src, size_t n, double *dst, std::st
 }
 
 void dev_free(DeviceCtx *c, void *p) {
-    if (!p) return;
-    (void)hipSetDevice(dev_device(c));
-    (void)hipStreamSynchronize(static_cast<hipStream_t>(dev_stream(c)));
-    (void)hipFree(p);
+    dev_mem_put(c, p);
 }
 
 // Device memory of the allocation-free product (mwg_multiply_noalloc): one
@@ -1183,10 +1176,9 @@ struct DevMulSession {
     bool borrowed_a = false, borrowed_b = false;
     ~DevMulSession() {
         if (noalloc) return;
-        for (double *p : {F, wsc, ws})
-            if (p) (void)hipFree(p);
-        if (pool_a && !borrowed_a) (void)hipFree(pool_a);
-        if (pool_b && !borrowed_b) (void)hipFree(pool_b);
+        for (double *p : {F, wsc, ws}) dev_mem_put(ctx, p);
+        if (!borrowed_a) dev_mem_put(ctx, pool_a);
+        if (!borrowed_b) dev_mem_put(ctx, pool_b);
     }
 };
 
@@ -1265,7 +1257,7 @@ int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a
     m->ctx = c;
     m->n = n;
     auto up = [&](const double *v, size_t nv, double **d) -> int {
-        HIP_TRY(hipMalloc((void **)d, sizeof(double) * std::max<size_t>(nv, 1)));
+        if (int rc = dev_mem(c, nv, d, err)) return rc;
         if (nv) HIP_TRY(hipMemcpyAsync(*d, v, sizeof(double) * nv, hipMemcpyHostToDevice, s));
         return 0;
     };
@@ -1284,13 +1276,7 @@ int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a
     }
     if (!rc) rc = up(mra.basis.F.data(), mra.basis.F.size(), &m->F);
     if (!rc) rc = up(wsc.data(), wsc.size(), &m->wsc);
-    if (!rc) {
-        hipError_t e = hipMalloc((void **)&m->ws, sizeof(double) * (size_t)kMulBlocks * 24 * n3);
-        if (e != hipSuccess) {
-            err = std::string("hipMalloc(work area): ") + hipGetErrorString(e);
-            rc = -2;
-        }
-    }
+    if (!rc) rc = dev_mem(c, (size_t)kMulBlocks * 24 * n3, &m->ws, err);
     if (rc) {
         (void)hipStreamSynchronize(s);
         delete m;
@@ -1324,14 +1310,14 @@ int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double co
     }
     MulNode *dn = nullptr;
     double *dout = out_on_device ? out_blocks : nullptr;
-    HIP_TRY(hipMalloc((void **)&dn, sizeof(MulNode) * nodes.size()));
-    hipError_t e = out_on_device ? hipSuccess : hipMalloc((void **)&dout, sizeof(double) * nodes.size() * 8 * n3);
-    if (e != hipSuccess) {
-        (void)hipFree(dn);
-        err = std::string("hipMalloc(out): ") + hipGetErrorString(e);
-        return -2;
+    if (int rc = dev_mem(m->ctx, nodes.size(), &dn, err)) return rc;
+    if (!out_on_device) {
+        if (int rc = dev_mem(m->ctx, nodes.size() * 8 * n3, &dout, err)) {
+            dev_mem_put(m->ctx, dn);
+            return rc;
+        }
     }
-    e = hipMemcpyAsync(dn, nodes.data(), sizeof(MulNode) * nodes.size(), hipMemcpyHostToDevice, s);
+    hipError_t e = hipMemcpyAsync(dn, nodes.data(), sizeof(MulNode) * nodes.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
         const int grid = (int)std::min<size_t>(nodes.size(), kMulBlocks);
         hipLaunchKernelGGL(k_mul_nodes, dim3(grid), dim3(kMulThreads), 0, s, m->n, dn, (int)nodes.size(), m->pool_a,
@@ -1342,8 +1328,8 @@ int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double co
     if (e == hipSuccess && !out_on_device)
         crc = dev_copy_d2h(m->ctx, out_blocks, dout, sizeof(double) * nodes.size() * 8 * n3, err);
     if (e == hipSuccess && out_on_device) e = hipStreamSynchronize(s);
-    (void)hipFree(dn);
-    if (!out_on_device) (void)hipFree(dout);
+    dev_mem_put(m->ctx, dn);
+    if (!out_on_device) dev_mem_put(m->ctx, dout);
     if (crc) return crc;
     if (e != hipSuccess) {
         err = std::string("multiply launch: ") + hipGetErrorString(e);
@@ -1364,8 +1350,7 @@ struct DevAddSession {
     int n = 0, n_in = 0;
     double *pool = nullptr, *coefs = nullptr, *F = nullptr, *ws = nullptr;
     ~DevAddSession() {
-        for (double *p : {pool, coefs, F, ws})
-            if (p) (void)hipFree(p);
+        for (double *p : {pool, coefs, F, ws}) dev_mem_put(ctx, p);
     }
 };
 
@@ -1379,16 +1364,16 @@ int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &
     m->n_in = (int)coefs.size();
     const int n3 = m->n * m->n * m->n;
     auto up = [&](const std::vector<double> &v, double **d) -> int {
-        HIP_TRY(hipMalloc((void **)d, sizeof(double) * std::max<size_t>(v.size(), 1)));
+        if (int rc = dev_mem(c, v.size(), d, err)) return rc;
         if (!v.empty()) HIP_TRY(hipMemcpyAsync(*d, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice, s));
         return 0;
     };
     // the pool: the sources one after another, copied from host or device
     size_t total = 0;
     for (const BlockSource &b : pool) total += b.n;
-    int rc = 0;
-    {
-        hipError_t e = hipMalloc((void **)&m->pool, sizeof(double) * std::max<size_t>(total, 1));
+    int rc = dev_mem(c, total, &m->pool, err);
+    if (!rc) {
+        hipError_t e = hipSuccess;
         size_t off = 0;
         for (const BlockSource &b : pool) {
             if (e != hipSuccess) break;
@@ -1404,13 +1389,7 @@ int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &
     }
     if (!rc) rc = up(coefs, &m->coefs);
     if (!rc) rc = up(mra.basis.F, &m->F);
-    if (!rc) {
-        hipError_t e = hipMalloc((void **)&m->ws, sizeof(double) * (size_t)kMulBlocks * 16 * n3);
-        if (e != hipSuccess) {
-            err = std::string("hipMalloc(work area): ") + hipGetErrorString(e);
-            rc = -2;
-        }
-    }
+    if (!rc) rc = dev_mem(c, (size_t)kMulBlocks * 16 * n3, &m->ws, err);
     if (rc) {
         (void)hipStreamSynchronize(s);
         delete m;
@@ -1433,14 +1412,14 @@ int dev_add_nodes(DevAddSession *m, const std::vector<AddSrc> &src, double *out_
     const int n3 = m->n * m->n * m->n;
     AddSrc *dsrc = nullptr;
     double *dout = out_on_device ? out_blocks : nullptr;
-    HIP_TRY(hipMalloc((void **)&dsrc, sizeof(AddSrc) * src.size()));
-    hipError_t e = out_on_device ? hipSuccess : hipMalloc((void **)&dout, sizeof(double) * n_nodes * 8 * n3);
-    if (e != hipSuccess) {
-        (void)hipFree(dsrc);
-        err = std::string("hipMalloc(out): ") + hipGetErrorString(e);
-        return -2;
+    if (int rc = dev_mem(m->ctx, src.size(), &dsrc, err)) return rc;
+    if (!out_on_device) {
+        if (int rc = dev_mem(m->ctx, n_nodes * 8 * n3, &dout, err)) {
+            dev_mem_put(m->ctx, dsrc);
+            return rc;
+        }
     }
-    e = hipMemcpyAsync(dsrc, src.data(), sizeof(AddSrc) * src.size(), hipMemcpyHostToDevice, s);
+    hipError_t e = hipMemcpyAsync(dsrc, src.data(), sizeof(AddSrc) * src.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
         const int grid = (int)std::min<size_t>(n_nodes, kMulBlocks);
         hipLaunchKernelGGL(k_add_nodes, dim3(grid), dim3(kMulThreads), 0, s, m->n, dsrc, m->n_in, (int)n_nodes,
@@ -1451,8 +1430,8 @@ int dev_add_nodes(DevAddSession *m, const std::vector<AddSrc> &src, double *out_
     if (e == hipSuccess && !out_on_device)
         crc = dev_copy_d2h(m->ctx, out_blocks, dout, sizeof(double) * n_nodes * 8 * n3, err);
     if (e == hipSuccess && out_on_device) e = hipStreamSynchronize(s);
-    (void)hipFree(dsrc);
-    if (!out_on_device) (void)hipFree(dout);
+    dev_mem_put(m->ctx, dsrc);
+    if (!out_on_device) dev_mem_put(m->ctx, dout);
     if (crc) return crc;
     if (e != hipSuccess) {
         err = std::string("add launch: ") + hipGetErrorString(e);

@@ -387,19 +387,18 @@ int fill_n(int N, const OpItem *items, int n, const OpConst &k, const OpScanOut 
 #undef MWG_CALL
 }
 
-// Device buffers freed on scope exit.
+// Device buffers put back on scope exit.
 struct DevBufs {
+    DeviceCtx *c;
     std::vector<void *> p;
     template <typename T>
     int alloc(size_t n, T **out, std::string &err) {
-        void *d = nullptr;
-        HIP_TRY(hipMalloc(&d, sizeof(T) * std::max<size_t>(n, 1)));
-        p.push_back(d);
-        *out = static_cast<T *>(d);
-        return 0;
+        const int rc = dev_mem(c, n, out, err);
+        if (!rc) p.push_back(*out);
+        return rc;
     }
     ~DevBufs() {
-        for (void *q : p) (void)hipFree(q);
+        for (void *q : p) dev_mem_put(c, q);
     }
 };
 
@@ -454,7 +453,7 @@ int dev_build_operators(DeviceCtx *c, const MRA &mra, const std::vector<OpBuildJ
     const double *qx = nullptr, *qw = nullptr;
     const int nq = N2 + 20;
     quad_rule01(nq, &qx, &qw);
-    DevBufs tmp;
+    DevBufs tmp{c, {}};
     double *dC, *dF, *dqx, *dqw, *dnrm;
     OpItem *ditems;
     OpScanOut *dscan;

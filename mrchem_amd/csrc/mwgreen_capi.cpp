@@ -2118,16 +2118,14 @@ int mwg_device_buffer_create(mwg_context ctx, long long bytes, void **dev) {
     return guarded_ctx(ctx, [&] {
         if (!ctx || !dev || bytes < 0) return fail(MWG_ERR_ARG, "bad arguments");
         std::string err;
-        double *p = nullptr;
-        dev_check(dev_alloc(ctx->dev, ((size_t)bytes + 7) / 8, &p, err), err);
-        *dev = p;
+        dev_check(dev_raw_alloc(ctx->dev, (size_t)bytes, dev, err), err);
         return (int)MWG_OK;
     });
 }
 
 int mwg_device_buffer_destroy(mwg_context ctx, void *dev) {
     if (!ctx) return fail(MWG_ERR_ARG, "null context");
-    dev_free(ctx->dev, dev);
+    dev_raw_free(ctx->dev, dev);
     return MWG_OK;
 }
 
