@@ -85,9 +85,9 @@ __device__ void pair_pass(int n, const double *F, const double *src, double *dst
 // pairs: dst[k] = sum_j H_bit[j][i] lo_k[j] + G_bit[j][i] hi_k[j] along dim,
 // with lo_k = src + lo_off[k] blocks, hi_k likewise (hi_off < 0: none).
 __device__ void child_pass(int n, const double *F, const double *src, const int *lo_blk, const int *hi_blk, int nb,
-                           double *dst, int dim, int bit, int tid, int nth = kMulThreads) {
+                           double *dst, int dim, int bit, int tid) {
     const int n2 = 2 * n, n3 = n * n * n;
-    for (int e = tid; e < nb * n3; e += nth) {
+    for (int e = tid; e < nb * n3; e += kMulThreads) {
         const int k = e / n3, rem = e % n3;
         int i, a, c;
         if (dim == 0) {
@@ -234,106 +234,6 @@ __global__ __launch_bounds__(kMulThreads) void k_add_nodes(int n, const AddSrc *
             }
         }
     }
-}
-
-// The generated children of one parent in an apply plan's pool: out[t] is
-// the scaling block of child t (null when child t is not generated), the
-// parent an input-tree node (full: its 8 components) or a generated node
-// (its scaling block only).
-struct GenGroup {
-    const double *src;
-    double *out[8];
-    int full, mask;
-};
-
-// Threads of a k_gen_fill workgroup: its LDS (6 n^3 doubles, 83 KB at
-// n = 12) allows one or two workgroups per compute unit, so a workgroup
-// brings 16 waves (64 Helmholtz applies at k = 11, adaptive on resident
-// trees: 1099 -> 1023 ms against 256 threads).
-constexpr int kGenThreads = 1024;
-
-// Generated nodes of one depth, grouped by parent (their parents are input
-// nodes or generated nodes of the depth above): one workgroup per parent
-// runs the z pass once per z half of the children it has, the y pass once
-// per (z, y) quarter and the x pass per child, through LDS (X: 4 blocks,
-// Y: 2); each output gets the operations it gets taken alone.
-__global__ __launch_bounds__(kGenThreads) void k_gen_fill(int n, const double *F, const GenGroup *groups,
-                                                          int n_groups) {
-    extern __shared__ double lds[];  // 6 n^3
-    const int tid = threadIdx.x, n3 = n * n * n;
-    double *X = lds, *Y = lds + 4 * n3;
-    for (int gi = blockIdx.x; gi < n_groups; gi += gridDim.x) {
-        const GenGroup &gr = groups[gi];
-        const int mask = gr.mask, full = gr.full;
-        const double *src = gr.src;
-        for (int zb = 0; zb < 2; zb++) {
-            if (!((mask >> (4 * zb)) & 0xf)) continue;
-            if (full) {
-                const int lo[4] = {0, 1, 2, 3}, hi[4] = {4, 5, 6, 7};
-                child_pass(n, F, src, lo, hi, 4, X, 2, zb, tid, kGenThreads);
-            } else {
-                const int lo[1] = {0}, none[1] = {-1};
-                child_pass(n, F, src, lo, none, 1, X, 2, zb, tid, kGenThreads);
-            }
-            __syncthreads();
-            for (int yb = 0; yb < 2; yb++) {
-                if (!((mask >> (4 * zb + 2 * yb)) & 0x3)) continue;
-                if (full) {
-                    const int lo2[2] = {0, 1}, hi2[2] = {2, 3};
-                    child_pass(n, F, X, lo2, hi2, 2, Y, 1, yb, tid, kGenThreads);
-                } else {
-                    const int lo[1] = {0}, none[1] = {-1};
-                    child_pass(n, F, X, lo, none, 1, Y, 1, yb, tid, kGenThreads);
-                }
-                __syncthreads();
-                for (int xb = 0; xb < 2; xb++) {
-                    const int t = xb | (yb << 1) | (zb << 2);
-                    if (!((mask >> t) & 1)) continue;
-                    if (full) {
-                        const int lo1[1] = {0}, hi1[1] = {1};
-                        child_pass(n, F, Y, lo1, hi1, 1, gr.out[t], 0, xb, tid, kGenThreads);
-                    } else {
-                        const int lo[1] = {0}, none[1] = {-1};
-                        child_pass(n, F, Y, lo, none, 1, gr.out[t], 0, xb, tid, kGenThreads);
-                    }
-                }
-                __syncthreads();
-            }
-        }
-    }
-}
-
-// One slot of an apply plan's pool: len doubles from src (an input node's
-// full block, or a generated node's scaling block) to dst, and the slot's 8
-// component norms to norms (wavelet norms 0 for a generated slot).
-struct SlotItem {
-    const double *src;
-    double *dst, *norms;
-    int len;
-};
-
-// The copies: one wave per slot.
-__global__ __launch_bounds__(64) void k_pool_fill(const SlotItem *items, int n_items) {
-    const int lane = threadIdx.x;
-    for (int s = blockIdx.x; s < n_items; s += gridDim.x) {
-        const SlotItem it = items[s];
-        for (int e = lane; e < it.len; e += 64) it.dst[e] = it.src[e];
-    }
-}
-
-// The norms: one lane per (slot, component), each summed in index order.
-__global__ __launch_bounds__(256) void k_slot_norms(int n, const SlotItem *items, int n_items) {
-    const int n3 = n * n * n;
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= 8LL * n_items) return;
-    const int s = (int)(i >> 3), comp = (int)(i & 7);
-    const SlotItem it = items[s];
-    double q = 0.0;
-    if (comp * n3 < it.len) {
-        const double *x = it.src + (size_t)comp * n3;
-        for (int e = 0; e < n3; e++) q += x[e] * x[e];
-    }
-    it.norms[comp] = sqrt(q);
 }
 
 // Squared norms of each node's scaling part and wavelet parts: one
@@ -809,6 +709,130 @@ static hipError_t post_level(hipStream_t s, int n, bool down, const PostPair *pa
     }
 }
 
+// One generated node of an apply plan's pool: the scaling block dst of child
+// `child` (bits x, y, z) of a parent with block src, an input-tree node
+// (full: its 8 components) or a generated node (its scaling block only).
+struct GenItem {
+    const double *src;
+    double *dst;
+    int child, full;
+};
+
+// Generated nodes of one depth (their parents are input nodes or generated
+// nodes of the depth above): one workgroup per child, the TopDown branch of
+// k_post_one without the addition.  Each pass keeps the half of its outputs
+// that leads to the child, one thread per line with the line in registers; a
+// launch holds few children and takes as long as one of them, so siblings
+// repeat the first passes rather than share them (one workgroup of 1024
+// threads per parent, a thread per output value: 80 -> 15 us a launch at
+// k = 9, 188 -> 42 us at k = 11).
+template <int N>
+__global__ __launch_bounds__(PostOneShape<N>::T) void k_gen_fill(const GenItem *items, const double *__restrict__ F) {
+    constexpr int N3 = N * N * N, NN = N * N, N2 = 2 * N;
+    __shared__ double X[4 * N3];
+    __shared__ double M[N2 * N2];
+    const int tid = threadIdx.x;
+    const GenItem it = items[blockIdx.x];
+    for (int e = tid; e < N2 * N2; e += PostOneShape<N>::T) M[e] = F[e];
+    const int hx = it.child & 1, hy = (it.child >> 1) & 1, hz = it.child >> 2;
+    double v[N2], o[N];
+    // a scaling-only parent has its first slot alone, and zero wavelet inputs
+    const int sh = it.full ? 0 : 2;
+    const int q = tid / NN, ac = tid % NN, a = ac % N, c = ac / N;
+#pragma unroll
+    for (int j = 0; j < N2; j++) v[j] = 0.0;
+    // z: slot q = (ty, tx) from components q and q | 4
+    if (tid < (4 >> sh) * NN) {
+#pragma unroll
+        for (int j = 0; j < N; j++) v[j] = it.src[q * N3 + post_index<N, 2>(a, c, j)];
+        if (it.full) {
+#pragma unroll
+            for (int j = 0; j < N; j++) v[N + j] = it.src[(q | 4) * N3 + post_index<N, 2>(a, c, j)];
+        }
+    }
+    __syncthreads();  // M in LDS
+    if (tid < (4 >> sh) * NN) {
+        post_half_line<N>(v, M, hz, o);
+#pragma unroll
+        for (int i = 0; i < N; i++) X[q * N3 + post_index<N, 2>(a, c, i)] = o[i];
+    }
+    __syncthreads();
+    // y: slot tx from slots tx and tx | 2
+    if (tid < (it.full ? 2 : 1) * NN) {
+#pragma unroll
+        for (int j = 0; j < N; j++) v[j] = X[q * N3 + post_index<N, 1>(a, c, j)];
+        if (it.full) {
+#pragma unroll
+            for (int j = 0; j < N; j++) v[N + j] = X[(q | 2) * N3 + post_index<N, 1>(a, c, j)];
+        }
+        post_half_line<N>(v, M, hy, o);
+    }
+    __syncthreads();  // the slots of every line read before any is written
+    if (tid < (it.full ? 2 : 1) * NN) {
+#pragma unroll
+        for (int i = 0; i < N; i++) X[q * N3 + post_index<N, 1>(a, c, i)] = o[i];
+    }
+    __syncthreads();
+    // x: slots 0 and 1
+    if (tid < NN) {
+#pragma unroll
+        for (int j = 0; j < N; j++) v[j] = X[post_index<N, 0>(a, c, j)];
+        if (it.full) {
+#pragma unroll
+            for (int j = 0; j < N; j++) v[N + j] = X[N3 + post_index<N, 0>(a, c, j)];
+        }
+        post_half_line<N>(v, M, hx, o);
+#pragma unroll
+        for (int i = 0; i < N; i++) it.dst[post_index<N, 0>(a, c, i)] = o[i];
+    }
+}
+
+static hipError_t gen_fill(hipStream_t s, int n, const GenItem *items, int cnt, const double *F) {
+#define MWG_GEN(NN)                                                                                          \
+    case NN:                                                                                                 \
+        hipLaunchKernelGGL((k_gen_fill<NN>), dim3(cnt), dim3(PostOneShape<NN>::T), 0, s, items, F);          \
+        break;
+    switch (n) {
+        MWG_GEN(2) MWG_GEN(3) MWG_GEN(4) MWG_GEN(5) MWG_GEN(6) MWG_GEN(7) MWG_GEN(8) MWG_GEN(9) MWG_GEN(10)
+        MWG_GEN(11) MWG_GEN(12)
+        default: return hipErrorInvalidValue;
+    }
+#undef MWG_GEN
+    return hipGetLastError();
+}
+
+// One slot of an apply plan's pool: len doubles from src (an input node's
+// full block, or a generated node's scaling block) to dst, and the slot's 8
+// component norms to norms (wavelet norms 0 for a generated slot).
+struct SlotItem {
+    const double *src;
+    double *dst, *norms;
+    int len;
+};
+
+// The copies and the norms in one pass: one wave per (slot, component), each
+// value read once (a copy launch and one thread per norm read them twice, the
+// norms in chains of n^3 dependent additions: 172 -> 14 us a launch at k = 9).
+__global__ __launch_bounds__(256) void k_pool_fill(int n3, const SlotItem *items, int n_items) {
+    const int s = blockIdx.x >> 1, comp = 4 * (blockIdx.x & 1) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (s >= n_items) return;
+    const SlotItem it = items[s];
+    double q = 0.0;
+    if (comp * n3 < it.len) {
+        const double *x = it.src + (size_t)comp * n3;
+        double *y = it.dst + (size_t)comp * n3;
+#pragma unroll 4
+        for (int e = lane; e < n3; e += 64) {
+            const double v = x[e];
+            y[e] = v;
+            q += v * v;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) q += __shfl_xor(q, o);
+    }
+    if (lane == 0) it.norms[comp] = sqrt(q);
+}
+
 int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &jobs, std::string &err) {
     if (jobs.empty()) return 0;
     HIP_TRY(hipSetDevice(dev_device(c)));
@@ -826,27 +850,20 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
         slot_at[i + 1] = slot_at[i] + pl.slot_src.size();
     }
     const size_t n_gen = gen_at[nj], n_slot = slot_at[nj];
-    if (n_gen >= (1u << 31) || n_slot >= (1u << 31)) {
+    if (n_gen >= (1u << 31) || n_slot >= (1u << 30)) {
         err = "pool fill: too many slots";
         return -1;
     }
-    // parent groups (runs of one parent within a depth: the plan orders the
-    // children of a parent next to each other) of depth lv:
-    // [lv_at[lv], lv_at[lv + 1])
-    auto n_groups = [&](const ApplyPlan &pl, size_t lv) {
-        size_t k = 0;
-        for (int g = pl.gen_level_off[lv]; g < pl.gen_level_off[lv + 1]; g++)
-            k += (g == pl.gen_level_off[lv] || pl.gen_parent[g] != pl.gen_parent[g - 1]);
-        return k;
-    };
+    // generated nodes of depth lv: items [lv_at[lv], lv_at[lv + 1])
     std::vector<size_t> lv_at(nlv + 1, 0);
     for (size_t lv = 0; lv < nlv; lv++) {
         size_t k = 0;
-        for (size_t i = 0; i < nj; i++)
-            if (lv + 1 < jobs[i].pl->gen_level_off.size()) k += n_groups(*jobs[i].pl, lv);
+        for (size_t i = 0; i < nj; i++) {
+            const std::vector<int> &lo = jobs[i].pl->gen_level_off;
+            if (lv + 1 < lo.size()) k += (size_t)(lo[lv + 1] - lo[lv]);
+        }
         lv_at[lv + 1] = lv_at[lv] + k;
     }
-    const size_t n_grp = lv_at[nlv];
     // one device allocation: [filter | gen items | slot items] (uploaded)
     // [generated scaling blocks of every job] [every slot's norms]
     size_t bytes = 0;
@@ -856,7 +873,7 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
         return off;
     };
     const size_t f_F = place(sizeof(double) * mra.basis.F.size());
-    const size_t f_gi = place(sizeof(GenGroup) * n_grp), f_si = place(sizeof(SlotItem) * n_slot);
+    const size_t f_gi = place(sizeof(GenItem) * n_gen), f_si = place(sizeof(SlotItem) * n_slot);
     const size_t up_bytes = bytes;
     const size_t f_gen = place(sizeof(double) * n_gen * (size_t)n3), f_nrm = place(sizeof(double) * 8 * n_slot);
     unsigned char *dev = nullptr;
@@ -864,7 +881,7 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
     double *gen_s = reinterpret_cast<double *>(dev + f_gen), *norms = reinterpret_cast<double *>(dev + f_nrm);
     std::vector<unsigned char, UninitAlloc<unsigned char>> stage(up_bytes);
     std::memcpy(stage.data() + f_F, mra.basis.F.data(), sizeof(double) * mra.basis.F.size());
-    GenGroup *gi = reinterpret_cast<GenGroup *>(stage.data() + f_gi);
+    GenItem *gi = reinterpret_cast<GenItem *>(stage.data() + f_gi);
     SlotItem *si = reinterpret_cast<SlotItem *>(stage.data() + f_si);
     // job i's generated node g is gen_s block gen_at[i] + g
     std::vector<size_t> lv_fill(lv_at.begin(), lv_at.end() - (nlv ? 1 : 0));
@@ -872,27 +889,12 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
         const ApplyPlan &pl = *jobs[i].pl;
         const double *inp = jobs[i].inp;
         double *gs = gen_s + gen_at[i] * (size_t)n3;
-        for (size_t lv = 0; lv + 1 < pl.gen_level_off.size(); lv++) {
-            GenGroup *cur = nullptr;
+        for (size_t lv = 0; lv + 1 < pl.gen_level_off.size(); lv++)
             for (int g = pl.gen_level_off[lv]; g < pl.gen_level_off[lv + 1]; g++) {
                 const int par = pl.gen_parent[g];
-                if (g == pl.gen_level_off[lv] || par != pl.gen_parent[g - 1]) {
-                    cur = &gi[lv_fill[lv]++];
-                    cur->src = par < 0 ? inp + (size_t)(-par - 1) * 8 * n3 : gs + (size_t)par * n3;
-                    for (int t = 0; t < 8; t++) cur->out[t] = nullptr;
-                    cur->full = par < 0;
-                    cur->mask = 0;
-                }
-                const int t = pl.gen_child[g];
-                if ((cur->mask >> t) & 1) {
-                    dev_mem_put(c, dev);
-                    err = "pool fill: a generated node twice";
-                    return -1;
-                }
-                cur->out[t] = gs + (size_t)g * n3;
-                cur->mask |= 1 << t;
+                gi[lv_fill[lv]++] = GenItem{par < 0 ? inp + (size_t)(-par - 1) * 8 * n3 : gs + (size_t)par * n3,
+                                            gs + (size_t)g * n3, pl.gen_child[g], par < 0};
             }
-        }
     }
     for (size_t i = 0; i < nj; i++) {
         const ApplyPlan &pl = *jobs[i].pl;
@@ -909,24 +911,16 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
     }
     std::vector<double, UninitAlloc<double>> norms_h(8 * n_slot);
     const double *F = reinterpret_cast<const double *>(dev + f_F);
-    const GenGroup *dgi = reinterpret_cast<const GenGroup *>(dev + f_gi);
+    const GenItem *dgi = reinterpret_cast<const GenItem *>(dev + f_gi);
     const SlotItem *dsi = reinterpret_cast<const SlotItem *>(dev + f_si);
     hipError_t e = hipMemcpyAsync(dev, stage.data(), up_bytes, hipMemcpyHostToDevice, s);
     for (size_t lv = 0; e == hipSuccess && lv < nlv; lv++) {
         const int cnt = (int)(lv_at[lv + 1] - lv_at[lv]);
         if (cnt == 0) continue;
-        hipLaunchKernelGGL(k_gen_fill, dim3(std::min(cnt, kMulBlocks)), dim3(kGenThreads), sizeof(double) * 6 * n3, s,
-                           n, F, dgi + lv_at[lv], cnt);
-        e = hipGetLastError();
+        e = gen_fill(s, n, dgi + lv_at[lv], cnt, F);
     }
     if (e == hipSuccess && n_slot > 0) {
-        hipLaunchKernelGGL(k_pool_fill, dim3((unsigned)std::min<size_t>(n_slot, 16384)), dim3(64), 0, s, dsi,
-                           (int)n_slot);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess && n_slot > 0) {
-        hipLaunchKernelGGL(k_slot_norms, dim3((unsigned)((8 * n_slot + 255) / 256)), dim3(256), 0, s, n, dsi,
-                           (int)n_slot);
+        hipLaunchKernelGGL(k_pool_fill, dim3((unsigned)(2 * n_slot)), dim3(256), 0, s, n3, dsi, (int)n_slot);
         e = hipGetLastError();
     }
     if (e == hipSuccess && n_slot > 0)
