@@ -351,7 +351,7 @@ int mwg_plan_finish(mwg_plan plan);
  * execution was mwg_plan_apply (its blocks are transformed in place). */
 int mwg_plan_download_ns(mwg_plan plan, double *ns, long long capacity);
 /* [0] output nodes, [1] input slots, [2] generated slots, [3] host plan ms,
- * [4] term-applications counted on the host with the screening rule,
+ * [4] term-applications counted with the screening rule when the plan was made,
  * [5] work segments (entries of the FP64 work queue), [6] applies,
  * [7] widest band half-width (translations |l| <= W per direction),
  * [8] FP64-class cut tau, [9] single-rounding ratio, [10] queue order. */

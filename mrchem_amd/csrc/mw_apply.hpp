@@ -1,0 +1,103 @@
+// Kernel arguments of an apply plan, shared by the per-node calculators
+// (mw_device.hip) and the kernels that count and cut a plan's work
+// (mw_count.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "mw_device.hpp"
+
+namespace mwg {
+
+// Per apply of a batched plan: its operator tables (device copies resident in
+// the context) and where its screening tables start.
+struct AppDesc {
+    const int *opL;                   // [m * ndepth + d]
+    const long long *op_boff, *op_noff;
+    const double *op_norms;
+    const double *blk64;              // FP64 blocks
+    const float *blk32;               // FP32 copy (mixed mode), or null
+    const _Float16 *blk_h;            // FP16 split rows (split mode), or null
+    const double *blk_hsc;            // their per-block scales
+    int M, ndepth;
+    long long bw_off;                 // start of this apply in bw
+    int act_base;                     // start of this apply in act_off
+    int mt_d0;                        // first output depth of mtab
+    double thr_floor;                 // positive floor of the class threshold
+    // pre-screen: per output depth d >= mt_d0, component combination
+    // cmb = cx | cy << 2 | cz << 4 and translation |l| <= mt_w, the largest
+    // ((N_x N_y) N_z) over the depth's active terms, [d - mt_d0][cmb][lz][ly][lx]
+    const double *mtab;
+    int mt_w, pad_;
+};
+
+struct KArgs {
+    // output nodes (all applies, concatenated)
+    const int *out_depth;
+    const int *out_app;               // apply of each output node
+    const double *out_thr;
+    const long long *band_off;
+    const int *band_w;
+    const int *band;
+    double *out_ns;
+    // input slots (all applies, concatenated)
+    const long long *slot_off;
+    const double *slot_norm;
+    // screening tables: active terms per depth, and their norms (k_term_norms)
+    // [c][l + w][active term] of the depth's band half-width w, from
+    // tn + tn_off[act_base + d]
+    const int *bw;
+    const int *act_off, *act_terms;
+    const double *tn;
+    const long long *tn_off;
+    const AppDesc *apps;
+    // [0] term-applications passing screening (algorithmic work)
+    unsigned long long *counters;
+    // work segments: job = 8*out + gt, (band position p, input component ft)
+    // pairs 8 p + ft in [p0, p1)
+    const int *seg_job, *seg_p0, *seg_p1;
+};
+
+// One depth of one apply in the norm and pre-screen tables.
+struct TermLevel {
+    int app, d, w;       // apply, output depth, band half-width there
+    int na, a0;          // its active terms: act_terms[a0, a0 + na)
+    int pad_;
+    long long tn;        // start of its norms in tn
+};
+
+// What the class lists of the mixed and split modes need of a segment: passing
+// terms and the smallest and largest passing bound.
+struct SegRec {
+    int job, p0, apps, pad_;
+    double lo, hi;
+};
+
+// Work counts and segments of a plan (mw_count.hip).
+struct CountArgs {
+    KArgs k{};
+    int n_out = 0, n_app = 0, n_share = 1;
+    const unsigned char *dense = nullptr;  // per output node: computed by the root kernels
+    // passing terms per (output component, band position) of every node,
+    // node q's at 8 band_off[q] + gt nb + p; with bounds the smallest and
+    // largest passing bound there
+    int *cnt = nullptr;
+    double *bmin = nullptr, *bmax = nullptr;
+    // per apply: passing terms, and those of dense nodes
+    unsigned long long *totals = nullptr;
+    // segments found: [0] pair ones, [1] fine ones (also past the capacity)
+    unsigned long long *n_seg = nullptr;
+    int cap[2] = {0, 0};
+    // pair segments at [0, cap[0]), fine ones at [cap[0], cap[0] + cap[1])
+    int *seg_job = nullptr, *seg_p0 = nullptr, *seg_p1 = nullptr;
+    SegRec *rec = nullptr;  // with bounds
+};
+// Norm and pre-screen tables of levels[0, n) (device array); mtab of each
+// apply is written through apps[app].mtab.  Launches only, on stream.
+int dev_term_tables(hipStream_t s, const KArgs &k, const TermLevel *levels, int n, double *tn, std::string &err);
+// Counts per position (bounds: the class bounds too), then the segments.
+// Launches only, on stream.
+int dev_count_terms(hipStream_t s, const CountArgs &c, bool bounds, std::string &err);
+int dev_cut_segments(hipStream_t s, const CountArgs &c, bool bounds, std::string &err);
+
+}  // namespace mwg

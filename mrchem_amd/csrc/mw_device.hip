@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <set>
 #include <string>
@@ -18,7 +19,7 @@
 #include <type_traits>
 #include <vector>
 
-#include "mw_device.hpp"
+#include "mw_apply.hpp"
 
 namespace mwg {
 
@@ -32,51 +33,6 @@ namespace mwg {
     } while (0)
 
 constexpr int kMaxActive = 4096;
-
-// Per apply of a batched plan: its operator tables (device copies resident in
-// the context) and where its screening tables start.
-struct AppDesc {
-    const int *opL;                   // [m * ndepth + d]
-    const long long *op_boff, *op_noff;
-    const double *op_norms;
-    const double *blk64;              // FP64 blocks
-    const float *blk32;               // FP32 copy (mixed mode), or null
-    const _Float16 *blk_h;            // FP16 split rows (split mode), or null
-    const double *blk_hsc;            // their per-block scales
-    int M, ndepth;
-    long long bw_off;                 // start of this apply in bw
-    int act_base;                     // start of this apply in act_off
-    int mt_d0;                        // first output depth of mtab
-    double thr_floor;                 // positive floor of the class threshold
-    // pre-screen: per output depth d >= mt_d0, component combination
-    // cmb = cx | cy << 2 | cz << 4 and translation |l| <= mt_w, the largest
-    // ((N_x N_y) N_z) over the depth's active terms, [d - mt_d0][cmb][lz][ly][lx]
-    const double *mtab;
-    int mt_w, pad_;
-};
-
-struct KArgs {
-    // output nodes (all applies, concatenated)
-    const int *out_depth;
-    const int *out_app;               // apply of each output node
-    const double *out_thr;
-    const long long *band_off;
-    const int *band_w;
-    const int *band;
-    double *out_ns;
-    // input slots (all applies, concatenated)
-    const long long *slot_off;
-    const double *slot_norm;
-    // screening tables
-    const int *bw;
-    const int *act_off, *act_terms;
-    const AppDesc *apps;
-    // [0] term-applications passing screening (algorithmic work)
-    unsigned long long *counters;
-    // work segments: job = 8*out + gt, (band position p, input component ft)
-    // pairs 8 p + ft in [p0, p1)
-    const int *seg_job, *seg_p0, *seg_p1;
-};
 
 template <typename T>
 __device__ __forceinline__ const T *op_blocks(const AppDesc &ad);
@@ -225,17 +181,10 @@ __device__ __forceinline__ void stage_terms(const KArgs &a, const AppDesc &ad, c
         ltab[e] = (e < cnt) ? ad.opL[m * j.ndepth + j.d] : -1;
         btab[e] = (e < cnt) ? ad.op_boff[m * j.ndepth + j.d] : 0;
     }
+    const double *tn = a.tn + a.tn_off[ad.act_base + j.d];
     for (int e = tid; e < 64 * 4 * j.nl; e += nth) {
-        const int ti = e / (4 * j.nl), c = (e / j.nl) % 4, li = e % j.nl, l = li - j.w;
-        double v = 0.0;
-        if (ti < cnt) {
-            const int m = a.act_terms[j.a0 + base + ti];
-            const int L = ad.opL[m * j.ndepth + j.d];
-            const int bwc = a.bw[ad.bw_off + ((long long)j.d * ad.M + m) * 4 + c];
-            if (abs(l) <= bwc && abs(l) <= L)
-                v = ad.op_norms[ad.op_noff[m * j.ndepth + j.d] + (long long)c * (2 * L + 1) + (l + L)];
-        }
-        nrm_s[ti * nrm_stride(j.nl) + c * j.nl + li] = v;
+        const int ti = e & 63, cl = e >> 6;
+        nrm_s[ti * nrm_stride(j.nl) + cl] = ti < cnt ? tn[(long long)cl * j.nact + base + ti] : 0.0;
     }
 }
 
@@ -1426,12 +1375,20 @@ void dev_raw_free(DeviceCtx *c, void *p) {
     (void)hipFree(p);
 }
 
+// One segment for the class lists: its index, passing terms, class cut base
+// thr_cls and the range of passing bounds.
+struct SegMeta {
+    int index, apps;
+    double thr, bmin, bmax;
+};
+
 struct DevicePlan {
     DeviceCtx *ctx = nullptr;
     std::vector<const void *> op_keys;  // per part
-    // segments: n_pseg pair ones (indices 0 .. n_pseg - 1), then n_fseg fine
-    // single-component ones
+    // segments: n_pseg pair ones (indices 0 .. n_pseg - 1) and n_fseg fine
+    // single-component ones (behind the room for pair ones)
     int n_out = 0, kp1 = 0, wmax = 0, n_pseg = 0, n_fseg = 0;
+    unsigned long long term_apps = 0;  // passing term-applications, counted when the plan was made
     long long npool = 0;
     double *pool = nullptr;
     float *pool32 = nullptr;
@@ -1442,10 +1399,8 @@ struct DevicePlan {
     AppDesc *d_apps = nullptr;
     std::vector<void *> bufs;
     size_t out_bytes = 0;
-    // per pair segment: class cut base thr_cls and the range of passing
-    // bounds; the same for the fine segments
-    std::vector<double> pseg_thr, pseg_bmin, pseg_bmax;
-    std::vector<double> fseg_thr, fseg_bmin, fseg_bmax;
+    // pair and fine segments in job order (mixed and split modes)
+    std::vector<SegMeta> psegs, fsegs;
     // segment lists of the two classes, for list_tau and list_mode (the FP64
     // class lists fine segments, the low class of the split mode pair ones)
     double list_tau = -1.0;
@@ -1455,7 +1410,6 @@ struct DevicePlan {
     // passing-term count first)
     double single_ratio = 16.0;
     int order = 0;
-    std::vector<int> pseg_apps, fseg_apps;  // passing terms per segment
     int *list_hi = nullptr, *list_lo = nullptr;
     int n_hi = 0, n_lo = 0;
     // post transforms in place (dev_plan_set_post): (branch, first child)
@@ -1791,8 +1745,8 @@ static int upload_at(T *dst, const std::vector<T, A> &v, hipStream_t s, std::str
     return 0;
 }
 
-int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan **out, std::string &err,
-                    double *adopt_pool) {
+int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, DevicePlan **out,
+                    std::string &err) {
     HIP_TRY(hipSetDevice(c->device));
     if (parts.empty()) {
         err = "empty plan";
@@ -1809,7 +1763,6 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
     }
     // sizes and validation
     long long n_out = 0, n_band = 0, n_slot = 0, n_pool = 0, n_bw = 0, n_actoff = 0, n_act = 0;
-    long long n_pseg = 0, n_fseg = 0;
     int wmax = 0;
     for (const PlanPart &pp : parts) {
         const ApplyPlan &pl = *pp.plan;
@@ -1832,75 +1785,48 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
         n_out += (long long)pl.out_node.size();
         n_band += (long long)pl.band.size();
         n_slot += (long long)pl.slot_off.size();
-        n_pool += pl.device_pool ? pl.pool_values : (long long)pl.in_coefs.size();
+        n_pool += pl.pool_values;
         n_bw += (long long)pl.bw.size();
         n_actoff += (long long)pl.active_off.size();
         n_act += (long long)pl.active_terms.size();
-        n_pseg += (long long)pl.pseg_job.size();
-        n_fseg += (long long)pl.fseg_job.size();
     }
-    const long long n_all = n_pseg + n_fseg;
-    if (n_out >= (1LL << 27) || n_all >= (1LL << 31) || n_slot >= (1LL << 31) || n_band >= (1LL << 31)) {
+    if (n_out >= (1LL << 27) || n_slot >= (1LL << 30) || n_band >= (1LL << 31)) {
         err = "batch too large for 32-bit node, segment or slot indices";
         return -1;
     }
-    auto *p = new DevicePlan;
+    std::unique_ptr<DevicePlan> p(new DevicePlan);
     p->ctx = c;
     p->n_out = (int)n_out;
     p->kp1 = N;
     p->wmax = wmax;
     p->npool = n_pool;
-    p->n_pseg = (int)n_pseg;
-    p->n_fseg = (int)n_fseg;
     KArgs &a = p->args;
     hipStream_t s = c->stream;
     int rc = 0;
-    // Every table of the plan but the pool and the output lives in one
-    // device arena, filled from one host staging buffer with one copy: a
-    // refinement level's plan costs one allocation and one upload however
-    // many applies it holds.
     std::vector<DevOper *> opers(parts.size(), nullptr);
-    std::vector<std::vector<double>> mtabs;
-    std::vector<std::pair<int, int>> mt_shape;
-    for (size_t ai = 0; ai < parts.size() && !rc; ai++) rc = get_oper(c, parts[ai].op_key, *parts[ai].flat, &opers[ai], err);
-    if (rc) {
-        delete p;
-        return rc;
-    }
-    {
-        std::vector<const ApplyPlan *> pls;
-        std::vector<const OperFlat *> fs;
-        for (const PlanPart &pp : parts) {
-            pls.push_back(pp.plan);
-            fs.push_back(pp.flat);
-        }
-        build_prescreens(pls, fs, mtabs, mt_shape);
-    }
-    size_t arena = 0;
-    auto place = [&](size_t bytes) {
-        const size_t off = arena;
-        arena += (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
-        return off;
-    };
-    const size_t f_out_depth = place(sizeof(int) * n_out), f_out_app = place(sizeof(int) * n_out);
-    const size_t f_thr = place(sizeof(double) * n_out), f_band_off = place(sizeof(long long) * n_out);
-    const size_t f_band_w = place(sizeof(int) * n_out), f_band = place(sizeof(int) * n_band);
-    const size_t f_slot_off = place(sizeof(long long) * n_slot), f_norm = place(sizeof(double) * 8 * n_slot);
-    const size_t f_bw = place(sizeof(int) * n_bw), f_act_off = place(sizeof(int) * n_actoff);
-    const size_t f_act = place(sizeof(int) * n_act);
-    const size_t f_sj = place(sizeof(int) * n_all), f_s0 = place(sizeof(int) * n_all), f_s1 = place(sizeof(int) * n_all);
-    const size_t f_apps = place(sizeof(AppDesc) * parts.size());
-    const size_t f_cnt = place(sizeof(unsigned long long) * 8);
-    // root boxes and (apply, term) items of the dense root kernels
+    for (size_t ai = 0; ai < parts.size(); ai++)
+        if ((rc = get_oper(c, parts[ai].op_key, *parts[ai].flat, &opers[ai], err))) return rc;
+    // The roots go to the dense root kernels in plain FP64, and in the mixed
+    // and split modes where no threshold is positive (then every term is of
+    // the FP64 class); with positive thresholds those modes class the roots'
+    // terms by bound, and the roots keep their segments.
+    auto dense = [&](const ApplyPlan &pl) { return !pl.root_q.empty() && (mode == 0 || pl.thr_floor == 0.0); };
+    // Root boxes and (apply, term) items of the dense root kernels, and the
+    // depths of every apply in the norm and pre-screen tables.
     std::vector<RootApp> root_apps;
     std::vector<RootItem> root_items;
     std::vector<long long> root_slot_off;
     std::vector<int> root_out;
+    std::vector<TermLevel> levels;
+    std::vector<long long> tn_off;
+    std::vector<std::pair<int, int>> mt_shape(parts.size());  // first depth, widest band
+    std::vector<size_t> mt_size(parts.size());
+    long long n_tn = 0;
     {
-        long long o_out = 0, o_pool = 0;
+        long long o_out = 0, o_pool = 0, o_act = 0;
         for (size_t ai = 0; ai < parts.size(); ai++) {
             const ApplyPlan &pl = *parts[ai].plan;
-            if (pl.root_dense) {
+            if (dense(pl)) {
                 const OperFlat &f = *parts[ai].flat;
                 for (int m = 0; m < f.M; m++)
                     if (f.L[(size_t)m * f.ndepth] >= 0) root_items.push_back(RootItem{(int)root_apps.size(), m});
@@ -1911,64 +1837,82 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
                     root_slot_off.push_back(o_pool + pl.slot_off[pl.root_slot[r]]);
                 }
                 p->root.geo = RootGeo{N, {pl.boxes[0], pl.boxes[1], pl.boxes[2]}};
-                p->root.apps_count += (unsigned long long)pl.root_apps;
+            }
+            std::vector<int> wd(pl.active_off.size(), -1);
+            int w = 0, d0 = 0, d1 = -1;
+            for (size_t q = 0; q < pl.out_depth.size(); q++) {
+                const int d = pl.out_depth[q];
+                wd[d] = pl.band_w[q];
+                w = std::max(w, pl.band_w[q]);
+                if (d1 < 0 || d < d0) d0 = d;
+                d1 = std::max(d1, d);
+            }
+            mt_shape[ai] = {d0, w};
+            mt_size[ai] = (size_t)(d1 - d0 + 1) * 64 * (2 * w + 1) * (2 * w + 1) * (2 * w + 1);
+            for (int d = 0; d < (int)pl.active_off.size(); d++) {
+                tn_off.push_back(n_tn);
+                if (d < d0 || d > d1) continue;
+                const int na = wd[d] >= 0 ? pl.active_off[d + 1] - pl.active_off[d] : 0, wl = std::max(wd[d], 0);
+                levels.push_back(TermLevel{(int)ai, d, wl, na, (int)o_act + pl.active_off[d], 0, n_tn});
+                n_tn += 4LL * (2 * wl + 1) * na;
             }
             o_out += (long long)pl.out_node.size();
-            o_pool += pl.device_pool ? pl.pool_values : (long long)pl.in_coefs.size();
+            o_pool += pl.pool_values;
+            o_act += (long long)pl.active_terms.size();
         }
     }
+    // Every table of the plan but the pool and the output lives in one
+    // device arena; what the host made of it is filled from one staging
+    // buffer with one copy, so that a refinement level's plan costs one
+    // upload however many applies it holds.
+    size_t arena = 0;
+    auto place = [&](size_t bytes) {
+        const size_t off = arena;
+        arena += (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+        return off;
+    };
+    const size_t f_out_depth = place(sizeof(int) * n_out), f_out_app = place(sizeof(int) * n_out);
+    const size_t f_thr = place(sizeof(double) * n_out), f_band_off = place(sizeof(long long) * n_out);
+    const size_t f_band_w = place(sizeof(int) * n_out), f_band = place(sizeof(int) * n_band);
+    const size_t f_slot_off = place(sizeof(long long) * n_slot);
+    const size_t f_bw = place(sizeof(int) * n_bw), f_act_off = place(sizeof(int) * n_actoff);
+    const size_t f_act = place(sizeof(int) * n_act);
+    const size_t f_apps = place(sizeof(AppDesc) * parts.size());
+    const size_t f_cnt = place(sizeof(unsigned long long) * 8);
+    // apply totals (terms, dense terms) and the two segment counts
+    const size_t n_tot = 2 * parts.size() + 2, f_tot = place(sizeof(unsigned long long) * n_tot);
     const size_t f_ra = place(sizeof(RootApp) * root_apps.size()), f_ri = place(sizeof(RootItem) * root_items.size());
     const size_t f_rs = place(sizeof(long long) * root_slot_off.size()), f_ro = place(sizeof(int) * root_out.size());
+    const size_t f_dense = place((size_t)n_out), f_tno = place(sizeof(long long) * tn_off.size());
+    const size_t f_lv = place(sizeof(TermLevel) * levels.size());
+    const size_t up_bytes = arena;
+    const size_t f_norm = place(sizeof(double) * 8 * n_slot), f_tn = place(sizeof(double) * n_tn);
     std::vector<size_t> f_mt(parts.size());
-    for (size_t ai = 0; ai < parts.size(); ai++) f_mt[ai] = place(sizeof(double) * mtabs[ai].size());
-    if (adopt_pool) {
-        // the parts' pools must sit one after another in it
-        long long off = 0;
-        for (const PlanPart &pp : parts) {
-            if (!pp.plan->device_pool || pp.dev_pool != adopt_pool + off) {
-                err = "adopted pool does not hold the parts' pools in order";
-                delete p;
-                return -1;
-            }
-            off += pp.plan->pool_values;
-        }
-    }
+    for (size_t ai = 0; ai < parts.size(); ai++) f_mt[ai] = place(sizeof(double) * mt_size[ai]);
     unsigned char *dev = nullptr;
-    rc = plan_alloc(p, arena, &dev, err);
-    if (!rc && adopt_pool) {
-        p->pool = adopt_pool;  // owned (in bufs) only once the plan is made
-    } else if (!rc) {
-        rc = plan_alloc(p, (size_t)std::max<long long>(n_pool, 1), &p->pool, err);
-    }
+    rc = plan_alloc(p.get(), arena, &dev, err);
+    if (!rc) rc = plan_alloc(p.get(), (size_t)std::max<long long>(n_pool, 1), &p->pool, err);
     p->out_bytes = sizeof(double) * (size_t)std::max<long long>(n_out, 1) * 8 * N * N * N;
-    if (!rc) rc = plan_alloc(p, p->out_bytes / sizeof(double), &a.out_ns, err);
+    if (!rc) rc = plan_alloc(p.get(), p->out_bytes / sizeof(double), &a.out_ns, err);
     if (!rc && !root_items.empty()) {
         size_t na = 0, ny = 0;
         root_work_values(N, p->root.geo.boxes, (long long)root_items.size(), &na, &ny);
-        rc = plan_alloc(p, na, &p->root.A, err);
-        if (!rc) rc = plan_alloc(p, ny, &p->root.Y, err);
+        rc = plan_alloc(p.get(), na, &p->root.A, err);
+        if (!rc) rc = plan_alloc(p.get(), ny, &p->root.Y, err);
     }
-    if (rc) {
-        delete p;
-        return rc;
-    }
-    std::vector<unsigned char, UninitAlloc<unsigned char>> stage(arena);
+    if (rc) return rc;
+    std::vector<unsigned char, UninitAlloc<unsigned char>> stage(up_bytes), fill_stage;
     auto at = [&](size_t f) { return stage.data() + f; };
     auto put = [&](size_t f, long long off, const auto &v) {
         using T = typename std::decay_t<decltype(v)>::value_type;
         if (!v.empty()) std::memcpy(at(f) + sizeof(T) * off, v.data(), sizeof(T) * v.size());
     };
+    std::memset(at(f_cnt), 0, sizeof(unsigned long long) * 8);
+    std::memset(at(f_tot), 0, sizeof(unsigned long long) * n_tot);
+    std::memset(at(f_dense), 0, (size_t)n_out);
     long long o_out = 0, o_band = 0, o_slot = 0, o_pool = 0, o_bw = 0, o_actoff = 0, o_act = 0;
-    long long o_pseg = 0, o_fseg = n_pseg;
-    // a segment list's jobs, shifted to the batch's output numbering
-    auto put_jobs = [&](long long o_dst, const std::vector<int> &jobs, const std::vector<int> &p0,
-                        const std::vector<int> &p1, long long o_o) {
-        int *sj = reinterpret_cast<int *>(at(f_sj)) + o_dst;
-        for (size_t i = 0; i < jobs.size(); i++) sj[i] = jobs[i] + (int)(8 * o_o);
-        put(f_s0, o_dst, p0);
-        put(f_s1, o_dst, p1);
-    };
-    for (size_t ai = 0; ai < parts.size() && !rc; ai++) {
+    std::vector<PoolFill> fills;
+    for (size_t ai = 0; ai < parts.size(); ai++) {
         const PlanPart &pp = parts[ai];
         const ApplyPlan &pl = *pp.plan;
         DevOper *o = opers[ai];
@@ -1989,7 +1933,6 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
         ad.thr_floor = pl.thr_floor;
         ad.mt_d0 = mt_shape[ai].first;
         ad.mt_w = mt_shape[ai].second;
-        put(f_mt[ai], 0, mtabs[ai]);
         ad.mtab = reinterpret_cast<const double *>(dev + f_mt[ai]);
         p->apps.push_back(ad);
         const size_t no = pl.out_node.size();
@@ -2004,27 +1947,14 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
             for (size_t i = 0; i < pl.band.size(); i++) bd[i] = pl.band[i] >= 0 ? pl.band[i] + (int)o_slot : pl.band[i];
         }
         put(f_band_w, o_out, pl.band_w);
+        if (dense(pl))
+            for (int q : pl.root_q) at(f_dense)[o_out + q] = 1;
         // inputs
         {
             long long *so = reinterpret_cast<long long *>(at(f_slot_off)) + o_slot;
             for (size_t i = 0; i < pl.slot_off.size(); i++) so[i] = pl.slot_off[i] + o_pool;
         }
-        if (pl.device_pool) {
-            if (!pp.dev_pool) {
-                err = "plan part without its device pool";
-                rc = -1;
-            } else if (pl.pool_values > 0 && !adopt_pool) {
-                hipError_t e = hipMemcpyAsync(p->pool + o_pool, pp.dev_pool, sizeof(double) * pl.pool_values,
-                                              hipMemcpyDeviceToDevice, s);
-                if (e != hipSuccess) {
-                    err = std::string("pool copy: ") + hipGetErrorString(e);
-                    rc = -2;
-                }
-            }
-        } else {
-            rc = upload_at(p->pool + o_pool, pl.in_coefs, s, err);
-        }
-        put(f_norm, o_slot * 8, pl.in_norms);
+        fills.push_back(PoolFill{pp.inp, &pl, p->pool + o_pool});
         // screening tables
         put(f_bw, o_bw, pl.bw);
         {
@@ -2032,52 +1962,21 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
             for (size_t i = 0; i < pl.active_off.size(); i++) ao[i] = pl.active_off[i] + (int)o_act;
         }
         put(f_act, o_act, pl.active_terms);
-        // segments
-        p->pseg_apps.insert(p->pseg_apps.end(), pl.pseg_apps.begin(), pl.pseg_apps.end());
-        p->fseg_apps.insert(p->fseg_apps.end(), pl.fseg_apps.begin(), pl.fseg_apps.end());
-        put_jobs(o_pseg, pl.pseg_job, pl.pseg_p0, pl.pseg_p1, o_out);
-        for (size_t i = 0; i < pl.pseg_job.size(); i++) {
-            const double t = pl.out_thr[pl.pseg_job[i] >> 3];
-            p->pseg_thr.push_back(t > pl.thr_floor ? t : pl.thr_floor);  // as the kernels form thr_cls
-            p->pseg_bmin.push_back(pl.pseg_bmin[i]);
-            p->pseg_bmax.push_back(pl.pseg_bmax[i]);
-        }
-        o_pseg += (long long)pl.pseg_job.size();
-        put_jobs(o_fseg, pl.fseg_job, pl.fseg_p0, pl.fseg_p1, o_out);
-        for (size_t i = 0; i < pl.fseg_job.size(); i++) {
-            const double t = pl.out_thr[pl.fseg_job[i] >> 3];
-            p->fseg_thr.push_back(t > pl.thr_floor ? t : pl.thr_floor);
-            p->fseg_bmin.push_back(pl.fseg_bmin[i]);
-            p->fseg_bmax.push_back(pl.fseg_bmax[i]);
-        }
-        o_fseg += (long long)pl.fseg_job.size();
         o_out += (long long)no;
         o_band += (long long)pl.band.size();
         o_slot += (long long)pl.slot_off.size();
-        o_pool += pl.device_pool ? pl.pool_values : (long long)pl.in_coefs.size();
+        o_pool += pl.pool_values;
         o_bw += (long long)pl.bw.size();
         o_actoff += (long long)pl.active_off.size();
         o_act += (long long)pl.active_terms.size();
     }
-    if (!rc) {
-        std::memcpy(at(f_apps), p->apps.data(), sizeof(AppDesc) * p->apps.size());
-        std::memset(at(f_cnt), 0, sizeof(unsigned long long) * 8);
-        put(f_ra, 0, root_apps);
-        put(f_ri, 0, root_items);
-        put(f_rs, 0, root_slot_off);
-        put(f_ro, 0, root_out);
-        hipError_t e = hipMemcpyAsync(dev, stage.data(), arena, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) {
-            err = std::string("upload: ") + hipGetErrorString(e);
-            rc = -2;
-        }
-    }
-    if (rc) {
-        (void)hipStreamSynchronize(s);
-        delete p;
-        return rc;
-    }
+    put(f_apps, 0, p->apps);
+    put(f_ra, 0, root_apps);
+    put(f_ri, 0, root_items);
+    put(f_rs, 0, root_slot_off);
+    put(f_ro, 0, root_out);
+    put(f_tno, 0, tn_off);
+    put(f_lv, 0, levels);
     p->d_apps = reinterpret_cast<AppDesc *>(dev + f_apps);
     a.counters = reinterpret_cast<unsigned long long *>(dev + f_cnt);
     a.out_depth = reinterpret_cast<const int *>(dev + f_out_depth);
@@ -2091,10 +1990,85 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
     a.bw = reinterpret_cast<const int *>(dev + f_bw);
     a.act_off = reinterpret_cast<const int *>(dev + f_act_off);
     a.act_terms = reinterpret_cast<const int *>(dev + f_act);
+    a.tn = reinterpret_cast<const double *>(dev + f_tn);
+    a.tn_off = reinterpret_cast<const long long *>(dev + f_tno);
     a.apps = p->d_apps;
-    a.seg_job = reinterpret_cast<const int *>(dev + f_sj);
-    a.seg_p0 = reinterpret_cast<const int *>(dev + f_s0);
-    a.seg_p1 = reinterpret_cast<const int *>(dev + f_s1);
+    // counts per (output component, band position)
+    const bool bounds = mode != 0;
+    struct Temp {
+        DeviceCtx *c;
+        std::vector<void *> p;
+        ~Temp() {
+            // the staging buffers of a failed plan may still be read
+            (void)hipStreamSynchronize(c->stream);
+            for (void *q : p) dev_mem_put(c, q);
+        }
+    } temp{c, {}};
+    auto tmp = [&](size_t n, auto **out) {
+        const int r = dev_mem(c, n, out, err);
+        if (!r) temp.p.push_back(*out);
+        return r;
+    };
+    CountArgs ca;
+    ca.n_out = (int)n_out;
+    ca.n_app = (int)parts.size();
+    ca.n_share = (int)parts.size();
+    ca.dense = dev + f_dense;
+    ca.totals = reinterpret_cast<unsigned long long *>(dev + f_tot);
+    ca.n_seg = ca.totals + 2 * parts.size();
+    if ((rc = tmp((size_t)(8 * n_band), &ca.cnt))) return rc;
+    if (bounds && ((rc = tmp((size_t)(8 * n_band), &ca.bmin)) || (rc = tmp((size_t)(8 * n_band), &ca.bmax)))) return rc;
+    HIP_TRY(hipMemcpyAsync(dev, stage.data(), up_bytes, hipMemcpyHostToDevice, s));
+    rc = dev_pool_fill(c, mra, fills, reinterpret_cast<double *>(dev + f_norm), fill_stage, err);
+    if (!rc)
+        rc = dev_term_tables(s, a, reinterpret_cast<const TermLevel *>(dev + f_lv), (int)levels.size(),
+                             reinterpret_cast<double *>(dev + f_tn), err);
+    ca.k = a;
+    if (!rc) rc = dev_count_terms(s, ca, bounds, err);
+    if (rc) return rc;
+    // Room for the segments: what a small launch can hold and 16 (fine ones
+    // 24) for each output node; the few plans that need more are cut again.
+    std::vector<unsigned long long> tot(n_tot);
+    long long cap[2] = {2048 + 16 * n_out, bounds ? 16384 + 24 * n_out : 0};
+    int *seg = nullptr;
+    SegRec *rec = nullptr;
+    for (int attempt = 0;; attempt++) {
+        const long long n_all = cap[0] + cap[1];
+        if (n_all >= (1LL << 31)) {
+            err = "batch too large for 32-bit node, segment or slot indices";
+            return -1;
+        }
+        if ((rc = plan_alloc(p.get(), (size_t)(3 * n_all), &seg, err))) return rc;
+        if (bounds && (rc = tmp((size_t)n_all, &rec))) return rc;
+        for (int i = 0; i < 2; i++) ca.cap[i] = (int)cap[i];
+        ca.seg_job = seg;
+        ca.seg_p0 = seg + n_all;
+        ca.seg_p1 = seg + 2 * n_all;
+        ca.rec = rec;
+        if (attempt) {
+            hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, ca.n_seg, 2);
+            HIP_TRY(hipGetLastError());
+        }
+        if ((rc = dev_cut_segments(s, ca, bounds, err))) return rc;
+        HIP_TRY(hipMemcpyAsync(tot.data(), ca.totals, sizeof(unsigned long long) * n_tot, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        const long long need[2] = {(long long)tot[n_tot - 2], (long long)tot[n_tot - 1]};
+        if (need[0] <= cap[0] && need[1] <= cap[1]) {
+            p->n_pseg = (int)need[0];
+            p->n_fseg = (int)need[1];
+            break;
+        }
+        for (int i = 0; i < 2; i++) cap[i] = std::max(cap[i], need[i]);
+        p->bufs.pop_back();
+        dev_mem_put(c, seg);
+    }
+    for (size_t ai = 0; ai < parts.size(); ai++) {
+        p->term_apps += tot[2 * ai];
+        p->root.apps_count += tot[2 * ai + 1];
+    }
+    a.seg_job = ca.seg_job;
+    a.seg_p0 = ca.seg_p0;
+    a.seg_p1 = ca.seg_p1;
     if (!root_items.empty()) {
         RootLaunch &r = p->root;
         r.apps = reinterpret_cast<const RootApp *>(dev + f_ra);
@@ -2105,9 +2079,39 @@ int dev_plan_create(DeviceCtx *c, const std::vector<PlanPart> &parts, DevicePlan
         r.pool = p->pool;
         r.counter = a.counters;
     }
-    if (adopt_pool) p->bufs.push_back(adopt_pool);
-    *out = p;
+    if (bounds) {
+        // what the class lists of the mixed and split modes are chosen from,
+        // in job order (the cut leaves the jobs in the order they finished)
+        std::vector<double> thr_cls;
+        for (const PlanPart &pp : parts)
+            for (double t : pp.plan->out_thr) thr_cls.push_back(std::max(t, pp.plan->thr_floor));
+        std::vector<SegRec, UninitAlloc<SegRec>> r((size_t)p->n_pseg + p->n_fseg);
+        if (p->n_pseg)
+            HIP_TRY(hipMemcpyAsync(r.data(), ca.rec, sizeof(SegRec) * p->n_pseg, hipMemcpyDeviceToHost, s));
+        if (p->n_fseg)
+            HIP_TRY(hipMemcpyAsync(r.data() + p->n_pseg, ca.rec + cap[0], sizeof(SegRec) * p->n_fseg,
+                                   hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        auto meta = [&](const SegRec *q, int n, int first, std::vector<SegMeta> &m) {
+            std::vector<std::pair<long long, int>> order(n);  // (job, start), segment
+            for (int i = 0; i < n; i++) order[i] = {((long long)q[i].job << 32) | (unsigned)q[i].p0, i};
+            std::sort(order.begin(), order.end());
+            m.reserve(n);
+            for (const auto &o : order) {
+                const SegRec &x = q[o.second];
+                m.push_back(SegMeta{first + o.second, x.apps, thr_cls[x.job >> 3], x.lo, x.hi});
+            }
+        };
+        meta(r.data(), p->n_pseg, 0, p->psegs);
+        meta(r.data() + p->n_pseg, p->n_fseg, (int)cap[0], p->fsegs);
+    }
+    *out = p.release();
     return 0;
+}
+
+void dev_plan_counts(const DevicePlan *p, unsigned long long *term_apps, int *segments) {
+    *term_apps = p->term_apps;
+    *segments = p->n_pseg;
 }
 
 int dev_plan_set_post(DevicePlan *p, const MRA &mra,
@@ -2243,22 +2247,21 @@ static int drop_graph(DevicePlan *p, std::string &err);
 
 static int make_lists(DevicePlan *p, int mode, double tau, std::string &err) {
     if (p->list_tau == tau && p->list_mode == mode && p->list_order == p->order) return 0;
-    std::vector<int> hi, lo;
-    for (int i = 0; i < p->n_fseg; i++)
-        if (p->fseg_bmax[i] > tau * p->fseg_thr[i] * (1.0 - 1e-9)) hi.push_back(p->n_pseg + i);
+    std::vector<SegMeta> shi, slo;
+    for (const SegMeta &m : p->fsegs)
+        if (m.bmax > tau * m.thr * (1.0 - 1e-9)) shi.push_back(m);
     if (mode == 1 || mode == 2)
-        for (int i = 0; i < p->n_pseg; i++)
-            if (p->pseg_bmin[i] <= tau * p->pseg_thr[i] * (1.0 + 1e-9)) lo.push_back(i);
+        for (const SegMeta &m : p->psegs)
+            if (m.bmin <= tau * m.thr * (1.0 + 1e-9)) slo.push_back(m);
     if (p->order == 1) {
-        // largest first (segment index -> its passing-term count)
-        auto apps = [&](int sg) {
-            if (sg < p->n_pseg) return p->pseg_apps[sg];
-            return p->fseg_apps[sg - p->n_pseg];
-        };
-        auto by_cost = [&](int x, int y) { return apps(x) > apps(y); };
-        std::stable_sort(hi.begin(), hi.end(), by_cost);
-        std::stable_sort(lo.begin(), lo.end(), by_cost);
+        // largest first
+        auto by_cost = [](const SegMeta &x, const SegMeta &y) { return x.apps > y.apps; };
+        std::stable_sort(shi.begin(), shi.end(), by_cost);
+        std::stable_sort(slo.begin(), slo.end(), by_cost);
     }
+    std::vector<int> hi, lo;
+    for (const SegMeta &m : shi) hi.push_back(m.index);
+    for (const SegMeta &m : slo) lo.push_back(m.index);
     // a captured step holds the old lists
     int rc0 = drop_graph(p, err);
     if (rc0) return rc0;

@@ -250,80 +250,32 @@ struct ApplyPlan {
     std::vector<int> band_w;        // band half-width W (band has (2W+1)^3 entries)
     std::vector<int> band;          // input slot or -1, order dz,dy,dx with dx fastest
     // input slots (real or generated nodes)
-    std::vector<long long> slot_off;  // offset of the slot's block in in_coefs
-    std::vector<double, UninitAlloc<double>> in_coefs;  // pool: full blocks (real) or scaling part (generated)
-    std::vector<double> in_norms;   // slots x 8 (wavelet norms 0 for generated slots)
-    std::vector<int> in_depth;
+    std::vector<long long> slot_off;  // offset of the slot's block in the pool (full: real node, scaling part: generated)
     // screening-derived bandwidths: w[(d*M + m)*4 + c]
     std::vector<int> bw;
     std::vector<int> active_off, active_terms;  // per depth, terms with any w >= 0
     long long n_generated = 0;
-    // Work segments of the output component pairs (gt, gt | 4), gt < 4:
-    // job = 8*out + gt; a segment covers the (band position p, input
-    // component ft) pairs 8 p + ft in [pseg_p0, pseg_p1) of one job (whole
-    // band positions, except in small launches, where a band position with
-    // more terms than a segment is cut by ft).  Jobs are cut so that no
-    // segment holds many more than
-    // `seg_target` term-applications of the two components (counted exactly
-    // here with the kernels' screening rule); jobs without any are left out.
-    // The kernels share the x and y passes of a pair.  Per segment: passing
-    // terms and the smallest / largest screening bound among them (for
-    // choosing the segments of each precision class).
-    std::vector<int> pseg_job, pseg_p0, pseg_p1, pseg_apps;
-    std::vector<double> pseg_bmin, pseg_bmax;
-    // Fine segments: single-component jobs cut at about seg_target / 8
-    // passing terms, for the launch of the FP64 class of the mixed and split
-    // modes, whose terms crowd into few segments (coarse output nodes).
-    std::vector<int> fseg_job, fseg_p0, fseg_p1, fseg_apps;
-    std::vector<double> fseg_bmin, fseg_bmax;
-    long long term_apps = 0;   // exact count of term-applications in the plan
     double thr_floor = 0.0;    // smallest positive threshold of the plan
-    // A pool made on the device (build_plan with device_pool): in_coefs
-    // stays empty; slot_src[s] is the slot's input-tree node (>= 0) or
+    // Sources of the pool: slot_src[s] is the slot's input-tree node (>= 0) or
     // generated node -(g + 1); generated node g is child gen_child[g] of
     // generated node gen_parent[g] (>= 0) or of input node -(gen_parent[g]
     // + 1), in order of depth, [gen_level_off[i], gen_level_off[i + 1]) one
-    // depth; slot_off[s] is the slot's offset in the pool as before.
-    bool device_pool = false;
+    // depth.
     std::vector<int> slot_src, gen_parent, gen_child, gen_level_off;
     long long pool_values = 0;  // doubles of the pool
     // The root boxes when all of them are output nodes with threshold zero
     // (an apply's first level) and their tensor fits the dense root kernels
     // (2 (k+1) boxes <= 48 per direction): output position and input slot of
-    // each box, x fastest; else empty.  root_dense (finish_plan_counts): the
-    // roots are computed by those kernels and hold no segments, root_apps
-    // their passing term-applications.
+    // each box, x fastest; else empty.
     int boxes[3] = {0, 0, 0};
     std::vector<int> root_q, root_slot;
-    bool root_dense = false;
-    long long root_apps = 0;
 };
 
-struct ApplyStats {
-    double term_apps = 0;      // term-applications passing screening
-    double candidates = 0;     // (f, ft, gt, m) candidates examined
-    double out_nodes = 0;
-    double in_slots = 0;
-    double generated = 0;
-};
-
-// Build the plan for output nodes `nodes` of `out` with screening parameter
-// thr_param (thr_g = thr_param * prec_fac[g]).
-// With device_pool the plan stops after the slots and their sources: the
-// pool and in_norms are made on the device (dev_pool_fill), then
-// finish_plan_counts adds the exact counts and the work segments.
-// in_cnorm8: the input tree's 8 component norms per node (tree order), when
-// the caller has them; otherwise computed here.
+// Build the plan for output nodes `nodes` of `out` with thresholds thr.
+// in_cnorm8: the input tree's 8 component norms per node (tree order).
 void build_plan(ApplyPlan &plan, const Operator &op, const Tree &inp, const Tree &out,
                 const std::vector<int> &nodes, const std::vector<double> &thr,
-                int max_band_w, int seg_target = 256, bool device_pool = false,
-                const double *in_cnorm8 = nullptr);
-// fine_segments: also cut the fine single-component segments (the FP64 class
-// of the mixed and split modes; plain FP64 runs over the pair segments only).
-// n_share: the number of plans of about this size launched together (the
-// applies of a batch level), which decides whether the launch is small.
-void finish_plan_counts(ApplyPlan &plan, const Operator &op, int seg_target = 256, bool fine_segments = true,
-                        int n_share = 1);
+                int max_band_w, const double *in_cnorm8);
 double oper_norm(const Operator &op, int m, int d, int c, long long l);
 
 // Operator tables flattened for the device: per (m, d) the half-width L, the
@@ -349,12 +301,5 @@ void prepare_operator(Operator &op, const MRA &mra, double mu, double build_prec
 bool term_depth_scan(const MRA &mra, double alpha, int d, double tau, long long &Lscan, double &peak);
 // Gauss-Legendre rule of n points on [0, 1] (cached).
 void quad_rule01(int n, const double **x, const double **w);
-// Pre-screen table of an apply plan for the device screening: for each
-// output depth d in [d0, d0 + nd), component combination cmb = cx | cy << 2 |
-// cz << 4 and translation |l| <= w (the plan's widest band), the largest
-// ((N_x N_y) N_z) over the depth's active terms.  The tables of all plans of
-// a batch are built in one parallel pass over (plan, depth, cmb).
-void build_prescreens(const std::vector<const ApplyPlan *> &pls, const std::vector<const OperFlat *> &fs,
-                      std::vector<std::vector<double>> &mts, std::vector<std::pair<int, int>> &shapes);
 
 }  // namespace mwg

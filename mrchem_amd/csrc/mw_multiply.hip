@@ -833,7 +833,8 @@ __global__ __launch_bounds__(256) void k_pool_fill(int n3, const SlotItem *items
     if (lane == 0) it.norms[comp] = sqrt(q);
 }
 
-int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &jobs, std::string &err) {
+int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &jobs, double *norms,
+                  std::vector<unsigned char, UninitAlloc<unsigned char>> &stage, std::string &err) {
     if (jobs.empty()) return 0;
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
@@ -865,7 +866,7 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
         lv_at[lv + 1] = lv_at[lv] + k;
     }
     // one device allocation: [filter | gen items | slot items] (uploaded)
-    // [generated scaling blocks of every job] [every slot's norms]
+    // [generated scaling blocks of every job]
     size_t bytes = 0;
     auto place = [&](size_t b) {
         const size_t off = bytes;
@@ -875,11 +876,11 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
     const size_t f_F = place(sizeof(double) * mra.basis.F.size());
     const size_t f_gi = place(sizeof(GenItem) * n_gen), f_si = place(sizeof(SlotItem) * n_slot);
     const size_t up_bytes = bytes;
-    const size_t f_gen = place(sizeof(double) * n_gen * (size_t)n3), f_nrm = place(sizeof(double) * 8 * n_slot);
+    const size_t f_gen = place(sizeof(double) * n_gen * (size_t)n3);
     unsigned char *dev = nullptr;
     if (int rc = dev_mem(c, bytes, &dev, err)) return rc;
-    double *gen_s = reinterpret_cast<double *>(dev + f_gen), *norms = reinterpret_cast<double *>(dev + f_nrm);
-    std::vector<unsigned char, UninitAlloc<unsigned char>> stage(up_bytes);
+    double *gen_s = reinterpret_cast<double *>(dev + f_gen);
+    stage.resize(up_bytes);
     std::memcpy(stage.data() + f_F, mra.basis.F.data(), sizeof(double) * mra.basis.F.size());
     GenItem *gi = reinterpret_cast<GenItem *>(stage.data() + f_gi);
     SlotItem *si = reinterpret_cast<SlotItem *>(stage.data() + f_si);
@@ -909,7 +910,6 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
             it.len = sr >= 0 ? 8 * n3 : n3;
         }
     }
-    std::vector<double, UninitAlloc<double>> norms_h(8 * n_slot);
     const double *F = reinterpret_cast<const double *>(dev + f_F);
     const GenItem *dgi = reinterpret_cast<const GenItem *>(dev + f_gi);
     const SlotItem *dsi = reinterpret_cast<const SlotItem *>(dev + f_si);
@@ -923,18 +923,11 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
         hipLaunchKernelGGL(k_pool_fill, dim3((unsigned)(2 * n_slot)), dim3(256), 0, s, n3, dsi, (int)n_slot);
         e = hipGetLastError();
     }
-    if (e == hipSuccess && n_slot > 0)
-        e = hipMemcpyAsync(norms_h.data(), norms, sizeof(double) * 8 * n_slot, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    // (put back at once: its next holder's work comes after these launches)
     dev_mem_put(c, dev);
     if (e != hipSuccess) {
         err = std::string("pool fill: ") + hipGetErrorString(e);
         return -2;
-    }
-    for (size_t i = 0; i < nj; i++) {
-        ApplyPlan &pl = *jobs[i].pl;
-        const size_t cnt = pl.slot_src.size() * 8;
-        if (cnt) std::memcpy(pl.in_norms.data(), norms_h.data() + slot_at[i] * 8, sizeof(double) * cnt);
     }
     return 0;
 }

@@ -445,78 +445,21 @@ struct InputBlocks {
     }
 };
 
-// The device pools of one plan's parts, one after another in one
-// allocation (the device plan adopts it; freed here otherwise).
-struct LevelPool {
-    DeviceCtx *c;
-    double *base = nullptr;
-    std::vector<double *> parts;
-    ~LevelPool() { dev_free(c, base); }
-    double *release() {
-        double *b = base;
-        base = nullptr;
-        return b;
-    }
-};
-
-// Host plans of `active` (in parallel across applies when there are several;
-// build_plan parallelises internally otherwise), their pools made on the
-// device from the input trees' blocks into one allocation, then the exact
-// counts and segments (the fine single-component ones only for a mode with
-// an FP64 class beside a low-precision one).
-void build_plans(mwg_context ctx, std::vector<Job *> &active, const std::vector<std::vector<int>> &nodes,
-                 const std::vector<std::vector<double>> &thr, InputBlocks &inputs, LevelPool &pools, int mode,
-                 double *ms3 = nullptr) {
+// Host plans of `active`, in parallel across applies when there are several.
+void build_plans(std::vector<Job *> &active, const std::vector<std::vector<int>> &nodes,
+                 const std::vector<std::vector<double>> &thr) {
     const int n = (int)active.size();
-    const double t0 = now_ms();
 #pragma omp parallel for num_threads(team_size()) schedule(dynamic, 1) if (n > 1)
     for (int i = 0; i < n; i++) {
         Job &j = *active[i];
         try {
-            build_plan(j.plan, j.op->op, *j.inp, j.out->tree, nodes[i], thr[i], 64, 256, true, j.inp_cn8);
+            build_plan(j.plan, j.op->op, *j.inp, j.out->tree, nodes[i], thr[i], 64, j.inp_cn8);
         } catch (const std::exception &e) {
             j.err = e.what();
         }
     }
     for (Job *j : active)
         if (!j->err.empty()) throw std::runtime_error(j->err);
-    const double t1 = now_ms();
-    const MRA &mra = *active[0]->out->tree.mra;
-    {
-        size_t total = 0;
-        for (Job *j : active) total += (size_t)j->plan.pool_values;
-        std::string err;
-        dev_free(pools.c, pools.base);
-        pools.base = nullptr;
-        dev_check(dev_alloc(pools.c, total, &pools.base, err), err);
-        pools.parts.assign(n, nullptr);
-        std::vector<PoolFill> fills(n);
-        size_t off = 0;
-        for (int i = 0; i < n; i++) {
-            Job &j = *active[i];
-            pools.parts[i] = pools.base + off;
-            off += (size_t)j.plan.pool_values;
-            fills[i] = PoolFill{inputs.of(ctx, j.inp_h), &j.plan, pools.parts[i]};
-        }
-        dev_check(dev_pool_fill(ctx->dev, mra, fills, err), err);
-    }
-    const double t2 = now_ms();
-#pragma omp parallel for num_threads(team_size()) schedule(dynamic, 1) if (n > 1)
-    for (int i = 0; i < n; i++) {
-        Job &j = *active[i];
-        try {
-            finish_plan_counts(j.plan, j.op->op, 256, mode != MWG_MODE_FP64, n);
-        } catch (const std::exception &e) {
-            j.err = e.what();
-        }
-    }
-    for (Job *j : active)
-        if (!j->err.empty()) throw std::runtime_error(j->err);
-    if (ms3) {
-        ms3[0] += t1 - t0;
-        ms3[1] += t2 - t1;
-        ms3[2] += now_ms() - t2;
-    }
 }
 
 // Adaptive applies with mrcpp::apply semantics per job; every refinement
@@ -563,7 +506,7 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
     double kms = 0.0, pms = 0.0, slots = 0.0, gen = 0.0, computed = 0.0, apps_total = 0.0;
     double t_dev = 0.0, t_split = 0.0;  // device plan create + run + download; host split checks
     double t_create = 0.0, t_run = 0.0;  // parts of t_dev: plan creation, run (both host wall time)
-    double plan3[3] = {0.0, 0.0, 0.0};   // parts of the plan time: grids and bands, device pools, counts
+    double t_inp = 0.0;                  // uploads of host input trees
     const double t_all = now_ms();
     int launches = 0;
     // Every level's output blocks stay on the device until the post
@@ -594,14 +537,14 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
                 thr[a][q] = j.prec * prec_factor(j.prec_trees, j.out->tree.keys[j.work[q]]) * std::sqrt(Nsq / M);
         }
         const double t0 = now_ms();
-        LevelPool pools{ctx->dev};
-        build_plans(ctx, active, nodes, thr, inputs, pools, ctx->mode, plan3);
+        build_plans(active, nodes, thr);
         pms += now_ms() - t0;
+        const double t0i = now_ms();
         std::vector<PlanPart> parts;
         size_t total = 0;
         for (size_t a = 0; a < active.size(); a++) {
             Job *j = active[a];
-            parts.push_back(PlanPart{j->op, &j->op->flat, &j->plan, pools.parts[a]});
+            parts.push_back(PlanPart{j->op, &j->op->flat, &j->plan, inputs.of(ctx, j->inp_h)});
             slots += (double)j->plan.slot_off.size();
             gen += (double)j->plan.n_generated;
             total += j->work.size();
@@ -609,9 +552,9 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         std::string err;
         DevicePlan *dp = nullptr;
         const double t1 = now_ms();
-        int rc = dev_plan_create(ctx->dev, parts, &dp, err, pools.base);
+        t_inp += t1 - t0i;
+        int rc = dev_plan_create(ctx->dev, mra, parts, ctx->mode, &dp, err);
         if (rc) return dev_fail(rc, err);
-        pools.release();  // the plan owns the pool now
         const double t1r = now_ms();
         t_create += t1r - t1;
         double ms = 0.0;
@@ -647,7 +590,6 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         for (int a = 0; a < na; a++) {
             Job &j = *active[a];
             try {
-                // j.plan stays: the next level's build reuses its pool storage
                 Tree &o = j.out->tree;
                 std::vector<NodeLoc> &loc = locs[&j - jobs.data()];
                 const int max_depth = std::min(mra.max_depth, j.op->op.max_depth);
@@ -789,9 +731,9 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
     st[10] = now_ms() - t_all;
     st[11] = t_create;
     st[12] = t_run;
-    st[13] = plan3[0];
-    st[14] = plan3[1];
-    st[15] = plan3[2];
+    st[13] = pms;
+    st[14] = t_inp;
+    st[15] = 0.0;
     return MWG_OK;
 }
 
@@ -828,17 +770,14 @@ int make_plan(mwg_context ctx, int n, const mwg_tree *out, const mwg_operator *o
     }
     const double t0 = now_ms();
     InputBlocks inputs(ctx);
-    LevelPool pools{ctx->dev};
-    build_plans(ctx, active, nodes, th, inputs, pools, mode);
+    build_plans(active, nodes, th);
     p->plan_ms = now_ms() - t0;
     std::vector<PlanPart> parts;
     for (int i = 0; i < n; i++) {
         const ApplyPlan &ap = jobs[i].plan;
-        parts.push_back(PlanPart{op[i], &op[i]->flat, &ap, pools.parts[i]});
+        parts.push_back(PlanPart{op[i], &op[i]->flat, &ap, inputs.of(ctx, inp[i])});
         p->slots += (double)ap.slot_off.size();
         p->gen += (double)ap.n_generated;
-        p->host_apps += (double)ap.term_apps;
-        p->segs += (double)ap.pseg_job.size();
         for (int w : ap.band_w) p->band_w = std::max(p->band_w, (double)w);
         p->outs.push_back(out[i]);
         p->ops.push_back(op[i]);
@@ -848,9 +787,15 @@ int make_plan(mwg_context ctx, int n, const mwg_tree *out, const mwg_operator *o
     }
     p->thr = std::move(th);
     std::string err;
-    int rc = dev_plan_create(ctx->dev, parts, &p->dev, err, pools.base);
+    int rc = dev_plan_create(ctx->dev, *out[0]->tree.mra, parts, mode, &p->dev, err);
     if (rc) return dev_fail(rc, err);
-    pools.release();  // the plan owns the pool now
+    {
+        unsigned long long apps = 0;
+        int segs = 0;
+        dev_plan_counts(p->dev, &apps, &segs);
+        p->host_apps = (double)apps;
+        p->segs = (double)segs;
+    }
     {
         // (branch, first child) pairs of every output grid, by depth, as
         // indices into the plan's concatenated output nodes
