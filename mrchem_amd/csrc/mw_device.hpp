@@ -94,6 +94,13 @@ struct OpBuildJob {
     OperFlat *flat;
     const void *key;
 };
+// Largest error |fit - K| r of every candidate fit on its grid of kFitPoints
+// points (kernel_fit_error on the device).
+struct FitCand {
+    const std::vector<GaussTerm> *terms;
+    double mu, r_min, r_max;
+};
+int dev_fit_errors(DeviceCtx *c, const std::vector<FitCand> &cands, std::vector<double> &errs, std::string &err);
 int dev_build_operators(DeviceCtx *c, const MRA &mra, const std::vector<OpBuildJob> &jobs, std::string &err);
 // Copy the device table of a device-built operator (f.device_blocks values).
 int dev_download_operator_blocks(DeviceCtx *c, const void *key, double *out, long long n, std::string &err);

@@ -85,6 +85,11 @@ struct GaussTerm {
 // mu > 0 gives exp(-mu r)/r.
 std::vector<GaussTerm> fit_kernel(double mu, double eps, double r_min, double r_max,
                                   double *achieved_err = nullptr);
+// The fit's search: step sizes 0.6 x 0.93^step, the first whose largest error
+// |fit - K| r over kFitPoints log-spaced points is at most eps / 2.
+constexpr int kFitSteps = 60, kFitPoints = 3000;
+std::vector<GaussTerm> kernel_terms(int step, double mu, double eps, double r_min, double r_max);
+void check_fit(double mu, double eps, double r_min, double r_max);
 double kernel_fit_error(const std::vector<GaussTerm> &t, double mu, double r_min, double r_max,
                         int npts);
 
@@ -295,6 +300,10 @@ double operator_tau(double build_prec);
 // Operator header without tables: world extent, kernel fit and the terms
 // (alpha, beta, coef1d), each with max_depth + 1 empty depths.
 void prepare_operator(Operator &op, const MRA &mra, double mu, double build_prec, int max_depth);
+// Its two parts: everything but the fit (the kernel is to be fitted to
+// build_prec / 10 on [r_min, r_max]), and the terms of a fit.
+void prepare_header(Operator &op, const MRA &mra, double mu, double build_prec, int max_depth);
+void set_terms(Operator &op, const std::vector<GaussTerm> &g, double fit_err);
 // Translation scan of one (term, depth): false when the depth stores nothing;
 // otherwise the scan bound Lscan and the position `peak` after which three
 // quiet translations end the scan.

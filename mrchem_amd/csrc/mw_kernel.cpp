@@ -97,18 +97,26 @@ double kernel_fit_error(const std::vector<GaussTerm> &t, double mu, double r_min
     return err;
 }
 
-std::vector<GaussTerm> fit_kernel(double mu, double eps, double r_min, double r_max, double *achieved_err) {
+std::vector<GaussTerm> kernel_terms(int step, double mu, double eps, double r_min, double r_max) {
+    double h = 0.6;
+    for (int it = 0; it < step; it++) h *= 0.93;
+    return make_terms(h, mu, eps, r_min, r_max);
+}
+
+void check_fit(double mu, double eps, double r_min, double r_max) {
     if (!(eps > 0 && eps < 1)) throw std::invalid_argument("fit_kernel: eps must be in (0,1)");
     if (!(r_min > 0 && r_max > r_min)) throw std::invalid_argument("fit_kernel: need 0 < r_min < r_max");
     if (mu < 0) throw std::invalid_argument("fit_kernel: mu must be >= 0");
-    double h = 0.6;
+}
+
+std::vector<GaussTerm> fit_kernel(double mu, double eps, double r_min, double r_max, double *achieved_err) {
+    check_fit(mu, eps, r_min, r_max);
     std::vector<GaussTerm> terms;
     double err = 1e300;
-    for (int it = 0; it < 60; it++) {
-        terms = make_terms(h, mu, eps, r_min, r_max);
-        err = kernel_fit_error(terms, mu, r_min, r_max, 3000);
+    for (int it = 0; it < kFitSteps; it++) {
+        terms = kernel_terms(it, mu, eps, r_min, r_max);
+        err = kernel_fit_error(terms, mu, r_min, r_max, kFitPoints);
         if (err <= 0.5 * eps) break;
-        h *= 0.93;
     }
     if (err > eps) throw std::runtime_error("fit_kernel: requested accuracy not reached");
     if (achieved_err) *achieved_err = err;

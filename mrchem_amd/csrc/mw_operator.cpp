@@ -196,7 +196,7 @@ bool term_depth_scan(const MRA &mra, double alpha, int d, double tau, long long 
 
 double operator_tau(double build_prec) { return std::min(1e-10, 1e-4 * build_prec); }
 
-void prepare_operator(Operator &op, const MRA &mra, double mu, double build_prec, int max_depth) {
+void prepare_header(Operator &op, const MRA &mra, double mu, double build_prec, int max_depth) {
     if (!(build_prec > 0)) throw std::invalid_argument("operator build precision must be > 0");
     if (max_depth < 0 || max_depth > mra.max_depth) max_depth = mra.max_depth;
     op.mra = &mra;
@@ -212,14 +212,24 @@ void prepare_operator(Operator &op, const MRA &mra, double mu, double build_prec
     double k_prec = build_prec / 10.0;
     double h_min = mra.box_size(mra.max_depth);
     op.r_min = std::sqrt(k_prec * h_min);
-    std::vector<GaussTerm> g = fit_kernel(mu, k_prec, op.r_min, op.r_max, &op.fit_err);
+}
+
+void set_terms(Operator &op, const std::vector<GaussTerm> &g, double fit_err) {
+    op.fit_err = fit_err;
     op.terms.assign(g.size(), OperTerm());
     for (size_t m = 0; m < g.size(); m++) {
         op.terms[m].alpha = g[m].alpha;
         op.terms[m].beta = g[m].beta;
         op.terms[m].coef1d = std::cbrt(g[m].beta);
-        op.terms[m].depth.assign(max_depth + 1, OperDepth());
+        op.terms[m].depth.assign(op.max_depth + 1, OperDepth());
     }
+}
+
+void prepare_operator(Operator &op, const MRA &mra, double mu, double build_prec, int max_depth) {
+    prepare_header(op, mra, mu, build_prec, max_depth);
+    double err = 0.0;
+    const std::vector<GaussTerm> g = fit_kernel(mu, build_prec / 10.0, op.r_min, op.r_max, &err);
+    set_terms(op, g, err);
 }
 
 void flatten_operator(const Operator &op, OperFlat &f) {

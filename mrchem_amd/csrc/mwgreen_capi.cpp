@@ -1057,18 +1057,63 @@ int mwg_operators_create_device(mwg_context ctx, mwg_mra mra, int n, const doubl
             if (!(mu[i] >= 0.0) || !std::isfinite(mu[i])) return fail(MWG_ERR_ARG, "mu must be finite and >= 0");
         std::vector<std::unique_ptr<mwg_operator_s>> made(n);
         for (int i = 0; i < n; i++) made[i].reset(new mwg_operator_s);
-        // kernel fits, one per operator, in parallel
-        std::vector<std::string> fit_err(n);
-#pragma omp parallel for num_threads(team_size()) schedule(dynamic, 1)
+        // Kernel fits: the terms of a run of step sizes of every operator on
+        // the host, in parallel, their errors on the device, until every
+        // operator has its first step within eps / 2.  An error that the
+        // device's rounding could put on the other side (both are sums of
+        // some hundred terms of total 1: within 1e-12, with room) is decided
+        // by the host's value.
+        const double eps = build_prec / 10.0;
+        std::vector<int> open;
         for (int i = 0; i < n; i++) {
-            try {
-                prepare_operator(made[i]->op, mra->mra, mu[i], build_prec, mra->mra.max_depth);
-            } catch (const std::exception &e) {
-                fit_err[i] = e.what();
-            }
+            prepare_header(made[i]->op, mra->mra, mu[i], build_prec, mra->mra.max_depth);
+            check_fit(mu[i], eps, made[i]->op.r_min, made[i]->op.r_max);
+            open.push_back(i);
         }
-        for (int i = 0; i < n; i++)
-            if (!fit_err[i].empty()) return fail(MWG_ERR_ARG, fit_err[i]);
+        constexpr int kRun = 15;
+        for (int s0 = 0; s0 < kFitSteps && !open.empty(); s0 += kRun) {
+            const int no = (int)open.size();
+            std::vector<std::vector<GaussTerm>> terms((size_t)no * kRun);
+            std::vector<std::string> fit_err((size_t)no * kRun);
+#pragma omp parallel for num_threads(team_size()) schedule(dynamic, 1)
+            for (int e = 0; e < no * kRun; e++) {
+                const Operator &op = made[open[e / kRun]]->op;
+                try {
+                    terms[e] = kernel_terms(s0 + e % kRun, op.mu, eps, op.r_min, op.r_max);
+                } catch (const std::exception &x) {
+                    fit_err[e] = x.what();
+                }
+            }
+            for (const std::string &x : fit_err)
+                if (!x.empty()) return fail(MWG_ERR_ARG, x);
+            std::vector<FitCand> cands;
+            for (int e = 0; e < no * kRun; e++) {
+                const Operator &op = made[open[e / kRun]]->op;
+                cands.push_back(FitCand{&terms[e], op.mu, op.r_min, op.r_max});
+            }
+            std::vector<double> errs;
+            std::string err;
+            dev_check(dev_fit_errors(ctx->dev, cands, errs, err), err);
+            std::vector<int> left;
+            for (int q = 0; q < no; q++) {
+                Operator &op = made[open[q]]->op;
+                bool done = false;
+                for (int k = 0; k < kRun && !done; k++) {
+                    const int e = q * kRun + k;
+                    double x = errs[e];
+                    if (std::fabs(x - 0.5 * eps) <= 1e-12)
+                        x = kernel_fit_error(terms[e], op.mu, op.r_min, op.r_max, kFitPoints);
+                    // the last step is taken up to eps
+                    if (x <= 0.5 * eps || (s0 + k == kFitSteps - 1 && x <= eps)) {
+                        set_terms(op, terms[e], x);
+                        done = true;
+                    }
+                }
+                if (!done) left.push_back(open[q]);
+            }
+            open.swap(left);
+        }
+        if (!open.empty()) return fail(MWG_ERR_ARG, "fit_kernel: requested accuracy not reached");
         std::vector<OpBuildJob> jobs;
         for (int i = 0; i < n; i++) {
             made[i]->dev_ctx = ctx;
