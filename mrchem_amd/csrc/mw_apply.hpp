@@ -50,11 +50,15 @@ struct KArgs {
     const int *act_off, *act_terms;
     const double *tn;
     const long long *tn_off;
+    // per active term (as act_terms): block id of component 0 at translation
+    // 0, and the distance of two components' blocks
+    const int2 *tb;
     const AppDesc *apps;
     // [0] term-applications passing screening (algorithmic work)
     unsigned long long *counters;
-    // work segments: job = 8*out + gt, (band position p, input component ft)
-    // pairs 8 p + ft in [p0, p1)
+    // work segments: job = 8*out + gt, [p0, p1) with ends (8 p + ft) << 12 | e:
+    // from active term e of the pair of band position p and input component ft
+    // (e = 0 but in plain FP64)
     const int *seg_job, *seg_p0, *seg_p1;
 };
 
@@ -92,9 +96,11 @@ struct CountArgs {
     int *seg_job = nullptr, *seg_p0 = nullptr, *seg_p1 = nullptr;
     SegRec *rec = nullptr;  // with bounds
 };
-// Norm and pre-screen tables of levels[0, n) (device array); mtab of each
-// apply is written through apps[app].mtab.  Launches only, on stream.
-int dev_term_tables(hipStream_t s, const KArgs &k, const TermLevel *levels, int n, double *tn, std::string &err);
+// Norm, block and pre-screen tables of levels[0, n) (device array), nn the
+// values of an operator block; mtab of each apply is written through
+// apps[app].mtab.  Launches only, on stream.
+int dev_term_tables(hipStream_t s, const KArgs &k, int nn, const TermLevel *levels, int n, double *tn, int2 *tb,
+                    std::string &err);
 // Counts per position (bounds: the class bounds too), then the segments.
 // Launches only, on stream.
 int dev_count_terms(hipStream_t s, const CountArgs &c, bool bounds, std::string &err);

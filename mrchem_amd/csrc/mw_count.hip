@@ -32,13 +32,19 @@ namespace {
 
 // 1D norms of one depth's active terms, [c][l + w][term] (term fastest, so
 // that a wave with one term per lane reads whole lines): zero outside the
-// term's bandwidth and stored width.  One workgroup per (level, component).
-__global__ __launch_bounds__(256) void k_term_norms(KArgs a, const TermLevel *levels, double *tn) {
+// term's bandwidth and stored width; and where its blocks lie.  One workgroup per (level, component).
+__global__ __launch_bounds__(256) void k_term_norms(KArgs a, int nn, const TermLevel *levels, double *tn,
+                                                    int2 *tb) {
     const TermLevel lv = levels[blockIdx.x];
     const int c = blockIdx.y, nl = 2 * lv.w + 1;
     if (lv.na == 0) return;
     const AppDesc &ad = a.apps[lv.app];
     double *dst = tn + lv.tn + (long long)c * nl * lv.na;
+    if (c == 0)
+        for (int ai = threadIdx.x; ai < lv.na; ai += 256) {
+            const int m = a.act_terms[lv.a0 + ai], L = ad.opL[m * ad.ndepth + lv.d];
+            tb[lv.a0 + ai] = int2{(int)(ad.op_boff[m * ad.ndepth + lv.d] / nn) + L, 2 * L + 1};
+        }
     for (int e = threadIdx.x; e < nl * lv.na; e += 256) {
         const int li = e / lv.na, ai = e % lv.na, l = li - lv.w;
         const int m = a.act_terms[lv.a0 + ai];
@@ -101,22 +107,30 @@ __device__ __forceinline__ NodeView node_view(const KArgs &a, int q) {
     return v;
 }
 
-// Passing terms of output component gt from input component ft (norm fn) of
-// band position p, counted by the whole wave (one term per lane); the
-// smallest and largest passing bound are folded into this lane's lo and hi.
-__device__ __forceinline__ int pair_terms(const NodeView &v, int gt, int p, int ft, double fn, int lane, double &lo,
-                                          double &hi) {
+// The norms of the three directions for output component gt and input
+// component ft of band position p, one value per active term.
+struct PairNorms {
+    const double *nx, *ny, *nz;
+};
+__device__ __forceinline__ PairNorms pair_norms(const NodeView &v, int gt, int p, int ft) {
     const int lx = p % v.side, ly = (p / v.side) % v.side, lz = p / (v.side * v.side);
     const int cx = 2 * (gt & 1) + (ft & 1), cy = (gt & 2) + ((ft >> 1) & 1), cz = 2 * (gt >> 2) + (ft >> 2);
-    const double *nx = v.tn + (long long)(cx * v.side + lx) * v.na;
-    const double *ny = v.tn + (long long)(cy * v.side + ly) * v.na;
-    const double *nz = v.tn + (long long)(cz * v.side + lz) * v.na;
+    return PairNorms{v.tn + (long long)(cx * v.side + lx) * v.na, v.tn + (long long)(cy * v.side + ly) * v.na,
+                     v.tn + (long long)(cz * v.side + lz) * v.na};
+}
+
+// Passing terms of the pair (norm fn of ft), counted by the whole wave (one
+// term per lane); the smallest and largest passing bound are folded into this
+// lane's lo and hi.
+__device__ __forceinline__ int pair_terms(const NodeView &v, int gt, int p, int ft, double fn, int lane, double &lo,
+                                          double &hi) {
+    const PairNorms n = pair_norms(v, gt, p, ft);
     int c = 0;
     for (int e0 = 0; e0 < v.na; e0 += 64) {
         const int e = e0 + lane;
         bool pass = false;
         if (e < v.na) {
-            const double b = ((nx[e] * ny[e]) * nz[e]) * fn;
+            const double b = ((n.nx[e] * n.ny[e]) * n.nz[e]) * fn;
             pass = b > v.thr;
             if (pass) {
                 lo = fmin(lo, b);
@@ -209,13 +223,20 @@ __global__ __launch_bounds__(512) void k_count(CountArgs c) {
 // Segment cut of one output node: one wave per job, the pair (gt, gt | 4)
 // (PAIR) or one component.  The positions are taken in order and a segment
 // closes at the first that brings it to the target; segments without passing
-// terms are left out.  Where `split` says so (below) a position holding more
-// than a segment is cut inside, at input-component boundaries.  Lane i
-// keeps the i-th segment found; every 64 and at the end the wave takes places
-// for them with one atomic and writes them side by side.
+// terms are left out.  A segment's ends are (8 p + ft) << 12 | term.  In the
+// mixed and split modes (BOUNDS) a small launch also cuts a position that
+// holds more than a segment at input-component boundaries.  Plain FP64 always
+// does, and inside a component at every 16th term: a (position, component)
+// pair of a coarse node holds all the depth's terms, and one wave working
+// through a hundred of them alone was the end of every level's launch.  (The
+// low-precision classes sum a segment in 32 bits and keep their segments.)
+// Lane i keeps the i-th segment found; every 64 and at the end the wave takes
+// places for them with one atomic and writes them side by side.
 constexpr int kSegTarget = 256;      // passing terms of a segment
 constexpr int kSegFloor = 32;        // the least in a small launch
 constexpr int kSegWanted = 2048;     // segments a small launch is cut into
+// plain FP64, whose segments are single waves (2048 of them resident)
+constexpr int kSegTarget64 = 64, kSegFloor64 = 16, kSegWanted64 = 8192;
 
 template <bool PAIR, bool BOUNDS>
 __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
@@ -226,14 +247,10 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
     const int app = a.out_app[v.q], kind = PAIR ? 0 : 1;
     // A launch with fewer than kSegWanted x kSegTarget passing terms (this
     // apply's count times the applies that share it) is cut into about
-    // kSegWanted segments, so that it still has work for every compute unit
-    // (one k = 9 apply, level kernels 12.8 -> 8.7 ms).
+    // kSegWanted segments, so that it still has work for every compute unit.
     const unsigned long long launch = (c.totals[2 * app] - c.totals[2 * app + 1]) * (unsigned long long)c.n_share;
-    const int whole = (int)min((unsigned long long)kSegTarget, max((unsigned long long)kSegFloor, launch / kSegWanted));
-    // positions above the target are cut inside in a small launch, and always
-    // in plain FP64 (no bounds), where a coarse node's position of thousands
-    // of terms taken late from the queue would end alone; the low-precision
-    // classes sum a segment in 32 bits and keep their segments
+    const unsigned long long most = BOUNDS ? kSegTarget : kSegTarget64, least = BOUNDS ? kSegFloor : kSegFloor64;
+    const int whole = (int)min(most, max(least, launch / (BOUNDS ? kSegWanted : kSegWanted64)));
     const bool split = !BOUNDS || whole < kSegTarget;
     const int target = PAIR ? whole : max(1, whole / 8);
     const int *c0 = c.cnt + 8 * a.band_off[v.q] + (long long)gt * v.nb, *c1 = c0 + 4LL * v.nb;
@@ -256,7 +273,7 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
         }
         n = 0;
     };
-    auto close = [&](int u1) {
+    auto close = [&](int u1) {  // u1 = end << 12 | term
         if (acc > 0) {
             if (lane == n) {
                 my_p0 = u0;
@@ -289,6 +306,26 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
                 for (int ft = 0; ft < 8; ft++) {
                     if (!((cm >> ft) & 0x101)) continue;
                     const double fn = __shfl(fl, ft);
+                    if constexpr (!BOUNDS) {
+                        const bool p0 = (cm >> ft) & 1, p1 = PAIR && ((cm >> (8 + ft)) & 1);
+                        const PairNorms q = pair_norms(v, gt, p, ft);
+                        const double *nz1 = q.nz + (long long)2 * v.side * v.na;
+                        for (int b0 = 0; b0 < v.na; b0 += 64) {
+                            const int e = b0 + lane;
+                            const bool in = e < v.na;
+                            const double xy = in ? q.nx[e] * q.ny[e] : 0.0;
+                            const unsigned long long m0 = __ballot(in && p0 && (xy * q.nz[in ? e : 0]) * fn > v.thr);
+                            const unsigned long long m1 = __ballot(in && p1 && (xy * nz1[in ? e : 0]) * fn > v.thr);
+                            for (int sb = 0; sb < 64; sb += 16) {
+                                acc += __popcll((m0 >> sb) & 0xffff) + __popcll((m1 >> sb) & 0xffff);
+                                if (acc >= target) {
+                                    const bool end = b0 + sb + 16 >= v.na;
+                                    close(((8 * p + ft + (end ? 1 : 0)) << 12) | (end ? 0 : b0 + sb + 16));
+                                }
+                            }
+                        }
+                        continue;
+                    }
                     double l = HUGE_VAL, h = 0.0;
                     int t = 0;
                     if ((cm >> ft) & 1) t = pair_terms(v, gt, p, ft, fn, lane, l, h);
@@ -298,7 +335,7 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
                     acc += t;
                     lo = fmin(lo, l);
                     hi = fmax(hi, h);
-                    if (acc >= target) close(8 * p + ft + 1);
+                    if (acc >= target) close((8 * p + ft + 1) << 12);
                 }
             } else {
                 acc += pc;
@@ -306,19 +343,20 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
                     lo = fmin(lo, PAIR ? fmin(l0[p], l0[4 * v.nb + p]) : l0[p]);
                     hi = fmax(hi, PAIR ? fmax(h0[p], h0[4 * v.nb + p]) : h0[p]);
                 }
-                if (acc >= target) close(8 * (p + 1));
+                if (acc >= target) close((8 * (p + 1)) << 12);
             }
         }
     }
-    close(8 * v.nb);
+    close((8 * v.nb) << 12);
     if (n > 0) flush();
 }
 
 }  // namespace
 
-int dev_term_tables(hipStream_t s, const KArgs &k, const TermLevel *levels, int n, double *tn, std::string &err) {
+int dev_term_tables(hipStream_t s, const KArgs &k, int nn, const TermLevel *levels, int n, double *tn, int2 *tb,
+                    std::string &err) {
     if (n == 0) return 0;
-    hipLaunchKernelGGL(k_term_norms, dim3(n, 4), dim3(256), 0, s, k, levels, tn);
+    hipLaunchKernelGGL(k_term_norms, dim3(n, 4), dim3(256), 0, s, k, nn, levels, tn, tb);
     HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(k_prescreen, dim3(n, 64), dim3(256), 0, s, k, levels);
     HIP_TRY(hipGetLastError());

@@ -34,19 +34,8 @@ namespace mwg {
 
 constexpr int kMaxActive = 4096;
 
-template <typename T>
-__device__ __forceinline__ const T *op_blocks(const AppDesc &ad);
-template <>
-__device__ __forceinline__ const double *op_blocks<double>(const AppDesc &ad) {
-    return ad.blk64;
-}
-template <>
-__device__ __forceinline__ const float *op_blocks<float>(const AppDesc &ad) {
-    return ad.blk32;
-}
-
-// One workgroup per job (output node g, output component gt, or the pair of
-// components gt and gt | 4 of a pair job); its NW waves share the job's
+// The FP32 class of the mixed mode.  One workgroup per pair job (output node
+// g, output components gt and gt | 4, gt < 4); its NW waves share the job's
 // 16-wide tiles (TW tiles each).
 //
 // Screening: the active terms of the job's depth are taken in chunks of 64
@@ -58,11 +47,10 @@ __device__ __forceinline__ const float *op_blocks<float>(const AppDesc &ad) {
 // gives the surviving terms, which are appended to an LDS worklist of
 // (band node, ft, term) items.  A term is taken by this launch when it
 // passes the reference rule (bound > thr) and falls in the launch's bound
-// class (bound > lo*thr and not bound > hi*thr), so launches with disjoint
-// classes together apply exactly the oracle's term set.
+// class (bound <= hi*thr), so launches with disjoint classes together apply
+// exactly the oracle's term set.
 //
-// Application: each item is three chains of 16x16x4 MFMAs in the launch's
-// arithmetic T (FP64 or FP32):
+// Application: each item is three chains of 16x16x4 FP32 MFMAs:
 //   x: X[(jz,jy)][ix]  = F[(jz,jy)][jx] . Ox^T[jx][ix]   F tiles in registers
 //   y: Y[iy][(jz,ix)]  = Oy[iy][jy] . X'[jy][(jz,ix)]
 //   z: acc[iz][(iy,ix)] += Oz[iz][jz] . Y''[jz][(iy,ix)]  acc tiles persist
@@ -71,35 +59,18 @@ __device__ __forceinline__ const float *op_blocks<float>(const AppDesc &ad) {
 // accumulators): 4 chains instead of 6 when both pass.
 // X and Y change layout through one padded LDS buffer (two at N >= 11)
 // whose lane addresses are a base plus a compile-time offset (padding
-// entries stay zero or finite and only meet zero operands).  While an item computes, the operator blocks
-// of the next item are loaded (registers, then a double-buffered LDS stage)
-// and, when the next item starts a new (f, ft) group, its F tiles too (into
-// the F registers, which the x chain no longer needs, during the y and z
-// chains).
+// entries stay zero or finite and only meet zero operands).  While an item
+// computes, the operator blocks of the next item are loaded (registers, then
+// a double-buffered LDS stage) and, when the next item starts a new (f, ft)
+// group, its F tiles too (into the F registers, which the x chain no longer
+// needs, during the y and z chains).
 // MFMA lane layouts (checked on gfx950): A[i][k] in lane i + 16k, B[k][j] in
-// lane j + 16k; FP64 D[i][j] in lane j + 16 (i mod 4), register i / 4; FP32
-// D[i][j] in lane j + 16 (i / 4), register i mod 4.
-typedef double mwg_double4 __attribute__((ext_vector_type(4)));
+// lane j + 16k, D[i][j] in lane j + 16 (i / 4), register i mod 4.
 typedef float mwg_float4 __attribute__((ext_vector_type(4)));
 
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<double> {
-    typedef mwg_double4 acc_t;
-    static __device__ __forceinline__ acc_t run(double a, double b, acc_t c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int drow(int lq, int r) { return lq + 4 * r; }
-};
-template <>
-struct Mfma<float> {
-    typedef mwg_float4 acc_t;
-    static __device__ __forceinline__ acc_t run(float a, float b, acc_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int drow(int lq, int r) { return 4 * lq + r; }
-};
+__device__ __forceinline__ mwg_float4 mfma32(float a, float b, mwg_float4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 
 template <int N>
 struct JobShape {
@@ -109,8 +80,7 @@ struct JobShape {
     // waves per job: at most 4 tiles each at N >= 9 (fewer tiles per wave
     // measured slower at N = 10, 12: each wave reads the item's operator
     // operands from LDS once), 2 of 2 tiles at N = 7, 8 (one wave per job
-    // left LDS-bound occupancy at 5 waves per CU: 136 exchange applies at
-    // k = 7, plain FP64 105.9 -> 97.6 ms)
+    // leaves LDS-bound occupancy at 5 waves per CU)
     static constexpr int NW = N == 7 || N == 8 ? (NT + 1) / 2 : (NT + 3) / 4;
     static constexpr int TW = (NT + NW - 1) / NW;  // tiles per wave
     static constexpr int T = 64 * NW;          // threads per job
@@ -122,9 +92,8 @@ struct JobShape {
     static constexpr int CP = 16 * NTP > 4 * KS * N ? 16 * NTP : 4 * KS * N;
     static constexpr int XSZ = XROWS * 16, YSZ = 16 * CP;
     // N >= 11: X and Y in buffers of their own, so that an item needs two
-    // barriers instead of four (64 Helmholtz applies at k = 11, plain FP64:
-    // 703 -> 679 ms); at N <= 10 the larger LDS footprint costs a workgroup
-    // per CU and one shared buffer is faster
+    // barriers instead of four; at N <= 10 the larger LDS footprint costs a
+    // workgroup per CU and one shared buffer is faster
     static constexpr bool SEP = N >= 11;
     static constexpr int BUF = SEP ? XSZ + YSZ : (XSZ > YSZ ? XSZ : YSZ);
     static constexpr int OB = 4 * N2;          // operator values per stage (Ox, Oy, Oz and Oz of gt | 4)
@@ -276,10 +245,10 @@ __device__ __forceinline__ int screen_scan(const KArgs &a, const AppDesc &ad, co
 
 // LDS of one job of apply_segment: the pass buffer, two operator stages,
 // the worklist and the staged term table.
-template <int N, typename T>
+template <int N>
 struct ApplySmem {
-    T buf[JobShape<N>::BUF];
-    T ops[2][JobShape<N>::OB];
+    float buf[JobShape<N>::BUF];
+    float ops[2][JobShape<N>::OB];
     int wl[kWorkCap];
     int ltab[64];
     long long btab[64];
@@ -295,12 +264,14 @@ struct ApplySmem {
 // computed once and its z pass once per passing component, into two
 // accumulators.  Worklist items are (p << 11) | (t1 << 10) | (t0 << 9) |
 // (ft << 6) | lane-term.
-template <int N, typename T, bool PAIR>
-__device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int seg, double lo_mult, double hi_mult,
-                                              int cls_counter, ApplySmem<N, T> &sm, double *nrm_s) {
+template <int N>
+__device__ __forceinline__ void apply_segment(const KArgs &a, const float *pool, int seg, double hi_mult,
+                                              ApplySmem<N> &sm, double *nrm_s) {
+    using T = float;
+    constexpr bool PAIR = true;
+    constexpr double lo_mult = 0.0;
     using S = JobShape<N>;
-    using MF = Mfma<T>;
-    using acc_t = typename MF::acc_t;
+    using acc_t = mwg_float4;
     constexpr int N2 = S::N2, N3 = S::N3, NT = S::NT, KS = S::KS, TW = S::TW, NTH = S::T;
     constexpr int CP = S::CP, BUF = S::BUF;
     constexpr int OB = (PAIR ? 4 : 3) * N2, OPL = (OB + NTH - 1) / NTH;
@@ -314,17 +285,16 @@ __device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int
     const int lc = lane & 15, lq = lane >> 4;
     for (int e = tid; e < BUF; e += NTH) xb[e] = T(0);
 
-    const int pi_begin = a.seg_p0[seg], pi_end = a.seg_p1[seg];
+    const int pi_begin = a.seg_p0[seg] >> 12, pi_end = a.seg_p1[seg] >> 12;
     const AppDesc ad = a.apps[a.out_app[a.seg_job[seg] >> 3]];
     const JobCtx j = job_ctx(a, ad, a.seg_job[seg], lo_mult, hi_mult);
     const int g = j.g, gt = j.gt, w = j.w, side = j.side;
     const long long boff = j.boff;
     const int *gb = j.gb;
-    const T *opblk = op_blocks<T>(ad);
+    const T *opblk = ad.blk32;
 
-    // this wave's tiles: t = wv*TW + tt; tiles t >= NT (N = 10: the eighth)
-    // are skipped (wave-uniform), their LDS entries keep finite values that
-    // only meet zero operator entries
+    // this wave's tiles: t = wv*TW + tt (a padding tile t >= NT is computed:
+    // skipping it costs more registers than its MFMAs)
     int ybase[TW], zbase[TW];
 #pragma unroll
     for (int tt = 0; tt < TW; tt++) {
@@ -333,9 +303,6 @@ __device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int
         ybase[tt] = (q * N + lq) * 16 + r;  // Xp[(jz*N + 4k + lq)][ix]
         zbase[tt] = q * CP + r + lq * N;    // Yp[iy][(4k + lq)*N + ix]
     }
-    // (in FP64 only: in FP32 the branches cost more registers than the
-    // padding tile's MFMAs)
-    auto live = [&](int tt) { return S::NTP == NT || !std::is_same<T, double>::value || wv * TW + tt < NT; };
     acc_t acc[TW], acc1[TW];  // acc1: gt | 4 (PAIR only)
 #pragma unroll
     for (int tt = 0; tt < TW; tt++) acc[tt] = acc1[tt] = acc_t{T(0), T(0), T(0), T(0)};
@@ -465,13 +432,12 @@ __device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int
                     for (int k = 0; k < KS; k++)
 #pragma unroll
                         for (int tt = 0; tt < TW; tt++)
-                            if (live(tt)) dx[tt] = MF::run(fa[tt][k], ox[k], dx[tt]);
+                            dx[tt] = mfma32(fa[tt][k], ox[k], dx[tt]);
 #pragma unroll
                     for (int tt = 0; tt < TW; tt++)
-                        if (live(tt))
 #pragma unroll
                             for (int r = 0; r < 4; r++)
-                                xb[(16 * (wv * TW + tt) + MF::drow(lq, r)) * 16 + lc] = dx[tt][r];
+                                xb[(16 * (wv * TW + tt) + 4 * lq + r) * 16 + lc] = dx[tt][r];
                 }
                 // the F tiles are dead after the x pass: those of the next
                 // item's group load during its y and z passes
@@ -486,16 +452,15 @@ __device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int
                     for (int k = 0; k < KS; k++)
 #pragma unroll
                         for (int tt = 0; tt < TW; tt++)
-                            if (live(tt)) dy[tt] = MF::run(oy[k], xb[ybase[tt] + 64 * k], dy[tt]);
+                            dy[tt] = mfma32(oy[k], xb[ybase[tt] + 64 * k], dy[tt]);
                     // one shared buffer: every wave has read X before Y
                     // overwrites it
                     if constexpr (!S::SEP) __syncthreads();
 #pragma unroll
                     for (int tt = 0; tt < TW; tt++)
-                        if (live(tt))
 #pragma unroll
                             for (int r = 0; r < 4; r++)
-                                yb[MF::drow(lq, r) * CP + 16 * (wv * TW + tt) + lc] = dy[tt][r];
+                                yb[(4 * lq + r) * CP + 16 * (wv * TW + tt) + lc] = dy[tt][r];
                 }
                 __syncthreads();
                 // z pass: B[jz][col'] = Yp[iy][jz*N + ix], col' = iy*N + ix,
@@ -505,23 +470,23 @@ __device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int
                     for (int k = 0; k < KS; k++)
 #pragma unroll
                         for (int tt = 0; tt < TW; tt++)
-                            if (live(tt)) {
+                            {
                                 const T yv = yb[zbase[tt] + 4 * k * N];
-                                acc[tt] = MF::run(oz[k], yv, acc[tt]);
-                                if (PAIR) acc1[tt] = MF::run(oz1[k], yv, acc1[tt]);
+                                acc[tt] = mfma32(oz[k], yv, acc[tt]);
+                                if (PAIR) acc1[tt] = mfma32(oz1[k], yv, acc1[tt]);
                             }
                 } else if (t0) {
 #pragma unroll
                     for (int k = 0; k < KS; k++)
 #pragma unroll
                         for (int tt = 0; tt < TW; tt++)
-                            if (live(tt)) acc[tt] = MF::run(oz[k], yb[zbase[tt] + 4 * k * N], acc[tt]);
+                            acc[tt] = mfma32(oz[k], yb[zbase[tt] + 4 * k * N], acc[tt]);
                 } else {
 #pragma unroll
                     for (int k = 0; k < KS; k++)
 #pragma unroll
                         for (int tt = 0; tt < TW; tt++)
-                            if (live(tt)) acc1[tt] = MF::run(oz1[k], yb[zbase[tt] + 4 * k * N], acc1[tt]);
+                            acc1[tt] = mfma32(oz1[k], yb[zbase[tt] + 4 * k * N], acc1[tt]);
                 }
                 it = nx;
                 stage ^= 1;
@@ -531,9 +496,9 @@ __device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int
     }
     if (tid == 0 && napps + napps1) {
         atomicAdd(&a.counters[0], napps + napps1);
-        if (cls_counter > 0) atomicAdd(&a.counters[cls_counter], napps + napps1);
+        atomicAdd(&a.counters[1], napps + napps1);
     }
-    // acc[tt][r] = out[iz = drow(lq, r)][col = 16t + lc], added in FP64 to the
+    // acc[tt][r] = out[iz = 4 lq + r][col = 16t + lc], added in FP64 to the
     // (zeroed) output: several segments and launches may share a job
     auto store = [&](const acc_t *ac, int comp) {
         double *dst = a.out_ns + (long long)g * 8 * N3 + (long long)comp * N3;
@@ -542,13 +507,484 @@ __device__ __forceinline__ void apply_segment(const KArgs &a, const T *pool, int
             const int col = 16 * (wv * TW + tt) + lc;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int iz = MF::drow(lq, r);
+                const int iz = 4 * lq + r;
                 if (col < N2 && iz < N) atomicAdd(&dst[iz * N2 + col], (double)ac[tt][r]);
             }
         }
     };
     if (napps) store(acc, gt);
     if (PAIR && napps1) store(acc1, gt | 4);
+}
+
+// Global-memory view of a pointer, so that loads through it are global, not
+// flat, loads.
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(1))) T *gmem(const T *p) {
+    return (const __attribute__((address_space(1))) T *)p;
+}
+
+// ------------------------------------------------------------ FP64 calculator
+//
+// One wave per job, on the 4 x 4 x 4 FP64 MFMA (four blocks b of 4 x 4 x 4;
+// gfx950 runs it at the FLOP rate of the 16 x 16 x 4 form: 68 against 70
+// TFLOP/s measured).  A 4-row tile pads the N rows of an operator to a
+// multiple of 4 where a 16-row tile pads to 16, and the data's N^2 columns
+// are packed 16 to an instruction:
+//   x: X[ix][(jz,jy)]  = Ox . F^T    F rows in registers as the B operand
+//   y: Y[iy][(jz,ix)]  = Oy . X
+//   z: acc[iz][(iy,ix)] += Oz . Y    for gt and, in a pair job, gt | 4
+// N = 10: 63 instructions of 16 cycles a chain where 21 of 64 were issued
+// (1008 cycles against 1344), N = 8 256 against 512, N = 12 1296 against 1728.
+// A wave owns its job, its LDS and its worklist alone, so an item needs no
+// barrier: a wave's LDS accesses run in order, and the second wave of the SIMD
+// computes while the first waits for its own.  What bounds the kernel is the
+// matrix unit: it is busy 69 % of the cycles a CU works at N = 10 (frozen plan
+// of 656 nodes; the rest waits for operands from LDS), and a refinement
+// level's launch ends with CUs idle while the last segments run.
+// Device time of the levels below the roots, against the 16 x 16 x 4 kernel
+// with two or three waves a job: six orbitals at k = 11 56.0 -> 25 ms, one k = 9
+// apply 5.7 -> 3.3 ms, ten exchange densities at k = 7 3.6 -> 1.7 ms, a frozen
+// k = 9 plan 5.0 -> 2.6 ms.  A pair job's z passes run one after the other over
+// one read of Oz each: side by side (one read of Y) they hold 18 more
+// registers and spill 250 at N = 12 (97 ms); without pairs, two single jobs a
+// segment, 34.8 ms against 33.5.
+// Lane layouts (checked on gfx950): A[b][i][k] in lane i + 4b + 16k, B[b][k][j]
+// in lane j + 4b + 16k, D[b][i][j] in lane j + 4b + 16i.  An operator operand
+// is the same for the four blocks; a data operand's 16 columns are 4b + j, so
+// D holds row lane / 16 of column lane % 16.
+// Where N is a multiple of 4 the x pass runs with the planes jz as the four
+// blocks (A = F rows (jz, jy), B = Ox^T): D then holds X[jy][ix] of plane jz in
+// exactly the lanes in which the y pass reads it as its B operand, and only Y
+// passes through LDS.
+// LDS pitch of a row: 16 CT rounded up to 20 mod 32 doubles, which puts both
+// the transposed stores and the reads on distinct banks but for a few lanes.
+template <int N>
+struct Job4 {
+    static constexpr int N2 = N * N, N3 = N2 * N;
+    static constexpr int G = (N + 3) / 4;       // 4-row groups of an operator, 4-deep k steps
+    static constexpr int NP = 4 * G;
+    static constexpr int CT = (N2 + 15) / 16;   // 16-column tiles
+    static constexpr int P = 16 * CT + (52 - 16 * CT % 32) % 32;
+    static constexpr int BUF = NP * P;
+    static constexpr bool CHAIN = N % 4 == 0;
+    static constexpr int LPD = (N2 + 63) / 64;  // loads of an operator block per lane
+    // worklist items of a batch (>= 64 + 64); N >= 11: eight waves' LDS fit a CU
+    static constexpr int CAP = N >= 11 ? 128 : 256;
+    // waves per SIMD the registers are held to: two at N >= 9 (accumulators
+    // and F rows alone take 126-162 of the 256), four below
+    static constexpr int WPE = N >= 9 ? 2 : 4;
+};
+
+// Worklist item: the operator block ids of translation 0, component 0, the
+// distance of two components' blocks, and the band position, input component
+// and which components of the job pass.
+struct Item4 {
+    int center, span, pos;  // pos = p << 5 | t1 << 4 | t0 << 3 | ft
+};
+
+template <int N>
+struct Smem4 {
+    double buf[Job4<N>::BUF];
+    double ops[4 * Job4<N>::NP * Job4<N>::NP];  // Ox, Oy, Oz, Oz of gt | 4, rows padded to NP
+    Item4 wl[Job4<N>::CAP];
+};
+
+// Keeps the compiler's scheduler from moving instructions past this point:
+// left alone it starts the operand reads of a whole pass ahead and spills.
+#define SCHED_STEP() __builtin_amdgcn_sched_barrier(0)
+
+// Orders this wave's LDS accesses for the compiler (the hardware runs a
+// wave's LDS accesses in order).
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Next items of a segment into the worklist: candidates as in screen_scan,
+// then for each the terms 64 at a time (one per lane), all of a pair before
+// the next pair, so that a pair's F rows load once.  Stops where 64 more items
+// may not fit and leaves the pair in pi and its first open term in e0.  Of pair
+// u_last only the terms before e_last belong to the segment.
+template <bool PAIR, int CAP>
+__device__ __forceinline__ int screen_items(const KArgs &a, const AppDesc &ad, const JobCtx &j, const double *tn,
+                                            const int2 *tb, int &pi, int pi_end, int &e0, int u_last, int e_last,
+                                            Item4 *wl, int lane, unsigned long long &apps0,
+                                            unsigned long long &apps1) {
+    const int S = 2 * ad.mt_w + 1;
+    const long long S3 = (long long)S * S * S;
+    const double *mt = ad.mtab + (long long)(j.d - ad.mt_d0) * 64 * S3;
+    int n = 0;
+    while (pi < pi_end) {
+        const int pr = pi + lane;
+        bool cand = false;
+        double fl = 0.0;
+        if (pr < pi_end) {
+            const int p = pr >> 3, ft = pr & 7;
+            const int s = a.band[j.boff + p];
+            // the NS form has no scaling-to-scaling part below the roots
+            const bool ex0 = j.d > 0 && ft == 0 && j.gt == 0;
+            if (s >= 0 && (PAIR || !ex0)) {
+                fl = a.slot_norm[(long long)s * 8 + ft];
+                const int lx = p % j.side - j.w, ly = (p / j.side) % j.side - j.w, lz = p / (j.side * j.side) - j.w;
+                const long long li = ((long long)(lz + ad.mt_w) * S + (ly + ad.mt_w)) * S + (lx + ad.mt_w);
+                const int cxy = (2 * j.gb[0] + (ft & 1)) | ((2 * j.gb[1] + ((ft >> 1) & 1)) << 2);
+                const int cz = 2 * j.gb[2] + ((ft >> 2) & 1);
+                double mb = ex0 ? 0.0 : mt[(cxy | (cz << 4)) * S3 + li] * fl;
+                if (PAIR) mb = fmax(mb, mt[(cxy | ((cz + 2) << 4)) * S3 + li] * fl);
+                cand = fl > 0.0 && mb > j.thr && mb > j.thr_lo;
+            }
+        }
+        unsigned long long cm = __ballot(cand);
+        while (cm) {
+            const int k = __builtin_ctzll(cm);
+            cm &= cm - 1;
+            const int p = (pi + k) >> 3, ft = (pi + k) & 7;
+            const double fn = __shfl(fl, k);
+            const int lx = p % j.side, ly = (p / j.side) % j.side, lz = p / (j.side * j.side);
+            const int cz = 2 * j.gb[2] + ((ft >> 2) & 1);
+            const double *nx = tn + (long long)((2 * j.gb[0] + (ft & 1)) * j.nl + lx) * j.nact;
+            const double *ny = tn + (long long)((2 * j.gb[1] + ((ft >> 1) & 1)) * j.nl + ly) * j.nact;
+            const double *nz = tn + (long long)(cz * j.nl + lz) * j.nact;
+            const double *nz1 = nz + (long long)2 * j.nl * j.nact;
+            const bool ex0 = PAIR && j.d > 0 && ft == 0 && j.gt == 0;
+            if (k > 0) e0 = 0;  // e0 belongs to the first pair alone
+            const int e1 = pi + k == u_last ? e_last : j.nact;
+            for (; e0 < e1; e0 += 64) {
+                if (n + 64 > CAP) {
+                    pi += k;
+                    return n;
+                }
+                const int e = e0 + lane;
+                bool t0 = false, t1 = false;
+                if (e < e1) {
+                    const double nxy = nx[e] * ny[e];
+                    const double b0 = (nxy * nz[e]) * fn;
+                    t0 = !ex0 && b0 > j.thr && b0 > j.thr_lo && !(b0 > j.thr_hi);
+                    if (PAIR) {
+                        const double b1 = (nxy * nz1[e]) * fn;
+                        t1 = b1 > j.thr && b1 > j.thr_lo && !(b1 > j.thr_hi);
+                    }
+                }
+                const unsigned long long mask = __ballot(t0 || t1);
+                if (PAIR) {
+                    apps0 += __popcll(__ballot(t0));
+                    apps1 += __popcll(__ballot(t1));
+                } else {
+                    apps0 += __popcll(mask);
+                }
+                if (t0 || t1) {
+                    const int2 b = tb[e];
+                    wl[n + __popcll(mask & ((1ull << lane) - 1ull))] =
+                        Item4{b.x, b.y, (p << 5) | ((int)t1 << 4) | ((int)t0 << 3) | ft};
+                }
+                n += __popcll(mask);
+            }
+            e0 = 0;
+        }
+        pi += 64;
+    }
+    return n;
+}
+
+template <int N, bool PAIR>
+__device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int seg, int comp, double lo_mult, double hi_mult,
+                                         Smem4<N> &sm) {
+    using S = Job4<N>;
+    constexpr int N2 = S::N2, N3 = S::N3, G = S::G, NP = S::NP, CT = S::CT, P = S::P, LPD = S::LPD;
+    const int lane = threadIdx.x, lc = lane & 15, lq = lane >> 4, l3 = lane & 3;
+    const AppDesc &ad = a.apps[a.out_app[a.seg_job[seg] >> 3]];
+    const JobCtx j = job_ctx(a, ad, a.seg_job[seg] | comp, lo_mult, hi_mult);
+    const int *gb = j.gb;
+    const double *tn = a.tn + a.tn_off[ad.act_base + j.d];
+    const int2 *tb = a.tb + j.a0;
+    double *const buf = sm.buf;
+    double *const ops = sm.ops;
+    const __attribute__((address_space(1))) double *const opblk = gmem(ad.blk64);
+
+    // per-lane offsets, fixed for the segment
+    int xw[S::CHAIN ? 1 : CT], yw[CT];
+#pragma unroll
+    for (int t = 0; t < CT; t++) {
+        const int e = 16 * t + lc;
+        if constexpr (!S::CHAIN) xw[t] = (e % N) * P + (e / N) * N + lq;
+        yw[t] = (e / N) * P + lq * N + e % N;
+    }
+    const int rd = lq * P + lc;             // y and z operand reads
+    const int ao = l3 * NP + lq;            // operator operand reads
+    int ow[LPD], og[LPD];                   // operator stage: LDS and block offsets
+#pragma unroll
+    for (int u = 0; u < LPD; u++) {
+        const int e = min(lane + 64 * u, N2 - 1);
+        og[u] = e;
+        ow[u] = (e / N) * NP + e % N;
+    }
+    const bool last = lane + 64 * (LPD - 1) < N2;
+
+    double acc[CT][G], acc1[PAIR ? CT : 1][G];
+#pragma unroll
+    for (int t = 0; t < CT; t++)
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            acc[t][g] = 0.0;
+            if constexpr (PAIR) acc1[t][g] = 0.0;
+        }
+    // F rows of an item's group.  CHAIN: f[(u G + g) G + k] = F[jz = 4u +
+    // block][jy = 4g + l3][jx = 4k + lq]; else f[t G + k] = F[(jz, jy) = 16 t
+    // + lc][jx = 4 k + lq]
+    constexpr int NF = S::CHAIN ? G * G * G : CT * G;
+    double f[NF];
+    auto load_f = [&](int pos) {
+        const int s = a.band[j.boff + (pos >> 5)];
+        const __attribute__((address_space(1))) double *src = gmem(pool) + a.slot_off[s] + (pos & 7) * N3;
+        if constexpr (S::CHAIN) {
+            const int base = ((lane >> 2) & 3) * N2 + l3 * N + lq;
+#pragma unroll
+            for (int u = 0; u < G; u++)
+#pragma unroll
+                for (int g = 0; g < G; g++)
+#pragma unroll
+                    for (int k = 0; k < G; k++)
+                        f[(u * G + g) * G + k] = src[base + 4 * u * N2 + 4 * g * N + 4 * k];
+        } else {
+#pragma unroll
+            for (int t = 0; t < CT; t++) {
+                const int e = 16 * t + lc;
+#pragma unroll
+                for (int k = 0; k < G; k++) {
+                    const bool in = (t + 1 < CT || e < N2) && (k + 1 < G || 4 * k + lq < N);
+                    f[t * G + k] = in ? src[e * N + 4 * k + lq] : 0.0;
+                }
+            }
+        }
+    };
+    // operator blocks of an item into registers, then into the stage; the z
+    // block of a component that does not pass is left as it is
+    double pre[PAIR ? 4 : 3][LPD];
+    auto fetch = [&](const Item4 &it) {
+        const int pos = it.pos, p = pos >> 5;
+        const int lx = p % j.side - j.w, ly = (p / j.side) % j.side - j.w, lz = p / (j.side * j.side) - j.w;
+        const int cx = (gb[0] << 1) | (pos & 1), cy = (gb[1] << 1) | ((pos >> 1) & 1), cz = (gb[2] << 1) | ((pos >> 2) & 1);
+        const int id[4] = {it.center + cx * it.span + lx, it.center + cy * it.span + ly, it.center + cz * it.span + lz,
+                           it.center + (cz + 2) * it.span + lz};
+#pragma unroll
+        for (int q = 0; q < (PAIR ? 4 : 3); q++) {
+            if (q == 2 && PAIR && !(pos & 8)) continue;
+            if (q == 3 && !(pos & 16)) continue;
+            const __attribute__((address_space(1))) double *b = opblk + (long long)id[q] * N2;
+#pragma unroll
+            for (int u = 0; u < LPD; u++) pre[q][u] = b[og[u]];
+        }
+    };
+    auto stage = [&](int pos) {
+#pragma unroll
+        for (int q = 0; q < (PAIR ? 4 : 3); q++) {
+            if (q == 2 && PAIR && !(pos & 8)) continue;
+            if (q == 3 && !(pos & 16)) continue;
+#pragma unroll
+            for (int u = 0; u < LPD; u++)
+                if (u + 1 < LPD || last) ops[q * NP * NP + ow[u]] = pre[q][u];
+        }
+    };
+    // operator q's operand: element (4 g + l3, 4 k + lq)
+    auto operand = [&](int q, double (&o)[G][G]) {
+#pragma unroll
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int k = 0; k < G; k++) o[g][k] = ops[q * NP * NP + 4 * g * NP + 4 * k + ao];
+    };
+    auto mfma = [](double x, double y, double c) { return __builtin_amdgcn_mfma_f64_4x4x4f64(x, y, c, 0, 0, 0); };
+    auto uniform = [&](int i) {
+        const Item4 v = sm.wl[i];
+        return Item4{__builtin_amdgcn_readfirstlane(v.center), __builtin_amdgcn_readfirstlane(v.span),
+                     __builtin_amdgcn_readfirstlane(v.pos)};
+    };
+
+    // the pair of the segment's end holds its terms before e_last only
+    const int u_last = a.seg_p1[seg] >> 12, e_last = a.seg_p1[seg] & 4095, pi_end = u_last + (e_last > 0 ? 1 : 0);
+    int pi = a.seg_p0[seg] >> 12, e0 = a.seg_p0[seg] & 4095;
+    unsigned long long napps = 0, napps1 = 0;
+    while (pi < pi_end) {
+        wave_order();
+        const int n = screen_items<PAIR, S::CAP>(a, ad, j, tn, tb, pi, pi_end, e0, e_last > 0 ? u_last : -1, e_last,
+                                                     sm.wl, lane, napps, napps1);
+        wave_order();
+        if (n == 0) continue;
+        Item4 it = uniform(0);
+        load_f(it.pos);
+        fetch(it);
+        stage(it.pos);
+        for (int i = 0; i < n; i++) {
+            const bool more = i + 1 < n;
+            const Item4 nx = uniform(more ? i + 1 : i);
+            const bool newgroup = more && ((nx.pos ^ it.pos) & ~24) != 0;
+            const bool t0 = !PAIR || (it.pos & 8), t1 = PAIR && (it.pos & 16);
+            wave_order();
+            double oy[G][G];
+            if constexpr (S::CHAIN) {
+                operand(1, oy);
+#pragma unroll
+                for (int u = 0; u < G; u++) {
+#pragma unroll
+                    for (int h = 0; h < G; h++) {
+                        double x[G], y[G], ox[G];  // rows 4g + lq of ix group h
+#pragma unroll
+                        for (int k = 0; k < G; k++) ox[k] = ops[4 * h * NP + 4 * k + ao];
+#pragma unroll
+                        for (int g = 0; g < G; g++) x[g] = y[g] = 0.0;
+#pragma unroll
+                        for (int k = 0; k < G; k++)
+#pragma unroll
+                            for (int g = 0; g < G; g++) x[g] = mfma(f[(u * G + g) * G + k], ox[k], x[g]);
+#pragma unroll
+                        for (int k = 0; k < G; k++)
+#pragma unroll
+                            for (int g = 0; g < G; g++) y[g] = mfma(oy[g][k], x[k], y[g]);
+                        // Y[jz = 4u + block][iy = 4g + lq][ix = 4h + l3]
+#pragma unroll
+                        for (int g = 0; g < G; g++)
+                            buf[(4 * u + ((lane >> 2) & 3)) * P + (4 * g + lq) * N + 4 * h + l3] = y[g];
+                        if (h & 1) SCHED_STEP();
+                    }
+                    SCHED_STEP();
+                }
+                if (newgroup) load_f(nx.pos);
+            } else {
+                double ox[G][G];
+                operand(0, ox);
+#pragma unroll
+                for (int t = 0; t < CT; t++) {
+                    double d[G];
+#pragma unroll
+                    for (int g = 0; g < G; g++) d[g] = 0.0;
+#pragma unroll
+                    for (int k = 0; k < G; k++)
+#pragma unroll
+                        for (int g = 0; g < G; g++) d[g] = mfma(ox[g][k], f[t * G + k], d[g]);
+                    // X[jy][(jz, ix)]; rows and columns past the last are not
+                    // stored (those of the buffer stay zero)
+                    if (t + 1 < CT || 16 * t + lc < N2) {
+#pragma unroll
+                        for (int g = 0; g < G; g++)
+                            if (g + 1 < G || 4 * g + lq < N) buf[xw[t] + 4 * g] = d[g];
+                    }
+                    if (t & 1) SCHED_STEP();
+                }
+                operand(1, oy);
+                // the F rows of the next group load during the other passes
+                if (newgroup) load_f(nx.pos);
+                wave_order();
+                SCHED_STEP();
+                double d[CT][G], bn[G];
+#pragma unroll
+                for (int k = 0; k < G; k++) bn[k] = buf[rd + 4 * k * P];
+#pragma unroll
+                for (int t = 0; t < CT; t++) {
+                    double b[G];
+#pragma unroll
+                    for (int k = 0; k < G; k++) {
+                        b[k] = bn[k];
+                        if (t + 1 < CT) bn[k] = buf[rd + 4 * k * P + 16 * (t + 1)];
+                    }
+#pragma unroll
+                    for (int g = 0; g < G; g++) d[t][g] = 0.0;
+#pragma unroll
+                    for (int k = 0; k < G; k++)
+#pragma unroll
+                        for (int g = 0; g < G; g++) d[t][g] = mfma(oy[g][k], b[k], d[t][g]);
+                    SCHED_STEP();
+                }
+                // Y[jz][(iy, ix)] in X's place, which every tile has read
+                wave_order();
+#pragma unroll
+                for (int t = 0; t < CT; t++)
+                    if (t + 1 < CT || 16 * t + lc < N2) {
+#pragma unroll
+                        for (int g = 0; g < G; g++)
+                            if (g + 1 < G || 4 * g + lq < N) buf[yw[t] + 4 * g * N] = d[t][g];
+                    }
+            }
+            SCHED_STEP();
+            if (more) fetch(nx);
+            wave_order();
+            // z, once per passing component (item-uniform branches)
+            auto z_pass = [&](auto both, auto &&c0, auto &&c1, int q0) {
+                constexpr bool BOTH = decltype(both)::value;
+                double oz[G][G], oz1[BOTH ? G : 1][G], bn[G];
+                operand(q0, oz);
+                if constexpr (BOTH) operand(3, oz1);
+#pragma unroll
+                for (int k = 0; k < G; k++) bn[k] = buf[rd + 4 * k * P];
+#pragma unroll
+                for (int t = 0; t < CT; t++) {
+                    double b[G];
+#pragma unroll
+                    for (int k = 0; k < G; k++) {
+                        b[k] = bn[k];
+                        if (t + 1 < CT) bn[k] = buf[rd + 4 * k * P + 16 * (t + 1)];
+                    }
+#pragma unroll
+                    for (int k = 0; k < G; k++)
+#pragma unroll
+                        for (int g = 0; g < G; g++) {
+                            c0[t][g] = mfma(oz[g][k], b[k], c0[t][g]);
+                            if constexpr (BOTH) c1[t][g] = mfma(oz1[g][k], b[k], c1[t][g]);
+                        }
+                    SCHED_STEP();
+                }
+            };
+            if constexpr (PAIR) {
+                if (t0) z_pass(std::false_type{}, acc, acc, 2);
+                SCHED_STEP();
+                if (t1) z_pass(std::false_type{}, acc1, acc1, 3);
+            } else {
+                z_pass(std::false_type{}, acc, acc, 2);
+            }
+            wave_order();
+            if (more) stage(nx.pos);
+            it = nx;
+        }
+    }
+    if (lane == 0 && napps + napps1) atomicAdd(&a.counters[0], napps + napps1);
+    // acc[t][g] = out[iz = 4 g + lq][16 t + lc], added to the (zeroed) output:
+    // several segments and launches may share a job
+    auto store = [&](const auto &ac, int comp) {
+        double *dst = a.out_ns + ((long long)j.g * 8 + comp) * N3;
+#pragma unroll
+        for (int t = 0; t < CT; t++)
+#pragma unroll
+            for (int g = 0; g < G; g++)
+                if ((t + 1 < CT || 16 * t + lc < N2) && (g + 1 < G || 4 * g + lq < N))
+                    atomicAdd(&dst[(4 * g + lq) * N2 + 16 * t + lc], ac[t][g]);
+    };
+    if (napps) store(acc, j.gt);
+    if constexpr (PAIR)
+        if (napps1) store(acc1, j.gt | 4);
+}
+
+// Persistent launch of one-wave workgroups over a queue of segments
+// seg_list[0, n) (or seg0 .. seg0 + n - 1 without a list), the terms in the
+// class (lo_mult thr_cls, hi_mult thr_cls].
+template <int N, bool PAIR>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Job4<N>::WPE))) void k_apply64(
+    KArgs a, const double *pool, const int *seg_list, int seg0, int n, double lo_mult, double hi_mult,
+    unsigned long long *head) {
+    __shared__ Smem4<N> sm;
+    // what the passes never write stays zero (padding rows, columns and
+    // operator elements)
+    for (int e = threadIdx.x; e < Job4<N>::BUF; e += 64) sm.buf[e] = 0.0;
+    for (int e = threadIdx.x; e < 4 * Job4<N>::NP * Job4<N>::NP; e += 64) sm.ops[e] = 0.0;
+    while (true) {
+        int e = 0;
+        if (threadIdx.x == 0) e = (int)atomicAdd(head, 1ull);
+        e = __builtin_amdgcn_readfirstlane(e);
+        if (e >= n) break;
+        const int seg = seg_list ? seg_list[e] : seg0 + e;
+        if constexpr (PAIR && N >= 99) {
+            for (int c = 0; c < 8; c += 4) segment4<N, false>(a, pool, seg, c, lo_mult, hi_mult, sm);
+        } else {
+            segment4<N, PAIR>(a, pool, seg, 0, lo_mult, hi_mult, sm);
+        }
+    }
 }
 
 // ------------------------------------------------------ FP16 split products
@@ -687,13 +1123,6 @@ __device__ __forceinline__ T &pick(T &a, T &b) {
         return b;
 }
 
-// Global-memory view of a pointer, so that loads through it are global, not
-// flat, loads.
-template <typename T>
-__device__ __forceinline__ const __attribute__((address_space(1))) T *gmem(const T *p) {
-    return (const __attribute__((address_space(1))) T *)p;
-}
-
 // Worklist item of the split kernel: the operator block ids (block = N x N
 // values of one term, depth, component and translation) of x, y and of z
 // for the output components gt and gt | 4, and the input group (band
@@ -766,7 +1195,7 @@ __device__ __forceinline__ void split_segment(const KArgs &a, const _Float16 *po
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int lc = lane & 15, lq = lane >> 4;
 
-    const int pi_begin = a.seg_p0[seg], pi_end = a.seg_p1[seg];
+    const int pi_begin = a.seg_p0[seg] >> 12, pi_end = a.seg_p1[seg] >> 12;
     const AppDesc ad = a.apps[a.out_app[a.seg_job[seg] >> 3]];
     const JobCtx j = job_ctx(a, ad, a.seg_job[seg], lo_mult, hi_mult);
     const double thr_single = (j.thr > ad.thr_floor ? j.thr : ad.thr_floor) * single_mult;
@@ -1152,24 +1581,18 @@ __device__ __forceinline__ int next_entry(unsigned long long *head, int *s_next)
     return __builtin_amdgcn_readfirstlane(*s_next);
 }
 
-// FP64 or FP32 per-node calculator over segments seg_list[0, n) (or segments
-// seg0 .. seg0 + n - 1 without a list) in the class (lo_mult thr_cls,
-// hi_mult thr_cls]; PAIR: the segments are pair segments.  Held to two waves
-// per SIMD: the FP64 pair jobs at N = 7, 10, 11 would otherwise take more
-// than 256 registers and run one wave per SIMD (N = 10: 8.4 ms against
-// 5.8 ms with 72 bytes per lane spilled, 116 Helmholtz terms at k = 9).
-template <int N, typename T, bool PAIR>
+// FP32 class over the pair segments seg_list[0, n): bounds at most hi_mult
+// thr_cls.  Held to two waves per SIMD.
+template <int N>
 __global__ __launch_bounds__(JobShape<N>::T) __attribute__((amdgpu_waves_per_eu(2))) void k_apply(
-    KArgs a, const T *pool, const int *seg_list, int seg0, int n, double lo_mult, double hi_mult, int cls_counter,
-    unsigned long long *head) {
-    __shared__ ApplySmem<N, T> sm;
+    KArgs a, const float *pool, const int *seg_list, int n, double hi_mult, unsigned long long *head) {
+    __shared__ ApplySmem<N> sm;
     extern __shared__ double nrm_s[];
     __shared__ int s_next;
     while (true) {
         const int e = next_entry(head, &s_next);
         if (e >= n) break;
-        apply_segment<N, T, PAIR>(a, pool, seg_list ? seg_list[e] : seg0 + e, lo_mult, hi_mult, cls_counter, sm,
-                                  nrm_s);
+        apply_segment<N>(a, pool, seg_list[e], hi_mult, sm, nrm_s);
     }
 }
 
@@ -1887,6 +2310,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     const size_t f_lv = place(sizeof(TermLevel) * levels.size());
     const size_t up_bytes = arena;
     const size_t f_norm = place(sizeof(double) * 8 * n_slot), f_tn = place(sizeof(double) * n_tn);
+    const size_t f_tb = place(sizeof(int2) * n_act);
     std::vector<size_t> f_mt(parts.size());
     for (size_t ai = 0; ai < parts.size(); ai++) f_mt[ai] = place(sizeof(double) * mt_size[ai]);
     unsigned char *dev = nullptr;
@@ -1992,6 +2416,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     a.act_terms = reinterpret_cast<const int *>(dev + f_act);
     a.tn = reinterpret_cast<const double *>(dev + f_tn);
     a.tn_off = reinterpret_cast<const long long *>(dev + f_tno);
+    a.tb = reinterpret_cast<const int2 *>(dev + f_tb);
     a.apps = p->d_apps;
     // counts per (output component, band position)
     const bool bounds = mode != 0;
@@ -2021,15 +2446,16 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     HIP_TRY(hipMemcpyAsync(dev, stage.data(), up_bytes, hipMemcpyHostToDevice, s));
     rc = dev_pool_fill(c, mra, fills, reinterpret_cast<double *>(dev + f_norm), fill_stage, err);
     if (!rc)
-        rc = dev_term_tables(s, a, reinterpret_cast<const TermLevel *>(dev + f_lv), (int)levels.size(),
-                             reinterpret_cast<double *>(dev + f_tn), err);
+        rc = dev_term_tables(s, a, N * N, reinterpret_cast<const TermLevel *>(dev + f_lv), (int)levels.size(),
+                             reinterpret_cast<double *>(dev + f_tn), reinterpret_cast<int2 *>(dev + f_tb), err);
     ca.k = a;
     if (!rc) rc = dev_count_terms(s, ca, bounds, err);
     if (rc) return rc;
     // Room for the segments: what a small launch can hold and 16 (fine ones
-    // 24) for each output node; the few plans that need more are cut again.
+    // 24, plain FP64's 64) for each output node; the few plans that need more
+    // are cut again.
     std::vector<unsigned long long> tot(n_tot);
-    long long cap[2] = {2048 + 16 * n_out, bounds ? 16384 + 24 * n_out : 0};
+    long long cap[2] = {bounds ? 2048 + 16 * n_out : 16384 + 64 * n_out, bounds ? 16384 + 24 * n_out : 0};
     int *seg = nullptr;
     SegRec *rec = nullptr;
     for (int attempt = 0;; attempt++) {
@@ -2197,45 +2623,67 @@ static int persistent_grid(DeviceCtx *c, const void *kernel, int threads, size_t
     return 0;
 }
 
-template <int N, typename T, bool PAIR>
-static int launch_nt(DeviceCtx *c, const KArgs &a, const T *pool, const int *list, int seg0, int n, int wmax,
-                     double lo, double hi, int cls, unsigned long long *head, hipStream_t s, std::string &err) {
+template <int N>
+static int launch32_n(DeviceCtx *c, const KArgs &a, const float *pool, const int *list, int n, int wmax, double hi,
+                      unsigned long long *head, hipStream_t s, std::string &err) {
     if (n == 0) return 0;
     const size_t shmem = nrm_bytes(wmax);
     int grid = 0;
-    int rc = persistent_grid(c, reinterpret_cast<const void *>(&k_apply<N, T, PAIR>), JobShape<N>::T,
-                             sizeof(ApplySmem<N, T>), shmem, n, &grid, err);
+    int rc = persistent_grid(c, reinterpret_cast<const void *>(&k_apply<N>), JobShape<N>::T, sizeof(ApplySmem<N>),
+                             shmem, n, &grid, err);
     if (rc) return rc;
-    hipLaunchKernelGGL((k_apply<N, T, PAIR>), dim3(grid), dim3(JobShape<N>::T), shmem, s, a, pool, list, seg0, n, lo,
-                       hi, cls, head);
+    hipLaunchKernelGGL((k_apply<N>), dim3(grid), dim3(JobShape<N>::T), shmem, s, a, pool, list, n, hi, head);
     HIP_TRY(hipGetLastError());
     return 0;
 }
 
-// Persistent launch of k_apply over seg_list[0, n) or, without a list,
-// segments seg0 .. seg0 + n - 1; pair: the segments are pair segments.
-template <typename T>
-static int launch_t(const DevicePlan *p, const T *pool, bool pair, const int *list, int seg0, int n, double lo,
-                    double hi, int cls, unsigned long long *head, std::string &err, hipStream_t s = nullptr) {
-    const KArgs &a = p->args;
-    if (!s) s = p->ctx->stream;
-#define MWG_LAUNCH(NN)                                                                                           \
-    (pair ? launch_nt<NN, T, true>(p->ctx, a, pool, list, seg0, n, p->wmax, lo, hi, cls, head, s, err)           \
-          : launch_nt<NN, T, false>(p->ctx, a, pool, list, seg0, n, p->wmax, lo, hi, cls, head, s, err))
-    switch (p->kp1) {
-        case 2: return MWG_LAUNCH(2);
-        case 3: return MWG_LAUNCH(3);
-        case 4: return MWG_LAUNCH(4);
-        case 5: return MWG_LAUNCH(5);
-        case 6: return MWG_LAUNCH(6);
-        case 7: return MWG_LAUNCH(7);
-        case 8: return MWG_LAUNCH(8);
-        case 9: return MWG_LAUNCH(9);
-        case 10: return MWG_LAUNCH(10);
-        case 11: return MWG_LAUNCH(11);
-        case 12: return MWG_LAUNCH(12);
-        default: err = "unsupported basis size"; return -1;
+template <int N, bool PAIR>
+static int launch64_n(DeviceCtx *c, const KArgs &a, const double *pool, const int *list, int seg0, int n, double lo,
+                      unsigned long long *head, hipStream_t s, std::string &err) {
+    if (n == 0) return 0;
+    int grid = 0;
+    int rc = persistent_grid(c, reinterpret_cast<const void *>(&k_apply64<N, PAIR>), 64, sizeof(Smem4<N>), 0, n, &grid,
+                             err);
+    if (rc) return rc;
+    hipLaunchKernelGGL((k_apply64<N, PAIR>), dim3(grid), dim3(64), 0, s, a, pool, list, seg0, n, lo, HUGE_VAL, head);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+#define MWG_SIZES(CALL)                                                                                     \
+    switch (p->kp1) {                                                                                       \
+        case 2: return CALL(2);                                                                             \
+        case 3: return CALL(3);                                                                             \
+        case 4: return CALL(4);                                                                             \
+        case 5: return CALL(5);                                                                             \
+        case 6: return CALL(6);                                                                             \
+        case 7: return CALL(7);                                                                             \
+        case 8: return CALL(8);                                                                             \
+        case 9: return CALL(9);                                                                             \
+        case 10: return CALL(10);                                                                           \
+        case 11: return CALL(11);                                                                           \
+        case 12: return CALL(12);                                                                           \
+        default: err = "unsupported basis size"; return -1;                                                 \
     }
+
+// Persistent launch of the FP32 class over the pair segments list[0, n):
+// bounds at most hi thr_cls.
+static int launch32(const DevicePlan *p, const int *list, int n, double hi, unsigned long long *head,
+                    std::string &err) {
+#define MWG_LAUNCH(NN) launch32_n<NN>(p->ctx, p->args, p->pool32, list, n, p->wmax, hi, head, p->ctx->stream, err)
+    MWG_SIZES(MWG_LAUNCH)
+#undef MWG_LAUNCH
+}
+
+// Persistent FP64 launch over the pair segments seg0 .. seg0 + n - 1 (no
+// list), or over the single-component segments list[0, n): bounds above lo
+// thr_cls.
+static int launch64(const DevicePlan *p, const int *list, int n, double lo, unsigned long long *head, hipStream_t s,
+                    std::string &err) {
+#define MWG_LAUNCH(NN)                                                                      \
+    (list ? launch64_n<NN, false>(p->ctx, p->args, p->pool, list, 0, n, lo, head, s, err)   \
+          : launch64_n<NN, true>(p->ctx, p->args, p->pool, nullptr, 0, n, lo, head, s, err))
+    MWG_SIZES(MWG_LAUNCH)
 #undef MWG_LAUNCH
 }
 
@@ -2450,13 +2898,12 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         rc = dev_root_launch(c->stream, p->root, err);
         if (rc) return rc;
     }
-    const double inf = HUGE_VAL;
     // queue heads of the persistent launches: counters[2] (first stream),
     // counters[3] (second stream)
     unsigned long long *head1 = p->args.counters + 2, *head2 = p->args.counters + 3;
     if (mode == 0) {
         // lo = 0: every term that passes screening, over the pair segments
-        rc = launch_t<double>(p, p->pool, true, nullptr, 0, p->n_pseg, 0.0, inf, 0, head1, err);
+        rc = launch64(p, nullptr, p->n_pseg, 0.0, head1, c->stream, err);
         if (rc) return rc;
     } else if (mode == 1) {
         // The FP64 class, then the FP32 class, on the first stream; both only
@@ -2467,11 +2914,11 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         // with the FP32 class instead of before it (64 Helmholtz applies at
         // k = 11, 119,968 output nodes: 316 ms against 394 ms a step).
         if (timed) HIP_TRY(hipEventRecord(c->ev2s, c->stream));
-        rc = launch_t<double>(p, p->pool, false, p->list_hi, 0, p->n_hi, tau, inf, 0, head2, err, c->stream);
+        rc = launch64(p, p->list_hi, p->n_hi, tau, head2, c->stream, err);
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(c->ev2e, c->stream));
         if (timed) HIP_TRY(hipEventRecord(c->evl, c->stream));
-        rc = launch_t<float>(p, p->pool32, true, p->list_lo, 0, p->n_lo, 0.0, tau, 1, head1, err);
+        rc = launch32(p, p->list_lo, p->n_lo, tau, head1, err);
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(c->evm, c->stream));
     } else {
@@ -2480,7 +2927,7 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         HIP_TRY(hipEventRecord(c->evz, c->stream));
         HIP_TRY(hipStreamWaitEvent(c->stream2, c->evz, 0));
         if (timed) HIP_TRY(hipEventRecord(c->ev2s, c->stream2));
-        rc = launch_t<double>(p, p->pool, false, p->list_hi, 0, p->n_hi, tau, inf, 0, head2, err, c->stream2);
+        rc = launch64(p, p->list_hi, p->n_hi, tau, head2, c->stream2, err);
         if (rc) return rc;
         HIP_TRY(hipEventRecord(c->ev2e, c->stream2));
         if (timed) HIP_TRY(hipEventRecord(c->evl, c->stream));

@@ -33,7 +33,7 @@ def test_more_segments_than_room(ctx, order, mode):
     ref, st = oracle.apply_fixed(mra, P.tables(), rho.nodes(), d, l, thr)
     info = plan.info()
     print("order %d %s: %d terms in %d segments" % (order, mode, st["term_apps"], info["segments"]))
-    assert info["segments"] > 2048 + 16 * len(d)
+    assert info["segments"] > (16384 + 64 * len(d) if mode == "fp64" else 2048 + 16 * len(d))
     r = plan.execute()
     assert r["term_apps"] == st["term_apps"] == info["host_term_apps"]
     plan.finish()
