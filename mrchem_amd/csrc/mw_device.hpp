@@ -219,12 +219,12 @@ int dev_raw_alloc(DeviceCtx *c, size_t bytes, void **p, std::string &err);
 void dev_raw_free(DeviceCtx *c, void *p);
 
 // Node-wise sums (mw_multiply.hip): for one output node and one input, the
-// input's source node (its deepest node on the path: block offset in the
-// concatenated pool of all inputs, or -1 when the input has no node on the
-// path), the levels from it down to the output node and the child index of
-// each level (3 bits per level, the first level below the source lowest).
+// input's source node (its deepest node on the path: its block on the device,
+// or null when the input has no node on the path), the levels from it down to
+// the output node and the child index of each level (3 bits per level, the
+// first level below the source lowest).
 struct AddSrc {
-    long long off;
+    const double *p;
     int dep, pad_;
     unsigned long long path;
 };
@@ -236,9 +236,11 @@ struct BlockSource {
     size_t n;
     bool on_device;
 };
-// The inputs' blocks are concatenated in order into the session's pool.
-int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &pool, const std::vector<double> &coefs,
-                  DevAddSession **out, std::string &err);
+// Uploads the host inputs; base receives where each input's blocks are on the
+// device (a device input is read in place).
+int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &inputs,
+                  const std::vector<double> &coefs, DevAddSession **out, std::vector<const double *> &base,
+                  std::string &err);
 // src: n_nodes x n_inputs entries (node-major); out_blocks: n_nodes x
 // 8(k+1)^3, on the host, or on the device with out_on_device.
 int dev_add_nodes(DevAddSession *m, const std::vector<AddSrc> &src, double *out_blocks, std::string &err,

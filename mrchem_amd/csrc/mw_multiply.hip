@@ -36,7 +36,7 @@ namespace mwg {
 namespace {
 
 constexpr int kMulThreads = 256;
-constexpr int kMulBlocks = 1024;  // resident workgroups, each with its own work area
+constexpr int kMulBlocks = 1024;  // resident workgroups of a launch
 
 // Index of the element at position i along dim of the line (a, c) in an
 // n^3 block (x fastest): the two other indices are a (the lower direction)
@@ -115,10 +115,13 @@ __device__ void child_pass(int n, const double *F, const double *src, const int 
     }
 }
 
+// Products and sums for n > 12, where a node's values do not fit LDS: one
+// thread per value of a pass, the passes through a work area in global memory.
+
 // Scaling block of the node `dep` >= 1 levels below the source node block
 // `src` (8 components) along `path` (3 bits per level, first level lowest)
 // into X[0, n^3); X holds 4 and Y 2 blocks of work area.
-__device__ void descend(int n, const double *F, const double *src, int dep, unsigned long long path, double *X,
+__device__ void descend_any(int n, const double *F, const double *src, int dep, unsigned long long path, double *X,
                         double *Y, int tid) {
     const int n3 = n * n * n;
     // first level: the full block (scaling and wavelet parts) towards child t
@@ -161,7 +164,7 @@ __device__ void children_of(int n, const double *F, const double *src, int dep, 
         for (int e = tid; e < 8 * n3; e += kMulThreads) Y[e] = src[e];
         __syncthreads();
     } else {
-        descend(n, F, src, dep, path, X, Y, tid);
+        descend_any(n, F, src, dep, path, X, Y, tid);
         // the work node's block: scaling part X[0], wavelet parts zero
         for (int e = tid; e < 8 * n3; e += kMulThreads) Y[e] = e < n3 ? X[e] : 0.0;
         __syncthreads();
@@ -177,7 +180,7 @@ __device__ void children_of(int n, const double *F, const double *src, int dep, 
 
 }  // namespace
 
-__global__ __launch_bounds__(kMulThreads) void k_mul_nodes(int n, const MulNode *nodes, int n_nodes,
+__global__ __launch_bounds__(kMulThreads) void k_mul_nodes_any(int n, const MulNode *nodes, int n_nodes,
                                                            const double *pool_a, const double *pool_b,
                                                            const double *F, const double *wsc, double coef,
                                                            double *ws, double *out) {
@@ -204,16 +207,9 @@ __global__ __launch_bounds__(kMulThreads) void k_mul_nodes(int n, const MulNode 
     }
 }
 
-// Sums: out block of node w = sum_i coefs[i] x (input i's block at the node,
-// or, below the input's finest node on the path, the scaling part
-// reconstructed from that node with zero wavelet parts).  src[w * n_in + i]
-// locates input i's source node (off < 0: the input has no node on the path
-// and contributes nothing).  Each workgroup owns its output blocks, so the
-// sums need no atomics; every thread adds into the same elements for every
-// input.
-__global__ __launch_bounds__(kMulThreads) void k_add_nodes(int n, const AddSrc *src, int n_in, int n_nodes,
-                                                           const double *pool, const double *coefs, const double *F,
-                                                           double *ws, double *out) {
+__global__ __launch_bounds__(kMulThreads) void k_add_nodes_any(int n, const AddSrc *src, int n_in, int n_nodes,
+                                                               const double *coefs, const double *F, double *ws,
+                                                               double *out) {
     const int tid = threadIdx.x;
     const int n3 = n * n * n;
     double *X = ws + (size_t)blockIdx.x * 16 * n3, *Y = X + 8 * n3;
@@ -222,13 +218,13 @@ __global__ __launch_bounds__(kMulThreads) void k_add_nodes(int n, const AddSrc *
         for (int e = tid; e < 8 * n3; e += kMulThreads) dst[e] = 0.0;
         for (int i = 0; i < n_in; i++) {
             const AddSrc sr = src[(size_t)w * n_in + i];
-            if (sr.off < 0) continue;
+            if (!sr.p) continue;
             const double c = coefs[i];
             if (sr.dep == 0) {
-                const double *b = pool + sr.off;
+                const double *b = sr.p;
                 for (int e = tid; e < 8 * n3; e += kMulThreads) dst[e] += c * b[e];
             } else {
-                descend(n, F, pool + sr.off, sr.dep, sr.path, X, Y, tid);
+                descend_any(n, F, sr.p, sr.dep, sr.path, X, Y, tid);
                 for (int e = tid; e < n3; e += kMulThreads) dst[e] += c * X[e];
                 __syncthreads();  // X is rewritten for the next input
             }
@@ -709,6 +705,71 @@ static hipError_t post_level(hipStream_t s, int n, bool down, const PostPair *pa
     }
 }
 
+// o[i] = sum over j of M[j][h N + i] v[j], j = 0 .. J - 1 in turn
+template <int N, int J>
+__device__ __forceinline__ void half_line(const double *v, const double *M, int h, double *o) {
+#pragma unroll
+    for (int i = 0; i < N; i++) o[i] = 0.0;
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+#pragma unroll
+        for (int i = 0; i < N; i++) o[i] = fma(M[j * 2 * N + h * N + i], v[j], o[i]);
+    }
+}
+
+// Scaling block of child `child` (bits x, y, z) of the node block src, its 8
+// components (FULL) or its scaling part alone, into X[0, N^3): the TopDown
+// branch of k_post_one without the addition.  Each pass keeps the half of its
+// outputs that leads to the child, one thread per line with the line in
+// registers.  src: global memory, or X itself; X holds 4 N^3 (FULL) or N^3
+// values, M the filter.  M and src must be in place before (a barrier);
+// ends with a barrier.  Threads: at least 4 N^2 (FULL) or N^2.
+template <int N, bool FULL>
+__device__ __forceinline__ void child_step(const double *src, double *X, const double *M, int child, int tid) {
+    constexpr int N3 = N * N * N, NN = N * N, J = FULL ? 2 * N : N;
+    const int q = tid / NN, ac = tid % NN, a = ac % N, c = ac / N;
+    double v[J], o[N];
+    // z: slot q = (ty, tx) from components q and q | 4
+    const bool lz = tid < (FULL ? 4 : 1) * NN;
+    if (lz) {
+#pragma unroll
+        for (int j = 0; j < J; j++) v[j] = src[(j < N ? q : q | 4) * N3 + post_index<N, 2>(a, c, j < N ? j : j - N)];
+        half_line<N, J>(v, M, child >> 2, o);
+    }
+    __syncthreads();  // src (which may be X) read before X is written
+    if (lz) {
+#pragma unroll
+        for (int i = 0; i < N; i++) X[q * N3 + post_index<N, 2>(a, c, i)] = o[i];
+    }
+    __syncthreads();
+    // y: slot tx from slots tx and tx | 2
+    const bool ly = tid < (FULL ? 2 : 1) * NN;
+    if (ly) {
+#pragma unroll
+        for (int j = 0; j < J; j++) v[j] = X[(j < N ? q : q | 2) * N3 + post_index<N, 1>(a, c, j < N ? j : j - N)];
+        half_line<N, J>(v, M, (child >> 1) & 1, o);
+    }
+    __syncthreads();
+    if (ly) {
+#pragma unroll
+        for (int i = 0; i < N; i++) X[q * N3 + post_index<N, 1>(a, c, i)] = o[i];
+    }
+    __syncthreads();
+    // x: slots 0 and 1
+    const bool lx = tid < NN;
+    if (lx) {
+#pragma unroll
+        for (int j = 0; j < J; j++) v[j] = X[(j < N ? 0 : 1) * N3 + post_index<N, 0>(a, c, j < N ? j : j - N)];
+        half_line<N, J>(v, M, child & 1, o);
+    }
+    __syncthreads();
+    if (lx) {
+#pragma unroll
+        for (int i = 0; i < N; i++) X[post_index<N, 0>(a, c, i)] = o[i];
+    }
+    __syncthreads();
+}
+
 // One generated node of an apply plan's pool: the scaling block dst of child
 // `child` (bits x, y, z) of a parent with block src, an input-tree node
 // (full: its 8 components) or a generated node (its scaling block only).
@@ -719,72 +780,23 @@ struct GenItem {
 };
 
 // Generated nodes of one depth (their parents are input nodes or generated
-// nodes of the depth above): one workgroup per child, the TopDown branch of
-// k_post_one without the addition.  Each pass keeps the half of its outputs
-// that leads to the child, one thread per line with the line in registers; a
-// launch holds few children and takes as long as one of them, so siblings
-// repeat the first passes rather than share them (one workgroup of 1024
-// threads per parent, a thread per output value: 80 -> 15 us a launch at
-// k = 9, 188 -> 42 us at k = 11).
+// nodes of the depth above): one workgroup per child.  A launch holds few
+// children and takes as long as one of them, so siblings repeat the first
+// passes rather than share them (one workgroup of 1024 threads per parent, a
+// thread per output value: 80 -> 15 us a launch at k = 9, 188 -> 42 us at
+// k = 11).
 template <int N>
 __global__ __launch_bounds__(PostOneShape<N>::T) void k_gen_fill(const GenItem *items, const double *__restrict__ F) {
-    constexpr int N3 = N * N * N, NN = N * N, N2 = 2 * N;
+    constexpr int N3 = N * N * N, N2 = 2 * N;
     __shared__ double X[4 * N3];
     __shared__ double M[N2 * N2];
     const int tid = threadIdx.x;
     const GenItem it = items[blockIdx.x];
     for (int e = tid; e < N2 * N2; e += PostOneShape<N>::T) M[e] = F[e];
-    const int hx = it.child & 1, hy = (it.child >> 1) & 1, hz = it.child >> 2;
-    double v[N2], o[N];
-    // a scaling-only parent has its first slot alone, and zero wavelet inputs
-    const int sh = it.full ? 0 : 2;
-    const int q = tid / NN, ac = tid % NN, a = ac % N, c = ac / N;
-#pragma unroll
-    for (int j = 0; j < N2; j++) v[j] = 0.0;
-    // z: slot q = (ty, tx) from components q and q | 4
-    if (tid < (4 >> sh) * NN) {
-#pragma unroll
-        for (int j = 0; j < N; j++) v[j] = it.src[q * N3 + post_index<N, 2>(a, c, j)];
-        if (it.full) {
-#pragma unroll
-            for (int j = 0; j < N; j++) v[N + j] = it.src[(q | 4) * N3 + post_index<N, 2>(a, c, j)];
-        }
-    }
-    __syncthreads();  // M in LDS
-    if (tid < (4 >> sh) * NN) {
-        post_half_line<N>(v, M, hz, o);
-#pragma unroll
-        for (int i = 0; i < N; i++) X[q * N3 + post_index<N, 2>(a, c, i)] = o[i];
-    }
     __syncthreads();
-    // y: slot tx from slots tx and tx | 2
-    if (tid < (it.full ? 2 : 1) * NN) {
-#pragma unroll
-        for (int j = 0; j < N; j++) v[j] = X[q * N3 + post_index<N, 1>(a, c, j)];
-        if (it.full) {
-#pragma unroll
-            for (int j = 0; j < N; j++) v[N + j] = X[(q | 2) * N3 + post_index<N, 1>(a, c, j)];
-        }
-        post_half_line<N>(v, M, hy, o);
-    }
-    __syncthreads();  // the slots of every line read before any is written
-    if (tid < (it.full ? 2 : 1) * NN) {
-#pragma unroll
-        for (int i = 0; i < N; i++) X[q * N3 + post_index<N, 1>(a, c, i)] = o[i];
-    }
-    __syncthreads();
-    // x: slots 0 and 1
-    if (tid < NN) {
-#pragma unroll
-        for (int j = 0; j < N; j++) v[j] = X[post_index<N, 0>(a, c, j)];
-        if (it.full) {
-#pragma unroll
-            for (int j = 0; j < N; j++) v[N + j] = X[N3 + post_index<N, 0>(a, c, j)];
-        }
-        post_half_line<N>(v, M, hx, o);
-#pragma unroll
-        for (int i = 0; i < N; i++) it.dst[post_index<N, 0>(a, c, i)] = o[i];
-    }
+    if (it.full) child_step<N, true>(it.src, X, M, it.child, tid);
+    else child_step<N, false>(it.src, X, M, it.child, tid);
+    for (int e = tid; e < N3; e += PostOneShape<N>::T) it.dst[e] = X[e];
 }
 
 static hipError_t gen_fill(hipStream_t s, int n, const GenItem *items, int cnt, const double *F) {
@@ -798,6 +810,173 @@ static hipError_t gen_fill(hipStream_t s, int n, const GenItem *items, int cnt, 
         default: return hipErrorInvalidValue;
     }
 #undef MWG_GEN
+    return hipGetLastError();
+}
+
+// Scaling block of the node `dep` >= 1 levels below the node block src (8
+// components) along `path` (3 bits per level, first level lowest) into
+// X[0, N^3); ends with a barrier.
+template <int N>
+__device__ __forceinline__ void descend(const double *src, int dep, unsigned long long path, double *X,
+                                        const double *M, int tid) {
+    child_step<N, true>(src, X, M, (int)(path & 7), tid);
+    for (int lv = 1; lv < dep; lv++) child_step<N, false>(X, X, M, (int)((path >> (3 * lv)) & 7), tid);
+}
+
+// Products: the block of output node w from both inputs' values at its 8
+// children's points.  One workgroup per node holds the 8 N^3 values in LDS,
+// every transform pass in place with the lines in registers (post_line_pass),
+// the first input's values in registers while the second's are made: the
+// inputs are read once and the output written once.  (1024 workgroups with a
+// work area of 24 N^3 values each in global memory and a thread per value of a
+// pass, N = 8, 990 nodes: 958 us; here 109 us, of which the LDS reads of the
+// filter are the larger part.)
+template <int N>
+__global__ __launch_bounds__(PostShape<N>::T) void k_mul_nodes(const MulNode *nodes, const double *pool_a,
+                                                            const double *pool_b, const double *__restrict__ F,
+                                                            const double *__restrict__ wsc, double coef,
+                                                            double *out) {
+    constexpr int N3 = N * N * N, N2 = 2 * N, T = PostShape<N>::T, E = 8 * N3, K = (E + T - 1) / T;
+    __shared__ double blk[E];
+    __shared__ double M[N2 * N2], MT[N2 * N2];  // the filter (reconstruct) and its transpose (compress)
+    const int tid = threadIdx.x;
+    const MulNode nd = nodes[blockIdx.x];
+    for (int e = tid; e < N2 * N2; e += T) {
+        M[e] = F[e];
+        MT[e] = F[(e % N2) * N2 + e / N2];
+    }
+    __syncthreads();
+    auto children = [&](const double *src, int dep, unsigned path) {
+        if (dep == 0) {
+#pragma unroll 8
+            for (int e = tid; e < E; e += T) blk[e] = src[e];
+        } else {
+            descend<N>(src, dep, path, blk, M, tid);
+            // the work node's block: its scaling part, wavelet parts zero
+            for (int e = N3 + tid; e < E; e += T) blk[e] = 0.0;
+        }
+        __syncthreads();
+        post_line_pass<N, 2>(blk, M, tid);
+        __syncthreads();
+        post_line_pass<N, 1>(blk, M, tid);
+        __syncthreads();
+        post_line_pass<N, 0>(blk, M, tid);
+        __syncthreads();
+    };
+    children(pool_a + nd.src_a, nd.dep_a, nd.path_a);
+    double va[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int e = tid + k * T;
+        va[k] = e < E ? coef * blk[e] : 0.0;
+    }
+    __syncthreads();
+    children(pool_b + nd.src_b, nd.dep_b, nd.path_b);
+    // the product at the children's points, back to coefficients
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int e = tid + k * T;
+        if (e < E) blk[e] = va[k] * blk[e] * nd.hfac * wsc[e % N3];
+    }
+    __syncthreads();
+    post_line_pass<N, 0>(blk, MT, tid);
+    __syncthreads();
+    post_line_pass<N, 1>(blk, MT, tid);
+    __syncthreads();
+    post_line_pass<N, 2>(blk, MT, tid);
+    __syncthreads();
+    double *dst = out + (size_t)blockIdx.x * E;
+#pragma unroll 8
+    for (int e = tid; e < E; e += T) dst[e] = blk[e];
+}
+
+// Sums: out block of node w = sum_i coefs[i] x (input i's block at the node,
+// or, below the input's finest node on the path, the scaling part
+// reconstructed from that node with zero wavelet parts).  src[w n_in + i]
+// locates input i's source block (null: the input has no node on the path and
+// contributes nothing).  One workgroup per node; each thread sums its values
+// of the node in registers over the inputs and stores them once.  (Summed in
+// global memory with the passes in a global work area, N = 8, 3160 nodes of 8
+// inputs: 2.15 ms; here 0.26 ms.)
+template <int N>
+__global__ __launch_bounds__(PostOneShape<N>::T) void k_add_nodes(const AddSrc *src, int n_in, const double *coefs,
+                                                               const double *__restrict__ F, double *out) {
+    constexpr int N3 = N * N * N, N2 = 2 * N, T = PostOneShape<N>::T, E = 8 * N3, K = (E + T - 1) / T;
+    __shared__ double X[4 * N3];
+    __shared__ double M[N2 * N2];
+    const int tid = threadIdx.x;
+    for (int e = tid; e < N2 * N2; e += T) M[e] = F[e];
+    __syncthreads();
+    double acc[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) acc[k] = 0.0;
+    for (int i = 0; i < n_in; i++) {
+        const AddSrc sr = src[(size_t)blockIdx.x * n_in + i];
+        if (!sr.p) continue;
+        const double c = coefs[i];
+        if (sr.dep == 0) {
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const int e = tid + k * T;
+                if (e < E) acc[k] += c * sr.p[e];
+            }
+        } else {
+            descend<N>(sr.p, sr.dep, sr.path, X, M, tid);
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const int e = tid + k * T;
+                if (e < N3) acc[k] += c * X[e];
+            }
+            __syncthreads();  // X is rewritten for the next input
+        }
+    }
+    double *dst = out + (size_t)blockIdx.x * E;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int e = tid + k * T;
+        if (e < E) dst[e] = acc[k];
+    }
+}
+
+#define MWG_NODE_SIZES(CASE) \
+    CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12)
+
+static hipError_t mul_nodes(hipStream_t s, int n, int cnt, const MulNode *nodes, const double *pa, const double *pb,
+                            const double *F, const double *wsc, double coef, double *ws, int ws_blocks, double *out) {
+    if (n > 12) {
+        hipLaunchKernelGGL(k_mul_nodes_any, dim3(std::min(cnt, ws_blocks)), dim3(kMulThreads), 0, s, n, nodes, cnt, pa,
+                           pb, F, wsc, coef, ws, out);
+        return hipGetLastError();
+    }
+#define MWG_CASE(NN)                                                                                            \
+    case NN:                                                                                                    \
+        hipLaunchKernelGGL((k_mul_nodes<NN>), dim3(cnt), dim3(PostShape<NN>::T), 0, s, nodes, pa, pb, F, wsc,   \
+                           coef, out);                                                                          \
+        break;
+    switch (n) {
+        MWG_NODE_SIZES(MWG_CASE)
+        default: return hipErrorInvalidValue;
+    }
+#undef MWG_CASE
+    return hipGetLastError();
+}
+
+static hipError_t add_nodes(hipStream_t s, int n, int cnt, const AddSrc *src, int n_in, const double *coefs,
+                            const double *F, double *ws, double *out) {
+    if (n > 12) {
+        hipLaunchKernelGGL(k_add_nodes_any, dim3(std::min(cnt, kMulBlocks)), dim3(kMulThreads), 0, s, n, src, n_in, cnt,
+                           coefs, F, ws, out);
+        return hipGetLastError();
+    }
+#define MWG_CASE(NN)                                                                                              \
+    case NN:                                                                                                      \
+        hipLaunchKernelGGL((k_add_nodes<NN>), dim3(cnt), dim3(PostOneShape<NN>::T), 0, s, src, n_in, coefs, F, out); \
+        break;
+    switch (n) {
+        MWG_NODE_SIZES(MWG_CASE)
+        default: return hipErrorInvalidValue;
+    }
+#undef MWG_CASE
     return hipGetLastError();
 }
 
@@ -1137,7 +1316,7 @@ void dev_free(DeviceCtx *c, void *p) {
 // host code its name is a host-side stand-in: kernels and copies get its
 // device address, taken once per device by dev_noalloc_init.
 constexpr size_t kNoAllocBytes = (size_t)128 << 20;
-constexpr int kNoAllocBlocks = 64;  // workgroups of an allocation-free launch
+constexpr int kNoAllocBlocks = 64;  // work areas reserved for an allocation-free launch (used at n > 12)
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
 int dev_noalloc_init(DeviceCtx *c, std::string &err) {
@@ -1263,7 +1442,7 @@ int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a
     }
     if (!rc) rc = up(mra.basis.F.data(), mra.basis.F.size(), &m->F);
     if (!rc) rc = up(wsc.data(), wsc.size(), &m->wsc);
-    if (!rc) rc = dev_mem(c, (size_t)kMulBlocks * 24 * n3, &m->ws, err);
+    if (!rc && n > 12) rc = dev_mem(c, (size_t)kMulBlocks * 24 * n3, &m->ws, err);
     if (rc) {
         (void)hipStreamSynchronize(s);
         delete m;
@@ -1285,10 +1464,8 @@ int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double co
         for (size_t c0 = 0; c0 < nodes.size(); c0 += m->chunk) {
             const size_t cn = std::min(m->chunk, nodes.size() - c0);
             HIP_TRY(hipMemcpyAsync(m->dn, nodes.data() + c0, sizeof(MulNode) * cn, hipMemcpyHostToDevice, s));
-            const int grid = (int)std::min<size_t>(cn, kNoAllocBlocks);
-            hipLaunchKernelGGL(k_mul_nodes, dim3(grid), dim3(kMulThreads), 0, s, m->n, m->dn, (int)cn, m->pool_a,
-                               m->pool_b, m->F, m->wsc, coef, m->ws, m->dout);
-            HIP_TRY(hipGetLastError());
+            HIP_TRY(mul_nodes(s, m->n, (int)cn, m->dn, m->pool_a, m->pool_b, m->F, m->wsc, coef, m->ws,
+                              kNoAllocBlocks, m->dout));
             HIP_TRY(hipMemcpyAsync(out_blocks + c0 * 8 * n3, m->dout, sizeof(double) * cn * 8 * n3,
                                    out_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
             HIP_TRY(hipStreamSynchronize(s));
@@ -1306,10 +1483,8 @@ int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double co
     }
     hipError_t e = hipMemcpyAsync(dn, nodes.data(), sizeof(MulNode) * nodes.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        const int grid = (int)std::min<size_t>(nodes.size(), kMulBlocks);
-        hipLaunchKernelGGL(k_mul_nodes, dim3(grid), dim3(kMulThreads), 0, s, m->n, dn, (int)nodes.size(), m->pool_a,
-                           m->pool_b, m->F, m->wsc, coef, m->ws, dout);
-        e = hipGetLastError();
+        e = mul_nodes(s, m->n, (int)nodes.size(), dn, m->pool_a, m->pool_b, m->F, m->wsc, coef, m->ws,
+                      kMulBlocks, dout);
     }
     int crc = 0;
     if (e == hipSuccess && !out_on_device)
@@ -1341,8 +1516,9 @@ struct DevAddSession {
     }
 };
 
-int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &pool, const std::vector<double> &coefs,
-                  DevAddSession **out, std::string &err) {
+int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &inputs,
+                  const std::vector<double> &coefs, DevAddSession **out, std::vector<const double *> &base,
+                  std::string &err) {
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
     auto *m = new DevAddSession;
@@ -1350,33 +1526,38 @@ int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &
     m->n = mra.kp1();
     m->n_in = (int)coefs.size();
     const int n3 = m->n * m->n * m->n;
-    auto up = [&](const std::vector<double> &v, double **d) -> int {
-        if (int rc = dev_mem(c, v.size(), d, err)) return rc;
-        if (!v.empty()) HIP_TRY(hipMemcpyAsync(*d, v.data(), sizeof(double) * v.size(), hipMemcpyHostToDevice, s));
+    auto up = [&](const double *v, size_t nv, double **d) -> int {
+        if (int rc = dev_mem(c, nv, d, err)) return rc;
+        if (nv) HIP_TRY(hipMemcpyAsync(*d, v, sizeof(double) * nv, hipMemcpyHostToDevice, s));
         return 0;
     };
-    // the pool: the sources one after another, copied from host or device
+    // host inputs one after another in the session's pool; device inputs are
+    // read in place
     size_t total = 0;
-    for (const BlockSource &b : pool) total += b.n;
-    int rc = dev_mem(c, total, &m->pool, err);
-    if (!rc) {
-        hipError_t e = hipSuccess;
-        size_t off = 0;
-        for (const BlockSource &b : pool) {
-            if (e != hipSuccess) break;
-            if (b.n)
-                e = hipMemcpyAsync(m->pool + off, b.p, sizeof(double) * b.n,
-                                   b.on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s);
-            off += b.n;
+    for (const BlockSource &b : inputs)
+        if (!b.on_device) total += b.n;
+    int rc = total ? dev_mem(c, total, &m->pool, err) : 0;
+    base.clear();
+    size_t off = 0;
+    for (const BlockSource &b : inputs) {
+        if (rc) break;
+        if (b.on_device) {
+            base.push_back(b.p);
+            continue;
         }
-        if (e != hipSuccess) {
-            err = std::string("add pool: ") + hipGetErrorString(e);
-            rc = -2;
+        if (b.n) {
+            hipError_t e = hipMemcpyAsync(m->pool + off, b.p, sizeof(double) * b.n, hipMemcpyHostToDevice, s);
+            if (e != hipSuccess) {
+                err = std::string("add pool: ") + hipGetErrorString(e);
+                rc = -2;
+            }
         }
+        base.push_back(m->pool + off);
+        off += b.n;
     }
-    if (!rc) rc = up(coefs, &m->coefs);
-    if (!rc) rc = up(mra.basis.F, &m->F);
-    if (!rc) rc = dev_mem(c, (size_t)kMulBlocks * 16 * n3, &m->ws, err);
+    if (!rc) rc = up(coefs.data(), coefs.size(), &m->coefs);
+    if (!rc) rc = up(mra.basis.F.data(), mra.basis.F.size(), &m->F);
+    if (!rc && m->n > 12) rc = dev_mem(c, (size_t)kMulBlocks * 16 * n3, &m->ws, err);
     if (rc) {
         (void)hipStreamSynchronize(s);
         delete m;
@@ -1408,10 +1589,7 @@ int dev_add_nodes(DevAddSession *m, const std::vector<AddSrc> &src, double *out_
     }
     hipError_t e = hipMemcpyAsync(dsrc, src.data(), sizeof(AddSrc) * src.size(), hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        const int grid = (int)std::min<size_t>(n_nodes, kMulBlocks);
-        hipLaunchKernelGGL(k_add_nodes, dim3(grid), dim3(kMulThreads), 0, s, m->n, dsrc, m->n_in, (int)n_nodes,
-                           m->pool, m->coefs, m->F, m->ws, dout);
-        e = hipGetLastError();
+        e = add_nodes(s, m->n, (int)n_nodes, dsrc, m->n_in, m->coefs, m->F, m->ws, dout);
     }
     int crc = 0;
     if (e == hipSuccess && !out_on_device)

@@ -1153,13 +1153,13 @@ bool mul_source(const Tree &f, const NodeKey &k, long long &off, int &dep, unsig
     return false;
 }
 
-// Source node of input f for the sum at output node k: f's deepest node on
-// the path, its block offset (base + index x block), the levels below it and
-// the child index of each level.  An input without any node on the path
-// (an empty tree) gets off = -1.  False when the node lies more than
+// Source node of input f (its blocks at base on the device) for the sum at
+// output node k: f's deepest node on the path, the levels below it and the
+// child index of each level.  An input without any node on the path (an empty
+// tree) gets p = null.  False when the node lies more than
 // kAddMaxLevels levels below f's finest node on the path.
-bool add_source(const Tree &f, const NodeKey &k, long long base, AddSrc &sr) {
-    sr.off = -1;
+bool add_source(const Tree &f, const NodeKey &k, const double *base, AddSrc &sr) {
+    sr.p = nullptr;
     sr.dep = 0;
     sr.pad_ = 0;
     sr.path = 0;
@@ -1175,7 +1175,7 @@ bool add_source(const Tree &f, const NodeKey &k, long long base, AddSrc &sr) {
             for (int q = 0; q < 3; q++) t |= (unsigned long long)((k.l[q] >> (k.depth - d - lv)) & 1) << q;
             sr.path |= t << (3 * (lv - 1));
         }
-        sr.off = base + (long long)idx * f.mra->block();
+        sr.p = base + (long long)idx * f.mra->block();
         return true;
     }
     return true;
@@ -1302,10 +1302,9 @@ int add_trees(mwg_context ctx, double prec, Tree &T, const std::vector<mwg_tree>
     const bool on_device = dres != nullptr;
     TempBlocks tb{ctx->dev, {}};
     std::vector<BlockSource> pool;
-    std::vector<long long> base(ins.size());
+    std::vector<const double *> base;
     size_t total = 0;
     for (size_t i = 0; i < ins.size(); i++) {
-        base[i] = (long long)total;
         bool on_dev = false;
         const double *p = input_blocks(ctx, ins[i], tb, false, on_dev);
         pool.push_back(BlockSource{p, tree_values(ins[i]), on_dev});
@@ -1331,7 +1330,7 @@ int add_trees(mwg_context ctx, double prec, Tree &T, const std::vector<mwg_tree>
     }
     std::string err;
     DevAddSession *m = nullptr;
-    dev_check(dev_add_begin(ctx->dev, mra, pool, coefs, &m, err), err);
+    dev_check(dev_add_begin(ctx->dev, mra, pool, coefs, &m, base, err), err);
     std::unique_ptr<DevAddSession, void (*)(DevAddSession *)> session(m, dev_add_end);
     DeviceLevels lv{ctx->dev, blk, mra.kp1(), {}, {}, {}, {}};
     const size_t n_in = ins.size();
