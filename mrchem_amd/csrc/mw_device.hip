@@ -687,13 +687,13 @@ __device__ __forceinline__ int screen_items(const KArgs &a, const AppDesc &ad, c
 }
 
 template <int N, bool PAIR>
-__device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int seg, int comp, double lo_mult, double hi_mult,
+__device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int seg, double lo_mult, double hi_mult,
                                          Smem4<N> &sm) {
     using S = Job4<N>;
     constexpr int N2 = S::N2, N3 = S::N3, G = S::G, NP = S::NP, CT = S::CT, P = S::P, LPD = S::LPD;
     const int lane = threadIdx.x, lc = lane & 15, lq = lane >> 4, l3 = lane & 3;
     const AppDesc &ad = a.apps[a.out_app[a.seg_job[seg] >> 3]];
-    const JobCtx j = job_ctx(a, ad, a.seg_job[seg] | comp, lo_mult, hi_mult);
+    const JobCtx j = job_ctx(a, ad, a.seg_job[seg], lo_mult, hi_mult);
     const int *gb = j.gb;
     const double *tn = a.tn + a.tn_off[ad.act_base + j.d];
     const int2 *tb = a.tb + j.a0;
@@ -962,12 +962,15 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
 }
 
 // Persistent launch of one-wave workgroups over a queue of segments
-// seg_list[0, n) (or seg0 .. seg0 + n - 1 without a list), the terms in the
-// class (lo_mult thr_cls, hi_mult thr_cls].
+// seg_list[0, n) (or 0 .. n - 1 without a list), the terms in the class
+// (lo_mult thr_cls, hi_mult thr_cls].  n_dev: the number of segments on the
+// device, n the room they had; with more than that nothing is done, the host
+// cuts again and launches again.
 template <int N, bool PAIR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Job4<N>::WPE))) void k_apply64(
-    KArgs a, const double *pool, const int *seg_list, int seg0, int n, double lo_mult, double hi_mult,
-    unsigned long long *head) {
+    KArgs a, const double *pool, const int *seg_list, const unsigned long long *n_dev, int n, double lo_mult,
+    double hi_mult, unsigned long long *head) {
+    if (n_dev) n = *n_dev <= (unsigned long long)n ? (int)*n_dev : 0;
     __shared__ Smem4<N> sm;
     // what the passes never write stays zero (padding rows, columns and
     // operator elements)
@@ -978,12 +981,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Job4<N>::WPE
         if (threadIdx.x == 0) e = (int)atomicAdd(head, 1ull);
         e = __builtin_amdgcn_readfirstlane(e);
         if (e >= n) break;
-        const int seg = seg_list ? seg_list[e] : seg0 + e;
-        if constexpr (PAIR && N >= 99) {
-            for (int c = 0; c < 8; c += 4) segment4<N, false>(a, pool, seg, c, lo_mult, hi_mult, sm);
-        } else {
-            segment4<N, PAIR>(a, pool, seg, 0, lo_mult, hi_mult, sm);
-        }
+        segment4<N, PAIR>(a, pool, seg_list ? seg_list[e] : e, lo_mult, hi_mult, sm);
     }
 }
 
@@ -1842,6 +1840,17 @@ struct DevicePlan {
     double *post_F = nullptr, *post_norms = nullptr;
     // the root level's dense products (n_items 0: none)
     RootLaunch root;
+    // The counts and the cut.  The result block on the device is [counters: 8]
+    // [totals: 2 per apply][segments: 2][squared norms: 2 n_out], so that a run
+    // brings what the host wants of it with one copy.  cut_open: the host has
+    // not seen the totals yet (a plan made to run once); until then the plan
+    // keeps what the enqueued work reads.
+    CountArgs count;
+    unsigned long long *result = nullptr;
+    size_t n_tot = 0;
+    bool cut_open = false;
+    std::vector<void *> temp;
+    std::vector<unsigned char, UninitAlloc<unsigned char>> stage, fill_stage;
     // the captured step (step_graph) and what it was captured for
     hipGraphExec_t graph = nullptr;
     int graph_mode = -1;
@@ -1850,6 +1859,8 @@ struct DevicePlan {
     unsigned ran_eager = 0;  // bit 2 mode + post: an eager run of that step happened
     ~DevicePlan() {
         if (graph) (void)hipGraphExecDestroy(graph);
+        if (cut_open) (void)hipStreamSynchronize(ctx->stream);
+        for (void *p : temp) dev_mem_put(ctx, p);
         for (void *p : bufs) dev_mem_put(ctx, p);
         for (void *p : {(void *)pool32, (void *)pool_h, (void *)pool_hsc, (void *)list_hi, (void *)list_lo})
             dev_mem_put(ctx, p);
@@ -2168,8 +2179,56 @@ static int upload_at(T *dst, const std::vector<T, A> &v, hipStream_t s, std::str
     return 0;
 }
 
-int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, DevicePlan **out,
-                    std::string &err) {
+// Room for cap segments and the cut into it (again: the counts of a first cut
+// are cleared).  Launches only.
+static int cut_plan(DevicePlan *p, const long long *cap, bool bounds, bool again, std::string &err) {
+    DeviceCtx *c = p->ctx;
+    CountArgs &ca = p->count;
+    const long long n_all = cap[0] + cap[1];
+    if (n_all >= (1LL << 31)) {
+        err = "batch too large for 32-bit node, segment or slot indices";
+        return -1;
+    }
+    int *seg = nullptr;
+    int rc = plan_alloc(p, (size_t)(3 * n_all), &seg, err);
+    if (rc) return rc;
+    if (bounds) {
+        if ((rc = dev_mem(c, (size_t)n_all, &ca.rec, err))) return rc;
+        p->temp.push_back(ca.rec);
+    }
+    for (int i = 0; i < 2; i++) ca.cap[i] = (int)cap[i];
+    p->args.seg_job = ca.seg_job = seg;
+    p->args.seg_p0 = ca.seg_p0 = seg + n_all;
+    p->args.seg_p1 = ca.seg_p1 = seg + 2 * n_all;
+    if (again) {
+        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, ca.n_seg, 2);
+        HIP_TRY(hipGetLastError());
+    }
+    return dev_cut_segments(c->stream, ca, bounds, err);
+}
+
+// The totals have come to the host: true when the segments fit their room.
+static bool cut_fits(DevicePlan *p, const unsigned long long *tot) {
+    const unsigned long long *n = tot + p->n_tot - 2;
+    if (n[0] > (unsigned long long)p->count.cap[0] || n[1] > (unsigned long long)p->count.cap[1]) return false;
+    p->n_pseg = (int)n[0];
+    p->n_fseg = (int)n[1];
+    p->term_apps = 0;
+    for (size_t i = 0; i + 2 < p->n_tot; i += 2) p->term_apps += tot[i];
+    return true;
+}
+
+// Frees what only the cut needed.
+static void cut_done(DevicePlan *p) {
+    p->cut_open = false;
+    for (void *q : p->temp) dev_mem_put(p->ctx, q);
+    p->temp.clear();
+    p->stage = decltype(p->stage)();
+    p->fill_stage = decltype(p->fill_stage)();
+}
+
+int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, bool once,
+                    DevicePlan **out, std::string &err) {
     HIP_TRY(hipSetDevice(c->device));
     if (parts.empty()) {
         err = "empty plan";
@@ -2301,14 +2360,17 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     const size_t f_bw = place(sizeof(int) * n_bw), f_act_off = place(sizeof(int) * n_actoff);
     const size_t f_act = place(sizeof(int) * n_act);
     const size_t f_apps = place(sizeof(AppDesc) * parts.size());
-    const size_t f_cnt = place(sizeof(unsigned long long) * 8);
-    // apply totals (terms, dense terms) and the two segment counts
-    const size_t n_tot = 2 * parts.size() + 2, f_tot = place(sizeof(unsigned long long) * n_tot);
+    // cleared counters, and per apply its terms and dense terms, and the two
+    // segment counts (the result block's head; its norms come behind it)
+    const size_t n_tot = 2 * parts.size() + 2;
     const size_t f_ra = place(sizeof(RootApp) * root_apps.size()), f_ri = place(sizeof(RootItem) * root_items.size());
     const size_t f_rs = place(sizeof(long long) * root_slot_off.size()), f_ro = place(sizeof(int) * root_out.size());
     const size_t f_dense = place((size_t)n_out), f_tno = place(sizeof(long long) * tn_off.size());
     const size_t f_lv = place(sizeof(TermLevel) * levels.size());
-    const size_t up_bytes = arena;
+    const size_t f_res = place(sizeof(unsigned long long) * (8 + n_tot));
+    const size_t up_bytes = f_res + sizeof(unsigned long long) * (8 + n_tot);
+    arena = up_bytes + sizeof(double) * 2 * n_out;
+    arena = (arena + 255) / 256 * 256;
     const size_t f_norm = place(sizeof(double) * 8 * n_slot), f_tn = place(sizeof(double) * n_tn);
     const size_t f_tb = place(sizeof(int2) * n_act);
     std::vector<size_t> f_mt(parts.size());
@@ -2325,14 +2387,14 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         if (!rc) rc = plan_alloc(p.get(), ny, &p->root.Y, err);
     }
     if (rc) return rc;
-    std::vector<unsigned char, UninitAlloc<unsigned char>> stage(up_bytes), fill_stage;
-    auto at = [&](size_t f) { return stage.data() + f; };
+    p->stage.resize(up_bytes);
+    p->cut_open = true;  // from here on the plan waits for the stream when it is dropped
+    auto at = [&](size_t f) { return p->stage.data() + f; };
     auto put = [&](size_t f, long long off, const auto &v) {
         using T = typename std::decay_t<decltype(v)>::value_type;
         if (!v.empty()) std::memcpy(at(f) + sizeof(T) * off, v.data(), sizeof(T) * v.size());
     };
-    std::memset(at(f_cnt), 0, sizeof(unsigned long long) * 8);
-    std::memset(at(f_tot), 0, sizeof(unsigned long long) * n_tot);
+    std::memset(at(f_res), 0, sizeof(unsigned long long) * (8 + n_tot));
     std::memset(at(f_dense), 0, (size_t)n_out);
     long long o_out = 0, o_band = 0, o_slot = 0, o_pool = 0, o_bw = 0, o_actoff = 0, o_act = 0;
     std::vector<PoolFill> fills;
@@ -2402,7 +2464,8 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     put(f_tno, 0, tn_off);
     put(f_lv, 0, levels);
     p->d_apps = reinterpret_cast<AppDesc *>(dev + f_apps);
-    a.counters = reinterpret_cast<unsigned long long *>(dev + f_cnt);
+    p->result = a.counters = reinterpret_cast<unsigned long long *>(dev + f_res);
+    p->n_tot = n_tot;
     a.out_depth = reinterpret_cast<const int *>(dev + f_out_depth);
     a.out_app = reinterpret_cast<const int *>(dev + f_out_app);
     a.out_thr = reinterpret_cast<const double *>(dev + f_thr);
@@ -2420,31 +2483,22 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     a.apps = p->d_apps;
     // counts per (output component, band position)
     const bool bounds = mode != 0;
-    struct Temp {
-        DeviceCtx *c;
-        std::vector<void *> p;
-        ~Temp() {
-            // the staging buffers of a failed plan may still be read
-            (void)hipStreamSynchronize(c->stream);
-            for (void *q : p) dev_mem_put(c, q);
-        }
-    } temp{c, {}};
-    auto tmp = [&](size_t n, auto **out) {
-        const int r = dev_mem(c, n, out, err);
-        if (!r) temp.p.push_back(*out);
+    auto tmp = [&](size_t n, auto **o) {
+        const int r = dev_mem(c, n, o, err);
+        if (!r) p->temp.push_back(*o);
         return r;
     };
-    CountArgs ca;
+    CountArgs &ca = p->count;
     ca.n_out = (int)n_out;
     ca.n_app = (int)parts.size();
     ca.n_share = (int)parts.size();
     ca.dense = dev + f_dense;
-    ca.totals = reinterpret_cast<unsigned long long *>(dev + f_tot);
+    ca.totals = p->result + 8;
     ca.n_seg = ca.totals + 2 * parts.size();
     if ((rc = tmp((size_t)(8 * n_band), &ca.cnt))) return rc;
     if (bounds && ((rc = tmp((size_t)(8 * n_band), &ca.bmin)) || (rc = tmp((size_t)(8 * n_band), &ca.bmax)))) return rc;
-    HIP_TRY(hipMemcpyAsync(dev, stage.data(), up_bytes, hipMemcpyHostToDevice, s));
-    rc = dev_pool_fill(c, mra, fills, reinterpret_cast<double *>(dev + f_norm), fill_stage, err);
+    HIP_TRY(hipMemcpyAsync(dev, p->stage.data(), up_bytes, hipMemcpyHostToDevice, s));
+    rc = dev_pool_fill(c, mra, fills, reinterpret_cast<double *>(dev + f_norm), p->fill_stage, err);
     if (!rc)
         rc = dev_term_tables(s, a, N * N, reinterpret_cast<const TermLevel *>(dev + f_lv), (int)levels.size(),
                              reinterpret_cast<double *>(dev + f_tn), reinterpret_cast<int2 *>(dev + f_tb), err);
@@ -2454,47 +2508,8 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     // Room for the segments: what a small launch can hold and 16 (fine ones
     // 24, plain FP64's 64) for each output node; the few plans that need more
     // are cut again.
-    std::vector<unsigned long long> tot(n_tot);
     long long cap[2] = {bounds ? 2048 + 16 * n_out : 16384 + 64 * n_out, bounds ? 16384 + 24 * n_out : 0};
-    int *seg = nullptr;
-    SegRec *rec = nullptr;
-    for (int attempt = 0;; attempt++) {
-        const long long n_all = cap[0] + cap[1];
-        if (n_all >= (1LL << 31)) {
-            err = "batch too large for 32-bit node, segment or slot indices";
-            return -1;
-        }
-        if ((rc = plan_alloc(p.get(), (size_t)(3 * n_all), &seg, err))) return rc;
-        if (bounds && (rc = tmp((size_t)n_all, &rec))) return rc;
-        for (int i = 0; i < 2; i++) ca.cap[i] = (int)cap[i];
-        ca.seg_job = seg;
-        ca.seg_p0 = seg + n_all;
-        ca.seg_p1 = seg + 2 * n_all;
-        ca.rec = rec;
-        if (attempt) {
-            hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, ca.n_seg, 2);
-            HIP_TRY(hipGetLastError());
-        }
-        if ((rc = dev_cut_segments(s, ca, bounds, err))) return rc;
-        HIP_TRY(hipMemcpyAsync(tot.data(), ca.totals, sizeof(unsigned long long) * n_tot, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        const long long need[2] = {(long long)tot[n_tot - 2], (long long)tot[n_tot - 1]};
-        if (need[0] <= cap[0] && need[1] <= cap[1]) {
-            p->n_pseg = (int)need[0];
-            p->n_fseg = (int)need[1];
-            break;
-        }
-        for (int i = 0; i < 2; i++) cap[i] = std::max(cap[i], need[i]);
-        p->bufs.pop_back();
-        dev_mem_put(c, seg);
-    }
-    for (size_t ai = 0; ai < parts.size(); ai++) {
-        p->term_apps += tot[2 * ai];
-        p->root.apps_count += tot[2 * ai + 1];
-    }
-    a.seg_job = ca.seg_job;
-    a.seg_p0 = ca.seg_p0;
-    a.seg_p1 = ca.seg_p1;
+    if ((rc = cut_plan(p.get(), cap, bounds, false, err))) return rc;
     if (!root_items.empty()) {
         RootLaunch &r = p->root;
         r.apps = reinterpret_cast<const RootApp *>(dev + f_ra);
@@ -2504,6 +2519,27 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         r.root_out = reinterpret_cast<const int *>(dev + f_ro);
         r.pool = p->pool;
         r.counter = a.counters;
+        r.totals = ca.totals;
+        r.n_totals = (int)parts.size();
+    }
+    // One wait per refinement level instead of three: the calculator starts
+    // behind the cut, and counters, segment counts and norms come back in one
+    // copy after it (single-Gaussian Coulomb apply at k = 7: 2.74 to 2.43 ms;
+    // the exchange applies of 4 orbitals in one batch: 12.0 to 10.5 ms, with
+    // the one-launch assembly of the trees).
+    if (once && !bounds) {
+        *out = p.release();
+        return 0;
+    }
+    std::vector<unsigned long long> tot(n_tot);
+    while (true) {
+        HIP_TRY(hipMemcpyAsync(tot.data(), ca.totals, sizeof(unsigned long long) * n_tot, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        if (cut_fits(p.get(), tot.data())) break;
+        for (int i = 0; i < 2; i++) cap[i] = std::max<long long>(cap[i], (long long)tot[n_tot - 2 + i]);
+        p->bufs.pop_back();
+        dev_mem_put(c, ca.seg_job);
+        if ((rc = cut_plan(p.get(), cap, bounds, true, err))) return rc;
     }
     if (bounds) {
         // what the class lists of the mixed and split modes are chosen from,
@@ -2531,6 +2567,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         meta(r.data(), p->n_pseg, 0, p->psegs);
         meta(r.data() + p->n_pseg, p->n_fseg, (int)cap[0], p->fsegs);
     }
+    cut_done(p.get());
     *out = p.release();
     return 0;
 }
@@ -2638,14 +2675,15 @@ static int launch32_n(DeviceCtx *c, const KArgs &a, const float *pool, const int
 }
 
 template <int N, bool PAIR>
-static int launch64_n(DeviceCtx *c, const KArgs &a, const double *pool, const int *list, int seg0, int n, double lo,
-                      unsigned long long *head, hipStream_t s, std::string &err) {
+static int launch64_n(DeviceCtx *c, const KArgs &a, const double *pool, const int *list,
+                      const unsigned long long *n_dev, int n, double lo, unsigned long long *head, hipStream_t s, std::string &err) {
     if (n == 0) return 0;
     int grid = 0;
     int rc = persistent_grid(c, reinterpret_cast<const void *>(&k_apply64<N, PAIR>), 64, sizeof(Smem4<N>), 0, n, &grid,
                              err);
     if (rc) return rc;
-    hipLaunchKernelGGL((k_apply64<N, PAIR>), dim3(grid), dim3(64), 0, s, a, pool, list, seg0, n, lo, HUGE_VAL, head);
+    hipLaunchKernelGGL((k_apply64<N, PAIR>), dim3(grid), dim3(64), 0, s, a, pool, list, n_dev, n, lo, HUGE_VAL,
+                       head);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -2675,14 +2713,14 @@ static int launch32(const DevicePlan *p, const int *list, int n, double hi, unsi
 #undef MWG_LAUNCH
 }
 
-// Persistent FP64 launch over the pair segments seg0 .. seg0 + n - 1 (no
-// list), or over the single-component segments list[0, n): bounds above lo
-// thr_cls.
-static int launch64(const DevicePlan *p, const int *list, int n, double lo, unsigned long long *head, hipStream_t s,
-                    std::string &err) {
+// Persistent FP64 launch over the pair segments 0 .. n - 1 (no list; n_dev: as
+// many as it holds, n at most), or over the single-component segments list[0, n):
+// bounds above lo thr_cls.
+static int launch64(const DevicePlan *p, const int *list, const unsigned long long *n_dev, int n, double lo,
+                    unsigned long long *head, hipStream_t s, std::string &err) {
 #define MWG_LAUNCH(NN)                                                                      \
-    (list ? launch64_n<NN, false>(p->ctx, p->args, p->pool, list, 0, n, lo, head, s, err)   \
-          : launch64_n<NN, true>(p->ctx, p->args, p->pool, nullptr, 0, n, lo, head, s, err))
+    (list ? launch64_n<NN, false>(p->ctx, p->args, p->pool, list, n_dev, n, lo, head, s, err)   \
+          : launch64_n<NN, true>(p->ctx, p->args, p->pool, list, n_dev, n, lo, head, s, err))
     MWG_SIZES(MWG_LAUNCH)
 #undef MWG_LAUNCH
 }
@@ -2903,7 +2941,8 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
     unsigned long long *head1 = p->args.counters + 2, *head2 = p->args.counters + 3;
     if (mode == 0) {
         // lo = 0: every term that passes screening, over the pair segments
-        rc = launch64(p, nullptr, p->n_pseg, 0.0, head1, c->stream, err);
+        rc = p->cut_open ? launch64(p, nullptr, p->count.n_seg, p->count.cap[0], 0.0, head1, c->stream, err)
+                         : launch64(p, nullptr, nullptr, p->n_pseg, 0.0, head1, c->stream, err);
         if (rc) return rc;
     } else if (mode == 1) {
         // The FP64 class, then the FP32 class, on the first stream; both only
@@ -2914,7 +2953,7 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         // with the FP32 class instead of before it (64 Helmholtz applies at
         // k = 11, 119,968 output nodes: 316 ms against 394 ms a step).
         if (timed) HIP_TRY(hipEventRecord(c->ev2s, c->stream));
-        rc = launch64(p, p->list_hi, p->n_hi, tau, head2, c->stream, err);
+        rc = launch64(p, p->list_hi, nullptr, p->n_hi, tau, head2, c->stream, err);
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(c->ev2e, c->stream));
         if (timed) HIP_TRY(hipEventRecord(c->evl, c->stream));
@@ -2927,7 +2966,7 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         HIP_TRY(hipEventRecord(c->evz, c->stream));
         HIP_TRY(hipStreamWaitEvent(c->stream2, c->evz, 0));
         if (timed) HIP_TRY(hipEventRecord(c->ev2s, c->stream2));
-        rc = launch64(p, p->list_hi, p->n_hi, tau, head2, c->stream2, err);
+        rc = launch64(p, p->list_hi, nullptr, p->n_hi, tau, head2, c->stream2, err);
         if (rc) return rc;
         HIP_TRY(hipEventRecord(c->ev2e, c->stream2));
         if (timed) HIP_TRY(hipEventRecord(c->evl, c->stream));
@@ -3066,7 +3105,7 @@ static int step_graph(DevicePlan *p, int mode, double tau, bool post, std::strin
 
 int dev_plan_run(DevicePlan *p, int mode, double tau, double *kernel_ms, unsigned long long *term_apps,
                  unsigned long long *lp_apps, std::string &err, double *split_ms, bool post, double *post_ms,
-                 bool graph) {
+                 bool graph, double *norms2) {
     DeviceCtx *c = p->ctx;
     HIP_TRY(hipSetDevice(c->device));
     if (post && !p->post_pairs) {
@@ -3094,21 +3133,41 @@ int dev_plan_run(DevicePlan *p, int mode, double tau, double *kernel_ms, unsigne
     }
     const unsigned bit = 1u << (2 * mode + (post ? 1 : 0));
     const bool replay = graph && (p->ran_eager & bit);
-    if (replay) {
-        int rc = step_graph(p, mode, tau, post, err);
+    // counters, and with an open cut or norms the rest of the result block
+    const size_t n_res = 8 + (norms2 ? p->n_tot + 2 * (size_t)p->n_out : p->cut_open ? p->n_tot : 0);
+    std::vector<unsigned long long, UninitAlloc<unsigned long long>> res(n_res);
+    const unsigned long long *cnt = res.data();
+    while (true) {
+        if (replay) {
+            int rc = step_graph(p, mode, tau, post, err);
+            if (rc) return rc;
+            HIP_TRY(hipEventRecord(c->ev0, c->stream));
+            HIP_TRY(hipGraphLaunch(p->graph, c->stream));
+        } else {
+            HIP_TRY(hipEventRecord(c->ev0, c->stream));
+            int rc = enqueue_step(p, mode, tau, post, true, err);
+            if (rc) return rc;
+            p->ran_eager |= bit;
+        }
+        HIP_TRY(hipEventRecord(c->ev1, c->stream));
+        if (norms2) {
+            double *nr = reinterpret_cast<double *>(p->result + 8 + p->n_tot);
+            int rc = dev_node_norms_launch(c->stream, p->kp1, p->args.out_ns, p->n_out, nr, nr + p->n_out, err);
+            if (rc) return rc;
+        }
+        HIP_TRY(hipMemcpyAsync(res.data(), p->result, sizeof(res[0]) * n_res, hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        if (!p->cut_open) break;
+        if (cut_fits(p, cnt + 8)) {
+            cut_done(p);
+            break;
+        }
+        // more segments than the room: cut again and run again
+        const long long cap[2] = {(long long)cnt[8 + p->n_tot - 2], p->count.cap[1]};
+        int rc = cut_plan(p, cap, false, true, err);
         if (rc) return rc;
-        HIP_TRY(hipEventRecord(c->ev0, c->stream));
-        HIP_TRY(hipGraphLaunch(p->graph, c->stream));
-    } else {
-        HIP_TRY(hipEventRecord(c->ev0, c->stream));
-        int rc = enqueue_step(p, mode, tau, post, true, err);
-        if (rc) return rc;
-        p->ran_eager |= bit;
     }
-    HIP_TRY(hipEventRecord(c->ev1, c->stream));
-    unsigned long long cnt[8];
-    HIP_TRY(hipMemcpyAsync(cnt, p->args.counters, sizeof(cnt), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (norms2) std::memcpy(norms2, res.data() + 8 + p->n_tot, sizeof(double) * 2 * (size_t)p->n_out);
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     if (kernel_ms) *kernel_ms = ms;

@@ -34,8 +34,10 @@ struct DevicePlan;
 // (dev_pool_fill), the norm and pre-screen tables, the exact counts and the
 // work segments (the fine single-component ones only for a mode with an FP64
 // class beside a low-precision one).  mode: the arithmetic the plan will run.
-int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, DevicePlan **out,
-                    std::string &err);
+// With once (plain FP64, a plan that is run once) the host does not wait for
+// the counts: the run reads the number of segments on the device.
+int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, bool once,
+                    DevicePlan **out, std::string &err);
 // Term-applications counted with the screening rule when the plan was made,
 // and its pair segments.
 void dev_plan_counts(const DevicePlan *p, unsigned long long *term_apps, int *segments);
@@ -53,9 +55,11 @@ void dev_plan_counts(const DevicePlan *p, unsigned long long *term_apps, int *se
 // With graph the step (zeroing, class launches, post) replays a hipGraph
 // captured on the plan for (mode, tau, post) after one eager run; a replay
 // reports the whole device time only (split_ms and post_ms stay 0).
+// norms2 (optional, 2 n_out values): the squared norms of the scaling part,
+// then of the wavelet parts, of every raw output block.
 int dev_plan_run(DevicePlan *p, int mode, double tau, double *kernel_ms, unsigned long long *term_apps,
                  unsigned long long *lp_apps, std::string &err, double *split_ms = nullptr, bool post = false,
-                 double *post_ms = nullptr, bool graph = false);
+                 double *post_ms = nullptr, bool graph = false, double *norms2 = nullptr);
 // Post transforms of the plan's output grid: levels[d] holds the (branch
 // node, first child) pairs at depth d as indices into the plan's output
 // nodes.  Uploads the pairs with their device addresses and the filter.
@@ -128,7 +132,8 @@ int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a
                   DevMulSession **out, std::string &err, bool noalloc = false, bool a_on_device = false,
                   bool b_on_device = false);
 // out_blocks: nodes.size() x 8(k+1)^3, on the host, or on the device with
-// out_on_device.
+// out_on_device (then launches only: nodes must live until the stream has run
+// them, as for dev_add_nodes).
 int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double coef, double *out_blocks,
                   std::string &err, bool out_on_device = false);
 void dev_mul_end(DevMulSession *m);
@@ -151,9 +156,6 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
 int dev_upload(DeviceCtx *c, const double *src, size_t n, double **dst, std::string &err);
 // n doubles of device memory (freed with dev_free).
 int dev_alloc(DeviceCtx *c, size_t n, double **dst, std::string &err);
-// Block i (blk doubles) of src to block dst_idx[i] of dst, on the device.
-int dev_scatter_blocks(DeviceCtx *c, const double *src, const std::vector<int> &dst_idx, int blk, double *dst,
-                       std::string &err);
 // Block src_idx[i] of src to block i of dst, on the device.
 int dev_gather_blocks(DeviceCtx *c, const double *src, const std::vector<int> &src_idx, int blk, double *dst,
                       std::string &err);
@@ -161,8 +163,6 @@ int dev_gather_blocks(DeviceCtx *c, const double *src, const std::vector<int> &s
 int dev_scale(DeviceCtx *c, double *p, size_t n, double f, std::string &err);
 // n doubles from host memory into device memory at dst, finished on return.
 int dev_upload_into(DeviceCtx *c, const double *src, size_t n, double *dst, std::string &err);
-// n doubles from device memory to device memory, finished on return.
-int dev_d2d(DeviceCtx *c, double *dst, const double *src, size_t n, std::string &err);
 
 // Node blocks resident on the device (mw_multiply.hip).  Per node of
 // blocks[0, n): its scaling part's and wavelet parts' squared norms.
@@ -183,6 +183,22 @@ struct PostPair {
 // leaves' scaling parts).
 int dev_post_transform(DeviceCtx *c, const MRA &mra, const std::vector<std::vector<PostPair>> &levels,
                        std::string &err, bool topdown = true);
+// The last step of a tree built level by level on the device, with one upload
+// and one wait: the blocks of `before` copied, the post transforms over
+// `levels` (none: empty), then the blocks of `after` copied (src == dst: left
+// in place) and normed: norms2 receives after.size() squared norms of the
+// scaling parts, then of the wavelet parts.
+struct BlockMove {
+    const double *src;
+    double *dst;
+};
+int dev_finish_blocks(DeviceCtx *c, const MRA &mra, const std::vector<BlockMove> &before,
+                      const std::vector<std::vector<PostPair>> &levels, bool topdown,
+                      const std::vector<BlockMove> &after, double *norms2, std::string &err);
+// A packed tree: head (host) and n doubles of blocks (device) into device
+// memory at dst, finished on return.
+int dev_pack(DeviceCtx *c, void *dst, const void *head, size_t head_bytes, const double *blocks, size_t n,
+             std::string &err);
 // The same TopDown/BottomUp sequence over pairs already on the device:
 // level d's pairs are pairs[lvl_off[d], lvl_off[d + 1]); F is the two-scale
 // filter on the device.  Launches only, on `stream`.
@@ -282,8 +298,10 @@ struct RootLaunch {
     const double *pool = nullptr;
     double *A = nullptr, *Y = nullptr;  // work areas (root_work_values)
     double *out_ns = nullptr;
-    unsigned long long *counter = nullptr;  // += apps_count
-    unsigned long long apps_count = 0;
+    // counter += the root terms of every apply, totals[2 i + 1], i < n_totals
+    unsigned long long *counter = nullptr;
+    const unsigned long long *totals = nullptr;
+    int n_totals = 0;
 };
 void root_work_values(int n, const int *boxes, long long n_items, size_t *a_values, size_t *y_values);
 // Launches only, on `stream`.

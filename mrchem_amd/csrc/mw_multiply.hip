@@ -1111,14 +1111,53 @@ int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &job
     return 0;
 }
 
-// Block src_idx[i] of src (blk doubles; i itself without src_idx) to block
-// dst_idx[i] of dst (i without dst_idx): one workgroup per block.
-__global__ __launch_bounds__(256) void k_move_blocks(const double *src, const int *src_idx, const int *dst_idx, int n,
-                                                     int blk, double *dst) {
+// Block src_idx[i] of src (blk doubles) to block i of dst: one workgroup per
+// block.
+__global__ __launch_bounds__(256) void k_gather_blocks(const double *src, const int *src_idx, int n, int blk,
+                                                       double *dst) {
     for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const double *a = src + (size_t)(src_idx ? src_idx[i] : i) * blk;
-        double *b = dst + (size_t)(dst_idx ? dst_idx[i] : i) * blk;
+        const double *a = src + (size_t)src_idx[i] * blk;
+        double *b = dst + (size_t)i * blk;
         for (int e = threadIdx.x; e < blk; e += 256) b[e] = a[e];
+    }
+}
+
+// Blocks copied (src == dst: left in place) and normed in one pass: one
+// workgroup per block, the sums as in k_node_norms.  Bound by memory; one
+// launch for the nodes of all trees in place of a copy and a wait for every
+// run of adjacent nodes (about 150 of them in a batch of exchange applies).
+__global__ __launch_bounds__(256) void k_move_norms(const BlockMove *moves, int n3, double *s2, double *w2) {
+    __shared__ double part[2][4];
+    const BlockMove m = moves[blockIdx.x];
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const bool copy = m.src != m.dst;
+    double s = 0.0, w = 0.0;
+#pragma unroll 4
+    for (int e = tid; e < n3; e += 256) {
+        const double v = m.src[e];
+        if (copy) m.dst[e] = v;
+        s += v * v;
+    }
+#pragma unroll 4
+    for (int e = n3 + tid; e < 8 * n3; e += 256) {
+        const double v = m.src[e];
+        if (copy) m.dst[e] = v;
+        w += v * v;
+    }
+    if (!s2) return;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o);
+        w += __shfl_xor(w, o);
+    }
+    if ((tid & 63) == 0) {
+        part[0][wave] = s;
+        part[1][wave] = w;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        s2[blockIdx.x] = (part[0][0] + part[0][1]) + (part[0][2] + part[0][3]);
+        w2[blockIdx.x] = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
     }
 }
 
@@ -1141,18 +1180,18 @@ int dev_alloc(DeviceCtx *c, size_t n, double **dst, std::string &err) {
     return dev_mem(c, n, dst, err);
 }
 
-static int move_blocks(DeviceCtx *c, const double *src, const std::vector<int> *src_idx,
-                       const std::vector<int> *dst_idx, size_t n, int blk, double *dst, std::string &err) {
+int dev_gather_blocks(DeviceCtx *c, const double *src, const std::vector<int> &src_idx, int blk, double *dst,
+                      std::string &err) {
+    const size_t n = src_idx.size();
     if (n == 0) return 0;
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
     int *d = nullptr;
     if (int rc = dev_mem(c, n, &d, err)) return rc;
-    const std::vector<int> &idx = src_idx ? *src_idx : *dst_idx;
-    hipError_t e = hipMemcpyAsync(d, idx.data(), sizeof(int) * n, hipMemcpyHostToDevice, s);
+    hipError_t e = hipMemcpyAsync(d, src_idx.data(), sizeof(int) * n, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_move_blocks, dim3((unsigned)std::min<size_t>(n, 4096)), dim3(256), 0, s, src,
-                           src_idx ? d : nullptr, src_idx ? nullptr : d, (int)n, blk, dst);
+        hipLaunchKernelGGL(k_gather_blocks, dim3((unsigned)std::min<size_t>(n, 4096)), dim3(256), 0, s, src, d, (int)n,
+                           blk, dst);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -1164,27 +1203,8 @@ static int move_blocks(DeviceCtx *c, const double *src, const std::vector<int> *
     return 0;
 }
 
-int dev_scatter_blocks(DeviceCtx *c, const double *src, const std::vector<int> &dst_idx, int blk, double *dst,
-                       std::string &err) {
-    return move_blocks(c, src, nullptr, &dst_idx, dst_idx.size(), blk, dst, err);
-}
-
-int dev_gather_blocks(DeviceCtx *c, const double *src, const std::vector<int> &src_idx, int blk, double *dst,
-                      std::string &err) {
-    return move_blocks(c, src, &src_idx, nullptr, src_idx.size(), blk, dst, err);
-}
-
 int dev_upload_into(DeviceCtx *c, const double *src, size_t n, double *dst, std::string &err) {
     return dev_copy_h2d(c, dst, src, sizeof(double) * n, err);
-}
-
-int dev_d2d(DeviceCtx *c, double *dst, const double *src, size_t n, std::string &err) {
-    if (n == 0) return 0;
-    HIP_TRY(hipSetDevice(dev_device(c)));
-    hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
-    HIP_TRY(hipMemcpyAsync(dst, src, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return 0;
 }
 
 int dev_upload(DeviceCtx *c, const double *src, size_t n, double **dst, std::string &err) {
@@ -1208,14 +1228,16 @@ int dev_node_norms(DeviceCtx *c, int kp1, const double *blocks, long long n, dou
     if (int rc = dev_mem(c, 2 * (size_t)n, &d, err)) return rc;
     hipLaunchKernelGGL(k_node_norms, dim3((unsigned)n), dim3(256), 0, s, blocks, n, kp1 * kp1 * kp1, d, d + n);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(host_s2, d, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(host_w2, d + n, sizeof(double) * n, hipMemcpyDeviceToHost, s);
+    std::vector<double, UninitAlloc<double>> h(2 * (size_t)n);
+    if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d, sizeof(double) * 2 * n, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     dev_mem_put(c, d);
     if (e != hipSuccess) {
         err = std::string("node norms: ") + hipGetErrorString(e);
         return -2;
     }
+    std::copy(h.begin(), h.begin() + n, host_s2);
+    std::copy(h.begin() + n, h.end(), host_w2);
     return 0;
 }
 
@@ -1276,6 +1298,75 @@ int dev_post_transform(DeviceCtx *c, const MRA &mra, const std::vector<std::vect
         err = std::string("post transforms: ") + hipGetErrorString(e);
         return -2;
     }
+    return 0;
+}
+
+int dev_finish_blocks(DeviceCtx *c, const MRA &mra, const std::vector<BlockMove> &before,
+                      const std::vector<std::vector<PostPair>> &levels, bool topdown,
+                      const std::vector<BlockMove> &after, double *norms2, std::string &err) {
+    HIP_TRY(hipSetDevice(dev_device(c)));
+    hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
+    const int n3 = mra.kp1_3();
+    std::vector<long long> off(1, 0);
+    for (const auto &l : levels) off.push_back(off.back() + (long long)l.size());
+    if (off.back() > 0 && mra.kp1() > 12) {
+        err = "post transforms: unsupported basis size";
+        return -1;
+    }
+    // [filter][pairs][before][after] from one staging buffer, then the norms
+    const size_t b_F = sizeof(double) * mra.basis.F.size(), b_p = sizeof(PostPair) * (size_t)off.back();
+    const size_t b_b = sizeof(BlockMove) * before.size(), b_a = sizeof(BlockMove) * after.size();
+    const size_t up = b_F + b_p + b_b + b_a, na = after.size();
+    std::vector<unsigned char, UninitAlloc<unsigned char>> stage(up);
+    std::memcpy(stage.data(), mra.basis.F.data(), b_F);
+    for (size_t l = 0; l < levels.size(); l++)
+        if (!levels[l].empty())
+            std::memcpy(stage.data() + b_F + sizeof(PostPair) * off[l], levels[l].data(),
+                        sizeof(PostPair) * levels[l].size());
+    if (b_b) std::memcpy(stage.data() + b_F + b_p, before.data(), b_b);
+    if (b_a) std::memcpy(stage.data() + b_F + b_p + b_b, after.data(), b_a);
+    unsigned char *dev = nullptr;
+    if (int rc = dev_mem(c, up + sizeof(double) * 2 * na, &dev, err)) return rc;
+    const double *F = reinterpret_cast<const double *>(dev);
+    const PostPair *pairs = reinterpret_cast<const PostPair *>(dev + b_F);
+    const BlockMove *mb = reinterpret_cast<const BlockMove *>(dev + b_F + b_p), *ma = mb + before.size();
+    double *nr = reinterpret_cast<double *>(dev + up);
+    hipError_t e = hipMemcpyAsync(dev, stage.data(), up, hipMemcpyHostToDevice, s);
+    int rc = 0;
+    if (e == hipSuccess && !before.empty()) {
+        hipLaunchKernelGGL(k_move_norms, dim3((unsigned)before.size()), dim3(256), 0, s, mb, n3,
+                           static_cast<double *>(nullptr), static_cast<double *>(nullptr));
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess && off.back() > 0) rc = dev_post_launch(s, mra.kp1(), pairs, off, F, err, topdown);
+    if (e == hipSuccess && !rc && na) {
+        hipLaunchKernelGGL(k_move_norms, dim3((unsigned)na), dim3(256), 0, s, ma, n3, nr, nr + na);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess && !rc && na) e = hipMemcpyAsync(norms2, nr, sizeof(double) * 2 * na, hipMemcpyDeviceToHost, s);
+    const hipError_t es = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = es;
+    dev_mem_put(c, dev);
+    if (rc) return rc;
+    if (e != hipSuccess) {
+        err = std::string("post transforms: ") + hipGetErrorString(e);
+        return -2;
+    }
+    return 0;
+}
+
+int dev_pack(DeviceCtx *c, void *dst, const void *head, size_t head_bytes, const double *blocks, size_t n,
+             std::string &err) {
+    HIP_TRY(hipSetDevice(dev_device(c)));
+    hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
+    HIP_TRY(hipMemcpyAsync(dst, head, head_bytes, hipMemcpyHostToDevice, s));
+    hipError_t e = hipSuccess;
+    if (n)
+        e = hipMemcpyAsync(static_cast<char *>(dst) + head_bytes, blocks, sizeof(double) * n, hipMemcpyDeviceToDevice,
+                           s);
+    const hipError_t es = hipStreamSynchronize(s);
+    HIP_TRY(e);
+    HIP_TRY(es);
     return 0;
 }
 
@@ -1489,7 +1580,6 @@ int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double co
     int crc = 0;
     if (e == hipSuccess && !out_on_device)
         crc = dev_copy_d2h(m->ctx, out_blocks, dout, sizeof(double) * nodes.size() * 8 * n3, err);
-    if (e == hipSuccess && out_on_device) e = hipStreamSynchronize(s);
     dev_mem_put(m->ctx, dn);
     if (!out_on_device) dev_mem_put(m->ctx, dout);
     if (crc) return crc;
@@ -1594,7 +1684,6 @@ int dev_add_nodes(DevAddSession *m, const std::vector<AddSrc> &src, double *out_
     int crc = 0;
     if (e == hipSuccess && !out_on_device)
         crc = dev_copy_d2h(m->ctx, out_blocks, dout, sizeof(double) * n_nodes * 8 * n3, err);
-    if (e == hipSuccess && out_on_device) e = hipStreamSynchronize(s);
     dev_mem_put(m->ctx, dsrc);
     if (!out_on_device) dev_mem_put(m->ctx, dout);
     if (crc) return crc;

@@ -159,18 +159,20 @@ __global__ __launch_bounds__(256) void k_root_xy(RootGeo geo, const RootApp *app
 // The z pass: out[iz][(iy, ix)] += sum over items and planes of A_z Y.  One
 // wave per (64 columns, run of per items); the accumulators are added into
 // the roots' output blocks (zeroed before) when the apply changes and at the
-// end of the run.  apps_count: the level's term-applications, added to the
-// plan's counter once.
+// end of the run.  totals: per apply of the plan its term-applications and
+// those of the roots; the latter are added to the plan's counter (n_totals 0:
+// not by this launch).
 template <int T, bool SAME>
 __global__ __launch_bounds__(256) void k_root_z(RootGeo geo, const RootApp *apps, const RootItem *items, int n_items,
                                                 int per, const int *root_out, const double *A, const double *Y,
                                                 double *out_ns, unsigned long long *counter,
-                                                unsigned long long apps_count) {
+                                                const unsigned long long *totals, int n_totals) {
     constexpr int K = 4 * T, SZ = T * K * 64, DP = 16 * T, nd = SAME ? 1 : 3;
     const int N = geo.n, N3 = N * N * N;
     const int D[3] = {2 * N * geo.boxes[0], 2 * N * geo.boxes[1], 2 * N * geo.boxes[2]};
     const int lane = threadIdx.x & 63, lc = lane & 15, lq = lane >> 4;
-    if (apps_count && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) atomicAdd(counter, apps_count);
+    if (blockIdx.x == 0 && blockIdx.y == 0)
+        for (int i = threadIdx.x; i < n_totals; i += 256) atomicAdd(counter, totals[2 * i + 1]);
     const int cg = 4 * blockIdx.y + (threadIdx.x >> 6);  // DP DP / 64 groups: a multiple of 4
     const int i0 = blockIdx.x * per, i1 = min(i0 + per, n_items);
     root_d4 acc[4][T];
@@ -229,7 +231,7 @@ __global__ __launch_bounds__(256) void k_root_z(RootGeo geo, const RootApp *apps
 }
 
 template <int T, bool SAME>
-hipError_t root_chunk(hipStream_t s, const RootLaunch &r, int item0, int n, unsigned long long apps_count) {
+hipError_t root_chunk(hipStream_t s, const RootLaunch &r, int item0, int n) {
     const int nd = SAME ? 1 : 3, dz = 2 * r.geo.n * r.geo.boxes[2], groups = 16 * T * T / 4;
     const RootItem *items = r.items + item0;
     hipLaunchKernelGGL((k_root_ops<T>), dim3(n, nd), dim3(256), 0, s, r.geo, r.apps, items, nd, r.A);
@@ -244,7 +246,7 @@ hipError_t root_chunk(hipStream_t s, const RootLaunch &r, int item0, int n, unsi
     const int runs = std::max(1, std::min((n + 3) / 4, 1024 / groups));
     const int per = (n + runs - 1) / runs;
     hipLaunchKernelGGL((k_root_z<T, SAME>), dim3((n + per - 1) / per, groups / 4), dim3(256), 0, s, r.geo, r.apps,
-                       items, n, per, r.root_out, r.A, r.Y, r.out_ns, r.counter, apps_count);
+                       items, n, per, r.root_out, r.A, r.Y, r.out_ns, r.counter, r.totals, item0 == 0 ? r.n_totals : 0);
     return hipGetLastError();
 }
 
@@ -277,11 +279,10 @@ int dev_root_launch(void *stream, const RootLaunch &r, std::string &err) {
     const int chunk = (int)root_chunk_items(r.geo.n, r.geo.boxes, r.n_items);
     for (int i = 0; i < r.n_items; i += chunk) {
         const int n = std::min(chunk, r.n_items - i);
-        const unsigned long long cnt = i == 0 ? r.apps_count : 0;
         hipError_t e = hipErrorInvalidValue;
-        if (t == 1) e = same ? root_chunk<1, true>(s, r, i, n, cnt) : root_chunk<1, false>(s, r, i, n, cnt);
-        if (t == 2) e = same ? root_chunk<2, true>(s, r, i, n, cnt) : root_chunk<2, false>(s, r, i, n, cnt);
-        if (t == 3) e = same ? root_chunk<3, true>(s, r, i, n, cnt) : root_chunk<3, false>(s, r, i, n, cnt);
+        if (t == 1) e = same ? root_chunk<1, true>(s, r, i, n) : root_chunk<1, false>(s, r, i, n);
+        if (t == 2) e = same ? root_chunk<2, true>(s, r, i, n) : root_chunk<2, false>(s, r, i, n);
+        if (t == 3) e = same ? root_chunk<3, true>(s, r, i, n) : root_chunk<3, false>(s, r, i, n);
         HIP_TRY(e);
     }
     return 0;

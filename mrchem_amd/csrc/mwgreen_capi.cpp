@@ -362,6 +362,8 @@ void check_finite(mwg_tree t, const char *what) {
 struct DeviceResult {
     DeviceCtx *c = nullptr;
     double *p = nullptr;
+    DeviceResult(DeviceCtx *ctx, double *q) : c(ctx), p(q) {}
+    DeviceResult(DeviceResult &&o) : c(o.c), p(o.release()) {}
     ~DeviceResult() { dev_free(c, p); }
     double *release() {
         double *q = p;
@@ -553,13 +555,16 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         DevicePlan *dp = nullptr;
         const double t1 = now_ms();
         t_inp += t1 - t0i;
-        int rc = dev_plan_create(ctx->dev, mra, parts, ctx->mode, &dp, err);
+        int rc = dev_plan_create(ctx->dev, mra, parts, ctx->mode, true, &dp, err);
         if (rc) return dev_fail(rc, err);
         const double t1r = now_ms();
         t_create += t1r - t1;
         double ms = 0.0;
         unsigned long long apps = 0;
-        rc = dev_plan_run(dp, ctx->mode, ctx->tau, &ms, &apps, nullptr, err, nullptr);
+        std::vector<double> norms(2 * total);  // squared: scaling parts, then wavelet parts
+        const double *s2 = norms.data(), *w2 = norms.data() + total;
+        rc = dev_plan_run(dp, ctx->mode, ctx->tau, &ms, &apps, nullptr, err, nullptr, false, nullptr, false,
+                          norms.data());
         t_run += now_ms() - t1r;
         // the level's blocks stay on the device; the host takes their norms
         double *lvl = rc ? nullptr : dev_plan_take_output(dp);
@@ -568,9 +573,6 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         const int level = (int)keep.bufs.size();
         keep.bufs.push_back(lvl);
         keep.count.push_back((long long)total);
-        std::vector<double> s2(total), w2(total);
-        rc = dev_node_norms(ctx->dev, mra.kp1(), lvl, (long long)total, s2.data(), w2.data(), err);
-        if (rc) return dev_fail(rc, err);
         t_dev += now_ms() - t1;
         const double t2 = now_ms();
         kms += ms;
@@ -657,63 +659,30 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
                 levels[o.keys[i].depth].push_back(PostPair{addr(loc[i]), addr(loc[c0])});
             }
         }
-        int rc = dev_post_transform(ctx->dev, mra, levels, err);
-        // norms of the transformed blocks, level by level
-        std::vector<std::vector<double>> s2(keep.bufs.size()), w2(keep.bufs.size());
-        for (size_t l = 0; l < keep.bufs.size() && !rc; l++) {
-            s2[l].resize(keep.count[l]);
-            w2[l].resize(keep.count[l]);
-            rc = dev_node_norms(ctx->dev, mra.kp1(), keep.bufs[l], keep.count[l], s2[l].data(), w2[l].data(), err);
+        // the transformed blocks into one array per tree, normed on the way:
+        // the device copy of an output resident on this context, else a
+        // temporary that is downloaded into the host tree
+        std::vector<DeviceResult> res;
+        for (size_t ji = 0; ji < jobs.size(); ji++) res.push_back(DeviceResult{ctx->dev, nullptr});
+        std::vector<BlockMove> moves;
+        for (size_t ji = 0; ji < jobs.size(); ji++) {
+            const Tree &o = jobs[ji].out->tree;
+            dev_check(dev_alloc(ctx->dev, (size_t)o.size() * blk, &res[ji].p, err), err);
+            for (int i = 0; i < o.size(); i++)
+                moves.push_back(BlockMove{addr(locs[ji][i]), res[ji].p + (size_t)i * blk});
         }
-        // the blocks into the trees, in runs of nodes adjacent in both: into
-        // the device copy of an output resident on this context, else
-        // downloaded into the host tree
-        for (size_t ji = 0; ji < jobs.size() && !rc; ji++) {
+        std::vector<double> nr(2 * moves.size());
+        dev_check(dev_finish_blocks(ctx->dev, mra, {}, levels, true, moves, nr.data(), err), err);
+        size_t at = 0;
+        for (size_t ji = 0; ji < jobs.size(); ji++) {
             mwg_tree out = jobs[ji].out;
-            Tree &o = out->tree;
-            const std::vector<NodeLoc> &loc = locs[ji];
-            const bool resident = out->dctx == ctx;
-            DeviceResult dres{ctx->dev, nullptr};
-            if (resident) {
-                rc = dev_alloc(ctx->dev, (size_t)o.size() * blk, &dres.p, err);
-            } else {
-                o.structure_only = false;
-                o.coefs.resize((size_t)o.size() * blk);  // every block is written below
-            }
-            int i = 0;
-            while (i < o.size() && !rc) {
-                int e = i + 1;
-                while (e < o.size() && loc[e].level == loc[i].level && loc[e].pos == loc[i].pos + (e - i)) e++;
-                const size_t nv = (size_t)(e - i) * blk;
-                if (resident) {
-                    rc = dev_d2d(ctx->dev, dres.p + (size_t)i * blk, addr(loc[i]), nv, err);
-                } else {
-                    rc = dev_download(ctx->dev, addr(loc[i]), nv, o.node(i), err);
-                    ctx->d2h_bytes += (long long)(sizeof(double) * nv);
-                }
-                i = e;
-            }
-            if (rc) break;
-            std::vector<double> ns2(o.size()), nw2(o.size());
-            for (int n = 0; n < o.size(); n++) {
-                const NodeLoc &l = loc[n];
-                ns2[n] = s2[l.level][l.pos];
-                nw2[n] = w2[l.level][l.pos];
-            }
-            if (resident) {
-                take_device_result(ctx, out, dres.release(), std::move(ns2), std::move(nw2));
-            } else {
-                double sq = 0.0;
-                for (int n = 0; n < o.size(); n++) sq += nw2[n] + (o.parent[n] < 0 ? ns2[n] : 0.0);
-                o.sqnorm = sq;
-                host_changed(out);
-                out->s2 = std::move(ns2);
-                out->w2 = std::move(nw2);
-                out->norms_valid = true;
-            }
+            const size_t n = (size_t)out->tree.size();
+            const double *ns2 = nr.data() + at, *nw2 = nr.data() + moves.size() + at;
+            take_device_result(ctx, out, res[ji].release(), std::vector<double>(ns2, ns2 + n),
+                               std::vector<double>(nw2, nw2 + n));
             out->apply_thr = jobs[ji].thr_all;
+            at += n;
         }
-        if (rc) return dev_fail(rc, err);
     }
     guard.done = true;
     auto &st = ctx->last_stats;
@@ -787,7 +756,7 @@ int make_plan(mwg_context ctx, int n, const mwg_tree *out, const mwg_operator *o
     }
     p->thr = std::move(th);
     std::string err;
-    int rc = dev_plan_create(ctx->dev, *out[0]->tree.mra, parts, mode, &p->dev, err);
+    int rc = dev_plan_create(ctx->dev, *out[0]->tree.mra, parts, mode, false, &p->dev, err);
     if (rc) return dev_fail(rc, err);
     {
         unsigned long long apps = 0;
@@ -1223,15 +1192,40 @@ struct DeviceLevels {
             w2[w[q]] = b[q];
         }
     }
-    // every level's blocks into one array of tree_size blocks in tree order
-    double *assemble(int tree_size) {
+    // every level's blocks into one array of tree_size blocks in tree order;
+    // with compress the branches of T are then recomputed from their children
+    // (BottomUp) and s2, w2 are the norms of the final blocks
+    double *assemble(const MRA &mra, const Tree &T, bool compress) {
         DeviceResult r{c, nullptr};
         std::string err;
-        dev_check(dev_alloc(c, (size_t)tree_size * blk, &r.p, err), err);
-        for (size_t l = 0; l < bufs.size(); l++) {
-            dev_check(dev_scatter_blocks(c, bufs[l], nodes[l], blk, r.p, err), err);
-            dev_free(c, bufs[l]);
-            bufs[l] = nullptr;
+        dev_check(dev_alloc(c, (size_t)T.size() * blk, &r.p, err), err);
+        std::vector<BlockMove> before, after;
+        for (size_t l = 0; l < bufs.size(); l++)
+            for (size_t q = 0; q < nodes[l].size(); q++)
+                before.push_back(BlockMove{bufs[l] + q * blk, r.p + (size_t)nodes[l][q] * blk});
+        std::vector<std::vector<PostPair>> levels;
+        std::vector<int> branch;
+        if (compress) {
+            levels.resize(T.max_depth() + 1);
+            for (int i = 0; i < T.size(); i++) {
+                if (T.child0[i] < 0) continue;
+                levels[T.keys[i].depth].push_back(
+                    PostPair{r.p + (size_t)i * blk, r.p + (size_t)T.child0[i] * blk});
+                after.push_back(BlockMove{r.p + (size_t)i * blk, r.p + (size_t)i * blk});
+                branch.push_back(i);
+            }
+        }
+        std::vector<double> nr(2 * after.size());
+        dev_check(dev_finish_blocks(c, mra, before, levels, false, after, nr.data(), err), err);
+        s2.resize(T.size(), 0.0);
+        w2.resize(T.size(), 0.0);
+        for (size_t i = 0; i < branch.size(); i++) {
+            s2[branch[i]] = nr[i];
+            w2[branch[i]] = nr[branch.size() + i];
+        }
+        for (double *&p : bufs) {
+            dev_free(c, p);
+            p = nullptr;
         }
         return r.release();
     }
@@ -1387,11 +1381,9 @@ int add_trees(mwg_context ctx, double prec, Tree &T, const std::vector<mwg_tree>
     session.reset();
     if (on_device) {
         // every node was computed once: its level's norms are its own
-        dres->blocks = lv.assemble(T.size());
+        dres->blocks = lv.assemble(mra, T, false);
         dres->s2 = std::move(lv.s2);
         dres->w2 = std::move(lv.w2);
-        dres->s2.resize(T.size(), 0.0);
-        dres->w2.resize(T.size(), 0.0);
     } else {
         T.sqnorm = tree_square_norm(T);
     }
@@ -1563,17 +1555,8 @@ int multiply_trees(mwg_context ctx, double prec, mwg_tree out, double coef, mwg_
         }
         session.reset();
         if (on_device) {
-            DeviceResult res{ctx->dev, lv.assemble(T.size())};
-            // BottomUp: every branch's block from its children's scaling parts
-            std::vector<std::vector<PostPair>> levels(T.max_depth() + 1);
-            for (int i = 0; i < T.size(); i++)
-                if (T.child0[i] >= 0)
-                    levels[T.keys[i].depth].push_back(
-                        PostPair{res.p + (size_t)i * blk, res.p + (size_t)T.child0[i] * blk});
-            dev_check(dev_post_transform(ctx->dev, mra, levels, err, false), err);
-            std::vector<double> s2(T.size()), w2(T.size());
-            dev_check(dev_node_norms(ctx->dev, mra.kp1(), res.p, T.size(), s2.data(), w2.data(), err), err);
-            take_device_result(ctx, out, res.release(), std::move(s2), std::move(w2));
+            double *res = lv.assemble(mra, T, true);
+            take_device_result(ctx, out, res, std::move(lv.s2), std::move(lv.w2));
         } else {
             tree_compress(T);
             T.sqnorm = tree_square_norm(T);
@@ -2090,15 +2073,9 @@ int mwg_tree_pack_device(mwg_tree t, mwg_context ctx, void *dst, long long bytes
         std::vector<char> head(head_bytes(n));
         pack_head(T, head.data());
         std::string err;
-        // the head as doubles: its size is a multiple of 8 bytes
-        dev_check(dev_upload_into(ctx->dev, reinterpret_cast<const double *>(head.data()), head.size() / 8,
-                                  static_cast<double *>(dst), err),
-                  err);
         TempBlocks tb{ctx->dev, {}};
         const double *blocks = tb.of(ctx, t);
-        dev_check(dev_d2d(ctx->dev, reinterpret_cast<double *>(static_cast<char *>(dst) + head.size()), blocks,
-                          tree_values(t), err),
-                  err);
+        dev_check(dev_pack(ctx->dev, dst, head.data(), head.size(), blocks, tree_values(t), err), err);
         return (int)MWG_OK;
     });
 }

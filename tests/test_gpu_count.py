@@ -41,6 +41,32 @@ def test_more_segments_than_room(ctx, order, mode):
     assert np.max(np.abs(out.nodes()[2] - ref)) < 1e-12 * np.max(np.abs(ref))
 
 
+@pytest.mark.parametrize("order", [2, 4])
+def test_adaptive_level_with_more_segments_than_room(ctx, order):
+    # an adaptive level starts its calculator before the host knows the
+    # number of segments; here the second level needs more than its room
+    mra = _mra(order)
+    P = mw.PoissonOperator(mra, 1e-10)
+    rho = mw.FunctionTree(mra).project_gaussians(1e-2, [1.0], [2.0], [[0.3, -0.2, 0.1]], max_depth=2)
+    out = mw.FunctionTree(mra)
+    mw.apply(1e-12, out, P, rho, max_iter=1, abs_prec=True, ctx=ctx)
+    stats = ctx.last_stats()
+    d, l, c = out.nodes()
+    thr = out.thresholds()
+    od, ol, othr, oc, st = oracle.apply_adaptive(mra, P.tables(), rho.nodes(), 1e-12, abs_prec=True, max_iter=1,
+                                                 max_depth=mra.max_depth)
+    np.testing.assert_array_equal(d, od)
+    np.testing.assert_array_equal(l, ol)
+    # estimates at roundoff of so small a threshold may fall on either side
+    assert abs(stats["term_apps"] - st["term_apps"]) < 1e-4 * st["term_apps"]
+    assert np.max(np.abs(c - oc)) < 1e-12 * np.max(np.abs(oc))
+    plan = mw.ApplyPlan(mw.FunctionTree(mra).set_nodes(d, l), P, rho, thr, ctx=ctx)
+    n1 = int((d == 1).sum())
+    print("order %d: %d nodes, %d segments" % (order, n1, plan.info()["segments"]))
+    assert plan.info()["segments"] > 16384 + 64 * n1
+    assert plan.execute()["term_apps"] == stats["term_apps"]
+
+
 @pytest.mark.parametrize("mode", ["fp64", "mixed"])
 def test_batch_of_unequal_counts(ctx, mode):
     mra = _mra(3)
