@@ -5,6 +5,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <string>
+#include <vector>
+
 #include "mw_device.hpp"
 
 namespace mwg {
@@ -61,6 +64,78 @@ struct KArgs {
     // (e = 0 but in plain FP64)
     const int *seg_job, *seg_p0, *seg_p1;
 };
+
+// A generated node of an apply plan's pool (mw_multiply.hip): scaling block dst
+// of child `child` of the node at src, a full block or a scaling block.
+struct GenItem {
+    const double *src;
+    double *dst;
+    int child, full;
+};
+
+// One slot of the pool: len doubles from src (an input node's full block, or a
+// generated node's scaling block) to dst, and the slot's 8 component norms to
+// norms (wavelet norms 0 for a generated slot).
+struct SlotItem {
+    const double *src;
+    double *dst, *norms;
+    int len;
+};
+
+// The pool from its items on the device: generated nodes level by level (of
+// level lv: gen[lv_off[lv], lv_off[lv + 1]), their parents in the input tree or
+// of level lv - 1), then every slot.  F: the basis' filter on the device.
+// Launches only, on stream.
+int dev_pool_fill(hipStream_t s, int n, const double *F, const GenItem *gen, const std::vector<int> &lv_off,
+                  const SlotItem *slots, int n_slot, std::string &err);
+
+// ---- Bands and slots of a plan (mw_band.hip) ----
+
+// The input tree of an apply: first child of every node (-1: none; the roots
+// are the first nodes, box x fastest) and the nodes' blocks.
+struct BandTree {
+    const int *child0;
+    const double *inp;
+};
+// Counters of the search: [0] real slots, [1] generated slots, [2] not 0: the
+// table was too small, [3 + lv] generated nodes lv generated levels below a
+// node of the input tree.
+constexpr int kBandLevels = 32, kBandCounts = 3 + kBandLevels;
+struct BandArgs {
+    const int *out_l, *out_depth, *out_app;  // out_l: 3 per output node
+    const long long *band_off;
+    const int *band_w;
+    const BandTree *trees;  // per apply
+    int corner[3], boxes[3];
+    int n_out;
+    long long n_band;
+    // table of cap cells (a power of two): name of the node, slot, generation
+    // level (-1: in the input tree) and, of a node in the tree, {its index, 0},
+    // of a generated one {parent's cell or -(tree node + 1), position in its
+    // level}
+    unsigned cap;
+    unsigned long long *rep;
+    int *slot;
+    int2 *gen;
+    signed char *lv;
+    int *cell;      // per band entry: its cell, or -1
+    unsigned *cnt;  // kBandCounts
+};
+// What the search found, as items: real slots are slots [0, n_real).
+struct BandItems {
+    int n3, n_real, n_roots;
+    int lv_off[kBandLevels];
+    double *gen_s, *pool, *norms;
+    GenItem *gen;
+    SlotItem *slots;
+    long long *slot_off;
+    int *band;
+    const int *root_out;  // output nodes of the dense root kernels
+    long long *root_off;  // pool offsets of their own slots
+};
+// Launches only, on stream.  widest: entries of the widest band.
+int dev_band_find(hipStream_t s, const BandArgs &a, long long widest, std::string &err);
+int dev_band_items(hipStream_t s, const BandArgs &a, const BandItems &o, std::string &err);
 
 // One depth of one apply in the norm and pre-screen tables.
 struct TermLevel {

@@ -1850,7 +1850,9 @@ struct DevicePlan {
     size_t n_tot = 0;
     bool cut_open = false;
     std::vector<void *> temp;
-    std::vector<unsigned char, UninitAlloc<unsigned char>> stage, fill_stage;
+    std::vector<unsigned char, UninitAlloc<unsigned char>> stage;
+    long long n_slot = 0, n_generated = 0;
+    unsigned found[kBandCounts];  // what the search for them counted
     // the captured step (step_graph) and what it was captured for
     hipGraphExec_t graph = nullptr;
     int graph_mode = -1;
@@ -2224,7 +2226,101 @@ static void cut_done(DevicePlan *p) {
     for (void *q : p->temp) dev_mem_put(p->ctx, q);
     p->temp.clear();
     p->stage = decltype(p->stage)();
-    p->fill_stage = decltype(p->fill_stage)();
+}
+
+// Bands, slots and pool of the plan: the search, then, its counts known, the
+// slot tables, the pool and the generated nodes.  beside: launches that need
+// none of it, which run while the host waits for the counts.
+template <typename F>
+static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n_band, long long widest,
+                     const int *out_l, const BandTree *trees, int *band, const double *filter, const int *root_out,
+                     int n_roots, long long *root_off, F &&beside, std::string &err) {
+    DeviceCtx *c = p->ctx;
+    hipStream_t s = c->stream;
+    const int N = p->kp1;
+    const size_t n3 = (size_t)N * N * N, blk = 8 * n3;
+    BandArgs b{};
+    b.out_l = out_l;
+    b.out_depth = p->args.out_depth;
+    b.out_app = p->args.out_app;
+    b.band_off = p->args.band_off;
+    b.band_w = p->args.band_w;
+    b.trees = trees;
+    for (int d = 0; d < 3; d++) {
+        b.corner[d] = (int)mra.corner[d];
+        b.boxes[d] = mra.boxes[d];
+    }
+    b.n_out = p->n_out;
+    b.n_band = n_band;
+    // work memory, put back below: its next holder's work comes after these
+    // launches on the stream
+    struct Held {
+        DeviceCtx *c;
+        std::vector<void *> v;
+        ~Held() {
+            for (void *q : v) dev_mem_put(c, q);
+        }
+    } held{c, {}};
+    auto get = [&](size_t n, auto **o) {
+        const int r = dev_mem(c, n, o, err);
+        if (!r) held.v.push_back(*o);
+        return r;
+    };
+    int rc = get((size_t)std::max<long long>(n_band, 1), &b.cell);
+    if (!rc) rc = get((size_t)kBandCounts, &b.cnt);
+    if (rc) return rc;
+    unsigned *cnt = p->found;
+    for (bool first = true;; first = false) {
+        if (cells > (1LL << 30)) {
+            err = "batch too large for 32-bit node, segment or slot indices";
+            return -1;
+        }
+        b.cap = (unsigned)cells;
+        if ((rc = get((size_t)cells, &b.rep)) || (rc = get((size_t)cells, &b.slot)) ||
+            (rc = get((size_t)cells, &b.gen)) || (rc = get((size_t)cells, &b.lv)) ||
+            (rc = dev_band_find(s, b, widest, err)))
+            return rc;
+        HIP_TRY(hipMemcpyAsync(cnt, b.cnt, sizeof(p->found), hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipEventRecord(c->evz, s));
+        if (first && (rc = beside())) return rc;
+        HIP_TRY(hipEventSynchronize(c->evz));
+        if (!cnt[2]) break;
+        cells *= 2;
+    }
+    const long long n_real = cnt[0], n_slot = n_real + cnt[1];
+    long long n_gen = 0;
+    BandItems o{};
+    std::vector<int> lv_off(1, 0);
+    for (int lv = 0; lv < kBandLevels; lv++) {
+        o.lv_off[lv] = (int)n_gen;
+        n_gen += cnt[3 + lv];
+        lv_off.push_back((int)n_gen);
+    }
+    if (n_slot >= (1LL << 30) || n_gen >= (1LL << 31)) {
+        err = "batch too large for 32-bit node, segment or slot indices";
+        return -1;
+    }
+    p->n_slot = n_slot;
+    p->n_generated = cnt[1];
+    p->npool = n_real * (long long)blk + (long long)cnt[1] * (long long)n3;
+    double *norms = nullptr;
+    if ((rc = plan_alloc(p, (size_t)std::max<long long>(p->npool, 1), &p->pool, err)) ||
+        (rc = plan_alloc(p, (size_t)(8 * n_slot + 8), &norms, err)) ||
+        (rc = plan_alloc(p, (size_t)n_slot + 1, &o.slot_off, err)) || (rc = get((size_t)n_slot + 1, &o.slots)) ||
+        (rc = get((size_t)n_gen + 1, &o.gen)) || (rc = get((size_t)n_gen * n3 + 1, &o.gen_s)))
+        return rc;
+    o.n3 = (int)n3;
+    o.n_real = (int)n_real;
+    o.n_roots = n_roots;
+    o.pool = p->pool;
+    o.norms = norms;
+    o.band = band;
+    o.root_out = root_out;
+    o.root_off = root_off;
+    p->args.slot_off = o.slot_off;
+    p->args.slot_norm = norms;
+    if ((rc = dev_band_items(s, b, o, err))) return rc;
+    return dev_pool_fill(s, N, filter, o.gen, lv_off, o.slots, (int)n_slot, err);
 }
 
 int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, bool once,
@@ -2244,7 +2340,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         return -1;
     }
     // sizes and validation
-    long long n_out = 0, n_band = 0, n_slot = 0, n_pool = 0, n_bw = 0, n_actoff = 0, n_act = 0;
+    long long n_out = 0, n_band = 0, n_bw = 0, n_actoff = 0, n_act = 0;
     int wmax = 0;
     for (const PlanPart &pp : parts) {
         const ApplyPlan &pl = *pp.plan;
@@ -2264,15 +2360,13 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
             }
             wmax = std::max(wmax, wq);
         }
-        n_out += (long long)pl.out_node.size();
-        n_band += (long long)pl.band.size();
-        n_slot += (long long)pl.slot_off.size();
-        n_pool += pl.pool_values;
+        n_out += (long long)pl.out_thr.size();
+        n_band += pl.n_band;
         n_bw += (long long)pl.bw.size();
         n_actoff += (long long)pl.active_off.size();
         n_act += (long long)pl.active_terms.size();
     }
-    if (n_out >= (1LL << 27) || n_slot >= (1LL << 30) || n_band >= (1LL << 31)) {
+    if (n_out >= (1LL << 27) || n_band >= (1LL << 31)) {
         err = "batch too large for 32-bit node, segment or slot indices";
         return -1;
     }
@@ -2281,7 +2375,6 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     p->n_out = (int)n_out;
     p->kp1 = N;
     p->wmax = wmax;
-    p->npool = n_pool;
     KArgs &a = p->args;
     hipStream_t s = c->stream;
     int rc = 0;
@@ -2297,7 +2390,6 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     // depths of every apply in the norm and pre-screen tables.
     std::vector<RootApp> root_apps;
     std::vector<RootItem> root_items;
-    std::vector<long long> root_slot_off;
     std::vector<int> root_out;
     std::vector<TermLevel> levels;
     std::vector<long long> tn_off;
@@ -2305,7 +2397,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     std::vector<size_t> mt_size(parts.size());
     long long n_tn = 0;
     {
-        long long o_out = 0, o_pool = 0, o_act = 0;
+        long long o_out = 0, o_act = 0;
         for (size_t ai = 0; ai < parts.size(); ai++) {
             const ApplyPlan &pl = *parts[ai].plan;
             if (dense(pl)) {
@@ -2314,10 +2406,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
                     if (f.L[(size_t)m * f.ndepth] >= 0) root_items.push_back(RootItem{(int)root_apps.size(), m});
                 root_apps.push_back(RootApp{opers[ai]->L, opers[ai]->boff, opers[ai]->blocks, f.ndepth,
                                             (int)root_out.size()});
-                for (size_t r = 0; r < pl.root_q.size(); r++) {
-                    root_out.push_back((int)o_out + pl.root_q[r]);
-                    root_slot_off.push_back(o_pool + pl.slot_off[pl.root_slot[r]]);
-                }
+                for (int q : pl.root_q) root_out.push_back((int)o_out + q);
                 p->root.geo = RootGeo{N, {pl.boxes[0], pl.boxes[1], pl.boxes[2]}};
             }
             std::vector<int> wd(pl.active_off.size(), -1);
@@ -2338,11 +2427,43 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
                 levels.push_back(TermLevel{(int)ai, d, wl, na, (int)o_act + pl.active_off[d], 0, n_tn});
                 n_tn += 4LL * (2 * wl + 1) * na;
             }
-            o_out += (long long)pl.out_node.size();
-            o_pool += pl.pool_values;
+            o_out += (long long)pl.out_thr.size();
             o_act += (long long)pl.active_terms.size();
         }
     }
+    // the distinct input trees, and twice as many cells as the bands can hold
+    // nodes: the 8 children of a node share a neighbourhood of (2w + 2)^3 of
+    // their level, which touches (floor((2w + 1) / 2^j) + 2)^3 ancestors j
+    // levels up; a root has the root boxes
+    std::vector<const Tree *> trees;
+    std::vector<size_t> tree_of, child_at;
+    long long n_child = 0, widest = 0;
+    double n_cell = 0.0;
+    for (const PlanPart &pp : parts) {
+        size_t t = 0;
+        while (t < trees.size() && trees[t] != pp.tree) t++;
+        if (t == trees.size()) {
+            trees.push_back(pp.tree);
+            child_at.push_back((size_t)n_child);
+            n_child += pp.tree->size();
+        }
+        tree_of.push_back(t);
+        for (size_t q = 0; q < pp.plan->band_w.size(); q++) {
+            const int side = 2 * pp.plan->band_w[q] + 1, d = pp.plan->out_depth[q];
+            widest = std::max(widest, (long long)side * side * side);
+            if (d == 0) {
+                n_cell += (double)mra.boxes[0] * mra.boxes[1] * mra.boxes[2];
+                continue;
+            }
+            n_cell += (side + 1.0) * (side + 1.0) * (side + 1.0) / 8.0;
+            for (int j = 1; j < d; j++) {
+                const double t = (side >> j) + 2;
+                n_cell += t * t * t / 8.0;
+            }
+        }
+    }
+    long long cells = 1024;
+    while (cells < 2.0 * n_cell && cells < (1LL << 30)) cells *= 2;
     // Every table of the plan but the pool and the output lives in one
     // device arena; what the host made of it is filled from one staging
     // buffer with one copy, so that a refinement level's plan costs one
@@ -2354,9 +2475,10 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         return off;
     };
     const size_t f_out_depth = place(sizeof(int) * n_out), f_out_app = place(sizeof(int) * n_out);
+    const size_t f_out_l = place(sizeof(int) * 3 * n_out), f_child = place(sizeof(int) * n_child);
+    const size_t f_trees = place(sizeof(BandTree) * parts.size()), f_F = place(sizeof(double) * mra.basis.F.size());
     const size_t f_thr = place(sizeof(double) * n_out), f_band_off = place(sizeof(long long) * n_out);
-    const size_t f_band_w = place(sizeof(int) * n_out), f_band = place(sizeof(int) * n_band);
-    const size_t f_slot_off = place(sizeof(long long) * n_slot);
+    const size_t f_band_w = place(sizeof(int) * n_out);
     const size_t f_bw = place(sizeof(int) * n_bw), f_act_off = place(sizeof(int) * n_actoff);
     const size_t f_act = place(sizeof(int) * n_act);
     const size_t f_apps = place(sizeof(AppDesc) * parts.size());
@@ -2364,20 +2486,20 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     // segment counts (the result block's head; its norms come behind it)
     const size_t n_tot = 2 * parts.size() + 2;
     const size_t f_ra = place(sizeof(RootApp) * root_apps.size()), f_ri = place(sizeof(RootItem) * root_items.size());
-    const size_t f_rs = place(sizeof(long long) * root_slot_off.size()), f_ro = place(sizeof(int) * root_out.size());
+    const size_t f_ro = place(sizeof(int) * root_out.size());
     const size_t f_dense = place((size_t)n_out), f_tno = place(sizeof(long long) * tn_off.size());
     const size_t f_lv = place(sizeof(TermLevel) * levels.size());
     const size_t f_res = place(sizeof(unsigned long long) * (8 + n_tot));
     const size_t up_bytes = f_res + sizeof(unsigned long long) * (8 + n_tot);
     arena = up_bytes + sizeof(double) * 2 * n_out;
     arena = (arena + 255) / 256 * 256;
-    const size_t f_norm = place(sizeof(double) * 8 * n_slot), f_tn = place(sizeof(double) * n_tn);
+    const size_t f_rs = place(sizeof(long long) * root_out.size()), f_band = place(sizeof(int) * n_band);
+    const size_t f_tn = place(sizeof(double) * n_tn);
     const size_t f_tb = place(sizeof(int2) * n_act);
     std::vector<size_t> f_mt(parts.size());
     for (size_t ai = 0; ai < parts.size(); ai++) f_mt[ai] = place(sizeof(double) * mt_size[ai]);
     unsigned char *dev = nullptr;
     rc = plan_alloc(p.get(), arena, &dev, err);
-    if (!rc) rc = plan_alloc(p.get(), (size_t)std::max<long long>(n_pool, 1), &p->pool, err);
     p->out_bytes = sizeof(double) * (size_t)std::max<long long>(n_out, 1) * 8 * N * N * N;
     if (!rc) rc = plan_alloc(p.get(), p->out_bytes / sizeof(double), &a.out_ns, err);
     if (!rc && !root_items.empty()) {
@@ -2396,8 +2518,10 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     };
     std::memset(at(f_res), 0, sizeof(unsigned long long) * (8 + n_tot));
     std::memset(at(f_dense), 0, (size_t)n_out);
-    long long o_out = 0, o_band = 0, o_slot = 0, o_pool = 0, o_bw = 0, o_actoff = 0, o_act = 0;
-    std::vector<PoolFill> fills;
+    for (size_t t = 0; t < trees.size(); t++) put(f_child, (long long)child_at[t], trees[t]->child0);
+    put(f_F, 0, mra.basis.F);
+    std::vector<BandTree> band_trees;
+    long long o_out = 0, o_band = 0, o_bw = 0, o_actoff = 0, o_act = 0;
     for (size_t ai = 0; ai < parts.size(); ai++) {
         const PlanPart &pp = parts[ai];
         const ApplyPlan &pl = *pp.plan;
@@ -2421,26 +2545,21 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         ad.mt_w = mt_shape[ai].second;
         ad.mtab = reinterpret_cast<const double *>(dev + f_mt[ai]);
         p->apps.push_back(ad);
-        const size_t no = pl.out_node.size();
+        const size_t no = pl.out_thr.size();
         // outputs
         put(f_out_depth, o_out, pl.out_depth);
+        put(f_out_l, 3 * o_out, pl.out_l);
         std::fill_n(reinterpret_cast<int *>(at(f_out_app)) + o_out, no, (int)ai);
         put(f_thr, o_out, pl.out_thr);
         {
             long long *bo = reinterpret_cast<long long *>(at(f_band_off)) + o_out;
             for (size_t i = 0; i < no; i++) bo[i] = pl.band_off[i] + o_band;
-            int *bd = reinterpret_cast<int *>(at(f_band)) + o_band;
-            for (size_t i = 0; i < pl.band.size(); i++) bd[i] = pl.band[i] >= 0 ? pl.band[i] + (int)o_slot : pl.band[i];
         }
         put(f_band_w, o_out, pl.band_w);
         if (dense(pl))
             for (int q : pl.root_q) at(f_dense)[o_out + q] = 1;
-        // inputs
-        {
-            long long *so = reinterpret_cast<long long *>(at(f_slot_off)) + o_slot;
-            for (size_t i = 0; i < pl.slot_off.size(); i++) so[i] = pl.slot_off[i] + o_pool;
-        }
-        fills.push_back(PoolFill{pp.inp, &pl, p->pool + o_pool});
+        // input
+        band_trees.push_back(BandTree{reinterpret_cast<const int *>(dev + f_child) + child_at[tree_of[ai]], pp.inp});
         // screening tables
         put(f_bw, o_bw, pl.bw);
         {
@@ -2449,9 +2568,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         }
         put(f_act, o_act, pl.active_terms);
         o_out += (long long)no;
-        o_band += (long long)pl.band.size();
-        o_slot += (long long)pl.slot_off.size();
-        o_pool += pl.pool_values;
+        o_band += pl.n_band;
         o_bw += (long long)pl.bw.size();
         o_actoff += (long long)pl.active_off.size();
         o_act += (long long)pl.active_terms.size();
@@ -2459,7 +2576,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     put(f_apps, 0, p->apps);
     put(f_ra, 0, root_apps);
     put(f_ri, 0, root_items);
-    put(f_rs, 0, root_slot_off);
+    put(f_trees, 0, band_trees);
     put(f_ro, 0, root_out);
     put(f_tno, 0, tn_off);
     put(f_lv, 0, levels);
@@ -2472,8 +2589,6 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     a.band_off = reinterpret_cast<const long long *>(dev + f_band_off);
     a.band_w = reinterpret_cast<const int *>(dev + f_band_w);
     a.band = reinterpret_cast<const int *>(dev + f_band);
-    a.slot_off = reinterpret_cast<const long long *>(dev + f_slot_off);
-    a.slot_norm = reinterpret_cast<const double *>(dev + f_norm);
     a.bw = reinterpret_cast<const int *>(dev + f_bw);
     a.act_off = reinterpret_cast<const int *>(dev + f_act_off);
     a.act_terms = reinterpret_cast<const int *>(dev + f_act);
@@ -2498,10 +2613,14 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     if ((rc = tmp((size_t)(8 * n_band), &ca.cnt))) return rc;
     if (bounds && ((rc = tmp((size_t)(8 * n_band), &ca.bmin)) || (rc = tmp((size_t)(8 * n_band), &ca.bmax)))) return rc;
     HIP_TRY(hipMemcpyAsync(dev, p->stage.data(), up_bytes, hipMemcpyHostToDevice, s));
-    rc = dev_pool_fill(c, mra, fills, reinterpret_cast<double *>(dev + f_norm), p->fill_stage, err);
-    if (!rc)
-        rc = dev_term_tables(s, a, N * N, reinterpret_cast<const TermLevel *>(dev + f_lv), (int)levels.size(),
-                             reinterpret_cast<double *>(dev + f_tn), reinterpret_cast<int2 *>(dev + f_tb), err);
+    rc = make_pool(p.get(), mra, cells, n_band, widest, reinterpret_cast<int *>(dev + f_out_l),
+                   reinterpret_cast<BandTree *>(dev + f_trees), reinterpret_cast<int *>(dev + f_band),
+                   reinterpret_cast<double *>(dev + f_F), reinterpret_cast<int *>(dev + f_ro), (int)root_out.size(),
+                   reinterpret_cast<long long *>(dev + f_rs), [&] {
+                       return dev_term_tables(s, a, N * N, reinterpret_cast<const TermLevel *>(dev + f_lv),
+                                              (int)levels.size(), reinterpret_cast<double *>(dev + f_tn),
+                                              reinterpret_cast<int2 *>(dev + f_tb), err);
+                   }, err);
     ca.k = a;
     if (!rc) rc = dev_count_terms(s, ca, bounds, err);
     if (rc) return rc;
@@ -2570,6 +2689,11 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     cut_done(p.get());
     *out = p.release();
     return 0;
+}
+
+void dev_plan_slots(const DevicePlan *p, long long *slots, long long *generated) {
+    *slots = p->n_slot;
+    *generated = p->n_generated;
 }
 
 void dev_plan_counts(const DevicePlan *p, unsigned long long *term_apps, int *segments) {

@@ -18,20 +18,21 @@ void dev_destroy(DeviceCtx *c);
 void dev_forget_operator(DeviceCtx *c, const void *key);
 
 // One apply of a (possibly batched) device plan: the operator (its host
-// tables, keyed for the context's resident copy), the host plan and the
-// input tree's blocks on the device (tree order).
+// tables, keyed for the context's resident copy), the host plan, the input
+// tree and its blocks on the device (tree order).
 struct PlanPart {
     const void *op_key;
     const OperFlat *flat;
     const ApplyPlan *plan;
+    const Tree *tree;
     const double *inp;
 };
 
 // A plan resident in device memory: band tables, input slots and output
 // blocks of one or more applies, run together in each launch.
 struct DevicePlan;
-// Uploads the host plans and makes the rest on the device: the input pools
-// (dev_pool_fill), the norm and pre-screen tables, the exact counts and the
+// Uploads the host plans and makes the rest on the device: the bands and input
+// slots (dev_band_find), the input pool (dev_pool_fill), the norm and pre-screen tables, the exact counts and the
 // work segments (the fine single-component ones only for a mode with an FP64
 // class beside a low-precision one).  mode: the arithmetic the plan will run.
 // With once (plain FP64, a plan that is run once) the host does not wait for
@@ -41,6 +42,8 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
 // Term-applications counted with the screening rule when the plan was made,
 // and its pair segments.
 void dev_plan_counts(const DevicePlan *p, unsigned long long *term_apps, int *segments);
+// Input slots of the plan, and how many of them are generated nodes.
+void dev_plan_slots(const DevicePlan *p, long long *slots, long long *generated);
 // Run the per-node calculator over the resident plan.  kernel_ms receives the
 // device time of the launches, term_apps the number of term-applications that
 // passed screening.
@@ -138,20 +141,6 @@ int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double co
                   std::string &err, bool out_on_device = false);
 void dev_mul_end(DevMulSession *m);
 
-// The input pools of apply plans (mw_multiply.hip), of every job in one
-// pass: generated nodes reconstructed from their parents and every slot's
-// block copied from the input tree's blocks on the device (inp: the input
-// tree's coefficients, 8 (k+1)^3 per node in tree order) into pool
-// (pl->pool_values doubles, the caller's); norms (device) receives the 8
-// component norms of every slot, jobs in order.  Launches only: stage holds
-// what they upload and must live until the stream has run them.
-struct PoolFill {
-    const double *inp;
-    const ApplyPlan *pl;
-    double *pool;
-};
-int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &jobs, double *norms,
-                  std::vector<unsigned char, UninitAlloc<unsigned char>> &stage, std::string &err);
 // A device copy of n doubles (freed with dev_free).
 int dev_upload(DeviceCtx *c, const double *src, size_t n, double **dst, std::string &err);
 // n doubles of device memory (freed with dev_free).

@@ -241,39 +241,29 @@ double tree_eval(const Tree &t, const double *r);
 bool split_check(const MRA &mra, int depth, double wnorm, double prec, double tnorm);
 
 // ----------------------------------------------------------- apply plan
-// Everything the per-node calculator needs, laid out flat: the output nodes
-// (one refinement level or a whole fixed grid), the input nodes of their
-// bands (real or generated by reconstruction), the dense band table, and the
-// screening thresholds.  Built on the host; consumed by the HIP kernels.
+// What the device makes a plan from, laid out flat: the output nodes (one
+// refinement level or a whole fixed grid), the widths of their bands, the
+// active terms and the screening thresholds.
 struct ApplyPlan {
     int kp1 = 0, ndepth = 0, M = 0;
-    // output nodes (in the order of out_idx)
-    std::vector<int> out_node;      // node index in output tree
-    std::vector<int> out_depth;
-    std::vector<double> out_thr;    // screening threshold per output node
-    std::vector<long long> band_off;  // offset of this node's band table entries
-    std::vector<int> band_w;        // band half-width W (band has (2W+1)^3 entries)
-    std::vector<int> band;          // input slot or -1, order dz,dy,dx with dx fastest
-    // input slots (real or generated nodes)
-    std::vector<long long> slot_off;  // offset of the slot's block in the pool (full: real node, scaling part: generated)
+    // output nodes
+    std::vector<int> out_depth, out_l;  // out_l: translations, 3 per node
+    std::vector<double> out_thr;        // screening threshold per output node
+    // entries of a node's band: (2W+1)^3 from band_off, order dz, dy, dx with
+    // dx fastest
+    std::vector<long long> band_off;
+    std::vector<int> band_w;
+    long long n_band = 0;
     // screening-derived bandwidths: w[(d*M + m)*4 + c]
     std::vector<int> bw;
     std::vector<int> active_off, active_terms;  // per depth, terms with any w >= 0
-    long long n_generated = 0;
     double thr_floor = 0.0;    // smallest positive threshold of the plan
-    // Sources of the pool: slot_src[s] is the slot's input-tree node (>= 0) or
-    // generated node -(g + 1); generated node g is child gen_child[g] of
-    // generated node gen_parent[g] (>= 0) or of input node -(gen_parent[g]
-    // + 1), in order of depth, [gen_level_off[i], gen_level_off[i + 1]) one
-    // depth.
-    std::vector<int> slot_src, gen_parent, gen_child, gen_level_off;
-    long long pool_values = 0;  // doubles of the pool
     // The root boxes when all of them are output nodes with threshold zero
     // (an apply's first level) and their tensor fits the dense root kernels
-    // (2 (k+1) boxes <= 48 per direction): output position and input slot of
-    // each box, x fastest; else empty.
+    // (2 (k+1) boxes <= 48 per direction): output position of each box, x
+    // fastest; else empty.
     int boxes[3] = {0, 0, 0};
-    std::vector<int> root_q, root_slot;
+    std::vector<int> root_q;
 };
 
 // Build the plan for output nodes `nodes` of `out` with thresholds thr.

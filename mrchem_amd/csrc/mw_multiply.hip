@@ -20,7 +20,7 @@
 #include <string>
 #include <vector>
 
-#include "mw_device.hpp"
+#include "mw_apply.hpp"
 
 namespace mwg {
 
@@ -770,15 +770,6 @@ __device__ __forceinline__ void child_step(const double *src, double *X, const d
     __syncthreads();
 }
 
-// One generated node of an apply plan's pool: the scaling block dst of child
-// `child` (bits x, y, z) of a parent with block src, an input-tree node
-// (full: its 8 components) or a generated node (its scaling block only).
-struct GenItem {
-    const double *src;
-    double *dst;
-    int child, full;
-};
-
 // Generated nodes of one depth (their parents are input nodes or generated
 // nodes of the depth above): one workgroup per child.  A launch holds few
 // children and takes as long as one of them, so siblings repeat the first
@@ -980,15 +971,6 @@ static hipError_t add_nodes(hipStream_t s, int n, int cnt, const AddSrc *src, in
     return hipGetLastError();
 }
 
-// One slot of an apply plan's pool: len doubles from src (an input node's
-// full block, or a generated node's scaling block) to dst, and the slot's 8
-// component norms to norms (wavelet norms 0 for a generated slot).
-struct SlotItem {
-    const double *src;
-    double *dst, *norms;
-    int len;
-};
-
 // The copies and the norms in one pass: one wave per (slot, component), each
 // value read once (a copy launch and one thread per norm read them twice, the
 // norms in chains of n^3 dependent additions: 172 -> 14 us a launch at k = 9).
@@ -1012,98 +994,15 @@ __global__ __launch_bounds__(256) void k_pool_fill(int n3, const SlotItem *items
     if (lane == 0) it.norms[comp] = sqrt(q);
 }
 
-int dev_pool_fill(DeviceCtx *c, const MRA &mra, const std::vector<PoolFill> &jobs, double *norms,
-                  std::vector<unsigned char, UninitAlloc<unsigned char>> &stage, std::string &err) {
-    if (jobs.empty()) return 0;
-    HIP_TRY(hipSetDevice(dev_device(c)));
-    hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
-    const int n = mra.kp1(), n3 = n * n * n;
-    const size_t nj = jobs.size();
-    // generated nodes of all jobs by depth (a job's depth lv after its depth
-    // lv - 1), then every job's slots
-    size_t nlv = 0;
-    std::vector<size_t> gen_at(nj + 1, 0), slot_at(nj + 1, 0);
-    for (size_t i = 0; i < nj; i++) {
-        const ApplyPlan &pl = *jobs[i].pl;
-        nlv = std::max(nlv, pl.gen_level_off.empty() ? (size_t)0 : pl.gen_level_off.size() - 1);
-        gen_at[i + 1] = gen_at[i] + pl.gen_parent.size();
-        slot_at[i + 1] = slot_at[i] + pl.slot_src.size();
-    }
-    const size_t n_gen = gen_at[nj], n_slot = slot_at[nj];
-    if (n_gen >= (1u << 31) || n_slot >= (1u << 30)) {
-        err = "pool fill: too many slots";
-        return -1;
-    }
-    // generated nodes of depth lv: items [lv_at[lv], lv_at[lv + 1])
-    std::vector<size_t> lv_at(nlv + 1, 0);
-    for (size_t lv = 0; lv < nlv; lv++) {
-        size_t k = 0;
-        for (size_t i = 0; i < nj; i++) {
-            const std::vector<int> &lo = jobs[i].pl->gen_level_off;
-            if (lv + 1 < lo.size()) k += (size_t)(lo[lv + 1] - lo[lv]);
-        }
-        lv_at[lv + 1] = lv_at[lv] + k;
-    }
-    // one device allocation: [filter | gen items | slot items] (uploaded)
-    // [generated scaling blocks of every job]
-    size_t bytes = 0;
-    auto place = [&](size_t b) {
-        const size_t off = bytes;
-        bytes += (std::max<size_t>(b, 8) + 255) / 256 * 256;
-        return off;
-    };
-    const size_t f_F = place(sizeof(double) * mra.basis.F.size());
-    const size_t f_gi = place(sizeof(GenItem) * n_gen), f_si = place(sizeof(SlotItem) * n_slot);
-    const size_t up_bytes = bytes;
-    const size_t f_gen = place(sizeof(double) * n_gen * (size_t)n3);
-    unsigned char *dev = nullptr;
-    if (int rc = dev_mem(c, bytes, &dev, err)) return rc;
-    double *gen_s = reinterpret_cast<double *>(dev + f_gen);
-    stage.resize(up_bytes);
-    std::memcpy(stage.data() + f_F, mra.basis.F.data(), sizeof(double) * mra.basis.F.size());
-    GenItem *gi = reinterpret_cast<GenItem *>(stage.data() + f_gi);
-    SlotItem *si = reinterpret_cast<SlotItem *>(stage.data() + f_si);
-    // job i's generated node g is gen_s block gen_at[i] + g
-    std::vector<size_t> lv_fill(lv_at.begin(), lv_at.end() - (nlv ? 1 : 0));
-    for (size_t i = 0; i < nj; i++) {
-        const ApplyPlan &pl = *jobs[i].pl;
-        const double *inp = jobs[i].inp;
-        double *gs = gen_s + gen_at[i] * (size_t)n3;
-        for (size_t lv = 0; lv + 1 < pl.gen_level_off.size(); lv++)
-            for (int g = pl.gen_level_off[lv]; g < pl.gen_level_off[lv + 1]; g++) {
-                const int par = pl.gen_parent[g];
-                gi[lv_fill[lv]++] = GenItem{par < 0 ? inp + (size_t)(-par - 1) * 8 * n3 : gs + (size_t)par * n3,
-                                            gs + (size_t)g * n3, pl.gen_child[g], par < 0};
-            }
-    }
-    for (size_t i = 0; i < nj; i++) {
-        const ApplyPlan &pl = *jobs[i].pl;
-        const double *inp = jobs[i].inp;
-        const double *gs = gen_s + gen_at[i] * (size_t)n3;
-        for (size_t q = 0; q < pl.slot_src.size(); q++) {
-            const int sr = pl.slot_src[q];
-            SlotItem &it = si[slot_at[i] + q];
-            it.src = sr >= 0 ? inp + (size_t)sr * 8 * n3 : gs + (size_t)(-sr - 1) * n3;
-            it.dst = jobs[i].pool + pl.slot_off[q];
-            it.norms = norms + (slot_at[i] + q) * 8;
-            it.len = sr >= 0 ? 8 * n3 : n3;
-        }
-    }
-    const double *F = reinterpret_cast<const double *>(dev + f_F);
-    const GenItem *dgi = reinterpret_cast<const GenItem *>(dev + f_gi);
-    const SlotItem *dsi = reinterpret_cast<const SlotItem *>(dev + f_si);
-    hipError_t e = hipMemcpyAsync(dev, stage.data(), up_bytes, hipMemcpyHostToDevice, s);
-    for (size_t lv = 0; e == hipSuccess && lv < nlv; lv++) {
-        const int cnt = (int)(lv_at[lv + 1] - lv_at[lv]);
-        if (cnt == 0) continue;
-        e = gen_fill(s, n, dgi + lv_at[lv], cnt, F);
-    }
+int dev_pool_fill(hipStream_t s, int n, const double *F, const GenItem *gen, const std::vector<int> &lv_off,
+                  const SlotItem *slots, int n_slot, std::string &err) {
+    hipError_t e = hipSuccess;
+    for (size_t lv = 0; e == hipSuccess && lv + 1 < lv_off.size(); lv++)
+        if (lv_off[lv + 1] > lv_off[lv]) e = gen_fill(s, n, gen + lv_off[lv], lv_off[lv + 1] - lv_off[lv], F);
     if (e == hipSuccess && n_slot > 0) {
-        hipLaunchKernelGGL(k_pool_fill, dim3((unsigned)(2 * n_slot)), dim3(256), 0, s, n3, dsi, (int)n_slot);
+        hipLaunchKernelGGL(k_pool_fill, dim3((unsigned)(2 * n_slot)), dim3(256), 0, s, n * n * n, slots, n_slot);
         e = hipGetLastError();
     }
-    // (put back at once: its next holder's work comes after these launches)
-    dev_mem_put(c, dev);
     if (e != hipSuccess) {
         err = std::string("pool fill: ") + hipGetErrorString(e);
         return -2;

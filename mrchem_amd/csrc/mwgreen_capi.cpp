@@ -546,9 +546,7 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         size_t total = 0;
         for (size_t a = 0; a < active.size(); a++) {
             Job *j = active[a];
-            parts.push_back(PlanPart{j->op, &j->op->flat, &j->plan, inputs.of(ctx, j->inp_h)});
-            slots += (double)j->plan.slot_off.size();
-            gen += (double)j->plan.n_generated;
+            parts.push_back(PlanPart{j->op, &j->op->flat, &j->plan, j->inp, inputs.of(ctx, j->inp_h)});
             total += j->work.size();
         }
         std::string err;
@@ -559,6 +557,10 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         if (rc) return dev_fail(rc, err);
         const double t1r = now_ms();
         t_create += t1r - t1;
+        long long n_slots = 0, n_gen = 0;
+        dev_plan_slots(dp, &n_slots, &n_gen);
+        slots += (double)n_slots;
+        gen += (double)n_gen;
         double ms = 0.0;
         unsigned long long apps = 0;
         std::vector<double> norms(2 * total);  // squared: scaling parts, then wavelet parts
@@ -744,9 +746,7 @@ int make_plan(mwg_context ctx, int n, const mwg_tree *out, const mwg_operator *o
     std::vector<PlanPart> parts;
     for (int i = 0; i < n; i++) {
         const ApplyPlan &ap = jobs[i].plan;
-        parts.push_back(PlanPart{op[i], &op[i]->flat, &ap, inputs.of(ctx, inp[i])});
-        p->slots += (double)ap.slot_off.size();
-        p->gen += (double)ap.n_generated;
+        parts.push_back(PlanPart{op[i], &op[i]->flat, &ap, jobs[i].inp, inputs.of(ctx, inp[i])});
         for (int w : ap.band_w) p->band_w = std::max(p->band_w, (double)w);
         p->outs.push_back(out[i]);
         p->ops.push_back(op[i]);
@@ -762,6 +762,10 @@ int make_plan(mwg_context ctx, int n, const mwg_tree *out, const mwg_operator *o
         unsigned long long apps = 0;
         int segs = 0;
         dev_plan_counts(p->dev, &apps, &segs);
+        long long n_slots = 0, n_gen = 0;
+        dev_plan_slots(p->dev, &n_slots, &n_gen);
+        p->slots = (double)n_slots;
+        p->gen = (double)n_gen;
         p->host_apps = (double)apps;
         p->segs = (double)segs;
     }
