@@ -180,5 +180,9 @@ int dev_term_tables(hipStream_t s, const KArgs &k, int nn, const TermLevel *leve
 // Launches only, on stream.
 int dev_count_terms(hipStream_t s, const CountArgs &c, bool bounds, std::string &err);
 int dev_cut_segments(hipStream_t s, const CountArgs &c, bool bounds, std::string &err);
+// The class lists of a cut with bounds (n: their two lengths, cleared before).
+// Launches only, on stream.
+int dev_class_lists(hipStream_t s, const CountArgs &c, double tau, int *lo, int *hi, unsigned long long *n,
+                    std::string &err);
 
 }  // namespace mwg

@@ -1579,14 +1579,16 @@ __device__ __forceinline__ int next_entry(unsigned long long *head, int *s_next)
     return __builtin_amdgcn_readfirstlane(*s_next);
 }
 
-// FP32 class over the pair segments seg_list[0, n): bounds at most hi_mult
-// thr_cls.  Held to two waves per SIMD.
+// FP32 class over the pair segments seg_list[0, n) (n_dev: as many as it
+// holds): bounds at most hi_mult thr_cls.  Held to two waves per SIMD.
 template <int N>
 __global__ __launch_bounds__(JobShape<N>::T) __attribute__((amdgpu_waves_per_eu(2))) void k_apply(
-    KArgs a, const float *pool, const int *seg_list, int n, double hi_mult, unsigned long long *head) {
+    KArgs a, const float *pool, const int *seg_list, const unsigned long long *n_dev, int n, double hi_mult,
+    unsigned long long *head) {
     __shared__ ApplySmem<N> sm;
     extern __shared__ double nrm_s[];
     __shared__ int s_next;
+    if (n_dev) n = (int)*n_dev;
     while (true) {
         const int e = next_entry(head, &s_next);
         if (e >= n) break;
@@ -1595,16 +1597,18 @@ __global__ __launch_bounds__(JobShape<N>::T) __attribute__((amdgpu_waves_per_eu(
 }
 
 // The split class of the split mode: one workgroup per pair segment of
-// seg_list (terms with bound <= tau thr_cls, FP16 split products).  It runs
+// seg_list (n_dev: as many as it holds; terms with bound <= tau thr_cls, FP16 split products).  It runs
 // beside the persistent FP64-class launch on the second stream.  A launch of
 // one grid per entry keeps this kernel at 128 VGPRs (4 waves per SIMD at
 // N <= 10); a persistent loop around the body, or the FP64 body in the same
 // kernel, costs registers and was measured slower.
 template <int N>
 __global__ __launch_bounds__(SplitShape<N>::T) __attribute__((amdgpu_waves_per_eu(SplitShape<N>::WPE))) void k_apply_h(
-    KArgs a, const _Float16 *pool_h, const double *pool_sc, const int *seg_list, double tau, double single_mult) {
+    KArgs a, const _Float16 *pool_h, const double *pool_sc, const int *seg_list, const unsigned long long *n_dev,
+    double tau, double single_mult) {
     __shared__ SplitSmem<N> sm;
     extern __shared__ double nrm_s[];
+    if (n_dev && blockIdx.x >= *n_dev) return;
     split_segment<N>(a, pool_h, pool_sc, seg_list[blockIdx.x], 0.0, tau, single_mult, 1, sm, nrm_s);
 }
 
@@ -1850,6 +1854,8 @@ struct DevicePlan {
     size_t n_tot = 0;
     bool cut_open = false;
     std::vector<void *> temp;
+    // a deferred plan's class lists (in temp); their lengths are counters 4, 5
+    int *dev_list[2] = {nullptr, nullptr};
     std::vector<unsigned char, UninitAlloc<unsigned char>> stage;
     long long n_slot = 0, n_generated = 0;
     unsigned found[kBandCounts];  // what the search for them counted
@@ -2181,9 +2187,38 @@ static int upload_at(T *dst, const std::vector<T, A> &v, hipStream_t s, std::str
     return 0;
 }
 
-// Room for cap segments and the cut into it (again: the counts of a first cut
+// Norm table bytes at the start of a job's LDS (16-byte aligned end).
+static int nrm_bytes(int wmax) { return (int)((sizeof(double) * 64 * nrm_stride(2 * wmax + 1) + 15) / 16 * 16); }
+
+// Whether the plan's widest band fits the norm table of the mode's
+// low-precision kernel beside its tiles; where it doesn't the host has to know
+// that no segment is of that class before the kernel is left out.
+template <int N>
+static bool lowp_fits_n(const DevicePlan *p, int mode) {
+    const size_t tiles = mode == 1 ? sizeof(ApplySmem<N>) : sizeof(SplitSmem<N>);
+    return tiles + (size_t)nrm_bytes(p->wmax) + 16 <= (size_t)p->ctx->lds_max;
+}
+
+static bool lowp_fits(const DevicePlan *p, int mode) {
+    switch (p->kp1) {
+        case 2: return lowp_fits_n<2>(p, mode);
+        case 3: return lowp_fits_n<3>(p, mode);
+        case 4: return lowp_fits_n<4>(p, mode);
+        case 5: return lowp_fits_n<5>(p, mode);
+        case 6: return lowp_fits_n<6>(p, mode);
+        case 7: return lowp_fits_n<7>(p, mode);
+        case 8: return lowp_fits_n<8>(p, mode);
+        case 9: return lowp_fits_n<9>(p, mode);
+        case 10: return lowp_fits_n<10>(p, mode);
+        case 11: return lowp_fits_n<11>(p, mode);
+        case 12: return lowp_fits_n<12>(p, mode);
+        default: return false;
+    }
+}
+
+// Room for cap segments (defer: and their class lists) and the cut into it (again: the counts of a first cut
 // are cleared).  Launches only.
-static int cut_plan(DevicePlan *p, const long long *cap, bool bounds, bool again, std::string &err) {
+static int cut_plan(DevicePlan *p, const long long *cap, bool bounds, bool defer, bool again, std::string &err) {
     DeviceCtx *c = p->ctx;
     CountArgs &ca = p->count;
     const long long n_all = cap[0] + cap[1];
@@ -2197,6 +2232,10 @@ static int cut_plan(DevicePlan *p, const long long *cap, bool bounds, bool again
     if (bounds) {
         if ((rc = dev_mem(c, (size_t)n_all, &ca.rec, err))) return rc;
         p->temp.push_back(ca.rec);
+        for (int i = 0; defer && i < 2; i++) {
+            if ((rc = dev_mem(c, (size_t)cap[i], &p->dev_list[i], err))) return rc;
+            p->temp.push_back(p->dev_list[i]);
+        }
     }
     for (int i = 0; i < 2; i++) ca.cap[i] = (int)cap[i];
     p->args.seg_job = ca.seg_job = seg;
@@ -2628,7 +2667,8 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     // 24, plain FP64's 64) for each output node; the few plans that need more
     // are cut again.
     long long cap[2] = {bounds ? 2048 + 16 * n_out : 16384 + 64 * n_out, bounds ? 16384 + 24 * n_out : 0};
-    if ((rc = cut_plan(p.get(), cap, bounds, false, err))) return rc;
+    const bool defer = once && (!bounds || lowp_fits(p.get(), mode));
+    if ((rc = cut_plan(p.get(), cap, bounds, defer, false, err))) return rc;
     if (!root_items.empty()) {
         RootLaunch &r = p->root;
         r.apps = reinterpret_cast<const RootApp *>(dev + f_ra);
@@ -2641,12 +2681,12 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         r.totals = ca.totals;
         r.n_totals = (int)parts.size();
     }
-    // One wait per refinement level instead of three: the calculator starts
-    // behind the cut, and counters, segment counts and norms come back in one
+    // One wait per refinement level instead of three: the calculator (in the
+    // low-precision modes the class lists first) starts behind the cut, and counters, segment counts and norms come back in one
     // copy after it (single-Gaussian Coulomb apply at k = 7: 2.74 to 2.43 ms;
     // the exchange applies of 4 orbitals in one batch: 12.0 to 10.5 ms, with
     // the one-launch assembly of the trees).
-    if (once && !bounds) {
+    if (defer) {
         *out = p.release();
         return 0;
     }
@@ -2658,7 +2698,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         for (int i = 0; i < 2; i++) cap[i] = std::max<long long>(cap[i], (long long)tot[n_tot - 2 + i]);
         p->bufs.pop_back();
         dev_mem_put(c, ca.seg_job);
-        if ((rc = cut_plan(p.get(), cap, bounds, true, err))) return rc;
+        if ((rc = cut_plan(p.get(), cap, bounds, false, true, err))) return rc;
     }
     if (bounds) {
         // what the class lists of the mixed and split modes are chosen from,
@@ -2754,9 +2794,6 @@ void dev_plan_destroy(DevicePlan *p) {
     delete p;
 }
 
-// Norm table bytes at the start of a job's LDS (16-byte aligned end).
-static int nrm_bytes(int wmax) { return (int)((sizeof(double) * 64 * nrm_stride(2 * wmax + 1) + 15) / 16 * 16); }
-
 // Grid of a persistent launch: the resident workgroups of `kernel` with
 // `static_lds` bytes of static and `shmem` bytes of dynamic LDS (occupancy
 // per CU x CUs), at most n.
@@ -2785,15 +2822,17 @@ static int persistent_grid(DeviceCtx *c, const void *kernel, int threads, size_t
 }
 
 template <int N>
-static int launch32_n(DeviceCtx *c, const KArgs &a, const float *pool, const int *list, int n, int wmax, double hi,
-                      unsigned long long *head, hipStream_t s, std::string &err) {
+static int launch32_n(DeviceCtx *c, const KArgs &a, const float *pool, const int *list,
+                      const unsigned long long *n_dev, int n, int wmax, double hi, unsigned long long *head,
+                      hipStream_t s, std::string &err) {
     if (n == 0) return 0;
     const size_t shmem = nrm_bytes(wmax);
     int grid = 0;
     int rc = persistent_grid(c, reinterpret_cast<const void *>(&k_apply<N>), JobShape<N>::T, sizeof(ApplySmem<N>),
                              shmem, n, &grid, err);
     if (rc) return rc;
-    hipLaunchKernelGGL((k_apply<N>), dim3(grid), dim3(JobShape<N>::T), shmem, s, a, pool, list, n, hi, head);
+    hipLaunchKernelGGL((k_apply<N>), dim3(grid), dim3(JobShape<N>::T), shmem, s, a, pool, list, n_dev, n, hi,
+                       head);
     HIP_TRY(hipGetLastError());
     return 0;
 }
@@ -2828,11 +2867,12 @@ static int launch64_n(DeviceCtx *c, const KArgs &a, const double *pool, const in
         default: err = "unsupported basis size"; return -1;                                                 \
     }
 
-// Persistent launch of the FP32 class over the pair segments list[0, n):
-// bounds at most hi thr_cls.
-static int launch32(const DevicePlan *p, const int *list, int n, double hi, unsigned long long *head,
-                    std::string &err) {
-#define MWG_LAUNCH(NN) launch32_n<NN>(p->ctx, p->args, p->pool32, list, n, p->wmax, hi, head, p->ctx->stream, err)
+// Persistent launch of the FP32 class over the pair segments list[0, n) (n_dev:
+// as many as it holds, n at most): bounds at most hi thr_cls.
+static int launch32(const DevicePlan *p, const int *list, const unsigned long long *n_dev, int n, double hi,
+                    unsigned long long *head, std::string &err) {
+#define MWG_LAUNCH(NN) \
+    launch32_n<NN>(p->ctx, p->args, p->pool32, list, n_dev, n, p->wmax, hi, head, p->ctx->stream, err)
     MWG_SIZES(MWG_LAUNCH)
 #undef MWG_LAUNCH
 }
@@ -3006,35 +3046,28 @@ static int ensure_h16(DevicePlan *p, std::string &err) {
 }
 
 template <int N>
-static int launch_h_n(const DevicePlan *p, double tau, std::string &err) {
-    if (p->n_lo == 0) return 0;
+static int launch_h_n(const DevicePlan *p, const int *list, const unsigned long long *n_dev, int n, double tau,
+                      std::string &err) {
+    if (n == 0) return 0;
     const size_t shmem = nrm_bytes(p->wmax);
     if (sizeof(SplitSmem<N>) + shmem + 16 > (size_t)p->ctx->lds_max) {
         err = "band half-width " + std::to_string(p->wmax) + " needs more LDS than the split kernel has at k+1 = " +
               std::to_string(N) + "; use the FP64 or mixed mode";
         return -1;
     }
-    hipLaunchKernelGGL((k_apply_h<N>), dim3(p->n_lo), dim3(SplitShape<N>::T), shmem, p->ctx->stream, p->args,
-                       p->pool_h, p->pool_hsc, p->list_lo, tau, p->single_ratio);
+    hipLaunchKernelGGL((k_apply_h<N>), dim3(n), dim3(SplitShape<N>::T), shmem, p->ctx->stream, p->args, p->pool_h,
+                       p->pool_hsc, list, n_dev, tau, p->single_ratio);
     HIP_TRY(hipGetLastError());
     return 0;
 }
 
-static int launch_h(const DevicePlan *p, double tau, std::string &err) {
-    switch (p->kp1) {
-        case 2: return launch_h_n<2>(p, tau, err);
-        case 3: return launch_h_n<3>(p, tau, err);
-        case 4: return launch_h_n<4>(p, tau, err);
-        case 5: return launch_h_n<5>(p, tau, err);
-        case 6: return launch_h_n<6>(p, tau, err);
-        case 7: return launch_h_n<7>(p, tau, err);
-        case 8: return launch_h_n<8>(p, tau, err);
-        case 9: return launch_h_n<9>(p, tau, err);
-        case 10: return launch_h_n<10>(p, tau, err);
-        case 11: return launch_h_n<11>(p, tau, err);
-        case 12: return launch_h_n<12>(p, tau, err);
-        default: err = "unsupported basis size"; return -1;
-    }
+// One workgroup per pair segment of list[0, n) (n_dev: as many as it holds, n
+// at most).
+static int launch_h(const DevicePlan *p, const int *list, const unsigned long long *n_dev, int n, double tau,
+                    std::string &err) {
+#define MWG_LAUNCH(NN) launch_h_n<NN>(p, list, n_dev, n, tau, err)
+    MWG_SIZES(MWG_LAUNCH)
+#undef MWG_LAUNCH
 }
 
 // The launch sequence of one step on the context's stream(s): counters and
@@ -3063,6 +3096,21 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
     // queue heads of the persistent launches: counters[2] (first stream),
     // counters[3] (second stream)
     unsigned long long *head1 = p->args.counters + 2, *head2 = p->args.counters + 3;
+    // the class lists: the host's, or a deferred plan's on the device
+    const int *lo = p->list_lo, *hi = p->list_hi;
+    const unsigned long long *n_lo_dev = nullptr, *n_hi_dev = nullptr;
+    int n_lo = p->n_lo, n_hi = p->n_hi;
+    if (mode != 0 && p->cut_open) {
+        unsigned long long *n = p->args.counters + 4;
+        rc = dev_class_lists(c->stream, p->count, tau, p->dev_list[0], p->dev_list[1], n, err);
+        if (rc) return rc;
+        lo = p->dev_list[0];
+        hi = p->dev_list[1];
+        n_lo_dev = n;
+        n_hi_dev = n + 1;
+        n_lo = p->count.cap[0];
+        n_hi = p->count.cap[1];
+    }
     if (mode == 0) {
         // lo = 0: every term that passes screening, over the pair segments
         rc = p->cut_open ? launch64(p, nullptr, p->count.n_seg, p->count.cap[0], 0.0, head1, c->stream, err)
@@ -3077,11 +3125,11 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         // with the FP32 class instead of before it (64 Helmholtz applies at
         // k = 11, 119,968 output nodes: 316 ms against 394 ms a step).
         if (timed) HIP_TRY(hipEventRecord(c->ev2s, c->stream));
-        rc = launch64(p, p->list_hi, nullptr, p->n_hi, tau, head2, c->stream, err);
+        rc = launch64(p, hi, n_hi_dev, n_hi, tau, head2, c->stream, err);
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(c->ev2e, c->stream));
         if (timed) HIP_TRY(hipEventRecord(c->evl, c->stream));
-        rc = launch32(p, p->list_lo, p->n_lo, tau, head1, err);
+        rc = launch32(p, lo, n_lo_dev, n_lo, tau, head1, err);
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(c->evm, c->stream));
     } else {
@@ -3090,11 +3138,11 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         HIP_TRY(hipEventRecord(c->evz, c->stream));
         HIP_TRY(hipStreamWaitEvent(c->stream2, c->evz, 0));
         if (timed) HIP_TRY(hipEventRecord(c->ev2s, c->stream2));
-        rc = launch64(p, p->list_hi, nullptr, p->n_hi, tau, head2, c->stream2, err);
+        rc = launch64(p, hi, n_hi_dev, n_hi, tau, head2, c->stream2, err);
         if (rc) return rc;
         HIP_TRY(hipEventRecord(c->ev2e, c->stream2));
         if (timed) HIP_TRY(hipEventRecord(c->evl, c->stream));
-        rc = launch_h(p, tau, err);
+        rc = launch_h(p, lo, n_lo_dev, n_lo, tau, err);
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(c->evm, c->stream));
         HIP_TRY(hipStreamWaitEvent(c->stream, c->ev2e, 0));
@@ -3252,7 +3300,7 @@ int dev_plan_run(DevicePlan *p, int mode, double tau, double *kernel_ms, unsigne
     }
     if (mode != 0) {
         int rc = mode == 1 ? ensure_f32(p, err) : ensure_h16(p, err);
-        if (!rc) rc = make_lists(p, mode, tau, err);
+        if (!rc && !p->cut_open) rc = make_lists(p, mode, tau, err);
         if (rc) return rc;
     }
     const unsigned bit = 1u << (2 * mode + (post ? 1 : 0));
@@ -3287,8 +3335,9 @@ int dev_plan_run(DevicePlan *p, int mode, double tau, double *kernel_ms, unsigne
             break;
         }
         // more segments than the room: cut again and run again
-        const long long cap[2] = {(long long)cnt[8 + p->n_tot - 2], p->count.cap[1]};
-        int rc = cut_plan(p, cap, false, true, err);
+        long long cap[2];
+        for (int i = 0; i < 2; i++) cap[i] = std::max<long long>(p->count.cap[i], (long long)cnt[8 + p->n_tot - 2 + i]);
+        int rc = cut_plan(p, cap, mode != 0, true, true, err);
         if (rc) return rc;
     }
     if (norms2) std::memcpy(norms2, res.data() + 8 + p->n_tot, sizeof(double) * 2 * (size_t)p->n_out);
