@@ -46,6 +46,7 @@ struct KArgs {
     // input slots (all applies, concatenated)
     const long long *slot_off;
     const double *slot_norm;
+    int n_real, pad_;                 // slots [0, n_real) hold full blocks
     // screening tables: active terms per depth, and their norms (k_term_norms)
     // [c][l + w][active term] of the depth's band half-width w, from
     // tn + tn_off[act_base + d]

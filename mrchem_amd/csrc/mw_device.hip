@@ -573,13 +573,14 @@ struct Job4 {
     // waves per SIMD the registers are held to: two at N >= 9 (accumulators
     // and F rows alone take 126-162 of the 256), four below
     static constexpr int WPE = N >= 9 ? 2 : 4;
+    static constexpr int AHEAD = WPE == 2 ? 4 : 2;  // screening steps whose norms load together
 };
 
-// Worklist item: the operator block ids of translation 0, component 0, the
-// distance of two components' blocks, and the band position, input component
-// and which components of the job pass.
+// Worklist item: active term, input slot, and the band position (lx, ly, lz from
+// the band's corner) with the input component and which components of the job
+// pass.
 struct Item4 {
-    int center, span, pos;  // pos = p << 5 | t1 << 4 | t0 << 3 | ft
+    int e, slot, pos;  // pos = lz << 21 | ly << 13 | lx << 5 | t1 << 4 | t0 << 3 | ft
 };
 
 template <int N>
@@ -604,64 +605,92 @@ __device__ __forceinline__ void wave_order() {
 // then for each the terms 64 at a time (one per lane), all of a pair before
 // the next pair, so that a pair's F rows load once.  Stops where 64 more items
 // may not fit and leaves the pair in pi and its first open term in e0.  Of pair
-// u_last only the terms before e_last belong to the segment.
-template <bool PAIR, int CAP>
+// u_last only the terms before e_last belong to the segment.  The norms of AHEAD
+// steps load together: a pair of a fine level holds one or two passing terms,
+// and one step's loads after the other's cost a microsecond each (frozen
+// 656-node Helmholtz plan at k = 9: 2.36 -> 2.28 ms; all levels of a k = 4
+// Coulomb apply: 0.58 -> 0.53 ms).
+template <bool PAIR, int CAP, int AHEAD>
 __device__ __forceinline__ int screen_items(const KArgs &a, const AppDesc &ad, const JobCtx &j, const double *tn,
-                                            const int2 *tb, int &pi, int pi_end, int &e0, int u_last, int e_last,
-                                            Item4 *wl, int lane, unsigned long long &apps0,
-                                            unsigned long long &apps1) {
+                                            int &pi, int pi_end, int &e0, int u_last, int e_last, Item4 *wl, int lane,
+                                            unsigned long long &apps0, unsigned long long &apps1) {
     const int S = 2 * ad.mt_w + 1;
     const long long S3 = (long long)S * S * S;
     const double *mt = ad.mtab + (long long)(j.d - ad.mt_d0) * 64 * S3;
+    const long long nz1 = (long long)2 * j.nl * j.nact;  // of gt | 4 from gt
     int n = 0;
     while (pi < pi_end) {
         const int pr = pi + lane;
         bool cand = false;
         double fl = 0.0;
+        int slot = -1, pos = 0, ox = 0, oy = 0, oz = 0;
         if (pr < pi_end) {
             const int p = pr >> 3, ft = pr & 7;
-            const int s = a.band[j.boff + p];
+            slot = a.band[j.boff + p];
             // the NS form has no scaling-to-scaling part below the roots
             const bool ex0 = j.d > 0 && ft == 0 && j.gt == 0;
-            if (s >= 0 && (PAIR || !ex0)) {
-                fl = a.slot_norm[(long long)s * 8 + ft];
-                const int lx = p % j.side - j.w, ly = (p / j.side) % j.side - j.w, lz = p / (j.side * j.side) - j.w;
-                const long long li = ((long long)(lz + ad.mt_w) * S + (ly + ad.mt_w)) * S + (lx + ad.mt_w);
-                const int cxy = (2 * j.gb[0] + (ft & 1)) | ((2 * j.gb[1] + ((ft >> 1) & 1)) << 2);
+            if (slot >= 0 && (PAIR || !ex0)) {
+                fl = a.slot_norm[(long long)slot * 8 + ft];
+                const int x = p % j.side, y = (p / j.side) % j.side, z = p / (j.side * j.side), dw = ad.mt_w - j.w;
+                const long long li = ((long long)(z + dw) * S + (y + dw)) * S + (x + dw);
+                const int cx = 2 * j.gb[0] + (ft & 1), cy = 2 * j.gb[1] + ((ft >> 1) & 1);
                 const int cz = 2 * j.gb[2] + ((ft >> 2) & 1);
+                const int cxy = cx | (cy << 2);
                 double mb = ex0 ? 0.0 : mt[(cxy | (cz << 4)) * S3 + li] * fl;
                 if (PAIR) mb = fmax(mb, mt[(cxy | ((cz + 2) << 4)) * S3 + li] * fl);
                 cand = fl > 0.0 && mb > j.thr && mb > j.thr_lo;
+                pos = z << 21 | y << 13 | x << 5 | ft;
+                ox = (cx * j.nl + x) * j.nact;
+                oy = (cy * j.nl + y) * j.nact;
+                oz = (cz * j.nl + z) * j.nact;
             }
         }
         unsigned long long cm = __ballot(cand);
+        if (!(cm & 1)) e0 = 0;  // e0 belongs to the first pair alone
         while (cm) {
-            const int k = __builtin_ctzll(cm);
-            cm &= cm - 1;
-            const int p = (pi + k) >> 3, ft = (pi + k) & 7;
-            const double fn = __shfl(fl, k);
-            const int lx = p % j.side, ly = (p / j.side) % j.side, lz = p / (j.side * j.side);
-            const int cz = 2 * j.gb[2] + ((ft >> 2) & 1);
-            const double *nx = tn + (long long)((2 * j.gb[0] + (ft & 1)) * j.nl + lx) * j.nact;
-            const double *ny = tn + (long long)((2 * j.gb[1] + ((ft >> 1) & 1)) * j.nl + ly) * j.nact;
-            const double *nz = tn + (long long)(cz * j.nl + lz) * j.nact;
-            const double *nz1 = nz + (long long)2 * j.nl * j.nact;
-            const bool ex0 = PAIR && j.d > 0 && ft == 0 && j.gt == 0;
-            if (k > 0) e0 = 0;  // e0 belongs to the first pair alone
-            const int e1 = pi + k == u_last ? e_last : j.nact;
-            for (; e0 < e1; e0 += 64) {
+            int sk[AHEAD], se[AHEAD];
+            double vx[AHEAD], vy[AHEAD], vz[AHEAD], vw[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                sk[u] = -1;
+                se[u] = 0;
+                if (cm) {
+                    const int k = __builtin_ctzll(cm);
+                    const int e1 = pi + k == u_last ? e_last : j.nact;
+                    sk[u] = k;
+                    se[u] = e0;
+                    e0 += 64;
+                    if (e0 >= e1) {
+                        cm &= cm - 1;
+                        e0 = 0;
+                    }
+                    const int e = min(se[u] + lane, j.nact - 1);
+                    vx[u] = tn[__builtin_amdgcn_readlane(ox, k) + e];
+                    vy[u] = tn[__builtin_amdgcn_readlane(oy, k) + e];
+                    const double *z = tn + __builtin_amdgcn_readlane(oz, k);
+                    vz[u] = z[e];
+                    if (PAIR) vw[u] = z[nz1 + e];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                if (sk[u] < 0) continue;
+                const int k = sk[u], e = se[u] + lane;
                 if (n + 64 > CAP) {
                     pi += k;
+                    e0 = se[u];
                     return n;
                 }
-                const int e = e0 + lane;
+                const int e1 = pi + k == u_last ? e_last : j.nact, ps = __builtin_amdgcn_readlane(pos, k);
+                const double fn = __shfl(fl, k);
+                const bool ex0 = PAIR && j.d > 0 && (ps & 7) == 0 && j.gt == 0;
                 bool t0 = false, t1 = false;
                 if (e < e1) {
-                    const double nxy = nx[e] * ny[e];
-                    const double b0 = (nxy * nz[e]) * fn;
+                    const double nxy = vx[u] * vy[u];
+                    const double b0 = (nxy * vz[u]) * fn;
                     t0 = !ex0 && b0 > j.thr && b0 > j.thr_lo && !(b0 > j.thr_hi);
                     if (PAIR) {
-                        const double b1 = (nxy * nz1[e]) * fn;
+                        const double b1 = (nxy * vw[u]) * fn;
                         t1 = b1 > j.thr && b1 > j.thr_lo && !(b1 > j.thr_hi);
                     }
                 }
@@ -672,15 +701,13 @@ __device__ __forceinline__ int screen_items(const KArgs &a, const AppDesc &ad, c
                 } else {
                     apps0 += __popcll(mask);
                 }
-                if (t0 || t1) {
-                    const int2 b = tb[e];
+                if (t0 || t1)
                     wl[n + __popcll(mask & ((1ull << lane) - 1ull))] =
-                        Item4{b.x, b.y, (p << 5) | ((int)t1 << 4) | ((int)t0 << 3) | ft};
-                }
+                        Item4{e, __builtin_amdgcn_readlane(slot, k), ps | ((int)t1 << 4) | ((int)t0 << 3)};
                 n += __popcll(mask);
             }
-            e0 = 0;
         }
+        e0 = 0;
         pi += 64;
     }
     return n;
@@ -733,9 +760,10 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
     // + lc][jx = 4 k + lq]
     constexpr int NF = S::CHAIN ? G * G * G : CT * G;
     double f[NF];
-    auto load_f = [&](int pos) {
-        const int s = a.band[j.boff + (pos >> 5)];
-        const __attribute__((address_space(1))) double *src = gmem(pool) + a.slot_off[s] + (pos & 7) * N3;
+    auto load_f = [&](const Item4 &it) {
+        // (as slot_off: full blocks of the real slots, then scaling blocks)
+        const long long b = it.slot < a.n_real ? 8LL * it.slot + (it.pos & 7) : 7LL * a.n_real + it.slot;
+        const __attribute__((address_space(1))) double *src = gmem(pool) + b * N3;
         if constexpr (S::CHAIN) {
             const int base = ((lane >> 2) & 3) * N2 + l3 * N + lq;
 #pragma unroll
@@ -760,12 +788,13 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
     // operator blocks of an item into registers, then into the stage; the z
     // block of a component that does not pass is left as it is
     double pre[PAIR ? 4 : 3][LPD];
-    auto fetch = [&](const Item4 &it) {
-        const int pos = it.pos, p = pos >> 5;
-        const int lx = p % j.side - j.w, ly = (p / j.side) % j.side - j.w, lz = p / (j.side * j.side) - j.w;
+    auto fetch = [&](const Item4 &it, int2 term) {
+        const int pos = it.pos, center = __builtin_amdgcn_readfirstlane(term.x),
+                  span = __builtin_amdgcn_readfirstlane(term.y);
+        const int lx = ((pos >> 5) & 255) - j.w, ly = ((pos >> 13) & 255) - j.w, lz = (pos >> 21) - j.w;
         const int cx = (gb[0] << 1) | (pos & 1), cy = (gb[1] << 1) | ((pos >> 1) & 1), cz = (gb[2] << 1) | ((pos >> 2) & 1);
-        const int id[4] = {it.center + cx * it.span + lx, it.center + cy * it.span + ly, it.center + cz * it.span + lz,
-                           it.center + (cz + 2) * it.span + lz};
+        const int id[4] = {center + cx * span + lx, center + cy * span + ly, center + cz * span + lz,
+                           center + (cz + 2) * span + lz};
 #pragma unroll
         for (int q = 0; q < (PAIR ? 4 : 3); q++) {
             if (q == 2 && PAIR && !(pos & 8)) continue;
@@ -795,7 +824,7 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
     auto mfma = [](double x, double y, double c) { return __builtin_amdgcn_mfma_f64_4x4x4f64(x, y, c, 0, 0, 0); };
     auto uniform = [&](int i) {
         const Item4 v = sm.wl[i];
-        return Item4{__builtin_amdgcn_readfirstlane(v.center), __builtin_amdgcn_readfirstlane(v.span),
+        return Item4{__builtin_amdgcn_readfirstlane(v.e), __builtin_amdgcn_readfirstlane(v.slot),
                      __builtin_amdgcn_readfirstlane(v.pos)};
     };
 
@@ -805,17 +834,18 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
     unsigned long long napps = 0, napps1 = 0;
     while (pi < pi_end) {
         wave_order();
-        const int n = screen_items<PAIR, S::CAP>(a, ad, j, tn, tb, pi, pi_end, e0, e_last > 0 ? u_last : -1, e_last,
+        const int n = screen_items<PAIR, S::CAP, S::AHEAD>(a, ad, j, tn, pi, pi_end, e0, e_last > 0 ? u_last : -1, e_last,
                                                      sm.wl, lane, napps, napps1);
         wave_order();
         if (n == 0) continue;
         Item4 it = uniform(0);
-        load_f(it.pos);
-        fetch(it);
+        load_f(it);
+        fetch(it, tb[it.e]);
         stage(it.pos);
         for (int i = 0; i < n; i++) {
             const bool more = i + 1 < n;
             const Item4 nx = uniform(more ? i + 1 : i);
+            const int2 nt = tb[nx.e];
             const bool newgroup = more && ((nx.pos ^ it.pos) & ~24) != 0;
             const bool t0 = !PAIR || (it.pos & 8), t1 = PAIR && (it.pos & 16);
             wave_order();
@@ -847,7 +877,7 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
                     }
                     SCHED_STEP();
                 }
-                if (newgroup) load_f(nx.pos);
+                if (newgroup) load_f(nx);
             } else {
                 double ox[G][G];
                 operand(0, ox);
@@ -871,7 +901,7 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
                 }
                 operand(1, oy);
                 // the F rows of the next group load during the other passes
-                if (newgroup) load_f(nx.pos);
+                if (newgroup) load_f(nx);
                 wave_order();
                 SCHED_STEP();
                 double d[CT][G], bn[G];
@@ -904,7 +934,7 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
                     }
             }
             SCHED_STEP();
-            if (more) fetch(nx);
+            if (more) fetch(nx, nt);
             wave_order();
             // z, once per passing component (item-uniform branches)
             auto z_pass = [&](auto both, auto &&c0, auto &&c1, int q0) {
@@ -2358,6 +2388,7 @@ static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n
     o.root_off = root_off;
     p->args.slot_off = o.slot_off;
     p->args.slot_norm = norms;
+    p->args.n_real = (int)n_real;
     if ((rc = dev_band_items(s, b, o, err))) return rc;
     return dev_pool_fill(s, N, filter, o.gen, lv_off, o.slots, (int)n_slot, err);
 }
