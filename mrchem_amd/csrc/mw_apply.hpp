@@ -157,6 +157,7 @@ struct SegRec {
 struct CountArgs {
     KArgs k{};
     int n_out = 0, n_app = 0, n_share = 1;
+    long long widest = 1;                  // positions of the widest band
     const unsigned char *dense = nullptr;  // per output node: computed by the root kernels
     // passing terms per (output component, band position) of every node,
     // node q's at 8 band_off[q] + gt nb + p; with bounds the smallest and

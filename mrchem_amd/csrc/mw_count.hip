@@ -161,23 +161,26 @@ __device__ __forceinline__ void wave_range(double &lo, double &hi) {
     }
 }
 
-// Counts of one output node: one wave per output component.  64 (position,
-// ft) pairs at a time are pre-screened against the depth's largest products
+// Counts of one output node: one wave per output component.  Up to 64
+// (position, ft) pairs at a time (step: a multiple of 8) are pre-screened against the depth's largest products
 // (rounding is monotone, so a pair whose largest bound does not pass holds no
-// passing term); the terms of each candidate are then counted by ballot.
+// passing term); the terms of each candidate are then counted by ballot, one
+// after the other: a microsecond of load latency each, which a launch of few
+// nodes shortens by sharing a node's steps among workgroups (grid y; with the
+// parts of k_cut 2.11 -> 1.96 ms for a Coulomb apply at k = 7).
 template <bool BOUNDS>
-__global__ __launch_bounds__(512) void k_count(CountArgs c) {
+__global__ __launch_bounds__(512) void k_count(CountArgs c, int step) {
     const KArgs &a = c.k;
     const NodeView v = node_view(a, blockIdx.x);
     const int gt = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long long base = 8 * a.band_off[v.q] + (long long)gt * v.nb;
     __shared__ unsigned long long part[8];
     unsigned long long total = 0;
-    for (int pi = 0; pi < 8 * v.nb; pi += 64) {
+    for (int pi = step * blockIdx.y; pi < 8 * v.nb; pi += step * gridDim.y) {
         const int p = (pi + lane) >> 3, ft = lane & 7;
         bool cand = false;
         double fn = 0.0;
-        if (p < v.nb) {
+        if (lane < step && p < v.nb) {
             const int s = v.band[p];
             if (s >= 0) {
                 fn = a.slot_norm[(long long)s * 8 + ft];
@@ -200,7 +203,7 @@ __global__ __launch_bounds__(512) void k_count(CountArgs c) {
                 mhi = fmax(mhi, hi);
             }
         }
-        if (lane < 8 && (pi >> 3) + lane < v.nb) {
+        if (lane < step >> 3 && (pi >> 3) + lane < v.nb) {
             const long long e = base + (pi >> 3) + lane;
             c.cnt[e] = my;
             if (BOUNDS) {
@@ -231,7 +234,9 @@ __global__ __launch_bounds__(512) void k_count(CountArgs c) {
 // through a hundred of them alone was the end of every level's launch.  (The
 // low-precision classes sum a segment in 32 bits and keep their segments.)
 // Lane i keeps the i-th segment found; every 64 and at the end the wave takes
-// places for them with one atomic and writes them side by side.
+// places for them with one atomic and writes them side by side.  Grid y: parts
+// of a node's positions, each cut by itself (never for the low-precision
+// classes' segments).
 constexpr int kSegTarget = 256;      // passing terms of a segment
 constexpr int kSegFloor = 32;        // the least in a small launch
 constexpr int kSegWanted = 2048;     // segments a small launch is cut into
@@ -256,7 +261,9 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
     const int *c0 = c.cnt + 8 * a.band_off[v.q] + (long long)gt * v.nb, *c1 = c0 + 4LL * v.nb;
     const double *l0 = BOUNDS ? c.bmin + 8 * a.band_off[v.q] + (long long)gt * v.nb : nullptr;
     const double *h0 = BOUNDS ? c.bmax + 8 * a.band_off[v.q] + (long long)gt * v.nb : nullptr;
-    int u0 = 0, acc = 0, n = 0;
+    const int part0 = (int)((long long)v.nb * blockIdx.y / gridDim.y);
+    const int part1 = (int)((long long)v.nb * (blockIdx.y + 1) / gridDim.y);
+    int u0 = (8 * part0) << 12, acc = 0, n = 0;
     double lo = HUGE_VAL, hi = 0.0;
     int my_p0 = 0, my_p1 = 0, my_acc = 0;  // the segment this lane keeps
     double my_lo = 0.0, my_hi = 0.0;
@@ -289,9 +296,9 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
         lo = HUGE_VAL;
         hi = 0.0;
     };
-    for (int pb = 0; pb < v.nb; pb += 64) {
+    for (int pb = part0; pb < part1; pb += 64) {
         const int pl = pb + lane;
-        const int mine = pl < v.nb ? c0[pl] + (PAIR ? c1[pl] : 0) : 0;
+        const int mine = pl < part1 ? c0[pl] + (PAIR ? c1[pl] : 0) : 0;
         unsigned long long m = __ballot(mine > 0);
         while (m) {
             const int k = __builtin_ctzll(m), p = pb + k;
@@ -347,7 +354,7 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
             }
         }
     }
-    close((8 * v.nb) << 12);
+    close((8 * part1) << 12);
     if (n > 0) flush();
 }
 
@@ -407,22 +414,30 @@ int dev_term_tables(hipStream_t s, const KArgs &k, int nn, const TermLevel *leve
 
 int dev_count_terms(hipStream_t s, const CountArgs &c, bool bounds, std::string &err) {
     if (c.n_out == 0) return 0;
+    // a node's steps shared among as many workgroups as keep a launch below
+    // 2048 of them, shorter steps where that leaves less than 1024
+    const long long pairs = 8 * c.widest;
+    const int step = c.n_out * ((pairs + 63) / 64) < 1024 ? 16 : 64;
+    const int y = (int)std::max<long long>(1, std::min<long long>((pairs + step - 1) / step, 2048 / c.n_out));
     if (bounds)
-        hipLaunchKernelGGL((k_count<true>), dim3(c.n_out), dim3(512), 0, s, c);
+        hipLaunchKernelGGL((k_count<true>), dim3(c.n_out, y), dim3(512), 0, s, c, step);
     else
-        hipLaunchKernelGGL((k_count<false>), dim3(c.n_out), dim3(512), 0, s, c);
+        hipLaunchKernelGGL((k_count<false>), dim3(c.n_out, y), dim3(512), 0, s, c, step);
     HIP_TRY(hipGetLastError());
     return 0;
 }
 
 int dev_cut_segments(hipStream_t s, const CountArgs &c, bool bounds, std::string &err) {
     if (c.n_out == 0) return 0;
+    // three positions a part at the least, and no more parts than fill the
+    // chip: each ends a segment
+    const int y = (int)std::max<long long>(1, std::min<long long>(c.widest / 3, 1024 / c.n_out));
     if (bounds) {
         hipLaunchKernelGGL((k_cut<true, true>), dim3(c.n_out), dim3(256), 0, s, c);
         HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL((k_cut<false, true>), dim3(c.n_out), dim3(512), 0, s, c);
+        hipLaunchKernelGGL((k_cut<false, true>), dim3(c.n_out, y), dim3(512), 0, s, c);
     } else {
-        hipLaunchKernelGGL((k_cut<true, false>), dim3(c.n_out), dim3(256), 0, s, c);
+        hipLaunchKernelGGL((k_cut<true, false>), dim3(c.n_out, y), dim3(256), 0, s, c);
     }
     HIP_TRY(hipGetLastError());
     return 0;

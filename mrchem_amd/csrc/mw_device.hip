@@ -1667,9 +1667,12 @@ __global__ void k_split_rows(const double *src, long long nblocks, int rows, _Fl
     }
 }
 
-__global__ void k_zero_f64(double *p, long long n) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0;
+// A step's counters and output blocks (n4 groups of four values; a block holds
+// 8 N^3).
+__global__ __launch_bounds__(256) void k_zero_step(unsigned long long *counters, double4 *p, long long n4) {
+    if (blockIdx.x == 0 && threadIdx.x < 8) counters[threadIdx.x] = 0;
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i < n4) p[i] = double4{0.0, 0.0, 0.0, 0.0};
 }
 
 // FP64 -> FP32 copy (input pool and operator tables of the FP32 launches)
@@ -2677,6 +2680,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     ca.n_out = (int)n_out;
     ca.n_app = (int)parts.size();
     ca.n_share = (int)parts.size();
+    ca.widest = std::max(widest, 1LL);
     ca.dense = dev + f_dense;
     ca.totals = p->result + 8;
     ca.n_seg = ca.totals + 2 * parts.size();
@@ -3110,12 +3114,10 @@ static int launch_h(const DevicePlan *p, const int *list, const unsigned long lo
 // are recorded).
 static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool timed, std::string &err) {
     DeviceCtx *c = p->ctx;
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c->stream, p->args.counters, 8);
-    HIP_TRY(hipGetLastError());
     {
         const long long nz = (long long)p->n_out * 8 * p->kp1 * p->kp1 * p->kp1;
-        const int bs = 256;
-        hipLaunchKernelGGL(k_zero_f64, dim3((unsigned)((nz + bs - 1) / bs)), dim3(bs), 0, c->stream, p->args.out_ns, nz);
+        hipLaunchKernelGGL(k_zero_step, dim3((unsigned)((nz / 4 + 255) / 256)), dim3(256), 0, c->stream,
+                           p->args.counters, reinterpret_cast<double4 *>(p->args.out_ns), nz / 4);
         HIP_TRY(hipGetLastError());
     }
     int rc = 0;
