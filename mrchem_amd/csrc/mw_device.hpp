@@ -233,7 +233,11 @@ struct AddSrc {
     int dep, pad_;
     unsigned long long path;
 };
-constexpr int kAddMaxLevels = 21;  // levels a 64-bit path holds
+// (a 64-bit path holds 21 levels, one more than the deepest tree has)
+// An output node: depth and translation.
+struct NodeAt {
+    int d, l[3];
+};
 struct DevAddSession;
 // One input's blocks: n doubles at p, in host or device memory.
 struct BlockSource {
@@ -241,14 +245,16 @@ struct BlockSource {
     size_t n;
     bool on_device;
 };
-// Uploads the host inputs; base receives where each input's blocks are on the
-// device (a device input is read in place).
+// Uploads the host inputs (a device input is read in place) and the structure
+// of the input trees.
 int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &inputs,
-                  const std::vector<double> &coefs, DevAddSession **out, std::vector<const double *> &base,
+                  const std::vector<const Tree *> &trees, const std::vector<double> &coefs, DevAddSession **out,
                   std::string &err);
-// src: n_nodes x n_inputs entries (node-major); out_blocks: n_nodes x
-// 8(k+1)^3, on the host, or on the device with out_on_device.
-int dev_add_nodes(DevAddSession *m, const std::vector<AddSrc> &src, double *out_blocks, std::string &err,
+// The sum at every node of nodes, each input's source found on the device.
+// out_blocks: nodes.size() x 8(k+1)^3, on the host, or on the device with
+// out_on_device (then launches only: nodes must live until the stream has run
+// them).
+int dev_add_nodes(DevAddSession *m, const std::vector<NodeAt> &nodes, double *out_blocks, std::string &err,
                   bool out_on_device = false);
 void dev_add_end(DevAddSession *m);
 

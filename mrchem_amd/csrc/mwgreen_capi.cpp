@@ -1126,34 +1126,6 @@ bool mul_source(const Tree &f, const NodeKey &k, long long &off, int &dep, unsig
     return false;
 }
 
-// Source node of input f (its blocks at base on the device) for the sum at
-// output node k: f's deepest node on the path, the levels below it and the
-// child index of each level.  An input without any node on the path (an empty
-// tree) gets p = null.  False when the node lies more than
-// kAddMaxLevels levels below f's finest node on the path.
-bool add_source(const Tree &f, const NodeKey &k, const double *base, AddSrc &sr) {
-    sr.p = nullptr;
-    sr.dep = 0;
-    sr.pad_ = 0;
-    sr.path = 0;
-    for (int d = k.depth; d >= 0; d--) {
-        long long l[3];
-        for (int q = 0; q < 3; q++) l[q] = k.l[q] >> (k.depth - d);
-        const int idx = f.find(d, l);
-        if (idx < 0) continue;
-        sr.dep = k.depth - d;
-        if (sr.dep > kAddMaxLevels) return false;
-        for (int lv = 1; lv <= sr.dep; lv++) {
-            unsigned long long t = 0;
-            for (int q = 0; q < 3; q++) t |= (unsigned long long)((k.l[q] >> (k.depth - d - lv)) & 1) << q;
-            sr.path |= t << (3 * (lv - 1));
-        }
-        sr.p = base + (long long)idx * f.mra->block();
-        return true;
-    }
-    return true;
-}
-
 // Nodes of f in order of depth, each after its parent.
 std::vector<int> by_depth(const Tree &f) {
     std::vector<int> order(f.size());
@@ -1300,7 +1272,6 @@ int add_trees(mwg_context ctx, double prec, Tree &T, const std::vector<mwg_tree>
     const bool on_device = dres != nullptr;
     TempBlocks tb{ctx->dev, {}};
     std::vector<BlockSource> pool;
-    std::vector<const double *> base;
     size_t total = 0;
     for (size_t i = 0; i < ins.size(); i++) {
         bool on_dev = false;
@@ -1328,24 +1299,25 @@ int add_trees(mwg_context ctx, double prec, Tree &T, const std::vector<mwg_tree>
     }
     std::string err;
     DevAddSession *m = nullptr;
-    dev_check(dev_add_begin(ctx->dev, mra, pool, coefs, &m, base, err), err);
+    std::vector<const Tree *> trees;
+    for (mwg_tree f : ins) trees.push_back(&f->tree);
+    dev_check(dev_add_begin(ctx->dev, mra, pool, trees, coefs, &m, err), err);
     std::unique_ptr<DevAddSession, void (*)(DevAddSession *)> session(m, dev_add_end);
     DeviceLevels lv{ctx->dev, blk, mra.kp1(), {}, {}, {}, {}};
-    const size_t n_in = ins.size();
     for (int iter = 0;; iter++) {
-        std::vector<AddSrc> src(work.size() * n_in);
-        for (size_t w = 0; w < work.size(); w++)
-            for (size_t i = 0; i < n_in; i++)
-                if (!add_source(ins[i]->tree, T.keys[work[w]], base[i], src[w * n_in + i]))
-                    return fail(MWG_ERR_ARG, "output node more than " + std::to_string(kAddMaxLevels) +
-                                                 " levels below an input's finest node");
+        std::vector<NodeAt> nodes;
+        nodes.reserve(work.size());
+        for (int w : work) {
+            const NodeKey &k = T.keys[w];
+            nodes.push_back(NodeAt{k.depth, {(int)k.l[0], (int)k.l[1], (int)k.l[2]}});
+        }
         if (on_device) {
             double *buf = lv.add_level(work);
-            dev_check(dev_add_nodes(m, src, buf, err, true), err);
+            dev_check(dev_add_nodes(m, nodes, buf, err, true), err);
             lv.level_norms(T.size());
         } else {
             std::vector<double> blocks(work.size() * (size_t)blk);
-            dev_check(dev_add_nodes(m, src, blocks.data(), err), err);
+            dev_check(dev_add_nodes(m, nodes, blocks.data(), err), err);
             ctx->d2h_bytes += (long long)(sizeof(double) * blocks.size());
 #pragma omp parallel for num_threads(team_size()) schedule(static)
             for (long long w = 0; w < (long long)work.size(); w++)
