@@ -112,6 +112,11 @@ int dev_build_operators(DeviceCtx *c, const MRA &mra, const std::vector<OpBuildJ
 // Copy the device table of a device-built operator (f.device_blocks values).
 int dev_download_operator_blocks(DeviceCtx *c, const void *key, double *out, long long n, std::string &err);
 
+// An output node of a product or sum: depth and translation.
+struct NodeAt {
+    int d, l[3];
+};
+
 // Node-wise products for the multiplication (mw_multiply.hip).  For one
 // output node: each input's source node (its deepest node on the path, block
 // offset in the input's coefficient pool), the levels from it down to the
@@ -131,14 +136,20 @@ struct DevMulSession;
 // a_on_device / b_on_device: that pool is device memory, used in place (or,
 // with noalloc, copied into the scratch array); otherwise it is host memory
 // and uploaded.
-int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a, const double *pool_b, size_t n_b,
-                  DevMulSession **out, std::string &err, bool noalloc = false, bool a_on_device = false,
-                  bool b_on_device = false);
-// out_blocks: nodes.size() x 8(k+1)^3, on the host, or on the device with
-// out_on_device (then launches only: nodes must live until the stream has run
-// them, as for dev_add_nodes).
+int dev_mul_begin(DeviceCtx *c, const MRA &mra, const Tree &a, const double *pool_a, size_t n_a, const Tree &b,
+                  const double *pool_b, size_t n_b, DevMulSession **out, std::string &err, bool noalloc = false,
+                  bool a_on_device = false, bool b_on_device = false);
+// The product at every node of nodes, the inputs' sources found on the device
+// (every node at most 10 levels below them: a 32-bit path; neither input
+// empty).  out_blocks: nodes.size() x 8(k+1)^3, on the host, or on the device
+// with out_on_device (then launches only: nodes must live until the stream has
+// run them, as for dev_add_nodes).
+int dev_mul_at(DevMulSession *m, const std::vector<NodeAt> &nodes, double coef, double *out_blocks, std::string &err,
+               bool out_on_device = false);
+// The same of an allocation-free session, from the host's descriptors into host
+// memory.
 int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double coef, double *out_blocks,
-                  std::string &err, bool out_on_device = false);
+                  std::string &err);
 void dev_mul_end(DevMulSession *m);
 
 // A device copy of n doubles (freed with dev_free).
@@ -234,10 +245,6 @@ struct AddSrc {
     unsigned long long path;
 };
 // (a 64-bit path holds 21 levels, one more than the deepest tree has)
-// An output node: depth and translation.
-struct NodeAt {
-    int d, l[3];
-};
 struct DevAddSession;
 // One input's blocks: n doubles at p, in host or device memory.
 struct BlockSource {

@@ -1317,6 +1317,99 @@ int dev_noalloc_init(DeviceCtx *c, std::string &err) {
     return 0;
 }
 
+// An input of a product or sum: first child of every node (-1: none; the roots
+// are the first nodes, box x fastest; size 0: an empty tree) and its blocks.
+struct AddTree {
+    const int *child0;
+    const double *base;
+    int size, pad_;
+};
+struct AddGeo {
+    int corner[3], boxes[3];
+};
+
+__device__ __forceinline__ int child_of(const NodeAt &k, int b) {
+    return ((k.l[0] >> b) & 1) | ((k.l[1] >> b) & 1) << 1 | ((k.l[2] >> b) & 1) << 2;
+}
+
+// The walk from the root box down to the input's deepest node on the path of k,
+// dep levels above it: a chain of at most 20 dependent loads.
+__device__ __forceinline__ int deepest_node(const AddGeo &geo, const AddTree &t, const NodeAt &k, int &dep) {
+    int node = (((k.l[2] >> k.d) - geo.corner[2]) * geo.boxes[1] + (k.l[1] >> k.d) - geo.corner[1]) * geo.boxes[0] +
+               (k.l[0] >> k.d) - geo.corner[0];
+    for (dep = k.d; dep > 0; dep--) {
+        const int c0 = t.child0[node];
+        if (c0 < 0) break;
+        node = c0 + child_of(k, dep - 1);
+    }
+    return node;
+}
+
+// The sources of n (node, input) pairs of a sum, a thread each.  Hash look-ups
+// from the finest level up on the host took 1.47 of 2.2 ms at 3448 nodes and 8
+// inputs.
+__global__ __launch_bounds__(256) void k_add_sources(AddGeo geo, const AddTree *trees, int n_in, const NodeAt *nodes,
+                                                     long long n, int blk, AddSrc *src) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const AddTree t = trees[i % n_in];
+    const NodeAt k = nodes[i / n_in];
+    AddSrc s{nullptr, 0, 0, 0};
+    if (t.size > 0) {
+        s.p = t.base + (long long)deepest_node(geo, t, k, s.dep) * blk;
+        for (int lv = 1; lv <= s.dep; lv++) s.path |= (unsigned long long)child_of(k, s.dep - lv) << (3 * (lv - 1));
+    }
+    src[i] = s;
+}
+
+// The descriptors of the output nodes of a product, a thread each (100 of 500
+// us on the host at 990 nodes).  hfac: by depth.
+struct MulFactors {
+    double hfac[24];
+};
+__global__ __launch_bounds__(256) void k_mul_sources(AddGeo geo, const AddTree *trees, const NodeAt *nodes, int n,
+                                                     int blk, MulFactors f, MulNode *out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const NodeAt k = nodes[i];
+    MulNode m{};
+    m.src_a = (long long)deepest_node(geo, trees[0], k, m.dep_a) * blk;
+    m.src_b = (long long)deepest_node(geo, trees[1], k, m.dep_b) * blk;
+    for (int lv = 1; lv <= m.dep_a; lv++) m.path_a |= (unsigned)child_of(k, m.dep_a - lv) << (3 * (lv - 1));
+    for (int lv = 1; lv <= m.dep_b; lv++) m.path_b |= (unsigned)child_of(k, m.dep_b - lv) << (3 * (lv - 1));
+    m.hfac = f.hfac[k.d];
+    out[i] = m;
+}
+
+// The structure of the inputs on the device: the AddTree of each, then their
+// child0 arrays, uploaded from stage (which lives until the stream has run it).
+static int upload_trees(DeviceCtx *c, const std::vector<const Tree *> &trees, const std::vector<const double *> &base,
+                        std::vector<unsigned char, UninitAlloc<unsigned char>> &stage, unsigned char **dev,
+                        std::string &err) {
+    size_t bytes = sizeof(AddTree) * trees.size(), at = bytes;
+    for (const Tree *t : trees) bytes += sizeof(int) * (size_t)t->size();
+    if (int rc = dev_mem(c, bytes + 1, dev, err)) return rc;
+    stage.resize(bytes);
+    for (size_t i = 0; i < trees.size(); i++) {
+        const size_t b = sizeof(int) * (size_t)trees[i]->size();
+        const AddTree t{reinterpret_cast<const int *>(*dev + at), base[i], trees[i]->size(), 0};
+        std::memcpy(stage.data() + sizeof(AddTree) * i, &t, sizeof(t));
+        if (b) std::memcpy(stage.data() + at, trees[i]->child0.data(), b);
+        at += b;
+    }
+    HIP_TRY(hipMemcpyAsync(*dev, stage.data(), bytes, hipMemcpyHostToDevice, static_cast<hipStream_t>(dev_stream(c))));
+    return 0;
+}
+
+static AddGeo add_geo(const MRA &mra) {
+    AddGeo g;
+    for (int d = 0; d < 3; d++) {
+        g.corner[d] = (int)mra.corner[d];
+        g.boxes[d] = mra.boxes[d];
+    }
+    return g;
+}
+
 struct DevMulSession {
     DeviceCtx *ctx = nullptr;
     int n = 0;
@@ -1330,16 +1423,23 @@ struct DevMulSession {
     double *dout = nullptr;
     // the pools are the caller's device blocks (not freed here)
     bool borrowed_a = false, borrowed_b = false;
+    // the inputs' structure (not of an allocation-free session)
+    AddGeo geo{};
+    MulFactors hfac{};
+    unsigned char *trees = nullptr;
+    std::vector<unsigned char, UninitAlloc<unsigned char>> stage;
     ~DevMulSession() {
         if (noalloc) return;
+        dev_mem_put(ctx, trees);
         for (double *p : {F, wsc, ws}) dev_mem_put(ctx, p);
         if (!borrowed_a) dev_mem_put(ctx, pool_a);
         if (!borrowed_b) dev_mem_put(ctx, pool_b);
     }
 };
 
-int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a, const double *pool_b, size_t n_b,
-                  DevMulSession **out, std::string &err, bool noalloc, bool a_on_device, bool b_on_device) {
+int dev_mul_begin(DeviceCtx *c, const MRA &mra, const Tree &a, const double *pool_a, size_t n_a, const Tree &b,
+                  const double *pool_b, size_t n_b, DevMulSession **out, std::string &err, bool noalloc,
+                  bool a_on_device, bool b_on_device) {
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
     if (mra.basis.type != BASIS_INTERPOLATING) {
@@ -1433,6 +1533,9 @@ int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a
     if (!rc) rc = up(mra.basis.F.data(), mra.basis.F.size(), &m->F);
     if (!rc) rc = up(wsc.data(), wsc.size(), &m->wsc);
     if (!rc && n > 12) rc = dev_mem(c, (size_t)kMulBlocks * 24 * n3, &m->ws, err);
+    m->geo = add_geo(mra);
+    for (int d = 0; d < 24; d++) m->hfac.hfac[d] = std::pow(mra.box_size(d + 1), -1.5);
+    if (!rc) rc = upload_trees(c, {&a, &b}, {m->pool_a, m->pool_b}, m->stage, &m->trees, err);
     if (rc) {
         (void)hipStreamSynchronize(s);
         delete m;
@@ -1443,35 +1546,52 @@ int dev_mul_begin(DeviceCtx *c, const MRA &mra, const double *pool_a, size_t n_a
 }
 
 int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double coef, double *out_blocks,
-                  std::string &err, bool out_on_device) {
+                  std::string &err) {
     if (nodes.empty()) return 0;
     HIP_TRY(hipSetDevice(dev_device(m->ctx)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(m->ctx));
     const int n3 = m->n * m->n * m->n;
-    if (m->noalloc) {
-        // chunk by chunk through the scratch array; each output node is one
-        // workgroup's, so the blocks equal those of the allocating path
-        for (size_t c0 = 0; c0 < nodes.size(); c0 += m->chunk) {
-            const size_t cn = std::min(m->chunk, nodes.size() - c0);
-            HIP_TRY(hipMemcpyAsync(m->dn, nodes.data() + c0, sizeof(MulNode) * cn, hipMemcpyHostToDevice, s));
-            HIP_TRY(mul_nodes(s, m->n, (int)cn, m->dn, m->pool_a, m->pool_b, m->F, m->wsc, coef, m->ws,
-                              kNoAllocBlocks, m->dout));
-            HIP_TRY(hipMemcpyAsync(out_blocks + c0 * 8 * n3, m->dout, sizeof(double) * cn * 8 * n3,
-                                   out_on_device ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
-        }
-        return 0;
+    // chunk by chunk through the scratch array; each output node is one
+    // workgroup's, so the blocks equal those of the allocating path
+    for (size_t c0 = 0; c0 < nodes.size(); c0 += m->chunk) {
+        const size_t cn = std::min(m->chunk, nodes.size() - c0);
+        HIP_TRY(hipMemcpyAsync(m->dn, nodes.data() + c0, sizeof(MulNode) * cn, hipMemcpyHostToDevice, s));
+        HIP_TRY(mul_nodes(s, m->n, (int)cn, m->dn, m->pool_a, m->pool_b, m->F, m->wsc, coef, m->ws, kNoAllocBlocks,
+                          m->dout));
+        HIP_TRY(hipMemcpyAsync(out_blocks + c0 * 8 * n3, m->dout, sizeof(double) * cn * 8 * n3, hipMemcpyDeviceToHost,
+                               s));
+        HIP_TRY(hipStreamSynchronize(s));
     }
+    return 0;
+}
+
+int dev_mul_at(DevMulSession *m, const std::vector<NodeAt> &nodes, double coef, double *out_blocks, std::string &err,
+               bool out_on_device) {
+    if (nodes.empty()) return 0;
+    HIP_TRY(hipSetDevice(dev_device(m->ctx)));
+    hipStream_t s = static_cast<hipStream_t>(dev_stream(m->ctx));
+    const int n3 = m->n * m->n * m->n;
     MulNode *dn = nullptr;
+    NodeAt *da = nullptr;
     double *dout = out_on_device ? out_blocks : nullptr;
     if (int rc = dev_mem(m->ctx, nodes.size(), &dn, err)) return rc;
+    if (int rc = dev_mem(m->ctx, nodes.size(), &da, err)) {
+        dev_mem_put(m->ctx, dn);
+        return rc;
+    }
     if (!out_on_device) {
         if (int rc = dev_mem(m->ctx, nodes.size() * 8 * n3, &dout, err)) {
             dev_mem_put(m->ctx, dn);
+            dev_mem_put(m->ctx, da);
             return rc;
         }
     }
-    hipError_t e = hipMemcpyAsync(dn, nodes.data(), sizeof(MulNode) * nodes.size(), hipMemcpyHostToDevice, s);
+    hipError_t e = hipMemcpyAsync(da, nodes.data(), sizeof(NodeAt) * nodes.size(), hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_mul_sources, dim3((unsigned)((nodes.size() + 255) / 256)), dim3(256), 0, s, m->geo,
+                           reinterpret_cast<const AddTree *>(m->trees), da, (int)nodes.size(), 8 * n3, m->hfac, dn);
+        e = hipGetLastError();
+    }
     if (e == hipSuccess) {
         e = mul_nodes(s, m->n, (int)nodes.size(), dn, m->pool_a, m->pool_b, m->F, m->wsc, coef, m->ws,
                       kMulBlocks, dout);
@@ -1480,6 +1600,7 @@ int dev_mul_nodes(DevMulSession *m, const std::vector<MulNode> &nodes, double co
     if (e == hipSuccess && !out_on_device)
         crc = dev_copy_d2h(m->ctx, out_blocks, dout, sizeof(double) * nodes.size() * 8 * n3, err);
     dev_mem_put(m->ctx, dn);
+    dev_mem_put(m->ctx, da);
     if (!out_on_device) dev_mem_put(m->ctx, dout);
     if (crc) return crc;
     if (e != hipSuccess) {
@@ -1494,45 +1615,6 @@ void dev_mul_end(DevMulSession *m) {
     (void)hipSetDevice(dev_device(m->ctx));
     (void)hipStreamSynchronize(static_cast<hipStream_t>(dev_stream(m->ctx)));
     delete m;
-}
-
-// An input of a sum: first child of every node (-1: none; the roots are the
-// first nodes, box x fastest; size 0: an empty tree) and its blocks.
-struct AddTree {
-    const int *child0;
-    const double *base;
-    int size, pad_;
-};
-struct AddGeo {
-    int corner[3], boxes[3];
-};
-
-// The sources of n_nodes x n_in (node, input) pairs, a thread each: the walk
-// from the root box down to the deepest node on the path.  A chain of at most
-// 20 dependent loads; hash look-ups from the finest level up on the host took
-// 1.47 of 2.2 ms at 3448 nodes and 8 inputs.
-__global__ __launch_bounds__(256) void k_add_sources(AddGeo geo, const AddTree *trees, int n_in, const NodeAt *nodes,
-                                                     long long n, int blk, AddSrc *src) {
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const AddTree t = trees[i % n_in];
-    const NodeAt k = nodes[i / n_in];
-    AddSrc s{nullptr, 0, 0, 0};
-    if (t.size > 0) {
-        int node = (((k.l[2] >> k.d) - geo.corner[2]) * geo.boxes[1] + (k.l[1] >> k.d) - geo.corner[1]) * geo.boxes[0] +
-                   (k.l[0] >> k.d) - geo.corner[0];
-        auto child = [&](int b) { return ((k.l[0] >> b) & 1) | ((k.l[1] >> b) & 1) << 1 | ((k.l[2] >> b) & 1) << 2; };
-        s.dep = k.d;
-        while (s.dep > 0) {
-            const int c0 = t.child0[node];
-            if (c0 < 0) break;
-            s.dep--;
-            node = c0 + child(s.dep);
-        }
-        for (int lv = 1; lv <= s.dep; lv++) s.path |= (unsigned long long)child(s.dep - lv) << (3 * (lv - 1));
-        s.p = t.base + (long long)node * blk;
-    }
-    src[i] = s;
 }
 
 struct DevAddSession {
@@ -1590,29 +1672,8 @@ int dev_add_begin(DeviceCtx *c, const MRA &mra, const std::vector<BlockSource> &
     if (!rc) rc = up(coefs.data(), coefs.size(), &m->coefs);
     if (!rc) rc = up(mra.basis.F.data(), mra.basis.F.size(), &m->F);
     if (!rc && m->n > 12) rc = dev_mem(c, (size_t)kMulBlocks * 16 * n3, &m->ws, err);
-    size_t bytes = sizeof(AddTree) * trees.size();
-    for (const Tree *t : trees) bytes += sizeof(int) * (size_t)t->size();
-    if (!rc) rc = dev_mem(c, bytes + 1, &m->trees, err);
-    if (!rc) {
-        for (int d = 0; d < 3; d++) {
-            m->geo.corner[d] = (int)mra.corner[d];
-            m->geo.boxes[d] = mra.boxes[d];
-        }
-        m->stage.resize(bytes);
-        size_t at = sizeof(AddTree) * trees.size();
-        for (size_t i = 0; i < trees.size(); i++) {
-            const size_t b = sizeof(int) * (size_t)trees[i]->size();
-            const AddTree t{reinterpret_cast<const int *>(m->trees + at), base[i], trees[i]->size(), 0};
-            std::memcpy(m->stage.data() + sizeof(AddTree) * i, &t, sizeof(t));
-            if (b) std::memcpy(m->stage.data() + at, trees[i]->child0.data(), b);
-            at += b;
-        }
-        const hipError_t e = hipMemcpyAsync(m->trees, m->stage.data(), bytes, hipMemcpyHostToDevice, s);
-        if (e != hipSuccess) {
-            err = std::string("add trees: ") + hipGetErrorString(e);
-            rc = -2;
-        }
-    }
+    m->geo = add_geo(mra);
+    if (!rc) rc = upload_trees(c, trees, base, m->stage, &m->trees, err);
     if (rc) {
         (void)hipStreamSynchronize(s);
         delete m;

@@ -12,6 +12,7 @@
 #include <atomic>
 #include <cstdio>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <exception>
@@ -1453,28 +1454,43 @@ int multiply_trees(mwg_context ctx, double prec, mwg_tree out, double coef, mwg_
         const double *pa = input_blocks(ctx, a, tb, noalloc, a_dev);
         const double *pb = input_blocks(ctx, b, tb, noalloc, b_dev);
         DevMulSession *m = nullptr;
-        dev_check(dev_mul_begin(ctx->dev, mra, pa, tree_values(a), pb, tree_values(b), &m, err, noalloc, a_dev, b_dev),
+        dev_check(dev_mul_begin(ctx->dev, mra, a->tree, pa, tree_values(a), b->tree, pb, tree_values(b), &m, err,
+                                noalloc, a_dev, b_dev),
                   err);
         std::unique_ptr<DevMulSession, void (*)(DevMulSession *)> session(m, dev_mul_end);
         const int blk = mra.block(), n3 = mra.kp1_3();
         DeviceLevels lv{ctx->dev, blk, mra.kp1(), {}, {}, {}, {}};
+        // no output node down to this depth is out of an input's reach
+        int reach = INT_MAX;
+        for (const Tree *f : {&a->tree, &b->tree}) {
+            if (f->size() == 0) reach = -1;
+            for (int i = 0; i < f->size(); i++)
+                if (f->child0[i] < 0) reach = std::min(reach, f->keys[i].depth + 10);
+        }
         for (int iter = 0;; iter++) {
-            std::vector<MulNode> nodes(work.size());
-            for (size_t w = 0; w < work.size(); w++) {
-                const NodeKey &k = T.keys[work[w]];
-                MulNode &nd = nodes[w];
-                if (!mul_source(a->tree, k, nd.src_a, nd.dep_a, nd.path_a) ||
-                    !mul_source(b->tree, k, nd.src_b, nd.dep_b, nd.path_b))
-                    return fail(MWG_ERR_ARG, "output node more than 10 levels below an input's finest node");
-                nd.hfac = std::pow(mra.box_size(k.depth + 1), -1.5);
+            std::vector<NodeAt> at;
+            std::vector<MulNode> nodes;  // of an allocation-free session
+            for (int w : work) {
+                const NodeKey &k = T.keys[w];
+                if (noalloc || k.depth > reach) {
+                    MulNode nd;
+                    if (!mul_source(a->tree, k, nd.src_a, nd.dep_a, nd.path_a) ||
+                        !mul_source(b->tree, k, nd.src_b, nd.dep_b, nd.path_b))
+                        return fail(MWG_ERR_ARG, "output node more than 10 levels below an input's finest node");
+                    nd.hfac = std::pow(mra.box_size(k.depth + 1), -1.5);
+                    if (noalloc) nodes.push_back(nd);
+                }
+                at.push_back(NodeAt{k.depth, {(int)k.l[0], (int)k.l[1], (int)k.l[2]}});
             }
             if (on_device) {
                 double *buf = lv.add_level(work);
-                dev_check(dev_mul_nodes(m, nodes, coef, buf, err, true), err);
+                dev_check(dev_mul_at(m, at, coef, buf, err, true), err);
                 lv.level_norms(T.size());
             } else {
                 std::vector<double> blocks(work.size() * (size_t)blk);
-                dev_check(dev_mul_nodes(m, nodes, coef, blocks.data(), err), err);
+                dev_check(noalloc ? dev_mul_nodes(m, nodes, coef, blocks.data(), err)
+                                  : dev_mul_at(m, at, coef, blocks.data(), err),
+                          err);
                 ctx->d2h_bytes += (long long)(sizeof(double) * blocks.size());
 #pragma omp parallel for num_threads(team_size()) schedule(static)
                 for (long long w = 0; w < (long long)work.size(); w++)
