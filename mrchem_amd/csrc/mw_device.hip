@@ -1747,6 +1747,8 @@ struct DeviceCtx {
     // on first use) and the events of their DMAs
     void *stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    // pinned: the counts of a plan's slot search (kBandCounts)
+    unsigned *found = nullptr;
 };
 
 namespace {
@@ -1891,7 +1893,7 @@ struct DevicePlan {
     int *dev_list[2] = {nullptr, nullptr};
     std::vector<unsigned char, UninitAlloc<unsigned char>> stage;
     long long n_slot = 0, n_generated = 0;
-    unsigned found[kBandCounts];  // what the search for them counted
+    bool cleared = false;  // counters and output are cleared for the first step
     // the captured step (step_graph) and what it was captured for
     hipGraphExec_t graph = nullptr;
     int graph_mode = -1;
@@ -1934,6 +1936,8 @@ int dev_create(int device, DeviceCtx **out, std::string &err) {
     if (e == hipSuccess) e = hipEventCreate(&c->ev2s);
     if (e == hipSuccess) e = hipEventCreate(&c->ev2e);
     if (e == hipSuccess) e = hipEventCreate(&c->evp);
+    if (e == hipSuccess)
+        e = hipHostMalloc(reinterpret_cast<void **>(&c->found), sizeof(unsigned) * kBandCounts, hipHostMallocDefault);
     if (e != hipSuccess) {
         err = std::string("stream/event creation: ") + hipGetErrorString(e);
         delete c;
@@ -1971,6 +1975,7 @@ void dev_destroy(DeviceCtx *c) {
     if (c->ev2s) (void)hipEventDestroy(c->ev2s);
     if (c->ev2e) (void)hipEventDestroy(c->ev2e);
     if (c->evp) (void)hipEventDestroy(c->evp);
+    if (c->found) (void)hipHostFree(c->found);
     for (int b = 0; b < 2; b++) {
         if (c->stage[b]) (void)hipHostFree(c->stage[b]);
         if (c->stage_ev[b]) (void)hipEventDestroy(c->stage_ev[b]);
@@ -2300,6 +2305,15 @@ static void cut_done(DevicePlan *p) {
     p->stage = decltype(p->stage)();
 }
 
+// Clears a step's counters and output.
+static int clear_step(DevicePlan *p, std::string &err) {
+    const long long n4 = (long long)p->n_out * 2 * p->kp1 * p->kp1 * p->kp1;
+    hipLaunchKernelGGL(k_zero_step, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, p->ctx->stream,
+                       p->args.counters, reinterpret_cast<double4 *>(p->args.out_ns), n4);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
 // Bands, slots and pool of the plan: the search, then, its counts known, the
 // slot tables, the pool and the generated nodes.  beside: launches that need
 // none of it, which run while the host waits for the counts.
@@ -2341,7 +2355,7 @@ static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n
     int rc = get((size_t)std::max<long long>(n_band, 1), &b.cell);
     if (!rc) rc = get((size_t)kBandCounts, &b.cnt);
     if (rc) return rc;
-    unsigned *cnt = p->found;
+    const unsigned *cnt = c->found;
     for (bool first = true;; first = false) {
         if (cells > (1LL << 30)) {
             err = "batch too large for 32-bit node, segment or slot indices";
@@ -2352,7 +2366,8 @@ static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n
             (rc = get((size_t)cells, &b.gen)) || (rc = get((size_t)cells, &b.lv)) ||
             (rc = dev_band_find(s, b, widest, err)))
             return rc;
-        HIP_TRY(hipMemcpyAsync(cnt, b.cnt, sizeof(p->found), hipMemcpyDeviceToHost, s));
+        // (into pinned memory: the host goes on to launch what runs beside)
+        HIP_TRY(hipMemcpyAsync(c->found, b.cnt, sizeof(unsigned) * kBandCounts, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipEventRecord(c->evz, s));
         if (first && (rc = beside())) return rc;
         HIP_TRY(hipEventSynchronize(c->evz));
@@ -2691,6 +2706,10 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
                    reinterpret_cast<BandTree *>(dev + f_trees), reinterpret_cast<int *>(dev + f_band),
                    reinterpret_cast<double *>(dev + f_F), reinterpret_cast<int *>(dev + f_ro), (int)root_out.size(),
                    reinterpret_cast<long long *>(dev + f_rs), [&] {
+                       if (once && n_out > 0) {
+                           if (int r = clear_step(p.get(), err)) return r;
+                           p->cleared = true;
+                       }
                        return dev_term_tables(s, a, N * N, reinterpret_cast<const TermLevel *>(dev + f_lv),
                                               (int)levels.size(), reinterpret_cast<double *>(dev + f_tn),
                                               reinterpret_cast<int2 *>(dev + f_tb), err);
@@ -3114,13 +3133,9 @@ static int launch_h(const DevicePlan *p, const int *list, const unsigned long lo
 // are recorded).
 static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool timed, std::string &err) {
     DeviceCtx *c = p->ctx;
-    {
-        const long long nz = (long long)p->n_out * 8 * p->kp1 * p->kp1 * p->kp1;
-        hipLaunchKernelGGL(k_zero_step, dim3((unsigned)((nz / 4 + 255) / 256)), dim3(256), 0, c->stream,
-                           p->args.counters, reinterpret_cast<double4 *>(p->args.out_ns), nz / 4);
-        HIP_TRY(hipGetLastError());
-    }
-    int rc = 0;
+    int rc = p->cleared ? 0 : clear_step(p, err);
+    if (rc) return rc;
+    p->cleared = false;
     if (p->root.n_items > 0) {
         p->root.out_ns = p->args.out_ns;
         rc = dev_root_launch(c->stream, p->root, err);
@@ -3350,7 +3365,7 @@ int dev_plan_run(DevicePlan *p, int mode, double tau, double *kernel_ms, unsigne
             HIP_TRY(hipGraphLaunch(p->graph, c->stream));
         } else {
             HIP_TRY(hipEventRecord(c->ev0, c->stream));
-            int rc = enqueue_step(p, mode, tau, post, true, err);
+            int rc = enqueue_step(p, mode, tau, post, split_ms || post_ms, err);
             if (rc) return rc;
             p->ran_eager |= bit;
         }
