@@ -18,10 +18,12 @@
 // plane) (k_root_z).  The work is a few Gflop, so the 16 x 16 x 4 FP64 MFMA
 // with the dimensions padded to 16 is near enough to its bound; what the
 // launches wait for is Y (8 D^3 bytes a term, written once and read once,
-// from the memory-side cache).  Device time of the root level, per-component
-// items -> these kernels: one apply at k = 7 (171 terms) 1.64 -> 0.08 ms, ten
-// exchange densities 5.96 -> 0.55 ms, six orbitals at k = 11 (145 terms each)
-// 11.2 -> 1.7 ms; one frozen k = 9 plan of 656 nodes as a whole 7.5 -> 5.3 ms.
+// from the memory-side cache): a SIMD holds one or two waves, so both passes
+// have their next operands on the way while they work (matrices through LDS,
+// Y in registers).  Device time of the root level, per-component items ->
+// these kernels: one apply at k = 7 (171 terms) 1.64 -> 0.06 ms (0.08 with
+// operands loaded as they are needed), ten exchange densities 5.96 -> 0.38 ms
+// (0.54), six orbitals at k = 11 (145 terms each) 11.2 -> 0.95 ms (1.7).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -90,7 +92,7 @@ __device__ __forceinline__ RootPos root_pos(int n, int q) { return RootPos{q / (
 // the lanes in which the y pass reads it as its B operand (D row lane / 16 +
 // 4 r of register r = the operand's row of step r), so no value passes
 // through LDS.  The four waves of a workgroup take four planes with the same
-// items, whose matrices they share in L1.
+// items, whose matrices they share in LDS.
 constexpr int kRootItems = 4;
 
 template <int T, bool SAME>
@@ -101,14 +103,31 @@ __global__ __launch_bounds__(256) void k_root_xy(RootGeo geo, const RootApp *app
     const int N = geo.n, N3 = N * N * N;
     const int D[3] = {2 * N * geo.boxes[0], 2 * N * geo.boxes[1], 2 * N * geo.boxes[2]};
     const int lane = threadIdx.x & 63, lc = lane & 15, lq = lane >> 4;
-    const int p = 4 * blockIdx.y + (threadIdx.x >> 6);
-    if (p >= D[2]) return;
+    const int p = min(4 * blockIdx.y + (int)(threadIdx.x >> 6), D[2] - 1);  // the last: maybe twice, same values
     const RootPos pz = root_pos(N, p);
     double fa[T][K];
     int cur = -1;
     const int i0 = blockIdx.x * kRootItems, i1 = min(i0 + kRootItems, n_items);
+    // the items' matrices (x, then y) in LDS, the next item's on its way in
+    // registers meanwhile
+    constexpr int NM = SAME ? 1 : 2, PER = NM * SZ / 256;
+    __shared__ double As[2][NM * SZ];
+    double next[PER];
+    auto fetch = [&](int it) {
+        const double *a = A + (size_t)it * nd * SZ + threadIdx.x;
+#pragma unroll
+        for (int e = 0; e < PER; e++) next[e] = a[256 * e];
+    };
+    auto keep = [&](int buf) {
+#pragma unroll
+        for (int e = 0; e < PER; e++) As[buf][threadIdx.x + 256 * e] = next[e];
+    };
+    fetch(i0);
+    keep(0);
+    __syncthreads();
     for (int it = i0; it < i1; it++) {
-        const int app = items[it].app;
+        if (it + 1 < i1) fetch(it + 1);
+        const int app = items[it].app, buf = (it - i0) & 1;
         if (app != cur) {
             cur = app;
             const long long *so = slot_off + apps[app].root0;
@@ -128,7 +147,7 @@ __global__ __launch_bounds__(256) void k_root_xy(RootGeo geo, const RootApp *app
                 }
             }
         }
-        const double *Ax = A + (size_t)it * nd * SZ, *Ay = SAME ? Ax : Ax + SZ;
+        const double *Ax = As[buf], *Ay = SAME ? Ax : Ax + SZ;
         double *y = Y + ((size_t)it * D[2] + p) * DP * DP;
 #pragma unroll 1
         for (int h = 0; h < T; h++) {
@@ -153,6 +172,8 @@ __global__ __launch_bounds__(256) void k_root_xy(RootGeo geo, const RootApp *app
 #pragma unroll
                 for (int r = 0; r < 4; r++) y[(16 * b + 4 * r + lq) * DP + 16 * h + lc] = d[b][r];
         }
+        if (it + 1 < i1) keep(buf ^ 1);
+        __syncthreads();
     }
 }
 
@@ -163,7 +184,7 @@ __global__ __launch_bounds__(256) void k_root_xy(RootGeo geo, const RootApp *app
 // those of the roots; the latter are added to the plan's counter (n_totals 0:
 // not by this launch).
 template <int T, bool SAME>
-__global__ __launch_bounds__(256) void k_root_z(RootGeo geo, const RootApp *apps, const RootItem *items, int n_items,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_root_z(RootGeo geo, const RootApp *apps, const RootItem *items, int n_items,
                                                 int per, const int *root_out, const double *A, const double *Y,
                                                 double *out_ns, unsigned long long *counter,
                                                 const unsigned long long *totals, int n_totals) {
@@ -184,7 +205,9 @@ __global__ __launch_bounds__(256) void k_root_z(RootGeo geo, const RootApp *apps
         const int *ro = root_out + apps[app].root0;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            const int col = 64 * cg + 16 * c + lc, iy = col / DP, ix = col % DP;
+            int cv = 16 * c + lc;  // (not to be worked out ahead of the steps)
+            asm volatile("" : "+v"(cv));
+            const int col = 64 * cg + cv, iy = col / DP, ix = col % DP;
             const RootPos py = root_pos(N, iy), px = root_pos(N, ix);
 #pragma unroll
             for (int t = 0; t < T; t++)
@@ -202,32 +225,51 @@ __global__ __launch_bounds__(256) void k_root_z(RootGeo geo, const RootApp *apps
                 }
         }
     };
-    int cur = items[i0].app;
-    for (int it = i0; it < i1; it++) {
-        const int app = items[it].app;
-        if (app != cur) {
-            flush(cur);
-            cur = app;
-        }
-        const double *Az = A + ((size_t)it * nd + (SAME ? 0 : 2)) * SZ;
-        const double *y = Y + (size_t)it * D[2] * DP * DP + 64 * cg + lc;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            if (4 * k >= D[2]) break;
+    // Steps (item, k) in order, the operands of the next AHEAD steps on their
+    // way: a SIMD holds one of these waves, and a step's loads come from the
+    // memory-side cache.
+    constexpr int AHEAD = 4;
+    const int ks = (D[2] + 3) / 4;
+    double a[AHEAD][T], b[AHEAD][4];
+    for (int s0 = i0; s0 < i1;) {
+        const int app = items[s0].app;
+        int s1 = s0 + 1;
+        while (s1 < i1 && items[s1].app == app) s1++;
+        int nit = s0, nk = 0;  // the next step to load (past the end: the last again)
+        auto load = [&](double (&a)[T], double (&b)[4]) {
+            const double *Az = A + ((size_t)nit * nd + (SAME ? 0 : 2)) * SZ + nk * 64 + lane;
             // rows past the last plane meet zero columns of A: any finite row
-            const double *yr = y + (size_t)min(4 * k + lq, D[2] - 1) * DP * DP;
-            double a[T], b[4];
+            const double *y = Y + ((size_t)nit * D[2] + min(4 * nk + lq, D[2] - 1)) * DP * DP + 64 * cg + lc;
 #pragma unroll
-            for (int t = 0; t < T; t++) a[t] = Az[(t * K + k) * 64 + lane];
+            for (int t = 0; t < T; t++) a[t] = Az[t * K * 64];
 #pragma unroll
-            for (int c = 0; c < 4; c++) b[c] = yr[16 * c];
+            for (int c = 0; c < 4; c++) b[c] = y[16 * c];
+            const bool wrap = nk + 1 == ks, end = wrap && nit + 1 == s1;
+            nk = end ? nk : wrap ? 0 : nk + 1;
+            nit += wrap && !end ? 1 : 0;
+        };
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) load(a[u], b[u]);
+        auto step = [&](int u) {
 #pragma unroll
             for (int c = 0; c < 4; c++)
 #pragma unroll
-                for (int t = 0; t < T; t++) acc[c][t] = root_mfma(a[t], b[c], acc[c][t]);
+                for (int t = 0; t < T; t++) acc[c][t] = root_mfma(a[u][t], b[u][c], acc[c][t]);
+        };
+        int left = (s1 - s0) * ks;
+        for (; left >= AHEAD; left -= AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                step(u);
+                load(a[u], b[u]);
+            }
         }
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++)
+            if (u < left) step(u);
+        flush(app);
+        s0 = s1;
     }
-    flush(cur);
 }
 
 template <int T, bool SAME>
@@ -257,11 +299,12 @@ int root_tiles(int n, const int *boxes) {
 
 bool root_same(const int *boxes) { return boxes[0] == boxes[1] && boxes[1] == boxes[2]; }
 
-// Terms of one chunk: Y of a chunk stays within 64 MB, so that the z pass
-// finds it in the memory-side cache.
+// Terms of one chunk: Y of a chunk stays within 128 MB, so that the z pass
+// finds it in the memory-side cache (with 64 MB the k = 11 chunks hold 75 terms
+// and half fill the chip: 0.74 against 0.51 ms of z passes).
 long long root_chunk_items(int n, const int *boxes, long long n_items) {
     const long long dp = 16 * root_tiles(n, boxes), y = 8LL * 2 * n * boxes[2] * dp * dp;
-    return std::max(1LL, std::min(n_items, (64LL << 20) / y));
+    return std::max(1LL, std::min(n_items, (128LL << 20) / y));
 }
 
 }  // namespace
