@@ -15,6 +15,12 @@
 //  pass 2 (k_op_fill): the kept blocks and norms of l in [-L, L], written
 //    straight into the flat operator table of the device.
 //
+// A step's time is LDS reads and shuffles: NS(-l) is NS(l) transposed, the
+// filter's products hold 3 x 3 values a lane at N = 12, and the moments' sums
+// are halved among the lanes (six operators of 145 terms at k = 11: scan
+// 3.28 -> 1.15 ms, fill 0.92 -> 0.36 ms against a transform for each sign, a
+// value per lane and a whole-wave sum per moment).
+//
 // Sums run in a different order than on the host, so values agree to a few
 // ulps; the tables stay resident on the device (the host keeps L and the
 // norms, which the apply planning reads).
@@ -69,6 +75,34 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
+// Wave-wide sums of n values, out[i] the sum of v[i] (added in wave_sum's
+// order): at each exchange a lane keeps one half of its values, [base, end) of
+// the whole.
+template <int n, int o>
+__device__ __forceinline__ void wave_sums(const double (&v)[n], double *out, int lane, int base, int end) {
+    constexpr int h = (n + 1) / 2;
+    const bool up = lane & o;
+    double r[h];
+    if constexpr (n == 1) {
+        r[0] = v[0] + __shfl_xor(v[0], o);
+    } else {
+#pragma unroll
+        for (int i = 0; i < h; i++) {
+            const double hi = h + i < n ? v[h + i] : 0.0;
+            r[i] = (up ? hi : v[i]) + __shfl_xor(up ? v[i] : hi, o);
+        }
+        if (up) base += h;
+        else end = min(end, base + h);
+    }
+    if constexpr (o > 1) {
+        wave_sums<h, o / 2>(r, out, lane, base, end);
+    } else {
+#pragma unroll
+        for (int i = 0; i < h; i++)
+            if (base + i < end) out[base + i] = r[i];
+    }
+}
+
 // Moments int_0^1 P~_p(u) exp(-A (u - c)^2) du, p < N2, of the normalised
 // shifted Legendre polynomials: the piecewise Gauss-Legendre rule of
 // gauss_moments01 (mw_math.cpp), points spread over the wave.
@@ -118,11 +152,9 @@ __device__ void moments(double A, double c, const OpConst &k, double *out, int l
             }
         }
     }
-#pragma unroll
-    for (int p = 0; p < N2; p++) {
-        const double s = wave_sum(acc[p]);
-        if (lane == 0) out[p] = s;
-    }
+    // wave-wide sums: the values are halved among the lanes at each exchange
+    // (24 of them: 30 shuffles, where a wave_sum of each needs 144)
+    wave_sums<N2, 32>(acc, out, lane, 0, N2);
 }
 
 // Rolling state of the scan over translations l = 0, 1, ...: moments
@@ -132,7 +164,7 @@ struct OpState {
     static constexpr int N2 = 2 * N, NN = N * N, MM = N2 * N2;
     double *mom;  // [3][N2]
     double *T;    // [3][NN]: T(2l-1), T(2l), T(2l+1)
-    double *Mf, *tmp, *Rp, *Rm;  // [MM] each
+    double *Mf, *tmp, *R, *F;  // [MM] each
 };
 
 // T(delta)[i][j] = pref sum_p C[i][j][p] M1[p] + (-1)^p C[j][i][p] M2[p], with
@@ -151,35 +183,53 @@ __device__ void t_block(const OpConst &k, double pref, const double *M1, const d
     }
 }
 
-// R = F Mf F^T with Mf = [[A, B], [Cb, A]] built from three N x N blocks, each
-// possibly transposed.
+// Z = X Y or X Y^T (TB), N2 x N2 in LDS: lane (i, j) of 8 x 8 holds rows i + 8 a
+// and columns j + 8 b, so that a step reads 2 TT values for TT^2 multiply-adds.
+template <int N2, bool TB>
+__device__ __forceinline__ void square_product(const double *X, const double *Y, double *Z, int lane) {
+    constexpr int TT = (N2 + 7) / 8;
+    const int li = lane >> 3, lj = lane & 7;
+    double z[TT][TT];
+#pragma unroll
+    for (int a = 0; a < TT; a++)
+#pragma unroll
+        for (int b = 0; b < TT; b++) z[a][b] = 0.0;
+#pragma unroll 4
+    for (int q = 0; q < N2; q++) {
+        double x[TT], y[TT];
+#pragma unroll
+        for (int a = 0; a < TT; a++) x[a] = X[min(li + 8 * a, N2 - 1) * N2 + q];
+#pragma unroll
+        for (int b = 0; b < TT; b++) {
+            const int c = min(lj + 8 * b, N2 - 1);
+            y[b] = TB ? Y[c * N2 + q] : Y[q * N2 + c];
+        }
+#pragma unroll
+        for (int a = 0; a < TT; a++)
+#pragma unroll
+            for (int b = 0; b < TT; b++) z[a][b] += x[a] * y[b];
+    }
+#pragma unroll
+    for (int a = 0; a < TT; a++)
+#pragma unroll
+        for (int b = 0; b < TT; b++)
+            if (li + 8 * a < N2 && lj + 8 * b < N2) Z[(li + 8 * a) * N2 + lj + 8 * b] = z[a][b];
+}
+
+// R = F M F^T with M = [[A, B], [C, A]] of three N x N blocks.
 template <int N>
-__device__ void ns_transform(const OpConst &k, const double *A, bool tA, const double *B, bool tB, const double *Cb,
-                             bool tC, double *Mf, double *tmp, double *R, int lane) {
+__device__ void ns_transform(const double *F, const double *A, const double *B, const double *C, double *M, double *tmp,
+                             double *R, int lane) {
     constexpr int N2 = 2 * N, MM = N2 * N2;
     for (int e = lane; e < MM; e += 64) {
         const int r = e / N2, c = e % N2;
-        const int bi = r % N, bj = c % N;
-        const double *src = (r < N) ? (c < N ? A : B) : (c < N ? Cb : A);
-        const bool tr = (r < N) ? (c < N ? tA : tB) : (c < N ? tC : tA);
-        Mf[e] = tr ? src[bj * N + bi] : src[bi * N + bj];
+        const double *src = (r < N) ? (c < N ? A : B) : (c < N ? C : A);
+        M[e] = src[(r % N) * N + c % N];
     }
     __syncthreads();
-    for (int e = lane; e < MM; e += 64) {
-        const int i = e / N2, j = e % N2;
-        double s = 0.0;
-#pragma unroll 4
-        for (int q = 0; q < N2; q++) s += k.F[i * N2 + q] * Mf[q * N2 + j];
-        tmp[e] = s;
-    }
+    square_product<N2, false>(F, M, tmp, lane);
     __syncthreads();
-    for (int e = lane; e < MM; e += 64) {
-        const int i = e / N2, j = e % N2;
-        double s = 0.0;
-#pragma unroll 4
-        for (int q = 0; q < N2; q++) s += tmp[i * N2 + q] * k.F[j * N2 + q];
-        R[e] = s;
-    }
+    square_product<N2, true>(tmp, F, R, lane);
     __syncthreads();
 }
 
@@ -200,7 +250,9 @@ __device__ void comp_norms(const double *R, double *nr, int lane) {
     }
 }
 
-// Advance the rolling state to translation l and form R+ = NS(l), R- = NS(-l).
+// Advance the rolling state to translation l and form R = NS(l).  The blocks of
+// NS(-l) before the filter, [[T(-2l), T(-2l+1)], [T(-2l-1), T(-2l)]] with T(-d) =
+// T(d)^T, are those of NS(l) transposed, and so NS(-l) = NS(l)^T.
 template <int N>
 __device__ void ns_step(const OpConst &k, const OpItem &it, OpState<N> &st, long long l, int lane) {
     constexpr int N2 = 2 * N, NN = N * N;
@@ -225,21 +277,20 @@ __device__ void ns_step(const OpConst &k, const OpItem &it, OpState<N> &st, long
         for (int e = lane; e < NN; e += 64) Tm[e] = Tp[(e % N) * N + e / N];
         __syncthreads();
     }
-    // NS(l): [[T(2l), T(2l+1)], [T(2l-1), T(2l)]]
-    ns_transform<N>(k, T0, false, Tp, false, Tm, false, st.Mf, st.tmp, st.Rp, lane);
-    // NS(-l): [[T(-2l), T(-2l+1)], [T(-2l-1), T(-2l)]] = transposes of T(2l), T(2l-1), T(2l+1)
-    ns_transform<N>(k, T0, true, Tm, true, Tp, true, st.Mf, st.tmp, st.Rm, lane);
+    // [[T(2l), T(2l+1)], [T(2l-1), T(2l)]]
+    ns_transform<N>(st.F, T0, Tp, Tm, st.Mf, st.tmp, st.R, lane);
 }
 
 template <int N>
-__device__ void setup_state(OpState<N> &st, double *lds) {
+__device__ void setup_state(OpState<N> &st, double *lds, const double *F, int lane) {
     constexpr int N2 = 2 * N, NN = N * N, MM = N2 * N2;
     st.mom = lds;
     st.T = st.mom + 3 * N2;
     st.Mf = st.T + 3 * NN;
     st.tmp = st.Mf + MM;
-    st.Rp = st.tmp + MM;
-    st.Rm = st.Rp + MM;
+    st.R = st.tmp + MM;
+    st.F = st.R + MM;
+    for (int e = lane; e < MM; e += 64) st.F[e] = F[e];
 }
 template <int N>
 constexpr int op_lds_doubles() {
@@ -254,7 +305,7 @@ __global__ __launch_bounds__(64) void k_op_scan(const OpItem *items, OpConst k, 
     const int lane = threadIdx.x;
     const OpItem it = items[blockIdx.x];
     OpState<N> st;
-    setup_state<N>(st, lds);
+    setup_state<N>(st, lds, k.F, lane);
     double ref = 0.0, wmax = 0.0;
     int quiet = 0;
     long long l = 0, nscan = 0;
@@ -265,9 +316,9 @@ __global__ __launch_bounds__(64) void k_op_scan(const OpItem *items, OpConst k, 
             break;
         }
         ns_step<N>(k, it, st, l, lane);
-        double a[4], b[4];
-        comp_norms<N>(st.Rp, a, lane);
-        comp_norms<N>(st.Rm, b, lane);
+        double a[4];
+        comp_norms<N>(st.R, a, lane);
+        const double b[4] = {a[0], a[2], a[1], a[3]};  // of NS(-l)
         if (lane == 0) {
 #pragma unroll
             for (int c = 0; c < 4; c++) {
@@ -315,15 +366,14 @@ __global__ __launch_bounds__(64) void k_op_fill(const OpItem *items, OpConst k, 
     if (so.L < 0) return;
     const int L = so.L, nl = 2 * L + 1;
     OpState<N> st;
-    setup_state<N>(st, lds);
+    setup_state<N>(st, lds, k.F, lane);
     for (long long l = 0; l <= L; l++) {
         ns_step<N>(k, it, st, l, lane);
-        double a[4], b[4];
-        comp_norms<N>(st.Rp, a, lane);
-        comp_norms<N>(st.Rm, b, lane);
+        double a[4];
+        comp_norms<N>(st.R, a, lane);
+        const double b[4] = {a[0], a[2], a[1], a[3]};  // of NS(-l)
 #pragma unroll
         for (int side = 0; side < 2; side++) {
-            const double *R = side == 0 ? st.Rp : st.Rm;
             const long long ls = side == 0 ? l : -l;
 #pragma unroll
             for (int c = 0; c < 4; c++) {
@@ -333,7 +383,8 @@ __global__ __launch_bounds__(64) void k_op_fill(const OpItem *items, OpConst k, 
                 const long long idx = (long long)c * nl + (ls + L);
                 const int r0 = (c >> 1) * N, c0 = (c & 1) * N;
                 for (int e = lane; e < NN; e += 64)
-                    it.blocks[it.boff + idx * NN + e] = R[(r0 + e / N) * N2 + c0 + e % N];
+                    it.blocks[it.boff + idx * NN + e] =
+                        side == 0 ? st.R[(r0 + e / N) * N2 + c0 + e % N] : st.R[(c0 + e % N) * N2 + r0 + e / N];
                 if (lane == 0) it.norms[it.noff + idx] = nr;
             }
         }
