@@ -342,9 +342,21 @@ __global__ __launch_bounds__(64) void k_op_scan(const OpItem *items, OpConst k, 
     }
     const double floor_w = it.tau * ref;
     const double floor_s = (it.d == 0) ? it.tau * ref : it.tau * ref * ref / fmax(wmax, 1e-300);
+    // stored half-width: the largest scanned translation with a component
+    // above its floor (build_term_depth)
+    __syncthreads();
+    int L = -1;
+    for (int q = lane; q < (int)nscan; q += 64) {
+        const double *n = nrm + it.nrm_off + 8LL * q;
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (fmax(n[c], n[4 + c]) > (c == 0 ? floor_s : floor_w)) L = q;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) L = max(L, __shfl_xor(L, o));
     if (lane == 0) {
         OpScanOut r;
-        r.L = -1;  // set by the host from the norms
+        r.L = L;
         r.nscan = (int)nscan;
         r.overflow = overflow;
         r.pad_ = 0;
@@ -592,25 +604,11 @@ int dev_build_operators(DeviceCtx *c, const MRA &mra, const std::vector<OpBuildJ
     std::vector<OpScanOut> scan(items.size());
     HIP_TRY(hipMemcpyAsync(scan.data(), dscan, sizeof(OpScanOut) * scan.size(), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
-    std::vector<double> nrm_h((size_t)nrm_total);
-    HIP_TRY(hipMemcpy(nrm_h.data(), dnrm, sizeof(double) * nrm_h.size(), hipMemcpyDeviceToHost));
-    for (int i = 0; i < n_items; i++) {
-        OpScanOut &so = scan[i];
+    for (const OpScanOut &so : scan)
         if (so.overflow) {
             err = "operator translation scan exceeded " + std::to_string(kOpScanCap) + " translations";
             return -1;
         }
-        // stored half-width: the largest scanned translation with a component
-        // above its floor (build_term_depth)
-        const double *nr = nrm_h.data() + items[i].nrm_off;
-        so.L = -1;
-        for (int l = 0; l < so.nscan; l++)
-            for (int c = 0; c < 4; c++) {
-                const double fl = c == 0 ? so.floor_s : so.floor_w;
-                if (nr[l * 8 + c] > fl || nr[l * 8 + 4 + c] > fl) so.L = l;
-            }
-    }
-    HIP_TRY(hipMemcpyAsync(dscan, scan.data(), sizeof(OpScanOut) * scan.size(), hipMemcpyHostToDevice, s));
     // flat layout of each operator (the order of flatten_operator)
     std::vector<std::vector<int>> Lmd(jobs.size());
     for (size_t jb = 0; jb < jobs.size(); jb++) {
