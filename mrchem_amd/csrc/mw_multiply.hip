@@ -705,15 +705,20 @@ static hipError_t post_level(hipStream_t s, int n, bool down, const PostPair *pa
     }
 }
 
-// o[i] = sum over j of M[j][h N + i] v[j], j = 0 .. J - 1 in turn
+// o[i] = sum over j of F[j][h N + i] v[j], j = 0 .. J - 1 in turn.  h is the
+// same for the whole wave, so from global memory the filter's rows come as
+// scalar loads (sum of 8 inputs at 3448 nodes, N = 8: 255 -> 166 us against
+// broadcasts from LDS; products, which have the filter in LDS for their other
+// passes, read it there: 108 against 154 us).
 template <int N, int J>
-__device__ __forceinline__ void half_line(const double *v, const double *M, int h, double *o) {
+__device__ __forceinline__ void half_line(const double *v, const double *__restrict__ F, int h, double *o) {
+    const double *Fh = F + __builtin_amdgcn_readfirstlane(h) * N;
 #pragma unroll
     for (int i = 0; i < N; i++) o[i] = 0.0;
 #pragma unroll
     for (int j = 0; j < J; j++) {
 #pragma unroll
-        for (int i = 0; i < N; i++) o[i] = fma(M[j * 2 * N + h * N + i], v[j], o[i]);
+        for (int i = 0; i < N; i++) o[i] = fma(Fh[j * 2 * N + i], v[j], o[i]);
     }
 }
 
@@ -722,10 +727,11 @@ __device__ __forceinline__ void half_line(const double *v, const double *M, int 
 // branch of k_post_one without the addition.  Each pass keeps the half of its
 // outputs that leads to the child, one thread per line with the line in
 // registers.  src: global memory, or X itself; X holds 4 N^3 (FULL) or N^3
-// values, M the filter.  M and src must be in place before (a barrier);
-// ends with a barrier.  Threads: at least 4 N^2 (FULL) or N^2.
+// values, F is the filter.  src (and F in LDS) must be in place before (a
+// barrier); ends with a barrier.  Threads: at least 4 N^2 (FULL) or N^2.
 template <int N, bool FULL>
-__device__ __forceinline__ void child_step(const double *src, double *X, const double *M, int child, int tid) {
+__device__ __forceinline__ void child_step(const double *src, double *X, const double *__restrict__ F, int child,
+                                           int tid) {
     constexpr int N3 = N * N * N, NN = N * N, J = FULL ? 2 * N : N;
     const int q = tid / NN, ac = tid % NN, a = ac % N, c = ac / N;
     double v[J], o[N];
@@ -734,7 +740,7 @@ __device__ __forceinline__ void child_step(const double *src, double *X, const d
     if (lz) {
 #pragma unroll
         for (int j = 0; j < J; j++) v[j] = src[(j < N ? q : q | 4) * N3 + post_index<N, 2>(a, c, j < N ? j : j - N)];
-        half_line<N, J>(v, M, child >> 2, o);
+        half_line<N, J>(v, F, child >> 2, o);
     }
     __syncthreads();  // src (which may be X) read before X is written
     if (lz) {
@@ -747,7 +753,7 @@ __device__ __forceinline__ void child_step(const double *src, double *X, const d
     if (ly) {
 #pragma unroll
         for (int j = 0; j < J; j++) v[j] = X[(j < N ? q : q | 2) * N3 + post_index<N, 1>(a, c, j < N ? j : j - N)];
-        half_line<N, J>(v, M, (child >> 1) & 1, o);
+        half_line<N, J>(v, F, (child >> 1) & 1, o);
     }
     __syncthreads();
     if (ly) {
@@ -760,7 +766,7 @@ __device__ __forceinline__ void child_step(const double *src, double *X, const d
     if (lx) {
 #pragma unroll
         for (int j = 0; j < J; j++) v[j] = X[(j < N ? 0 : 1) * N3 + post_index<N, 0>(a, c, j < N ? j : j - N)];
-        half_line<N, J>(v, M, child & 1, o);
+        half_line<N, J>(v, F, child & 1, o);
     }
     __syncthreads();
     if (lx) {
@@ -778,15 +784,12 @@ __device__ __forceinline__ void child_step(const double *src, double *X, const d
 // k = 11).
 template <int N>
 __global__ __launch_bounds__(PostOneShape<N>::T) void k_gen_fill(const GenItem *items, const double *__restrict__ F) {
-    constexpr int N3 = N * N * N, N2 = 2 * N;
+    constexpr int N3 = N * N * N;
     __shared__ double X[4 * N3];
-    __shared__ double M[N2 * N2];
     const int tid = threadIdx.x;
     const GenItem it = items[blockIdx.x];
-    for (int e = tid; e < N2 * N2; e += PostOneShape<N>::T) M[e] = F[e];
-    __syncthreads();
-    if (it.full) child_step<N, true>(it.src, X, M, it.child, tid);
-    else child_step<N, false>(it.src, X, M, it.child, tid);
+    if (it.full) child_step<N, true>(it.src, X, F, it.child, tid);
+    else child_step<N, false>(it.src, X, F, it.child, tid);
     for (int e = tid; e < N3; e += PostOneShape<N>::T) it.dst[e] = X[e];
 }
 
@@ -809,9 +812,9 @@ static hipError_t gen_fill(hipStream_t s, int n, const GenItem *items, int cnt, 
 // X[0, N^3); ends with a barrier.
 template <int N>
 __device__ __forceinline__ void descend(const double *src, int dep, unsigned long long path, double *X,
-                                        const double *M, int tid) {
-    child_step<N, true>(src, X, M, (int)(path & 7), tid);
-    for (int lv = 1; lv < dep; lv++) child_step<N, false>(X, X, M, (int)((path >> (3 * lv)) & 7), tid);
+                                        const double *__restrict__ F, int tid) {
+    child_step<N, true>(src, X, F, (int)(path & 7), tid);
+    for (int lv = 1; lv < dep; lv++) child_step<N, false>(X, X, F, (int)((path >> (3 * lv)) & 7), tid);
 }
 
 // Products: the block of output node w from both inputs' values at its 8
@@ -888,16 +891,13 @@ __global__ __launch_bounds__(PostShape<N>::T) void k_mul_nodes(const MulNode *no
 // contributes nothing).  One workgroup per node; each thread sums its values
 // of the node in registers over the inputs and stores them once.  (Summed in
 // global memory with the passes in a global work area, N = 8, 3160 nodes of 8
-// inputs: 2.15 ms; here 0.26 ms.)
+// inputs: 2.15 ms; here 0.17 ms.)
 template <int N>
 __global__ __launch_bounds__(PostOneShape<N>::T) void k_add_nodes(const AddSrc *src, int n_in, const double *coefs,
                                                                const double *__restrict__ F, double *out) {
-    constexpr int N3 = N * N * N, N2 = 2 * N, T = PostOneShape<N>::T, E = 8 * N3, K = (E + T - 1) / T;
+    constexpr int N3 = N * N * N, T = PostOneShape<N>::T, E = 8 * N3, K = (E + T - 1) / T;
     __shared__ double X[4 * N3];
-    __shared__ double M[N2 * N2];
     const int tid = threadIdx.x;
-    for (int e = tid; e < N2 * N2; e += T) M[e] = F[e];
-    __syncthreads();
     double acc[K];
 #pragma unroll
     for (int k = 0; k < K; k++) acc[k] = 0.0;
@@ -912,7 +912,7 @@ __global__ __launch_bounds__(PostOneShape<N>::T) void k_add_nodes(const AddSrc *
                 if (e < E) acc[k] += c * sr.p[e];
             }
         } else {
-            descend<N>(sr.p, sr.dep, sr.path, X, M, tid);
+            descend<N>(sr.p, sr.dep, sr.path, X, F, tid);
 #pragma unroll
             for (int k = 0; k < K; k++) {
                 const int e = tid + k * T;
