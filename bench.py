@@ -331,7 +331,7 @@ def main():
                      "kernel": kname},
         "fp64_path": {"value": n_out / (ms64 * 1e-3), "ms_per_step": ms64, "kernel_ms": res["fp64"]["kernel_ms"],
                       "roofline": {"achieved": ach64, "peak": PEAK_TFLOPS["f64"], "unit": "TFLOP/s",
-                                   "frac": ach64 / PEAK_TFLOPS["f64"], "kernel": "k_apply<%d, double>" % (k + 1)}},
+                                   "frac": ach64 / PEAK_TFLOPS["f64"], "kernel": "k_apply64<%d>" % (k + 1)}},
         "adaptive_apply": {"value": n_out / t_adapt, "unit": "nodes/s", "wall_ms": 1e3 * t_adapt,
                            "note": "the adaptive drop-in call (mwg_apply_batch, FP64) that fixed the grid, second "
                                    "call of the process: host refinement loop, per-level plans and launches, post "
