@@ -130,6 +130,7 @@ __global__ __launch_bounds__(256) void k_band_find(BandArgs a) {
     const int q = blockIdx.x, side = 2 * a.band_w[q] + 1, nb = side * side * side;
     const BandTree &t = a.trees[a.out_app[q]];
     int *cells = a.cell + a.band_off[q];
+    __shared__ int taken[2][4], first[2];
     for (int p0 = 256 * blockIdx.y; p0 < nb; p0 += 256 * gridDim.y) {
         const int p = p0 + threadIdx.x;
         int c = -1;
@@ -163,19 +164,49 @@ __global__ __launch_bounds__(256) void k_band_find(BandArgs a) {
             }
             real = da == k.d;
         }
-        const int ir = take_ids(claim && real, &a.cnt[0]), ig = take_ids(claim && !real, &a.cnt[1]);
-        if (claim) a.slot[c] = real ? ir : -(ig + 3);
+        // slot ids, one addition a workgroup (to one address they take about
+        // 10 ns each from all over the chip: 34 -> 23 us a launch on the
+        // exchange applies of 4 orbitals against one a wave and node)
+        const unsigned long long mr = __ballot(claim && real), mg = __ballot(claim && !real);
+        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+        if (lane == 0) {
+            taken[0][wv] = (int)__popcll(mr);
+            taken[1][wv] = (int)__popcll(mg);
+        }
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            int sum = 0;
+            for (int w = 0; w < 4; w++) sum += taken[threadIdx.x][w];
+            first[threadIdx.x] = sum ? (int)atomicAdd(&a.cnt[threadIdx.x], (unsigned)sum) : 0;
+        }
+        __syncthreads();
+        if (claim) {
+            int id = first[real ? 0 : 1] + (int)__popcll((real ? mr : mg) & ((1ull << lane) - 1));
+            for (int w = 0; w < wv; w++) id += taken[real ? 0 : 1][w];
+            a.slot[c] = real ? id : -(id + 3);
+        }
+        __syncthreads();  // read before the next entries' are written
         if (fresh && real) {
             a.lv[c] = -1;
             a.gen[c] = make_int2(node, 0);
         }
+        // positions of the entries' own generated nodes, a level at a time
+        const int lv0 = fresh && !real ? k.d - da - 1 : -1;
+        int pos = 0;
+        unsigned long long todo = __ballot(lv0 >= 0);
+        while (todo) {
+            const int lv = __builtin_amdgcn_readlane(lv0, __ffsll(todo) - 1);
+            const int id = take_ids(lv0 == lv, &a.cnt[3 + lv]);
+            if (lv0 == lv) pos = id;
+            todo &= ~__ballot(lv0 == lv);
+        }
         if (fresh && !real) {
             // the generated nodes from the entry's up to the child of the
             // ancestor that is there; a known one has the rest of its own
-            int lv = k.d - da - 1, at = c;
+            int lv = lv0, at = c;
             for (int up = 1;; up++, lv--) {
                 a.lv[at] = (signed char)lv;
-                const int pos = (int)atomicAdd(&a.cnt[3 + lv], 1u);
+                if (up > 1) pos = (int)atomicAdd(&a.cnt[3 + lv], 1u);
                 if (lv == 0) {
                     a.gen[at] = make_int2(-(node + 1), pos);
                     break;

@@ -233,8 +233,10 @@ __global__ __launch_bounds__(512) void k_count(CountArgs c, int step) {
 // pair of a coarse node holds all the depth's terms, and one wave working
 // through a hundred of them alone was the end of every level's launch.  (The
 // low-precision classes sum a segment in 32 bits and keep their segments.)
-// Lane i keeps the i-th segment found; every 64 and at the end the wave takes
-// places for them with one atomic and writes them side by side.  Grid y: parts
+// Lane i keeps the i-th segment found; every 64 the wave, and at the end the
+// workgroup, takes places for them with one addition (to one address they take
+// about 10 ns each, the time of a launch of some thousand waves) and they are
+// written side by side.  Grid y: parts
 // of a node's positions, each cut by itself (never for the low-precision
 // classes' segments).
 constexpr int kSegTarget = 256;      // passing terms of a segment
@@ -267,10 +269,8 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
     double lo = HUGE_VAL, hi = 0.0;
     int my_p0 = 0, my_p1 = 0, my_acc = 0;  // the segment this lane keeps
     double my_lo = 0.0, my_hi = 0.0;
-    auto flush = [&]() {
-        int at = 0;
-        if (lane == 0) at = (int)atomicAdd(&c.n_seg[kind], (unsigned long long)n);
-        at = __shfl(at, 0) + lane;
+    auto write = [&](int at) {  // the wave's n segments to places at, at + 1, ...
+        at += lane;
         if (lane < n && at < c.cap[kind]) {
             const int e = (PAIR ? 0 : c.cap[0]) + at;
             c.seg_job[e] = v.q * 8 + gt;
@@ -279,6 +279,11 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
             if (BOUNDS) c.rec[e] = SegRec{v.q * 8 + gt, my_p0, my_acc, 0, my_lo, my_hi};
         }
         n = 0;
+    };
+    auto flush = [&]() {
+        int at = 0;
+        if (lane == 0) at = (int)atomicAdd(&c.n_seg[kind], (unsigned long long)n);
+        write(__shfl(at, 0));
     };
     auto close = [&](int u1) {  // u1 = end << 12 | term
         if (acc > 0) {
@@ -355,7 +360,20 @@ __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
         }
     }
     close((8 * part1) << 12);
-    if (n > 0) flush();
+    // what is left, with one addition for the workgroup
+    constexpr int WAVES = PAIR ? 4 : 8;
+    __shared__ int left[WAVES], base;
+    if (lane == 0) left[gt] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int sum = 0;
+        for (int w = 0; w < WAVES; w++) sum += left[w];
+        base = sum ? (int)atomicAdd(&c.n_seg[kind], (unsigned long long)sum) : 0;
+    }
+    __syncthreads();
+    int at = base;
+    for (int w = 0; w < gt; w++) at += left[w];
+    write(at);
 }
 
 // The class lists of the low-precision modes (pair segments with a term of the
@@ -415,10 +433,12 @@ int dev_term_tables(hipStream_t s, const KArgs &k, int nn, const TermLevel *leve
 int dev_count_terms(hipStream_t s, const CountArgs &c, bool bounds, std::string &err) {
     if (c.n_out == 0) return 0;
     // a node's steps shared among as many workgroups as keep a launch below
-    // 2048 of them, shorter steps where that leaves less than 1024
+    // 768 of them (each adds to its apply's total, 10 ns for an addition to
+    // one address: 17 -> 15 us a level at k = 9 against 2048), shorter steps
+    // where whole ones leave less than 1024
     const long long pairs = 8 * c.widest;
     const int step = c.n_out * ((pairs + 63) / 64) < 1024 ? 16 : 64;
-    const int y = (int)std::max<long long>(1, std::min<long long>((pairs + step - 1) / step, 2048 / c.n_out));
+    const int y = (int)std::max<long long>(1, std::min<long long>((pairs + step - 1) / step, 768 / c.n_out));
     if (bounds)
         hipLaunchKernelGGL((k_count<true>), dim3(c.n_out, y), dim3(512), 0, s, c, step);
     else
