@@ -285,9 +285,9 @@ int mwg_apply_fixed(mwg_context ctx, mwg_tree out, mwg_operator op, mwg_tree inp
  * wall milliseconds of [7] device plan creation, runs and downloads,
  * [8] the host split checks, [9] the post transforms (TopDown, BottomUp,
  * norms), [10] the whole apply, of the parts of [7]: [11] device plan
- * creation, [12] runs, and of the parts of [4]: [13] bands and slots,
- * [14] input pools on the device, [15] exact counts and segments (adaptive
- * applies; frozen-grid calls leave [11..15] 0). */
+ * creation (bands, slots, pools, counts, segments), [12] runs; [13] the host
+ * plans as [4], [14] uploads of host inputs, [15] 0 (adaptive applies;
+ * frozen-grid calls leave [11..15] 0). */
 int mwg_last_apply_stats(mwg_context ctx, double *stats, int n);
 
 /* Frozen-grid apply split into a resident device plan (bands, input slots,

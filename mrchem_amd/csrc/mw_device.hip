@@ -792,7 +792,8 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
         const int pos = it.pos, center = __builtin_amdgcn_readfirstlane(term.x),
                   span = __builtin_amdgcn_readfirstlane(term.y);
         const int lx = ((pos >> 5) & 255) - j.w, ly = ((pos >> 13) & 255) - j.w, lz = (pos >> 21) - j.w;
-        const int cx = (gb[0] << 1) | (pos & 1), cy = (gb[1] << 1) | ((pos >> 1) & 1), cz = (gb[2] << 1) | ((pos >> 2) & 1);
+        const int cx = (gb[0] << 1) | (pos & 1), cy = (gb[1] << 1) | ((pos >> 1) & 1);
+        const int cz = (gb[2] << 1) | ((pos >> 2) & 1);
         const int id[4] = {center + cx * span + lx, center + cy * span + ly, center + cz * span + lz,
                            center + (cz + 2) * span + lz};
 #pragma unroll
@@ -834,8 +835,8 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
     unsigned long long napps = 0, napps1 = 0;
     while (pi < pi_end) {
         wave_order();
-        const int n = screen_items<PAIR, S::CAP, S::AHEAD>(a, ad, j, tn, pi, pi_end, e0, e_last > 0 ? u_last : -1, e_last,
-                                                     sm.wl, lane, napps, napps1);
+        const int n = screen_items<PAIR, S::CAP, S::AHEAD>(a, ad, j, tn, pi, pi_end, e0, e_last > 0 ? u_last : -1,
+                                                           e_last, sm.wl, lane, napps, napps1);
         wave_order();
         if (n == 0) continue;
         Item4 it = uniform(0);
@@ -2741,11 +2742,12 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         r.totals = ca.totals;
         r.n_totals = (int)parts.size();
     }
-    // One wait per refinement level instead of three: the calculator (in the
-    // low-precision modes the class lists first) starts behind the cut, and counters, segment counts and norms come back in one
-    // copy after it (single-Gaussian Coulomb apply at k = 7: 2.74 to 2.43 ms;
-    // the exchange applies of 4 orbitals in one batch: 12.0 to 10.5 ms, with
-    // the one-launch assembly of the trees).
+    // One wait for a level's work instead of three: the calculator (in the
+    // low-precision modes the class lists first) starts behind the cut, and
+    // counters, segment counts and norms come back in one copy after it
+    // (single-Gaussian Coulomb apply at k = 7: 2.74 to 2.43 ms; the exchange
+    // applies of 4 orbitals in one batch: 12.0 to 10.5 ms, with the one-launch
+    // assembly of the trees).
     if (defer) {
         *out = p.release();
         return 0;
@@ -2899,7 +2901,8 @@ static int launch32_n(DeviceCtx *c, const KArgs &a, const float *pool, const int
 
 template <int N, bool PAIR>
 static int launch64_n(DeviceCtx *c, const KArgs &a, const double *pool, const int *list,
-                      const unsigned long long *n_dev, int n, double lo, unsigned long long *head, hipStream_t s, std::string &err) {
+                      const unsigned long long *n_dev, int n, double lo, unsigned long long *head, hipStream_t s,
+                      std::string &err) {
     if (n == 0) return 0;
     int grid = 0;
     int rc = persistent_grid(c, reinterpret_cast<const void *>(&k_apply64<N, PAIR>), 64, sizeof(Smem4<N>), 0, n, &grid,
@@ -2949,12 +2952,13 @@ static int launch64(const DevicePlan *p, const int *list, const unsigned long lo
 #undef MWG_LAUNCH
 }
 
-// Segment lists of the mixed mode: segments holding a term with bound above
-// tau * thr_cls (the FP64 class) and segments holding one at or below it.  The
-// lists are widened by a relative 1e-9 so that rounding can only add segments;
-// the kernel's own class test decides each term.
 static int drop_graph(DevicePlan *p, std::string &err);
 
+// Segment lists of a kept plan's low-precision mode, in its tuned order:
+// segments holding a term with bound above tau * thr_cls (the FP64 class) and
+// segments holding one at or below it.  The lists are widened by a relative
+// 1e-9 so that rounding can only add segments; the kernel's own class test
+// decides each term.
 static int make_lists(DevicePlan *p, int mode, double tau, std::string &err) {
     if (p->list_tau == tau && p->list_mode == mode && p->list_order == p->order) return 0;
     std::vector<SegMeta> shi, slo;

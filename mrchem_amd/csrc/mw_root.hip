@@ -184,10 +184,9 @@ __global__ __launch_bounds__(256) void k_root_xy(RootGeo geo, const RootApp *app
 // those of the roots; the latter are added to the plan's counter (n_totals 0:
 // not by this launch).
 template <int T, bool SAME>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_root_z(RootGeo geo, const RootApp *apps, const RootItem *items, int n_items,
-                                                int per, const int *root_out, const double *A, const double *Y,
-                                                double *out_ns, unsigned long long *counter,
-                                                const unsigned long long *totals, int n_totals) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_root_z(
+    RootGeo geo, const RootApp *apps, const RootItem *items, int n_items, int per, const int *root_out, const double *A,
+    const double *Y, double *out_ns, unsigned long long *counter, const unsigned long long *totals, int n_totals) {
     constexpr int K = 4 * T, SZ = T * K * 64, DP = 16 * T, nd = SAME ? 1 : 3;
     const int N = geo.n, N3 = N * N * N;
     const int D[3] = {2 * N * geo.boxes[0], 2 * N * geo.boxes[1], 2 * N * geo.boxes[2]};
