@@ -103,11 +103,11 @@ struct BandTree {
 // node of the input tree.
 constexpr int kBandLevels = 32, kBandCounts = 3 + kBandLevels;
 struct BandArgs {
-    const int *out_l, *out_depth, *out_app;  // out_l: 3 per output node
+    const int *out_l, *out_depth, *out_app;  // out_l: 3 per output node, from the world's corner
     const long long *band_off;
     const int *band_w;
     const BandTree *trees;  // per apply
-    int corner[3], boxes[3];
+    int boxes[3];
     int n_out;
     long long n_band;
     // table of cap cells (a power of two): name of the node, slot, generation

@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void k_band_find(BandArgs a) {
             bool in = true;
 #pragma unroll
             for (int d = 0; d < 3; d++) {
-                const int b = (k.l[d] >> k.d) - a.corner[d];
+                const int b = k.l[d] >> k.d;
                 in = in && b >= 0 && b < a.boxes[d];
             }
             if (in) c = locate(a, k, rep_of(q, p, 0), fresh, found);
@@ -155,8 +155,7 @@ __global__ __launch_bounds__(256) void k_band_find(BandArgs a) {
         int node = -1, da = 0;
         if (fresh) {
             // (the roots are a tree's first nodes, box x fastest)
-            node = (((k.l[2] >> k.d) - a.corner[2]) * a.boxes[1] + (k.l[1] >> k.d) - a.corner[1]) * a.boxes[0] +
-                   (k.l[0] >> k.d) - a.corner[0];
+            node = ((k.l[2] >> k.d) * a.boxes[1] + (k.l[1] >> k.d)) * a.boxes[0] + (k.l[0] >> k.d);
             for (; da < k.d; da++) {
                 const int c0 = t.child0[node], b = k.d - 1 - da;
                 if (c0 < 0) break;

@@ -2339,10 +2339,7 @@ static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n
     b.band_off = p->args.band_off;
     b.band_w = p->args.band_w;
     b.trees = trees;
-    for (int d = 0; d < 3; d++) {
-        b.corner[d] = (int)mra.corner[d];
-        b.boxes[d] = mra.boxes[d];
-    }
+    for (int d = 0; d < 3; d++) b.boxes[d] = mra.boxes[d];
     b.n_out = p->n_out;
     b.n_band = n_band;
     // work memory, put back below: its next holder's work comes after these

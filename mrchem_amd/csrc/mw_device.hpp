@@ -112,7 +112,7 @@ int dev_build_operators(DeviceCtx *c, const MRA &mra, const std::vector<OpBuildJ
 // Copy the device table of a device-built operator (f.device_blocks values).
 int dev_download_operator_blocks(DeviceCtx *c, const void *key, double *out, long long n, std::string &err);
 
-// An output node of a product or sum: depth and translation.
+// An output node of a product or sum: depth and world_translation.
 struct NodeAt {
     int d, l[3];
 };

@@ -184,6 +184,14 @@ using UninitAlloc = BigAlloc<T, false>;
 // uninitialised (add_node fills its block with zeros explicitly).
 using CoefVec = std::vector<double, BigAlloc<double, false>>;
 
+// A node's translations from the world's lower corner, as the device walks
+// trees and bands: below 2^21 (at most 2 boxes and depth 20), where the
+// absolute ones, corner 2^depth and up, pass 32 bits for a corner a few
+// thousand boxes from the origin.  The bits below the root box are the same.
+inline void world_translation(const MRA &mra, const NodeKey &k, int *l) {
+    for (int d = 0; d < 3; d++) l[d] = (int)(k.l[d] - mra.tlo(k.depth, d));
+}
+
 struct Tree {
     const MRA *mra = nullptr;
     std::vector<NodeKey> keys;
@@ -247,7 +255,7 @@ bool split_check(const MRA &mra, int depth, double wnorm, double prec, double tn
 struct ApplyPlan {
     int kp1 = 0, ndepth = 0, M = 0;
     // output nodes
-    std::vector<int> out_depth, out_l;  // out_l: translations, 3 per node
+    std::vector<int> out_depth, out_l;  // out_l: 3 per node (world_translation)
     std::vector<double> out_thr;        // screening threshold per output node
     // entries of a node's band: (2W+1)^3 from band_off, order dz, dy, dx with
     // dx fastest

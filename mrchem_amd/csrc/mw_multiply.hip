@@ -1325,7 +1325,7 @@ struct AddTree {
     int size, pad_;
 };
 struct AddGeo {
-    int corner[3], boxes[3];
+    int boxes[3];
 };
 
 __device__ __forceinline__ int child_of(const NodeAt &k, int b) {
@@ -1335,8 +1335,7 @@ __device__ __forceinline__ int child_of(const NodeAt &k, int b) {
 // The walk from the root box down to the input's deepest node on the path of k,
 // dep levels above it: a chain of at most 20 dependent loads.
 __device__ __forceinline__ int deepest_node(const AddGeo &geo, const AddTree &t, const NodeAt &k, int &dep) {
-    int node = (((k.l[2] >> k.d) - geo.corner[2]) * geo.boxes[1] + (k.l[1] >> k.d) - geo.corner[1]) * geo.boxes[0] +
-               (k.l[0] >> k.d) - geo.corner[0];
+    int node = ((k.l[2] >> k.d) * geo.boxes[1] + (k.l[1] >> k.d)) * geo.boxes[0] + (k.l[0] >> k.d);
     for (dep = k.d; dep > 0; dep--) {
         const int c0 = t.child0[node];
         if (c0 < 0) break;
@@ -1403,10 +1402,7 @@ static int upload_trees(DeviceCtx *c, const std::vector<const Tree *> &trees, co
 
 static AddGeo add_geo(const MRA &mra) {
     AddGeo g;
-    for (int d = 0; d < 3; d++) {
-        g.corner[d] = (int)mra.corner[d];
-        g.boxes[d] = mra.boxes[d];
-    }
+    for (int d = 0; d < 3; d++) g.boxes[d] = mra.boxes[d];
     return g;
 }
 

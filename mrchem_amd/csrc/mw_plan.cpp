@@ -109,7 +109,7 @@ void build_plan(ApplyPlan &plan, const Operator &op, const Tree &inp, const Tree
         const NodeKey &k = out.keys[nodes[q]];
         const int side = 2 * W[k.depth] + 1;
         plan.out_depth[q] = k.depth;
-        for (int d = 0; d < 3; d++) plan.out_l[3 * q + d] = (int)k.l[d];
+        world_translation(mra, k, &plan.out_l[3 * q]);
         plan.band_w[q] = W[k.depth];
         plan.band_off[q] = plan.n_band;
         plan.n_band += (long long)side * side * side;

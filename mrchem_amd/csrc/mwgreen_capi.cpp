@@ -1127,6 +1127,12 @@ bool mul_source(const Tree &f, const NodeKey &k, long long &off, int &dep, unsig
     return false;
 }
 
+NodeAt node_at(const MRA &mra, const NodeKey &k) {
+    NodeAt n{k.depth, {0, 0, 0}};
+    world_translation(mra, k, n.l);
+    return n;
+}
+
 // Nodes of f in order of depth, each after its parent.
 std::vector<int> by_depth(const Tree &f) {
     std::vector<int> order(f.size());
@@ -1310,7 +1316,7 @@ int add_trees(mwg_context ctx, double prec, Tree &T, const std::vector<mwg_tree>
         nodes.reserve(work.size());
         for (int w : work) {
             const NodeKey &k = T.keys[w];
-            nodes.push_back(NodeAt{k.depth, {(int)k.l[0], (int)k.l[1], (int)k.l[2]}});
+            nodes.push_back(node_at(mra, k));
         }
         if (on_device) {
             double *buf = lv.add_level(work);
@@ -1480,7 +1486,7 @@ int multiply_trees(mwg_context ctx, double prec, mwg_tree out, double coef, mwg_
                     nd.hfac = std::pow(mra.box_size(k.depth + 1), -1.5);
                     if (noalloc) nodes.push_back(nd);
                 }
-                at.push_back(NodeAt{k.depth, {(int)k.l[0], (int)k.l[1], (int)k.l[2]}});
+                at.push_back(node_at(mra, k));
             }
             if (on_device) {
                 double *buf = lv.add_level(work);
