@@ -3192,6 +3192,15 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         // beside the split class on the first, as in the mixed mode
         HIP_TRY(hipEventRecord(c->evz, c->stream));
         HIP_TRY(hipStreamWaitEvent(c->stream2, c->evz, 0));
+        // Blocks of the memory pool are handed on in the order of the
+        // context's stream, so the second stream is never left unjoined: a
+        // step that fails before the join waits for it here.
+        struct Fork {
+            hipStream_t s;
+            ~Fork() {
+                if (s) (void)hipStreamSynchronize(s);
+            }
+        } fork{c->stream2};
         if (timed) HIP_TRY(hipEventRecord(c->ev2s, c->stream2));
         rc = launch64(p, hi, n_hi_dev, n_hi, tau, head2, c->stream2, err);
         if (rc) return rc;
@@ -3201,6 +3210,7 @@ static int enqueue_step(DevicePlan *p, int mode, double tau, bool post, bool tim
         if (rc) return rc;
         if (timed) HIP_TRY(hipEventRecord(c->evm, c->stream));
         HIP_TRY(hipStreamWaitEvent(c->stream, c->ev2e, 0));
+        fork.s = nullptr;
     }
     // end of the calculator (both classes joined)
     if (timed) HIP_TRY(hipEventRecord(c->evp, c->stream));
