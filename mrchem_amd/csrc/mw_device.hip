@@ -1759,15 +1759,37 @@ struct DeviceCtx {
 };
 
 namespace {
-// contexts of the process, for dev_mem_get's second try
+// contexts of the process
 std::mutex g_ctx_mtx;
 std::set<DeviceCtx *> g_ctxs;
 
-void mem_trim(MemPool &m) {
+// The idle blocks of a context back to the driver (hipFree waits for the
+// device, so also for work of this context that still uses them).
+void mem_trim(DeviceCtx *c) {
+    MemPool &m = c->mem;
     std::lock_guard<std::mutex> g(m.mtx);
     for (auto &kv : m.idle) (void)hipFree(kv.second);
     m.idle.clear();
     m.idle_bytes = 0;
+}
+
+// Of every context of c's device.
+void mem_trim_device(DeviceCtx *c) {
+    std::lock_guard<std::mutex> g(g_ctx_mtx);
+    for (DeviceCtx *o : g_ctxs)
+        if (o->device == c->device) mem_trim(o);
+}
+
+// hipMalloc on c's device, tried again without any idle memory when refused.
+hipError_t device_malloc(DeviceCtx *c, size_t bytes, void **p) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        mem_trim_device(c);
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) *p = nullptr;
+    return e;
 }
 }  // namespace
 
@@ -1775,7 +1797,7 @@ int dev_mem_get(DeviceCtx *c, size_t bytes, void **p, std::string &err) {
     *p = nullptr;
     HIP_TRY(hipSetDevice(c->device));
     MemPool &m = c->mem;
-    const size_t cls = MemPool::size_class(bytes);
+    size_t cls = MemPool::size_class(bytes);
     {
         std::lock_guard<std::mutex> g(m.mtx);
         auto it = m.idle.lower_bound(cls);
@@ -1788,14 +1810,11 @@ int dev_mem_get(DeviceCtx *c, size_t bytes, void **p, std::string &err) {
             return 0;
         }
     }
-    hipError_t e = hipMalloc(p, cls);
-    if (e != hipSuccess) {
+    hipError_t e = device_malloc(c, cls, p);
+    if (e != hipSuccess && cls > bytes && bytes > 0) {
+        // the card may hold what was asked for, if not its class
         (void)hipGetLastError();
-        {
-            std::lock_guard<std::mutex> g(g_ctx_mtx);
-            for (DeviceCtx *o : g_ctxs)
-                if (o->device == c->device) mem_trim(o->mem);
-        }
+        cls = bytes;
         e = hipMalloc(p, cls);
     }
     if (e != hipSuccess) {
@@ -1831,7 +1850,7 @@ void dev_mem_put(DeviceCtx *c, void *p) {
 int dev_raw_alloc(DeviceCtx *c, size_t bytes, void **p, std::string &err) {
     *p = nullptr;
     HIP_TRY(hipSetDevice(c->device));
-    HIP_TRY(hipMalloc(p, std::max<size_t>(bytes, 8)));
+    HIP_TRY(device_malloc(c, std::max<size_t>(bytes, 8), p));
     return 0;
 }
 
@@ -1995,7 +2014,7 @@ void dev_destroy(DeviceCtx *c) {
         std::lock_guard<std::mutex> g(g_ctx_mtx);
         g_ctxs.erase(c);
     }
-    mem_trim(c->mem);
+    mem_trim(c);
     for (auto &kv : c->mem.live) (void)hipFree(kv.first);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;

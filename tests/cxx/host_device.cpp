@@ -286,10 +286,39 @@ void split_step_fails() {
     check(unjoined() == 0, "the second stream is joined");
 }
 
+// Memory that lies idle in a context's pool is given back for every kind of
+// allocation, and a block whose size class does not fit is tried at its size.
+void idle_memory_is_given_back() {
+    mwg_mra m = world(7, 8);
+    mwg_context a = nullptr, b = nullptr;
+    check(mwg_context_create(0, &a) == MWG_OK && mwg_context_create(0, &b) == MWG_OK, "contexts");
+    mwg_tree f = gaussian(m, 1e-4, 40.0);
+    int n = 0;
+    check(mwg_tree_size(f, &n) == MWG_OK, "size");
+    const size_t bytes = (size_t)n * 8 * 512 * sizeof(double);
+    long long size = 0;
+    check(mwg_tree_pack_size(f, &size) == MWG_OK, "pack size");
+    std::vector<char> packed(size);
+    // (each uploads the blocks and puts them back)
+    for (mwg_context c : {a, b}) check(mwg_tree_pack_device(f, c, packed.data(), size) == MWG_OK, "pack");
+    std::printf("%d nodes, %zu bytes of blocks, %zu held by the pools\n", n, bytes, g_used);
+    check(g_used >= 2 * bytes, "both pools hold their blocks");
+    // room for the tree's blocks once, but not beside what lies idle
+    g_capacity = g_used + bytes / 2;
+    void *buf = nullptr;
+    check(mwg_device_buffer_create(a, (long long)bytes, &buf) == MWG_OK, "a caller's buffer");
+    check(mwg_device_buffer_destroy(a, buf) == MWG_OK, "destroy");
+    // room for the blocks to the byte, less than their class
+    g_capacity = g_used + bytes;
+    check(mwg_tree_pack_device(f, a, packed.data(), size) == MWG_OK, "blocks on a card they just fit");
+    check(g_used <= g_capacity, "within the card");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
-    const std::map<std::string, void (*)()> scenarios = {{"split_step_fails", split_step_fails}};
+    const std::map<std::string, void (*)()> scenarios = {{"split_step_fails", split_step_fails},
+                                                            {"idle_memory_is_given_back", idle_memory_is_given_back}};
     const auto it = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return 2;
     it->second();
