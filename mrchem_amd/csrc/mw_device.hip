@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -1712,10 +1713,11 @@ struct DevOper {
 // densities at k = 7 43.9 -> 31.3 ms, one k = 7 product 2.24 -> 1.39 ms).
 // Blocks are kept by
 // size class (an eighth of a power of two, so at most 12.5 % is unused) and
-// given back to the driver when more than kIdleMax bytes are idle, when an
-// allocation fails on any context of the device, and with the context.
+// given back to the driver when more than kIdleMax bytes are idle on the
+// device, those of other contexts first, when an allocation fails on any
+// context of the device, and with the context.
 struct MemPool {
-    static constexpr size_t kIdleMax = (size_t)8 << 30;
+    static constexpr size_t kIdleMax = (size_t)8 << 30;  // of all contexts of a device
     std::mutex mtx;
     std::map<void *, size_t> live;         // handed out: class size
     std::multimap<size_t, void *> idle;
@@ -1759,9 +1761,12 @@ struct DeviceCtx {
 };
 
 namespace {
-// contexts of the process
+// contexts of the process, and the idle bytes of all their pools by device
 std::mutex g_ctx_mtx;
 std::set<DeviceCtx *> g_ctxs;
+constexpr int kDevices = 64;
+std::atomic<size_t> g_idle[kDevices];
+std::atomic<size_t> &idle_of(const DeviceCtx *c) { return g_idle[c->device % kDevices]; }
 
 // The idle blocks of a context back to the driver (hipFree waits for the
 // device, so also for work of this context that still uses them).
@@ -1770,14 +1775,15 @@ void mem_trim(DeviceCtx *c) {
     std::lock_guard<std::mutex> g(m.mtx);
     for (auto &kv : m.idle) (void)hipFree(kv.second);
     m.idle.clear();
+    idle_of(c) -= m.idle_bytes;
     m.idle_bytes = 0;
 }
 
-// Of every context of c's device.
-void mem_trim_device(DeviceCtx *c) {
+// Of every context of c's device, or of every one but c.
+void mem_trim_device(DeviceCtx *c, bool others) {
     std::lock_guard<std::mutex> g(g_ctx_mtx);
     for (DeviceCtx *o : g_ctxs)
-        if (o->device == c->device) mem_trim(o);
+        if (o->device == c->device && !(others && o == c)) mem_trim(o);
 }
 
 // hipMalloc on c's device, tried again without any idle memory when refused.
@@ -1785,7 +1791,7 @@ hipError_t device_malloc(DeviceCtx *c, size_t bytes, void **p) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        mem_trim_device(c);
+        mem_trim_device(c, false);
         e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) *p = nullptr;
@@ -1805,6 +1811,7 @@ int dev_mem_get(DeviceCtx *c, size_t bytes, void **p, std::string &err) {
         if (it != m.idle.end() && it->first <= cls + cls / 7) {
             *p = it->second;
             m.idle_bytes -= it->first;
+            idle_of(c) -= it->first;
             m.live[*p] = it->first;
             m.idle.erase(it);
             return 0;
@@ -1830,18 +1837,27 @@ int dev_mem_get(DeviceCtx *c, size_t bytes, void **p, std::string &err) {
 void dev_mem_put(DeviceCtx *c, void *p) {
     if (!p) return;
     MemPool &m = c->mem;
+    size_t cls = 0;
     {
         std::lock_guard<std::mutex> g(m.mtx);
         auto it = m.live.find(p);
         if (it == m.live.end()) return;
-        const size_t cls = it->second;
+        cls = it->second;
         m.live.erase(it);
-        if (m.idle_bytes + cls <= MemPool::kIdleMax) {
-            m.idle.emplace(cls, p);
-            m.idle_bytes += cls;
-            return;
-        }
     }
+    std::atomic<size_t> &idle = idle_of(c);
+    bool keep = idle.fetch_add(cls) + cls <= MemPool::kIdleMax;
+    if (!keep && cls <= MemPool::kIdleMax) {
+        mem_trim_device(c, true);
+        keep = idle <= MemPool::kIdleMax;
+    }
+    if (keep) {
+        std::lock_guard<std::mutex> g(m.mtx);
+        m.idle.emplace(cls, p);
+        m.idle_bytes += cls;
+        return;
+    }
+    idle -= cls;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     (void)hipFree(p);

@@ -22,7 +22,8 @@
 namespace {
 
 std::recursive_mutex g_mtx;
-size_t g_capacity = (size_t)4 << 30, g_used = 0, g_peak = 0;
+size_t g_capacity = (size_t)4 << 30, g_used = 0, g_peak = 0, g_copy_max = ~(size_t)0;
+long long g_mallocs = 0;
 std::map<void *, size_t> g_mem;
 // by host function (registered before this program's own objects are made)
 std::map<const void *, std::string> &kernels() {
@@ -142,6 +143,7 @@ hipError_t hipMalloc(void **p, size_t n) {
     *p = nullptr;
     if (g_used + n > g_capacity) return result(hipErrorOutOfMemory);
     *p = std::calloc(n, 1);
+    g_mallocs++;
     g_mem[*p] = n;
     g_used += n;
     g_peak = std::max(g_peak, g_used);
@@ -175,7 +177,7 @@ hipError_t hipGetSymbolAddress(void **p, const void *) {
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t s) {
-    std::memcpy(dst, src, n);
+    if (n <= g_copy_max) std::memcpy(dst, src, n);
     std::lock_guard<std::recursive_mutex> g(g_mtx);
     of(s)->queued++;
     return hipSuccess;
@@ -314,11 +316,45 @@ void idle_memory_is_given_back() {
     check(g_used <= g_capacity, "within the card");
 }
 
+// What the contexts of a device hold idle is bounded for all of them together,
+// and a context that works after many others still keeps its own.
+void idle_memory_is_bounded() {
+    mwg_mra m = world(11, 4);
+    g_capacity = (size_t)64 << 30;
+    g_copy_max = (size_t)1 << 20;  // larger transfers move nothing
+    const size_t bound = (size_t)8 << 30;
+    mwg_tree f = nullptr;
+    const double c = 1.0, e = 0.05, pos[3] = {0.3, -0.2, 0.1};
+    check(mwg_tree_create(m, &f) == MWG_OK, "tree");
+    check(mwg_tree_project_gaussians(f, 1e-30, 1, 3, 1, &c, &e, pos) == MWG_OK, "projection");
+    int n = 0;
+    long long size = 0;
+    check(mwg_tree_size(f, &n) == MWG_OK && mwg_tree_pack_size(f, &size) == MWG_OK, "size");
+    const size_t bytes = (size_t)n * 8 * 1728 * sizeof(double);
+    char *dst = static_cast<char *>(std::malloc(size));
+    size_t most = 0;
+    long long last = 0;
+    const int contexts = (int)(bound / bytes) + 4;
+    for (int i = 0; i < contexts; i++) {
+        mwg_context ctx = nullptr;
+        check(mwg_context_create(0, &ctx) == MWG_OK, "context");
+        check(mwg_tree_pack_device(f, ctx, dst, size) == MWG_OK, "pack");
+        most = std::max(most, g_used);
+        last = g_mallocs;
+        check(mwg_tree_pack_device(f, ctx, dst, size) == MWG_OK, "pack again");
+        last = g_mallocs - last;
+    }
+    std::printf("%d nodes, %zu bytes of blocks, %d contexts: at most %zu bytes idle\n", n, bytes, contexts, most);
+    check(most > bound / 2 && most <= bound, "idle memory of all contexts");
+    check(last == 0, "the last context's block is kept for its next call");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const std::map<std::string, void (*)()> scenarios = {{"split_step_fails", split_step_fails},
-                                                            {"idle_memory_is_given_back", idle_memory_is_given_back}};
+                                                            {"idle_memory_is_given_back", idle_memory_is_given_back},
+                                                            {"idle_memory_is_bounded", idle_memory_is_bounded}};
     const auto it = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return 2;
     it->second();

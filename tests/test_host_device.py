@@ -20,7 +20,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("scenario", ["split_step_fails", "idle_memory_is_given_back"])
+@pytest.mark.parametrize("scenario", ["split_step_fails", "idle_memory_is_given_back", "idle_memory_is_bounded"])
 def test_scenario(exe, scenario):
     r = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=100)
     print(r.stdout, r.stderr)
