@@ -1254,6 +1254,42 @@ int dev_finish_blocks(DeviceCtx *c, const MRA &mra, const std::vector<BlockMove>
     return 0;
 }
 
+int dev_download_blocks(DeviceCtx *c, const MRA &mra, const std::vector<const double *> &src, double *dst,
+                        std::string &err) {
+    if (src.empty()) return 0;
+    HIP_TRY(hipSetDevice(dev_device(c)));
+    hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
+    const size_t n = src.size(), blk = (size_t)mra.block();
+    // several of the 64 MB chunks in which large copies overlap with the host's
+    const size_t per = std::min(n, std::max<size_t>(1, ((size_t)256 << 20) / (sizeof(double) * blk)));
+    double *room = nullptr;
+    BlockMove *dm = nullptr;
+    int rc = dev_mem(c, per * blk, &room, err);
+    if (!rc) rc = dev_mem(c, n, &dm, err);
+    hipError_t e = hipSuccess;
+    if (!rc) {
+        std::vector<BlockMove> moves(n);
+        for (size_t i = 0; i < n; i++) moves[i] = BlockMove{src[i], room + i % per * blk};
+        e = hipMemcpyAsync(dm, moves.data(), sizeof(BlockMove) * n, hipMemcpyHostToDevice, s);
+        for (size_t i = 0; i < n && !rc && e == hipSuccess; i += per) {
+            const size_t cnt = std::min(per, n - i);
+            hipLaunchKernelGGL(k_move_norms, dim3((unsigned)cnt), dim3(256), 0, s, dm + i, mra.kp1_3(),
+                               static_cast<double *>(nullptr), static_cast<double *>(nullptr));
+            e = hipGetLastError();
+            if (e == hipSuccess) rc = dev_copy_d2h(c, dst + i * blk, room, sizeof(double) * cnt * blk, err);
+        }
+        if (e != hipSuccess || rc) (void)hipStreamSynchronize(s);  // moves is read until then
+    }
+    dev_mem_put(c, room);
+    dev_mem_put(c, dm);
+    if (rc) return rc;
+    if (e != hipSuccess) {
+        err = std::string("block download: ") + hipGetErrorString(e);
+        return -2;
+    }
+    return 0;
+}
+
 int dev_pack(DeviceCtx *c, void *dst, const void *head, size_t head_bytes, const double *blocks, size_t n,
              std::string &err) {
     HIP_TRY(hipSetDevice(dev_device(c)));

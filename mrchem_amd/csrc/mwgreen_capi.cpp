@@ -317,6 +317,18 @@ void ensure_norms(mwg_tree t) {
     t->norms_valid = true;
 }
 
+// The norms of t's new blocks.
+void take_norms(mwg_tree t, std::vector<double> &&s2, std::vector<double> &&w2) {
+    Tree &T = t->tree;
+    double sq = 0.0;
+    for (int i = 0; i < T.size(); i++) sq += w2[i] + (T.parent[i] < 0 ? s2[i] : 0.0);
+    T.sqnorm = sq;
+    t->s2 = std::move(s2);
+    t->w2 = std::move(w2);
+    t->norms_valid = true;
+    t->cn8_valid = false;
+}
+
 // A result computed on the device by a call on ctx: t's blocks (tree order,
 // tree_values(t) doubles, owned by the call until handed over here) and their
 // norms.  Kept as t's resident copy when t is resident on ctx, else
@@ -343,13 +355,7 @@ void take_device_result(mwg_context ctx, mwg_tree t, double *blocks, std::vector
         t->host_valid = true;
         t->dev_valid = false;
     }
-    double sq = 0.0;
-    for (int i = 0; i < T.size(); i++) sq += w2[i] + (T.parent[i] < 0 ? s2[i] : 0.0);
-    T.sqnorm = sq;
-    t->s2 = std::move(s2);
-    t->w2 = std::move(w2);
-    t->norms_valid = true;
-    t->cn8_valid = false;
+    take_norms(t, std::move(s2), std::move(w2));
 }
 
 // An input must hold finite values (checked on its node norms).
@@ -662,17 +668,21 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
                 levels[o.keys[i].depth].push_back(PostPair{addr(loc[i]), addr(loc[c0])});
             }
         }
-        // the transformed blocks into one array per tree, normed on the way:
-        // the device copy of an output resident on this context, else a
-        // temporary that is downloaded into the host tree
+        // the transformed blocks normed, and on the way those of an output
+        // resident on this context into its device copy; a host tree's are
+        // downloaded from where they are, so that its blocks are on the
+        // device once
         std::vector<DeviceResult> res;
         for (size_t ji = 0; ji < jobs.size(); ji++) res.push_back(DeviceResult{ctx->dev, nullptr});
         std::vector<BlockMove> moves;
         for (size_t ji = 0; ji < jobs.size(); ji++) {
             const Tree &o = jobs[ji].out->tree;
-            dev_check(dev_alloc(ctx->dev, (size_t)o.size() * blk, &res[ji].p, err), err);
-            for (int i = 0; i < o.size(); i++)
-                moves.push_back(BlockMove{addr(locs[ji][i]), res[ji].p + (size_t)i * blk});
+            const bool resident = jobs[ji].out->dctx == ctx;
+            if (resident) dev_check(dev_alloc(ctx->dev, (size_t)o.size() * blk, &res[ji].p, err), err);
+            for (int i = 0; i < o.size(); i++) {
+                double *at = addr(locs[ji][i]);
+                moves.push_back(BlockMove{at, resident ? res[ji].p + (size_t)i * blk : at});
+            }
         }
         std::vector<double> nr(2 * moves.size());
         dev_check(dev_finish_blocks(ctx->dev, mra, {}, levels, true, moves, nr.data(), err), err);
@@ -680,9 +690,20 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         for (size_t ji = 0; ji < jobs.size(); ji++) {
             mwg_tree out = jobs[ji].out;
             const size_t n = (size_t)out->tree.size();
-            const double *ns2 = nr.data() + at, *nw2 = nr.data() + moves.size() + at;
-            take_device_result(ctx, out, res[ji].release(), std::vector<double>(ns2, ns2 + n),
-                               std::vector<double>(nw2, nw2 + n));
+            std::vector<double> ns2(nr.begin() + at, nr.begin() + at + n);
+            std::vector<double> nw2(nr.begin() + moves.size() + at, nr.begin() + moves.size() + at + n);
+            if (res[ji].p) {
+                take_device_result(ctx, out, res[ji].release(), std::move(ns2), std::move(nw2));
+            } else {
+                std::vector<const double *> src(n);
+                for (size_t i = 0; i < n; i++) src[i] = moves[at + i].src;
+                out->tree.structure_only = false;
+                out->tree.coefs.resize(tree_values(out));  // every block is written
+                host_changed(out);
+                dev_check(dev_download_blocks(ctx->dev, mra, src, out->tree.coefs.data(), err), err);
+                ctx->d2h_bytes += (long long)(sizeof(double) * tree_values(out));
+                take_norms(out, std::move(ns2), std::move(nw2));
+            }
             out->apply_thr = jobs[ji].thr_all;
             at += n;
         }

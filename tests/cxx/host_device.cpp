@@ -1,12 +1,12 @@
 // The library's host code on a device of host memory: this program defines the
 // HIP calls that libmwgreen.so imports (the executable's definitions come
 // first), with memory that is counted against a capacity, streams and events
-// that keep account of what waits for what, and kernels that do nothing but
-// can be made to fail.  So the host's error paths and its use of memory are
+// that keep account of what waits for what, and kernels that do nothing (norms
+// are all one, and a search finds no slot) but can be made to fail.  So the host's error paths and its use of memory are
 // checked without a GPU (tests/test_host_device.py).
 //
 //   host_device <scenario>
-#include <hip/hip_runtime_api.h>
+#include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdio>
@@ -17,6 +17,9 @@
 #include <string>
 #include <vector>
 
+#define _Float16 short  // (g++ has none; only pointers to it are declared)
+#include "mw_apply.hpp"
+#undef _Float16
 #include "mwgreen.h"
 
 namespace {
@@ -105,7 +108,7 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shmem, hip
     *stream = d.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t, hipStream_t s) {
     std::lock_guard<std::recursive_mutex> g(g_mtx);
     // the work items of a launch are counted in 32 bits
     if ((unsigned long long)grid.x * block.x >= (1ull << 32) || grid.x == 0 || grid.y == 0 || grid.y > 65535)
@@ -114,6 +117,15 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **, size_t
         g_failed++;
         return result(hipErrorLaunchFailure);
     }
+    const std::string &name = kernels()[f];
+    auto ones = [&](int s2) {
+        for (int a = s2; a < s2 + 2; a++)
+            if (double *p = *static_cast<double **>(args[a])) std::fill_n(p, grid.x, 1.0);
+    };
+    if (name.find("k_node_norms") != std::string::npos) ones(3);
+    if (name.find("k_move_norms") != std::string::npos) ones(2);
+    if (name.find("k_band_clear") != std::string::npos)
+        std::fill_n(static_cast<mwg::BandArgs *>(args[0])->cnt, mwg::kBandCounts, 0u);
     of(s)->queued++;
     return hipSuccess;
 }
@@ -349,12 +361,33 @@ void idle_memory_is_bounded() {
     check(last == 0, "the last context's block is kept for its next call");
 }
 
+// An apply to a host tree holds its output's blocks on the device once.
+void host_output_memory() {
+    mwg_mra m = world(5, 4);
+    mwg_context ctx = nullptr;
+    check(mwg_context_create(0, &ctx) == MWG_OK, "context");
+    mwg_operator P = nullptr;
+    check(mwg_poisson_create(m, 1e-2, &P) == MWG_OK, "operator");
+    mwg_tree f = gaussian(m, 1e-2, 1.0), V = nullptr;
+    check(mwg_tree_create(m, &V) == MWG_OK, "tree");
+    g_copy_max = (size_t)16 << 20;  // larger transfers move nothing
+    // every wavelet norm is one: the grid grows to the full depth
+    check(mwg_apply(ctx, 0.1, V, P, f, -1, 1) == MWG_OK, "apply");
+    int n = 0;
+    check(mwg_tree_size(V, &n) == MWG_OK, "size");
+    const size_t bytes = (size_t)n * 8 * 216 * sizeof(double);
+    std::printf("%d nodes, %zu bytes of blocks, at most %zu bytes on the device\n", n, bytes, g_peak);
+    check(n == 8 * 4681, "the whole grid");
+    check(g_peak < bytes + bytes * 4 / 5, "blocks on the device once, and a part of them to copy from");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const std::map<std::string, void (*)()> scenarios = {{"split_step_fails", split_step_fails},
                                                             {"idle_memory_is_given_back", idle_memory_is_given_back},
-                                                            {"idle_memory_is_bounded", idle_memory_is_bounded}};
+                                                            {"idle_memory_is_bounded", idle_memory_is_bounded},
+                                                            {"host_output_memory", host_output_memory}};
     const auto it = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return 2;
     it->second();
