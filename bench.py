@@ -185,11 +185,12 @@ def main():
     adaptive(False)  # first call: code objects, allocator and operator tables warm up
     outs, t_adapt, ast = adaptive(False)
     n_out = sum(o.size() for o in outs)
-    log("adaptive apply: %d output nodes in %.1f ms (kernel %.1f ms, bands %.1f ms, input uploads %.1f ms, %d "
-        "launches; device plan create %.1f + run %.1f of %.1f ms, split checks %.1f ms, post transforms + download "
-        "%.1f ms)" %
-        (n_out, 1e3 * t_adapt, ast["kernel_ms"], ast["plan_grid_ms"], ast["plan_pool_ms"], ast["launches"],
-         ast["device_create_ms"], ast["device_run_ms"], ast["device_ms"], ast["split_ms"], ast["post_ms"]))
+    log("adaptive apply: %d output nodes in %.1f ms (kernel %.1f ms, plan %.1f ms = bands %.1f + pools %.1f + "
+        "counts %.1f, %d launches; device plan create %.1f + run %.1f of %.1f ms, split checks %.1f ms, post "
+        "transforms + download %.1f ms)" %
+        (n_out, 1e3 * t_adapt, ast["kernel_ms"], ast["plan_ms"], ast["plan_grid_ms"], ast["plan_pool_ms"],
+         ast["plan_counts_ms"], ast["launches"], ast["device_create_ms"], ast["device_run_ms"], ast["device_ms"],
+         ast["split_ms"], ast["post_ms"]))
     adaptive(True)  # uploads the inputs once
     routs, t_res, rst = adaptive(True)
     log("adaptive apply, trees resident on the device: %.1f ms (plan %.1f ms, device %.1f ms, post %.1f ms)" %

@@ -280,14 +280,16 @@ int mwg_apply_fixed(mwg_context ctx, mwg_tree out, mwg_operator op, mwg_tree inp
 
 /* Statistics of the last apply on this context: [0] kernel milliseconds,
  * [1] output nodes computed, [2] input slots, [3] generated slots,
- * [4] host plan milliseconds, [5] kernel launches, [6] term-applications
+ * [4] plan milliseconds, [5] kernel launches, [6] term-applications
  * that passed screening (each 6(k+1)^4 flops of algorithmic work),
  * wall milliseconds of [7] device plan creation, runs and downloads,
  * [8] the host split checks, [9] the post transforms (TopDown, BottomUp,
  * norms), [10] the whole apply, of the parts of [7]: [11] device plan
- * creation (bands, slots, pools, counts, segments), [12] runs; [13] the host
- * plans as [4], [14] uploads of host inputs, [15] 0 (adaptive applies;
- * frozen-grid calls leave [11..15] 0). */
+ * creation, [12] runs, and of the parts of [4]: [13] bands and slots,
+ * [14] input pools on the device (with the uploads of host inputs), [15] exact
+ * counts and segments (adaptive applies; frozen-grid calls leave [11..15] 0).
+ * All are the host's time: device work of [14] and [15] that it does not wait
+ * for is part of [12]. */
 int mwg_last_apply_stats(mwg_context ctx, double *stats, int n);
 
 /* Frozen-grid apply split into a resident device plan (bands, input slots,

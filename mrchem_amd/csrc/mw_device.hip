@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -2356,13 +2357,18 @@ static int clear_step(DevicePlan *p, std::string &err) {
     return 0;
 }
 
+static double host_ms() {
+    return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
 // Bands, slots and pool of the plan: the search, then, its counts known, the
 // slot tables, the pool and the generated nodes.  beside: launches that need
 // none of it, which run while the host waits for the counts.
 template <typename F>
 static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n_band, long long widest,
                      const int *out_l, const BandTree *trees, int *band, const double *filter, const int *root_out,
-                     int n_roots, long long *root_off, F &&beside, std::string &err) {
+                     int n_roots, long long *root_off, F &&beside, double *plan_ms, std::string &err) {
+    const double t0 = host_ms();
     DeviceCtx *c = p->ctx;
     hipStream_t s = c->stream;
     const int N = p->kp1;
@@ -2413,6 +2419,8 @@ static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n
         if (!cnt[2]) break;
         cells *= 2;
     }
+    const double t1 = host_ms();
+    plan_ms[0] += t1 - t0;
     const long long n_real = cnt[0], n_slot = n_real + cnt[1];
     long long n_gen = 0;
     BandItems o{};
@@ -2447,11 +2455,15 @@ static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n
     p->args.slot_norm = norms;
     p->args.n_real = (int)n_real;
     if ((rc = dev_band_items(s, b, o, err))) return rc;
-    return dev_pool_fill(s, N, filter, o.gen, lv_off, o.slots, (int)n_slot, err);
+    rc = dev_pool_fill(s, N, filter, o.gen, lv_off, o.slots, (int)n_slot, err);
+    plan_ms[1] += host_ms() - t1;
+    return rc;
 }
 
 int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, bool once,
-                    DevicePlan **out, std::string &err) {
+                    DevicePlan **out, std::string &err, double *plan_ms) {
+    double unused[3] = {0.0, 0.0, 0.0};
+    if (!plan_ms) plan_ms = unused;
     HIP_TRY(hipSetDevice(c->device));
     if (parts.empty()) {
         err = "empty plan";
@@ -2752,7 +2764,8 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
                        return dev_term_tables(s, a, N * N, reinterpret_cast<const TermLevel *>(dev + f_lv),
                                               (int)levels.size(), reinterpret_cast<double *>(dev + f_tn),
                                               reinterpret_cast<int2 *>(dev + f_tb), err);
-                   }, err);
+                   }, plan_ms, err);
+    const double t_count = host_ms();
     ca.k = a;
     if (!rc) rc = dev_count_terms(s, ca, bounds, err);
     if (rc) return rc;
@@ -2780,10 +2793,12 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     // (single-Gaussian Coulomb apply at k = 7: 2.74 to 2.43 ms; the exchange
     // applies of 4 orbitals in one batch: 12.0 to 10.5 ms, with the one-launch
     // assembly of the trees).
+    plan_ms[2] += host_ms() - t_count;
     if (defer) {
         *out = p.release();
         return 0;
     }
+    const double t_wait = host_ms();
     std::vector<unsigned long long> tot(n_tot);
     while (true) {
         HIP_TRY(hipMemcpyAsync(tot.data(), ca.totals, sizeof(unsigned long long) * n_tot, hipMemcpyDeviceToHost, s));
@@ -2821,6 +2836,7 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
         meta(r.data() + p->n_pseg, p->n_fseg, (int)cap[0], p->fsegs);
     }
     cut_done(p.get());
+    plan_ms[2] += host_ms() - t_wait;
     *out = p.release();
     return 0;
 }

@@ -512,10 +512,11 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         j.thr_all.assign(o.size(), 0.0);
     }
     InputBlocks inputs(ctx);
-    double kms = 0.0, pms = 0.0, slots = 0.0, gen = 0.0, computed = 0.0, apps_total = 0.0;
+    double kms = 0.0, slots = 0.0, gen = 0.0, computed = 0.0, apps_total = 0.0;
     double t_dev = 0.0, t_split = 0.0;  // device plan create + run + download; host split checks
     double t_create = 0.0, t_run = 0.0;  // parts of t_dev: plan creation, run (both host wall time)
-    double t_inp = 0.0;                  // uploads of host input trees
+    // parts of the plan time: bands and slots, pools, counts and segments
+    double plan3[3] = {0.0, 0.0, 0.0};
     const double t_all = now_ms();
     int launches = 0;
     // Every level's output blocks stay on the device until the post
@@ -547,8 +548,8 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         }
         const double t0 = now_ms();
         build_plans(active, nodes, thr);
-        pms += now_ms() - t0;
         const double t0i = now_ms();
+        plan3[0] += t0i - t0;
         std::vector<PlanPart> parts;
         size_t total = 0;
         for (size_t a = 0; a < active.size(); a++) {
@@ -559,11 +560,14 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         std::string err;
         DevicePlan *dp = nullptr;
         const double t1 = now_ms();
-        t_inp += t1 - t0i;
-        int rc = dev_plan_create(ctx->dev, mra, parts, ctx->mode, true, &dp, err);
+        plan3[1] += t1 - t0i;  // uploads of host inputs
+        double dev3[3] = {0.0, 0.0, 0.0};
+        int rc = dev_plan_create(ctx->dev, mra, parts, ctx->mode, true, &dp, err, dev3);
         if (rc) return dev_fail(rc, err);
         const double t1r = now_ms();
-        t_create += t1r - t1;
+        const double t_plan = dev3[0] + dev3[1] + dev3[2];
+        for (int i = 0; i < 3; i++) plan3[i] += dev3[i];
+        t_create += t1r - t1 - t_plan;
         long long n_slots = 0, n_gen = 0;
         dev_plan_slots(dp, &n_slots, &n_gen);
         slots += (double)n_slots;
@@ -582,7 +586,7 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
         const int level = (int)keep.bufs.size();
         keep.bufs.push_back(lvl);
         keep.count.push_back((long long)total);
-        t_dev += now_ms() - t1;
+        t_dev += now_ms() - t1 - t_plan;
         const double t2 = now_ms();
         kms += ms;
         apps_total += (double)apps;
@@ -715,7 +719,7 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
     st[1] = computed;
     st[2] = slots;
     st[3] = gen;
-    st[4] = pms;
+    st[4] = plan3[0] + plan3[1] + plan3[2];
     st[5] = launches;
     st[6] = apps_total;
     st[7] = t_dev;
@@ -724,9 +728,7 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
     st[10] = now_ms() - t_all;
     st[11] = t_create;
     st[12] = t_run;
-    st[13] = pms;
-    st[14] = t_inp;
-    st[15] = 0.0;
+    for (int i = 0; i < 3; i++) st[13 + i] = plan3[i];
     return MWG_OK;
 }
 

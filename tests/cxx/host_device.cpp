@@ -381,13 +381,34 @@ void host_output_memory() {
     check(g_peak < bytes + bytes * 4 / 5, "blocks on the device once, and a part of them to copy from");
 }
 
+// The stages of an apply's plan make up its plan time, each under its own name.
+void apply_stages() {
+    mwg_mra m = world(3, 3);
+    mwg_context ctx = nullptr;
+    check(mwg_context_create(0, &ctx) == MWG_OK, "context");
+    mwg_operator P = nullptr;
+    check(mwg_poisson_create(m, 1e-2, &P) == MWG_OK, "operator");
+    mwg_tree f = gaussian(m, 1e-2, 4.0), V = nullptr;
+    check(mwg_tree_create(m, &V) == MWG_OK, "tree");
+    check(mwg_apply(ctx, 1e-2, V, P, f, -1, 1) == MWG_OK, "apply");
+    double st[16];
+    check(mwg_last_apply_stats(ctx, st, 16) == MWG_OK, "stats");
+    std::printf("plan %g ms = bands %g + pools %g + counts %g; create %g + run %g of %g; apply %g\n", st[4], st[13],
+                st[14], st[15], st[11], st[12], st[7], st[10]);
+    for (int i : {11, 12, 13, 14, 15}) check(st[i] > 0.0, "every stage takes time");
+    const double sum = st[13] + st[14] + st[15];
+    check(sum > st[4] * (1.0 - 1e-12) && sum < st[4] * (1.0 + 1e-12), "bands, pools and counts are the plan");
+    check(st[11] + st[12] <= st[7] && st[4] + st[7] + st[8] + st[9] <= st[10], "no time counted twice");
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     const std::map<std::string, void (*)()> scenarios = {{"split_step_fails", split_step_fails},
                                                             {"idle_memory_is_given_back", idle_memory_is_given_back},
                                                             {"idle_memory_is_bounded", idle_memory_is_bounded},
-                                                            {"host_output_memory", host_output_memory}};
+                                                            {"host_output_memory", host_output_memory},
+                                                            {"apply_stages", apply_stages}};
     const auto it = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return 2;
     it->second();
