@@ -156,7 +156,7 @@ struct SegRec {
 // Work counts and segments of a plan (mw_count.hip).
 struct CountArgs {
     KArgs k{};
-    int n_out = 0, n_app = 0, n_share = 1;
+    int n_out = 0, n_share = 1;
     long long widest = 1;                  // positions of the widest band
     const unsigned char *dense = nullptr;  // per output node: computed by the root kernels
     // passing terms per (output component, band position) of every node,

@@ -940,11 +940,9 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
             if (more) fetch(nx, nt);
             wave_order();
             // z, once per passing component (item-uniform branches)
-            auto z_pass = [&](auto both, auto &&c0, auto &&c1, int q0) {
-                constexpr bool BOTH = decltype(both)::value;
-                double oz[G][G], oz1[BOTH ? G : 1][G], bn[G];
+            auto z_pass = [&](auto &&c0, int q0) {
+                double oz[G][G], bn[G];
                 operand(q0, oz);
-                if constexpr (BOTH) operand(3, oz1);
 #pragma unroll
                 for (int k = 0; k < G; k++) bn[k] = buf[rd + 4 * k * P];
 #pragma unroll
@@ -958,19 +956,16 @@ __device__ __forceinline__ void segment4(const KArgs &a, const double *pool, int
 #pragma unroll
                     for (int k = 0; k < G; k++)
 #pragma unroll
-                        for (int g = 0; g < G; g++) {
-                            c0[t][g] = mfma(oz[g][k], b[k], c0[t][g]);
-                            if constexpr (BOTH) c1[t][g] = mfma(oz1[g][k], b[k], c1[t][g]);
-                        }
+                        for (int g = 0; g < G; g++) c0[t][g] = mfma(oz[g][k], b[k], c0[t][g]);
                     SCHED_STEP();
                 }
             };
             if constexpr (PAIR) {
-                if (t0) z_pass(std::false_type{}, acc, acc, 2);
+                if (t0) z_pass(acc, 2);
                 SCHED_STEP();
-                if (t1) z_pass(std::false_type{}, acc1, acc1, 3);
+                if (t1) z_pass(acc1, 3);
             } else {
-                z_pass(std::false_type{}, acc, acc, 2);
+                z_pass(acc, 2);
             }
             wave_order();
             if (more) stage(nx.pos);
@@ -2744,7 +2739,6 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     };
     CountArgs &ca = p->count;
     ca.n_out = (int)n_out;
-    ca.n_app = (int)parts.size();
     ca.n_share = (int)parts.size();
     ca.widest = std::max(widest, 1LL);
     ca.dense = dev + f_dense;

@@ -222,9 +222,6 @@ struct Tree {
 //           out = [s, d1..d7] (component bit d set = wavelet along d).
 void mw_compress(const Basis &b, const double *in, double *out);
 void mw_reconstruct(const Basis &b, const double *in, double *out);
-// Scaling block of child t alone (t = bx + 2 by + 4 bz); `in` is a full
-// compressed block, or only its scaling part when s_only.
-void mw_child_scaling(const Basis &b, const double *in, bool s_only, int t, double *out);
 void component_norms(const MRA &mra, const double *blk, double *norms8);
 double tree_square_norm(const Tree &t);
 double tree_dot(const Tree &a, const Tree &b);
