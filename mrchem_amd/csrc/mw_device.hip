@@ -2456,7 +2456,7 @@ static int make_pool(DevicePlan *p, const MRA &mra, long long cells, long long n
 }
 
 int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, bool once,
-                    DevicePlan **out, std::string &err, double *plan_ms) {
+                    DevicePlan **out, std::string &err, double *plan_ms, long long first_cells) {
     double unused[3] = {0.0, 0.0, 0.0};
     if (!plan_ms) plan_ms = unused;
     HIP_TRY(hipSetDevice(c->device));
@@ -2596,8 +2596,9 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
             }
         }
     }
-    long long cells = 1024;
-    while (cells < 2.0 * n_cell && cells < (1LL << 30)) cells *= 2;
+    long long cells = first_cells;
+    if (cells <= 0)
+        for (cells = 1024; cells < 2.0 * n_cell && cells < (1LL << 30);) cells *= 2;
     // Every table of the plan but the pool and the output lives in one
     // device arena; what the host made of it is filled from one staging
     // buffer with one copy, so that a refinement level's plan costs one

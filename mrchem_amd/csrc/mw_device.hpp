@@ -32,16 +32,19 @@ struct PlanPart {
 // blocks of one or more applies, run together in each launch.
 struct DevicePlan;
 // Uploads the host plans and makes the rest on the device: the bands and input
-// slots (dev_band_find), the input pool (dev_pool_fill), the norm and pre-screen tables, the exact counts and the
-// work segments (the fine single-component ones only for a mode with an FP64
-// class beside a low-precision one).  mode: the arithmetic the plan will run.
+// slots (dev_band_find), the input pool (dev_pool_fill), the norm and
+// pre-screen tables, the exact counts and the work segments (the fine
+// single-component ones only for a mode with an FP64 class beside a
+// low-precision one).  mode: the arithmetic the plan will run.
 // With once (a plan that is run once) the host does not wait for the counts:
 // the run reads the number of segments on the device.
 // plan_ms (optional): the host's time for bands and slots, for the pool, and
 // for counts and segments is added to plan_ms[0..2] (device work that the host
 // does not wait for is in the run's time).
+// first_cells: cells of the slot search's first table, a power of two (0: twice
+// what the bands can hold); a table that is too small is doubled.
 int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &parts, int mode, bool once,
-                    DevicePlan **out, std::string &err, double *plan_ms = nullptr);
+                    DevicePlan **out, std::string &err, double *plan_ms = nullptr, long long first_cells = 0);
 // Term-applications counted with the screening rule when the plan was made,
 // and its pair segments.
 void dev_plan_counts(const DevicePlan *p, unsigned long long *term_apps, int *segments);
