@@ -108,7 +108,7 @@ struct BandArgs {
     const int *band_w;
     const BandTree *trees;  // per apply
     int boxes[3];
-    int n_out;
+    int n_out, q0;  // q0: output node of the launch's first workgroups
     long long n_band;
     // table of cap cells (a power of two): name of the node, slot, generation
     // level (-1: in the input tree) and, of a node in the tree, {its index, 0},
@@ -157,6 +157,7 @@ struct SegRec {
 struct CountArgs {
     KArgs k{};
     int n_out = 0, n_share = 1;
+    int q0 = 0;                            // output node of the launch's first workgroups
     long long widest = 1;                  // positions of the widest band
     const unsigned char *dense = nullptr;  // per output node: computed by the root kernels
     // passing terms per (output component, band position) of every node,

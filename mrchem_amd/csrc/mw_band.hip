@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void k_band_clear(BandArgs a) {
 // slot's id (>= 0), -(id + 3) for a generated slot, -2 while its id is being
 // taken, -1 for a node that is no slot (a generated ancestor).
 __global__ __launch_bounds__(256) void k_band_find(BandArgs a) {
-    const int q = blockIdx.x, side = 2 * a.band_w[q] + 1, nb = side * side * side;
+    const int q = a.q0 + (int)blockIdx.x, side = 2 * a.band_w[q] + 1, nb = side * side * side;
     const BandTree &t = a.trees[a.out_app[q]];
     int *cells = a.cell + a.band_off[q];
     __shared__ int taken[2][4], first[2];
@@ -276,11 +276,14 @@ int dev_band_find(hipStream_t s, const BandArgs &a, long long widest, std::strin
     hipLaunchKernelGGL(k_band_clear, dim3((unsigned)((std::max(a.cap, (unsigned)kBandCounts) + 255) / 256)), dim3(256),
                        0, s, a);
     HIP_TRY(hipGetLastError());
-    if (a.n_out == 0) return 0;
     const unsigned y = (unsigned)std::min<long long>((widest + 255) / 256, 64);
-    hipLaunchKernelGGL(k_band_find, dim3((unsigned)a.n_out, y), dim3(256), 0, s, a);
-    HIP_TRY(hipGetLastError());
-    return 0;
+    return in_launches(a.n_out, 256, [&](long long first, long long n) {
+        BandArgs part = a;
+        part.q0 = (int)first;
+        hipLaunchKernelGGL(k_band_find, dim3((unsigned)n, y), dim3(256), 0, s, part);
+        HIP_TRY(hipGetLastError());
+        return 0;
+    });
 }
 
 int dev_band_items(hipStream_t s, const BandArgs &a, const BandItems &o, std::string &err) {

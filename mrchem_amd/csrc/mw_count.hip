@@ -171,7 +171,7 @@ __device__ __forceinline__ void wave_range(double &lo, double &hi) {
 template <bool BOUNDS>
 __global__ __launch_bounds__(512) void k_count(CountArgs c, int step) {
     const KArgs &a = c.k;
-    const NodeView v = node_view(a, blockIdx.x);
+    const NodeView v = node_view(a, c.q0 + (int)blockIdx.x);
     const int gt = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long long base = 8 * a.band_off[v.q] + (long long)gt * v.nb;
     __shared__ unsigned long long part[8];
@@ -248,8 +248,8 @@ constexpr int kSegTarget64 = 64, kSegFloor64 = 16, kSegWanted64 = 8192;
 template <bool PAIR, bool BOUNDS>
 __global__ __launch_bounds__(PAIR ? 256 : 512) void k_cut(CountArgs c) {
     const KArgs &a = c.k;
-    if (c.dense[blockIdx.x]) return;
-    const NodeView v = node_view(a, blockIdx.x);
+    if (c.dense[c.q0 + (int)blockIdx.x]) return;
+    const NodeView v = node_view(a, c.q0 + (int)blockIdx.x);
     const int gt = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int app = a.out_app[v.q], kind = PAIR ? 0 : 1;
     // A launch with fewer than kSegWanted x kSegTarget passing terms (this
@@ -439,12 +439,16 @@ int dev_count_terms(hipStream_t s, const CountArgs &c, bool bounds, std::string 
     const long long pairs = 8 * c.widest;
     const int step = c.n_out * ((pairs + 63) / 64) < 1024 ? 16 : 64;
     const int y = (int)std::max<long long>(1, std::min<long long>((pairs + step - 1) / step, 768 / c.n_out));
-    if (bounds)
-        hipLaunchKernelGGL((k_count<true>), dim3(c.n_out, y), dim3(512), 0, s, c, step);
-    else
-        hipLaunchKernelGGL((k_count<false>), dim3(c.n_out, y), dim3(512), 0, s, c, step);
-    HIP_TRY(hipGetLastError());
-    return 0;
+    return in_launches(c.n_out, 512, [&](long long first, long long n) {
+        CountArgs part = c;
+        part.q0 = (int)first;
+        if (bounds)
+            hipLaunchKernelGGL((k_count<true>), dim3((unsigned)n, y), dim3(512), 0, s, part, step);
+        else
+            hipLaunchKernelGGL((k_count<false>), dim3((unsigned)n, y), dim3(512), 0, s, part, step);
+        HIP_TRY(hipGetLastError());
+        return 0;
+    });
 }
 
 int dev_cut_segments(hipStream_t s, const CountArgs &c, bool bounds, std::string &err) {
@@ -452,15 +456,19 @@ int dev_cut_segments(hipStream_t s, const CountArgs &c, bool bounds, std::string
     // three positions a part at the least, and no more parts than fill the
     // chip: each ends a segment
     const int y = (int)std::max<long long>(1, std::min<long long>(c.widest / 3, 1024 / c.n_out));
-    if (bounds) {
-        hipLaunchKernelGGL((k_cut<true, true>), dim3(c.n_out), dim3(256), 0, s, c);
+    return in_launches(c.n_out, 512, [&](long long first, long long n) {
+        CountArgs part = c;
+        part.q0 = (int)first;
+        if (bounds) {
+            hipLaunchKernelGGL((k_cut<true, true>), dim3((unsigned)n), dim3(256), 0, s, part);
+            HIP_TRY(hipGetLastError());
+            hipLaunchKernelGGL((k_cut<false, true>), dim3((unsigned)n, y), dim3(512), 0, s, part);
+        } else {
+            hipLaunchKernelGGL((k_cut<true, false>), dim3((unsigned)n, y), dim3(256), 0, s, part);
+        }
         HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL((k_cut<false, true>), dim3(c.n_out, y), dim3(512), 0, s, c);
-    } else {
-        hipLaunchKernelGGL((k_cut<true, false>), dim3(c.n_out, y), dim3(256), 0, s, c);
-    }
-    HIP_TRY(hipGetLastError());
-    return 0;
+        return 0;
+    });
 }
 
 }  // namespace mwg

@@ -1638,12 +1638,13 @@ __global__ __launch_bounds__(JobShape<N>::T) __attribute__((amdgpu_waves_per_eu(
 // kernel, costs registers and was measured slower.
 template <int N>
 __global__ __launch_bounds__(SplitShape<N>::T) __attribute__((amdgpu_waves_per_eu(SplitShape<N>::WPE))) void k_apply_h(
-    KArgs a, const _Float16 *pool_h, const double *pool_sc, const int *seg_list, const unsigned long long *n_dev,
-    double tau, double single_mult) {
+    KArgs a, const _Float16 *pool_h, const double *pool_sc, const int *seg_list, long long first,
+    const unsigned long long *n_dev, double tau, double single_mult) {
     __shared__ SplitSmem<N> sm;
     extern __shared__ double nrm_s[];
-    if (n_dev && blockIdx.x >= *n_dev) return;
-    split_segment<N>(a, pool_h, pool_sc, seg_list[blockIdx.x], 0.0, tau, single_mult, 1, sm, nrm_s);
+    const unsigned long long e = (unsigned long long)first + blockIdx.x;
+    if (n_dev && e >= *n_dev) return;
+    split_segment<N>(a, pool_h, pool_sc, seg_list[e], 0.0, tau, single_mult, 1, sm, nrm_s);
 }
 
 // FP16 split rows of FP64 blocks (rows x N values each, row-major), data or
@@ -2767,7 +2768,9 @@ int dev_plan_create(DeviceCtx *c, const MRA &mra, const std::vector<PlanPart> &p
     // Room for the segments: what a small launch can hold and 16 (fine ones
     // 24, plain FP64's 64) for each output node; the few plans that need more
     // are cut again.
-    long long cap[2] = {bounds ? 2048 + 16 * n_out : 16384 + 64 * n_out, bounds ? 16384 + 24 * n_out : 0};
+    const long long most = (1LL << 30) - 1;  // of each kind: 32-bit places
+    long long cap[2] = {std::min(most, bounds ? 2048 + 16 * n_out : 16384 + 64 * n_out),
+                        bounds ? std::min(most, 16384 + 24 * n_out) : 0};
     const bool defer = once && (!bounds || lowp_fits(p.get(), mode));
     if ((rc = cut_plan(p.get(), cap, bounds, defer, false, err))) return rc;
     if (!root_items.empty()) {
@@ -3162,10 +3165,12 @@ static int launch_h_n(const DevicePlan *p, const int *list, const unsigned long 
               std::to_string(N) + "; use the FP64 or mixed mode";
         return -1;
     }
-    hipLaunchKernelGGL((k_apply_h<N>), dim3(n), dim3(SplitShape<N>::T), shmem, p->ctx->stream, p->args, p->pool_h,
-                       p->pool_hsc, list, n_dev, tau, p->single_ratio);
-    HIP_TRY(hipGetLastError());
-    return 0;
+    return in_launches(n, SplitShape<N>::T, [&](long long first, long long cnt) {
+        hipLaunchKernelGGL((k_apply_h<N>), dim3((unsigned)cnt), dim3(SplitShape<N>::T), shmem, p->ctx->stream, p->args,
+                           p->pool_h, p->pool_hsc, list, first, n_dev, tau, p->single_ratio);
+        HIP_TRY(hipGetLastError());
+        return 0;
+    });
 }
 
 // One workgroup per pair segment of list[0, n) (n_dev: as many as it holds, n

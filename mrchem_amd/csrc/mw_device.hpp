@@ -10,6 +10,19 @@ namespace mwg {
 
 struct DeviceCtx;
 
+// Workgroups of `threads` that one launch can hold: its work items are counted
+// in 32 bits.  Launches of a workgroup per node, slot or segment run in parts
+// of that many.
+constexpr long long launch_room(int threads) { return ((1LL << 32) - 1) / threads; }
+// launch(first, count) over [0, n) in parts a launch can hold.
+template <typename F>
+int in_launches(long long n, int threads, F &&launch) {
+    const long long room = launch_room(threads);
+    for (long long i = 0; i < n; i += room)
+        if (const int rc = launch(i, n - i < room ? n - i : room)) return rc;
+    return 0;
+}
+
 // Returns 0 on success; on failure a negative code and a message in err
 // (-1: invalid argument, -2: device error).
 int dev_create(int device, DeviceCtx **out, std::string &err);

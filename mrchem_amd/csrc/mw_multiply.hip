@@ -996,18 +996,19 @@ __global__ __launch_bounds__(256) void k_pool_fill(int n3, const SlotItem *items
 
 int dev_pool_fill(hipStream_t s, int n, const double *F, const GenItem *gen, const std::vector<int> &lv_off,
                   const SlotItem *slots, int n_slot, std::string &err) {
-    hipError_t e = hipSuccess;
-    for (size_t lv = 0; e == hipSuccess && lv + 1 < lv_off.size(); lv++)
-        if (lv_off[lv + 1] > lv_off[lv]) e = gen_fill(s, n, gen + lv_off[lv], lv_off[lv + 1] - lv_off[lv], F);
-    if (e == hipSuccess && n_slot > 0) {
-        hipLaunchKernelGGL(k_pool_fill, dim3((unsigned)(2 * n_slot)), dim3(256), 0, s, n * n * n, slots, n_slot);
-        e = hipGetLastError();
+    for (size_t lv = 0; lv + 1 < lv_off.size(); lv++) {
+        // (1024: at least the threads of every size's workgroups)
+        const int rc = in_launches(lv_off[lv + 1] - lv_off[lv], 1024, [&](long long first, long long cnt) {
+            HIP_TRY(gen_fill(s, n, gen + lv_off[lv] + first, (int)cnt, F));
+            return 0;
+        });
+        if (rc) return rc;
     }
-    if (e != hipSuccess) {
-        err = std::string("pool fill: ") + hipGetErrorString(e);
-        return -2;
-    }
-    return 0;
+    return in_launches(n_slot, 512, [&](long long first, long long cnt) {
+        hipLaunchKernelGGL(k_pool_fill, dim3((unsigned)(2 * cnt)), dim3(256), 0, s, n * n * n, slots + first, (int)cnt);
+        HIP_TRY(hipGetLastError());
+        return 0;
+    });
 }
 
 // Block src_idx[i] of src (blk doubles) to block i of dst: one workgroup per
@@ -1231,17 +1232,18 @@ int dev_finish_blocks(DeviceCtx *c, const MRA &mra, const std::vector<BlockMove>
     const BlockMove *mb = reinterpret_cast<const BlockMove *>(dev + b_F + b_p), *ma = mb + before.size();
     double *nr = reinterpret_cast<double *>(dev + up);
     hipError_t e = hipMemcpyAsync(dev, stage.data(), up, hipMemcpyHostToDevice, s);
+    auto move = [&](const BlockMove *m, size_t n, double *s2, double *w2) {
+        return in_launches((long long)n, 256, [&](long long first, long long cnt) {
+            hipLaunchKernelGGL(k_move_norms, dim3((unsigned)cnt), dim3(256), 0, s, m + first, n3,
+                               s2 ? s2 + first : nullptr, w2 ? w2 + first : nullptr);
+            HIP_TRY(hipGetLastError());
+            return 0;
+        });
+    };
     int rc = 0;
-    if (e == hipSuccess && !before.empty()) {
-        hipLaunchKernelGGL(k_move_norms, dim3((unsigned)before.size()), dim3(256), 0, s, mb, n3,
-                           static_cast<double *>(nullptr), static_cast<double *>(nullptr));
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess && off.back() > 0) rc = dev_post_launch(s, mra.kp1(), pairs, off, F, err, topdown);
-    if (e == hipSuccess && !rc && na) {
-        hipLaunchKernelGGL(k_move_norms, dim3((unsigned)na), dim3(256), 0, s, ma, n3, nr, nr + na);
-        e = hipGetLastError();
-    }
+    if (e == hipSuccess) rc = move(mb, before.size(), nullptr, nullptr);
+    if (e == hipSuccess && !rc && off.back() > 0) rc = dev_post_launch(s, mra.kp1(), pairs, off, F, err, topdown);
+    if (e == hipSuccess && !rc) rc = move(ma, na, nr, nr + na);
     if (e == hipSuccess && !rc && na) e = hipMemcpyAsync(norms2, nr, sizeof(double) * 2 * na, hipMemcpyDeviceToHost, s);
     const hipError_t es = hipStreamSynchronize(s);
     if (e == hipSuccess) e = es;

@@ -33,6 +33,7 @@ std::map<const void *, std::string> &kernels() {
     static std::map<const void *, std::string> k;
     return k;
 }
+std::map<std::string, long long> g_groups;  // workgroups (x) launched, by kernel
 std::string g_fail;  // launches of kernels with this in their names fail
 int g_failed = 0;
 hipError_t g_last = hipSuccess;
@@ -126,6 +127,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, si
     if (name.find("k_move_norms") != std::string::npos) ones(2);
     if (name.find("k_band_clear") != std::string::npos)
         std::fill_n(static_cast<mwg::BandArgs *>(args[0])->cnt, mwg::kBandCounts, 0u);
+    g_groups[name] += grid.x;
     of(s)->queued++;
     return hipSuccess;
 }
@@ -401,6 +403,39 @@ void apply_stages() {
     check(st[11] + st[12] <= st[7] && st[4] + st[7] + st[8] + st[9] <= st[10], "no time counted twice");
 }
 
+// More nodes and slots than one launch has work items for: the launches are
+// split, and together hold a workgroup for each.
+void more_than_a_launch() {
+    hipStream_t stream = nullptr;
+    check(hipStreamCreateWithFlags(&stream, 0) == hipSuccess, "stream");
+    std::string err;
+    const int n = 20 << 20;  // times 256 threads: past 32 bits
+    auto groups = [](const char *kernel) {
+        long long sum = 0;
+        for (const auto &g : g_groups)
+            if (g.first.find(kernel) != std::string::npos) sum += g.second;
+        return sum;
+    };
+    mwg::BandArgs b{};
+    std::vector<unsigned> cnt(mwg::kBandCounts);
+    b.n_out = n;
+    b.cap = 1024;
+    b.cnt = cnt.data();
+    check(mwg::dev_band_find(stream, b, 27, err) == 0 && groups("k_band_find") == n, "bands");
+    mwg::CountArgs c;
+    c.n_out = n;
+    c.widest = 27;
+    for (bool bounds : {false, true}) {
+        g_groups.clear();
+        check(mwg::dev_count_terms(stream, c, bounds, err) == 0 && groups("k_count") == n, "counts");
+        check(mwg::dev_cut_segments(stream, c, bounds, err) == 0 && groups("k_cut") == (bounds ? 2LL : 1LL) * n, "cuts");
+    }
+    check(mwg::dev_pool_fill(stream, 2, nullptr, nullptr, {0, n, 2 * n}, nullptr, n, err) == 0 &&
+              groups("k_gen_fill") == 2LL * n && groups("k_pool_fill") == 2LL * n,
+          "pool");
+    std::printf("%d nodes: %s\n", n, err.c_str());
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -408,7 +443,8 @@ int main(int argc, char **argv) {
                                                             {"idle_memory_is_given_back", idle_memory_is_given_back},
                                                             {"idle_memory_is_bounded", idle_memory_is_bounded},
                                                             {"host_output_memory", host_output_memory},
-                                                            {"apply_stages", apply_stages}};
+                                                            {"apply_stages", apply_stages},
+                                                            {"more_than_a_launch", more_than_a_launch}};
     const auto it = argc > 1 ? scenarios.find(argv[1]) : scenarios.end();
     if (it == scenarios.end()) return 2;
     it->second();

@@ -21,7 +21,7 @@ def exe(tmp_path_factory):
 
 
 @pytest.mark.parametrize("scenario", ["split_step_fails", "idle_memory_is_given_back", "idle_memory_is_bounded",
-                                      "host_output_memory", "apply_stages"])
+                                      "host_output_memory", "apply_stages", "more_than_a_launch"])
 def test_scenario(exe, scenario):
     r = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=100)
     print(r.stdout, r.stderr)
