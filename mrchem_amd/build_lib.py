@@ -23,7 +23,11 @@ HIP_SOURCES = ["mw_device.hip", "mw_opbuild.hip", "mw_multiply.hip", "mw_root.hi
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                "-mllvm", "-amdgpu-mfma-vgpr-form"]
-CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fopenmp", "-march=x86-64-v3", "-Wall", "-Wno-unused-function"]
+# Functions and loops are aligned: by default one more entry of the procedure
+# linkage table moves the inner loops across fetch blocks, and the evaluation of
+# 64 points at k = 8 took 6.1 instead of 5.0 ms with the same instructions.
+CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fopenmp", "-march=x86-64-v3", "-falign-functions=64", "-falign-loops=32",
+             "-Wall", "-Wno-unused-function"]
 
 
 def _run(cmd):
