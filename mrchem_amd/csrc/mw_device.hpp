@@ -215,9 +215,16 @@ int dev_finish_blocks(DeviceCtx *c, const MRA &mra, const std::vector<BlockMove>
                       const std::vector<std::vector<PostPair>> &levels, bool topdown,
                       const std::vector<BlockMove> &after, double *norms2, std::string &err);
 // Blocks on the device (8 (k+1)^3 values each), wherever they lie, one after
-// another into host memory, through at most 256 MB of device memory.
-int dev_download_blocks(DeviceCtx *c, const MRA &mra, const std::vector<const double *> &src, double *dst,
-                        std::string &err);
+// another into host memory: n of them to dst, for each of `to` in turn.  They
+// pass through `room`, kDownloadRoom bytes of device memory at most, which
+// holds `per` blocks; the first `per` are there already.
+constexpr size_t kDownloadRoom = (size_t)256 << 20;
+struct HostBlocks {
+    double *dst;
+    size_t n;
+};
+int dev_download_blocks(DeviceCtx *c, const MRA &mra, const std::vector<const double *> &src, double *room, size_t per,
+                        const std::vector<HostBlocks> &to, std::string &err);
 // A packed tree: head (host) and n doubles of blocks (device) into device
 // memory at dst, finished on return.
 int dev_pack(DeviceCtx *c, void *dst, const void *head, size_t head_bytes, const double *blocks, size_t n,

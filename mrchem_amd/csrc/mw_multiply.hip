@@ -1256,33 +1256,37 @@ int dev_finish_blocks(DeviceCtx *c, const MRA &mra, const std::vector<BlockMove>
     return 0;
 }
 
-int dev_download_blocks(DeviceCtx *c, const MRA &mra, const std::vector<const double *> &src, double *dst,
-                        std::string &err) {
-    if (src.empty()) return 0;
+int dev_download_blocks(DeviceCtx *c, const MRA &mra, const std::vector<const double *> &src, double *room, size_t per,
+                        const std::vector<HostBlocks> &to, std::string &err) {
     HIP_TRY(hipSetDevice(dev_device(c)));
     hipStream_t s = static_cast<hipStream_t>(dev_stream(c));
     const size_t n = src.size(), blk = (size_t)mra.block();
-    // several of the 64 MB chunks in which large copies overlap with the host's
-    const size_t per = std::min(n, std::max<size_t>(1, ((size_t)256 << 20) / (sizeof(double) * blk)));
-    double *room = nullptr;
     BlockMove *dm = nullptr;
-    int rc = dev_mem(c, per * blk, &room, err);
-    if (!rc) rc = dev_mem(c, n, &dm, err);
+    std::vector<BlockMove> moves;  // of the blocks after the first per
+    for (size_t i = per; i < n; i++) moves.push_back(BlockMove{src[i], room + i % per * blk});
+    int rc = moves.empty() ? 0 : dev_mem(c, moves.size(), &dm, err);
     hipError_t e = hipSuccess;
-    if (!rc) {
-        std::vector<BlockMove> moves(n);
-        for (size_t i = 0; i < n; i++) moves[i] = BlockMove{src[i], room + i % per * blk};
-        e = hipMemcpyAsync(dm, moves.data(), sizeof(BlockMove) * n, hipMemcpyHostToDevice, s);
-        for (size_t i = 0; i < n && !rc && e == hipSuccess; i += per) {
-            const size_t cnt = std::min(per, n - i);
-            hipLaunchKernelGGL(k_move_norms, dim3((unsigned)cnt), dim3(256), 0, s, dm + i, mra.kp1_3(),
+    if (!rc && dm) e = hipMemcpyAsync(dm, moves.data(), sizeof(BlockMove) * moves.size(), hipMemcpyHostToDevice, s);
+    size_t t = 0, done = 0;  // the target at work, and its blocks that are there
+    for (size_t i = 0; i < n && !rc && e == hipSuccess; i += per) {
+        const size_t cnt = std::min(per, n - i);
+        if (i > 0) {
+            hipLaunchKernelGGL(k_move_norms, dim3((unsigned)cnt), dim3(256), 0, s, dm + (i - per), mra.kp1_3(),
                                static_cast<double *>(nullptr), static_cast<double *>(nullptr));
             e = hipGetLastError();
-            if (e == hipSuccess) rc = dev_copy_d2h(c, dst + i * blk, room, sizeof(double) * cnt * blk, err);
         }
-        if (e != hipSuccess || rc) (void)hipStreamSynchronize(s);  // moves is read until then
+        for (size_t at = 0; at < cnt && !rc && e == hipSuccess;) {
+            const size_t m = std::min(cnt - at, to[t].n - done);
+            rc = dev_copy_d2h(c, to[t].dst + done * blk, room + at * blk, sizeof(double) * m * blk, err);
+            at += m;
+            done += m;
+            if (done == to[t].n) {
+                t++;
+                done = 0;
+            }
+        }
     }
-    dev_mem_put(c, room);
+    if (e != hipSuccess || rc) (void)hipStreamSynchronize(s);  // moves is read until then
     dev_mem_put(c, dm);
     if (rc) return rc;
     if (e != hipSuccess) {

@@ -673,23 +673,32 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
             }
         }
         // the transformed blocks normed, and on the way those of an output
-        // resident on this context into its device copy; a host tree's are
-        // downloaded from where they are, so that its blocks are on the
-        // device once
+        // resident on this context into its device copy and as many of the
+        // host trees' as its room holds into an array to download from; the
+        // others follow from where they are
         std::vector<DeviceResult> res;
         for (size_t ji = 0; ji < jobs.size(); ji++) res.push_back(DeviceResult{ctx->dev, nullptr});
+        size_t n_host = 0;
+        for (Job &j : jobs) n_host += j.out->dctx == ctx ? 0 : (size_t)j.out->tree.size();
+        const size_t per = std::min(n_host, std::max<size_t>(1, kDownloadRoom / (sizeof(double) * blk)));
+        DeviceResult room{ctx->dev, nullptr};
+        if (per > 0) dev_check(dev_alloc(ctx->dev, per * blk, &room.p, err), err);
         std::vector<BlockMove> moves;
+        std::vector<const double *> src;  // the host trees' blocks
         for (size_t ji = 0; ji < jobs.size(); ji++) {
             const Tree &o = jobs[ji].out->tree;
             const bool resident = jobs[ji].out->dctx == ctx;
             if (resident) dev_check(dev_alloc(ctx->dev, (size_t)o.size() * blk, &res[ji].p, err), err);
             for (int i = 0; i < o.size(); i++) {
                 double *at = addr(locs[ji][i]);
-                moves.push_back(BlockMove{at, resident ? res[ji].p + (size_t)i * blk : at});
+                double *dst = resident ? res[ji].p + (size_t)i * blk : src.size() < per ? room.p + src.size() * blk : at;
+                moves.push_back(BlockMove{at, dst});
+                if (!resident) src.push_back(at);
             }
         }
         std::vector<double> nr(2 * moves.size());
         dev_check(dev_finish_blocks(ctx->dev, mra, {}, levels, true, moves, nr.data(), err), err);
+        std::vector<HostBlocks> to;
         size_t at = 0;
         for (size_t ji = 0; ji < jobs.size(); ji++) {
             mwg_tree out = jobs[ji].out;
@@ -699,18 +708,17 @@ int apply_batch(mwg_context ctx, std::vector<Job> &jobs) {
             if (res[ji].p) {
                 take_device_result(ctx, out, res[ji].release(), std::move(ns2), std::move(nw2));
             } else {
-                std::vector<const double *> src(n);
-                for (size_t i = 0; i < n; i++) src[i] = moves[at + i].src;
                 out->tree.structure_only = false;
-                out->tree.coefs.resize(tree_values(out));  // every block is written
+                out->tree.coefs.resize(tree_values(out));  // every block is written below
                 host_changed(out);
-                dev_check(dev_download_blocks(ctx->dev, mra, src, out->tree.coefs.data(), err), err);
-                ctx->d2h_bytes += (long long)(sizeof(double) * tree_values(out));
                 take_norms(out, std::move(ns2), std::move(nw2));
+                to.push_back(HostBlocks{out->tree.coefs.data(), n});
+                ctx->d2h_bytes += (long long)(sizeof(double) * tree_values(out));
             }
             out->apply_thr = jobs[ji].thr_all;
             at += n;
         }
+        if (per > 0) dev_check(dev_download_blocks(ctx->dev, mra, src, room.p, per, to, err), err);
     }
     guard.done = true;
     auto &st = ctx->last_stats;
