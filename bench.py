@@ -314,7 +314,7 @@ def main():
         cpu = cpu_baseline(mra, ops, inps, outs, thr, ns64, args.cpu_seconds, check)
 
     peak_key = "f16" if head == "split16" else "f32"
-    kname = ("k_apply_h<%d>" if head == "split16" else "k_apply<%d, float>") % (k + 1)
+    kname = ("k_apply_h<%d>" if head == "split16" else "k_apply<%d>") % (k + 1)
     line = {
         "metric": METRIC,
         "value": n_out / (msmx * 1e-3),

@@ -11,7 +11,7 @@
 // slots and generated nodes known, writes the copy and generation items of the
 // pool and the band table.
 //
-// Nothing here moves more than the table and the band entries (24 and 8 bytes
+// Nothing here moves more than the table and the band entries (21 and 8 bytes
 // each): both launches are bound by the latency of dependent loads and
 // compare-and-swaps, so every entry has its own thread, and a node that is in
 // the table costs its later finders one load.  Hash maps on the host took 330 us

@@ -540,9 +540,9 @@ __device__ __forceinline__ const __attribute__((address_space(1))) T *gmem(const
 // A wave owns its job, its LDS and its worklist alone, so an item needs no
 // barrier: a wave's LDS accesses run in order, and the second wave of the SIMD
 // computes while the first waits for its own.  What bounds the kernel is the
-// matrix unit: it is busy 69 % of the cycles a CU works at N = 10 (frozen plan
-// of 656 nodes; the rest waits for operands from LDS), and a refinement
-// level's launch ends with CUs idle while the last segments run.
+// matrix unit: it is busy 67 % of the cycles a CU works at N = 10 (frozen plan
+// of 656 nodes; the rest waits for operands from LDS), 78 % at N = 12, and a
+// refinement level's launch ends with CUs idle while the last segments run.
 // Device time of the levels below the roots, against the 16 x 16 x 4 kernel
 // with two or three waves a job: six orbitals at k = 11 56.0 -> 25 ms, one k = 9
 // apply 5.7 -> 3.3 ms, ten exchange densities at k = 7 3.6 -> 1.7 ms, a frozen

@@ -4,8 +4,9 @@
 // operators at once: HelmholtzVector rebuilds one HelmholtzOperator per
 // orbital in every SCF iteration (src/scf_solver/HelmholtzVector.cpp:144),
 // and PoissonOperator is rebuilt in the SAD guess and the surface forces
-// (src/driver.cpp:1131,1283).  The kernel fit stays on the host (a 1D fit of
-// tens of terms); every (operator, term, depth) item becomes one wavefront:
+// (src/driver.cpp:1131,1283).  The terms of the kernel fit's steps come from the
+// host, their errors from the device (k_fit_error); every (operator, term, depth)
+// item becomes one wavefront:
 //
 //  pass 1 (k_op_scan): the translation scan of the host build, l = 0, 1, ...,
 //    with the s<-s blocks T^{d+1}_delta from Gaussian moments (the same
